@@ -146,12 +146,11 @@ typedef struct {
                                      kernel directly.  Either way the bonded terms and the
                                      displaced-state chain run beside the pair kernel on
                                      two side streams. */
-    int32_t pair_newton3;         /* block kernel only.  1: each pair once (half tile list,
-                                     j-force scatter); 0: each ordered pair (no atomics) */
-    int32_t pair_group;           /* 0: block kernel (one 64-atom i-block per wave, shared
-                                     j stream); 16 or 8: grouped kernel (the wave's i-block
-                                     split into groups of 16 or 8 atoms, each with its own j
-                                     stream, each pair once) */
+    int32_t pair_newton3;         /* 0 or 1: accepted for callers that choose between pair
+                                     kernels.  One kernel (each pair once) serves both;
+                                     with 0 an i-block has one wave */
+    int32_t pair_group;           /* 0, 8 or 16: as pair_newton3; with 8 or 16 an i-block has
+                                     one wave and list_skin is ignored */
     int32_t sort_interval;        /* steps between full spatial sorts (1: every step); the
                                      steps in between keep the slot order and only refresh
                                      the coordinates and block boxes.  Results differ only
@@ -163,14 +162,13 @@ typedef struct {
                                      1: on every step.  The pair energies are FP64 sums
                                      over the FP64 positions (their own kernel); the
                                      forces are FP32 pair arithmetic. */
-    int32_t pair_split;           /* block Newton-3 kernel only: 1, 2, 4 (the default), 8,
-                                     16 or 32 waves per i-block, each taking every
+    int32_t pair_split;           /* with pair_newton3 1 and pair_group 0: 1, 2, 4 (the
+                                     default), 8, 16 or 32 waves per i-block, each taking every
                                      pair_split-th tile, so that short tile lists do not
                                      leave the GPU waiting on long ones and small batches
                                      fill it.
                                      Results differ only in rounding: each wave's i forces
-                                     and pair energies are summed on their own before they
-                                     are added up. */
+                                     are summed on their own before they are added up. */
     int32_t side_fork;            /* where the restraints, force-field terms and the
                                      displaced-state chain run: 0 on two side streams
                                      forked after the tile lists (beside the pair kernel),
@@ -185,7 +183,7 @@ typedef struct {
                                      sort, one more fork event per step); with 2 they
                                      run with the rest.  Same results. */
     float list_skin;              /* Verlet skin of the tile lists in nm, 0 to
-                                     SDM_MAX_LIST_SKIN (block pair kernels only; 0, the
+                                     SDM_MAX_LIST_SKIN (pair_group 0 only; 0, the
                                      default, builds them on every evaluation).  Lists
                                      are built for r_c + list_skin and kept while every
                                      atom of the replica has moved less than list_skin / 2
@@ -419,13 +417,12 @@ int sdm_count_pairs(sdm_context* ctx, int64_t* p0, int64_t* pdelta /* [n_replica
    afterwards. */
 int sdm_time_pair_kernel(sdm_context* ctx, int32_t nsteps, double* avg_ms);
 
-/* Launch-configuration search (project-written autotuner): times each candidate (pair
-   kernel, waves per workgroup and per i-block, sort grid) on the context's own replicas
+/* Launch-configuration search (project-written autotuner): times each candidate (waves
+   per workgroup and per i-block of the pair kernel, sort grid) on the context's own replicas
    for `steps` steps, then times the three fastest, each with and without graph replay
    and with each of the five placements of the side work (side_fork), for 3 x `steps`
-   steps in two rounds, and keeps the one with the smallest total; with a block pair
-   kernel it then times that one with list_skin 0, 0.01, 0.02, 0.03 and 0.04 nm the same
-   way.  The state the context had before the call is restored. */
+   steps in two rounds, and keeps the one with the smallest total; it then times that one
+   with list_skin 0, 0.01, 0.02, 0.03 and 0.04 nm the same way.  The state the context had before the call is restored. */
 int sdm_autotune(sdm_context* ctx, int32_t steps, sdm_tuning* chosen);
 int sdm_get_tuning(sdm_context* ctx, sdm_tuning* t);
 int sdm_set_tuning(sdm_context* ctx, const sdm_tuning* t);

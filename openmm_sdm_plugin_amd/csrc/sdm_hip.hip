@@ -109,12 +109,15 @@ struct sdm_context {
     double* Fb = nullptr;  // [R][3][Np] FP64 bonded forces, atom order
     // per replica
     double *x64 = nullptr, *v64 = nullptr;
-    float4* posq_s = nullptr;
-    float2* par_s = nullptr;
-    float4* arec = nullptr;  // [R][Np][2] slot records of the grouped pair kernel
+    float4* arec = nullptr;  // [R][Np][2] slot records of the pair kernel, coordinates
+                             // relative to the block's reference
+    double4* bref = nullptr; // [R][NB] the blocks' references (first atom)
     int *orig_s = nullptr, *slot_of = nullptr, *key = nullptr;
     int *ccount = nullptr, *cstart = nullptr, *cfill = nullptr;
     float4 *bb_lo = nullptr, *bb_hi = nullptr;
+    int* exs = nullptr;      // [R][NB][max_ex][64] exclusion partners in slot order (k_bbox)
+    unsigned long long* exblocks = nullptr;  // [R][NB] set of the j-blocks that hold any
+    float4* cbox = nullptr;  // [R][NB][16] centres and half extents of the 8-slot clusters
     int *tiles = nullptr, *ntiles = nullptr;
     unsigned long long* tmask = nullptr;
     int* cmap = nullptr;    // [R][NB] block -> candidate index of k_ligcand (-1: none)
@@ -124,7 +127,7 @@ struct sdm_context {
                             // displacement of the replica's atoms since then (k_refresh),
                             // or stale after a sort (k_bbox)
     long long* F = nullptr;
-    double *e_pair = nullptr, *e_bond = nullptr, *u_part = nullptr;
+    double *e_bond = nullptr, *u_part = nullptr;
     double* e64 = nullptr;  // [R][NB * E64_SPLIT] FP64 pair-energy slots
     // SDMUtils restraints (group 1): centroid and alignment terms, their group atoms and
     // normalized weights, and one energy slot per (replica, restraint)
@@ -358,10 +361,9 @@ int setup_cells(sdm_context* c, int per_dim) {
 
 dim3 g2(int n, int per, int R) { return dim3((unsigned)((n + per - 1) / per), (unsigned)R); }
 
-// Tile lists are kept over steps (tuning.list_skin > 0) with the block pair kernels only:
-// there every slot refresh is followed by a k_tiles launch, which rebuilds after a sort,
-// so the build coordinates (xb) always belong to the lists in use.  The grouped kernel
-// builds lists on energy evaluations only; they are built every time.
+// Tile lists are kept over steps (tuning.list_skin > 0) except where tuning asks for the
+// grouped form.  Every slot refresh is followed by a k_tiles launch, which rebuilds after a
+// sort, so the build coordinates (xb) always belong to the lists in use.
 bool lists_kept(const sdm_context* c) { return c->tune.list_skin > 0.f && c->tune.pair_group == 0; }
 
 // slot order (a full spatial sort, or the last sort's order refreshed) and block boxes
@@ -371,22 +373,23 @@ void enqueue_order(sdm_context* c, bool full, bool energy = false) {
     hipStream_t s = c->stream;
     int N = c->N, Np = c->Np, R = c->R;
     Rec64* rec = energy ? c->rec64 : nullptr;
+#define SDM_REFRESH(SORT)                                                                      \
+    k_refresh<SORT><<<dim3(c->NB, R), 64, 0, s>>>(                                             \
+        N, Np, c->NB, c->x64, c->orig_s, c->qs, c->sh, c->se, c->g, c->arec, c->bref, c->F,    \
+        c->bb_lo, c->bb_hi, c->cbox, c->par64, rec, lists_kept(c) ? c->xb : nullptr, c->dmax,  \
+        c->slot_of, c->ex_start, c->ex_list, c->max_ex, c->exs, c->exblocks)
     if (!full) {
-        k_refresh<<<dim3(c->NB, R), 64, 0, s>>>(N, Np, c->NB, c->x64, c->orig_s, c->qs, c->g,
-                                                c->posq_s, c->arec, c->F, c->bb_lo, c->bb_hi,
-                                                c->par64, rec,
-                                                lists_kept(c) ? c->xb : nullptr,
-                                                c->dmax);
-    } else {
+        SDM_REFRESH(false);
+        return;
+    }
     k_bin<<<g2(N, 256, R), 256, 0, s>>>(N, Np, c->x64, c->key, c->ccount, c->cellrank, c->g,
                                         c->ncx, c->ncy, c->ncz, c->NC);
     k_scan<<<R, 1024, 0, s>>>(c->NC, c->ccount, c->cstart, c->cfill);
     k_scatter<<<g2(N, 256, R), 256, 0, s>>>(N, Np, c->NC, c->key, c->cstart, c->cfill, c->orig_s);
-    k_cellsort<<<g2(c->NC, 128, R), 128, 0, s>>>(N, Np, c->NC, c->cstart, c->orig_s, c->slot_of,
-                                                c->x64, c->qs, c->sh, c->se, c->posq_s,
-                                                c->par_s, c->arec, c->F, c->g, c->par64, rec);
-    k_bbox<<<dim3(c->NB, R), 64, 0, s>>>(N, Np, c->NB, c->posq_s, c->bb_lo, c->bb_hi, c->dmax);
-    }
+    k_cellsort<<<g2(c->NC, 128, R), 128, 0, s>>>(N, Np, c->NC, c->cstart, c->orig_s);
+    k_blockorder<<<dim3(c->NB, R), 64, 0, s>>>(N, Np, c->x64, c->orig_s, c->slot_of, c->g);
+    SDM_REFRESH(true);
+#undef SDM_REFRESH
 }
 
 // whether a launch of one workgroup per (replica, 64-atom block) leaves the GPU short of
@@ -406,13 +409,9 @@ TileRadius tile_radius(const sdm_context* c) {
     return tr;
 }
 
-// tile lists of the block pair kernels and of the FP64 energy kernel (the grouped
-// kernel finds its j-blocks itself: with it, lists are built for energy evaluations only,
-// as half lists).  With a skin, k_tiles keeps a replica's lists while its atoms have
-// moved less than half the skin since they were built.
-void enqueue_tiles(sdm_context* c, bool energy) {
-    if (c->tune.pair_group != 0 && !energy) return;
-    const int half = c->tune.pair_group != 0 ? 1 : c->tune.pair_newton3;
+// tile lists of the pair and energy kernels.  With a skin, k_tiles keeps a replica's lists
+// while its atoms have moved less than half the skin since they were built.
+void enqueue_tiles(sdm_context* c) {
     const TileRadius tr = tile_radius(c);
     // One workgroup per (replica, i-block).  Its time is the serial path through it, so
     // when the workgroups do not fill the GPU (fewer than 8 per CU) each gets 8 waves for
@@ -420,8 +419,8 @@ void enqueue_tiles(sdm_context* c, bool energy) {
     // replicas -1% with 8).
 #define SDM_TILES(NW)                                                                         \
     k_tiles<NW><<<dim3(c->NB, c->R), 64 * NW, 0, c->stream>>>(                                \
-        c->N, c->Np, c->NB, c->maxj, c->posq_s, c->bb_lo, c->bb_hi, c->tiles, c->tmask,       \
-        c->ntiles, c->dmax, c->xb, tr, c->g, half, c->flags)
+        c->N, c->Np, c->NB, c->maxj, c->arec, c->bref, c->bb_lo, c->bb_hi, c->cbox, c->tiles,  \
+        c->tmask, c->ntiles, c->dmax, c->xb, tr, c->g, c->flags)
     if (few_blocks(c)) SDM_TILES(8);
     else SDM_TILES(4);
 #undef SDM_TILES
@@ -430,113 +429,48 @@ void enqueue_tiles(sdm_context* c, bool energy) {
 // slot order, block boxes and tile lists
 void enqueue_sort(sdm_context* c, bool full) {
     enqueue_order(c, full);
-    enqueue_tiles(c, false);
+    enqueue_tiles(c);
 }
 
 // FP64 pair energies into e64 (needs the tile lists and FP64 records of this evaluation)
 void enqueue_energy64(sdm_context* c, hipStream_t st) {
-    const int half = c->tune.pair_group != 0 ? 1 : c->tune.pair_newton3;
     unsigned waves = (unsigned)(c->R * c->NB * E64_SPLIT);
-    size_t lds = (size_t)std::max(1, c->max_ex) * 64 * sizeof(int);
-    k_energy64<<<waves, 64, lds, st>>>(c->R, c->N, c->Np, c->NB, c->maxj, E64_SPLIT,
-                                              half, c->arec, c->rec64, c->orig_s, c->slot_of,
-                                              c->tiles, c->tmask, c->ntiles, c->bb_lo,
-                                              c->bb_hi, c->ex_start, c->ex_list, c->max_ex,
-                                              c->e64, c->g);
+    k_energy64<<<waves, 64, 0, st>>>(c->R, c->N, c->Np, c->NB, c->maxj, E64_SPLIT, c->rec64,
+                                     c->tiles, c->tmask, c->ntiles, c->bb_lo, c->bb_hi, c->exs,
+                                     c->exblocks, c->max_ex, c->e64, c->g);
 }
 
-// ring capacity (entries per group) of the grouped pair kernel
-template <int G>
-constexpr int grp_cap() {
-    return G == 16 ? 256 : 128;
+// waves per i-block of the pair kernel (tuning.pair_split; 1 where tuning asks for the full
+// tile lists or the grouped form, for which pair_split has no meaning)
+int pair_waves(const sdm_context* c) {
+    return c->tune.pair_group == 0 && c->tune.pair_newton3 ? c->tune.pair_split : 1;
 }
 
-template <int G, int W>
-void launch_pair_grp(sdm_context* c, bool count, unsigned long long* pc) {
-    constexpr int CAP = grp_cap<G>();
-    int waves = c->R * c->NB;
-    dim3 gr((waves + W - 1) / W);
-    // per wave: rings, exclusion partners, group boxes (the staging buffers are static)
-    size_t lds = (size_t)W * ((64 / G) * (CAP + 8) + c->max_ex * 64) * sizeof(unsigned);
-#define SDM_GRP_ARGS                                                                            \
-    c->R, c->N, c->Np, c->NB, c->arec, c->orig_s, c->slot_of, c->bb_lo, c->bb_hi, c->ex_start, \
-        c->ex_list, c->max_ex, c->F, c->e_pair, c->flags, pc, c->list_r2, c->g
-    if (count) k_pair_grp<G, CAP, W, true><<<gr, 64 * W, lds, c->stream>>>(SDM_GRP_ARGS);
-    else k_pair_grp<G, CAP, W, false><<<gr, 64 * W, lds, c->stream>>>(SDM_GRP_ARGS);
-#undef SDM_GRP_ARGS
+template <int W, bool GEO>
+void launch_pair(sdm_context* c, bool count) {
+    const int split = pair_waves(c), waves = c->R * c->NB * split;
+    const dim3 gr((waves + W - 1) / W);
+#define SDM_PAIR(COUNT)                                                                       \
+    k_pair<W, COUNT, GEO><<<gr, 64 * W, 0, c->stream>>>(                                      \
+        c->R, c->N, c->Np, c->NB, c->maxj, split, c->arec, c->bref, c->tiles, c->tmask,       \
+        c->ntiles, c->bb_lo, c->bb_hi, c->exs, c->exblocks, c->max_ex, c->F, c->flags, c->counters, c->g)
+    if (count) SDM_PAIR(true);
+    else SDM_PAIR(false);
+#undef SDM_PAIR
 }
 
-template <int G>
-void launch_pair_grp_w(sdm_context* c, bool count, unsigned long long* pc) {
-    switch (c->tune.pair_waves_per_group) {
-        case 2: launch_pair_grp<G, 2>(c, count, pc); break;
-        case 4: launch_pair_grp<G, 4>(c, count, pc); break;
-        default: launch_pair_grp<G, 1>(c, count, pc); break;
-    }
-}
-
-// energy = false (block Newton-3 kernel only): forces without the pair energies
-void enqueue_pair(sdm_context* c, bool count, bool energy = true) {
-    hipStream_t s = c->stream;
-    int waves = c->R * c->NB;
-    unsigned long long* pc = count ? c->counters : nullptr;
-    if (c->tune.pair_group == 16) return launch_pair_grp_w<16>(c, count, pc);
-    if (c->tune.pair_group == 8) return launch_pair_grp_w<8>(c, count, pc);
-    if (c->tune.pair_newton3) {
-        size_t lds = (size_t)c->tune.pair_waves_per_group * c->max_ex * 64 * sizeof(int);
-        const int split = c->tune.pair_split;
-        waves *= split;
-#define SDM_N3_ARGS                                                                             \
-    c->R, c->N, c->Np, c->NB, c->maxj, split, c->arec, c->orig_s, c->slot_of, c->tiles,         \
-        c->tmask,                                                                           \
-        c->ntiles, c->bb_lo, c->bb_hi, c->ex_start, c->ex_list, c->max_ex, c->F, c->e_pair, \
-        c->flags, pc, c->g
-#define SDM_LAUNCH_N3_G(W, GEO)                                                               \
-    do {                                                                                      \
-        dim3 gr((waves + W - 1) / W);                                                         \
-        if (count) k_pair_n3<W, true, true, GEO><<<gr, 64 * W, lds, s>>>(SDM_N3_ARGS);       \
-        else if (energy) k_pair_n3<W, false, true, GEO><<<gr, 64 * W, lds, s>>>(SDM_N3_ARGS); \
-        else k_pair_n3<W, false, false, GEO><<<gr, 64 * W, lds, s>>>(SDM_N3_ARGS);           \
-    } while (0)
-#define SDM_LAUNCH_N3(W)                                                                      \
-    do {                                                                                      \
-        if (c->g.geo) SDM_LAUNCH_N3_G(W, true);                                               \
-        else SDM_LAUNCH_N3_G(W, false);                                                       \
-    } while (0)
+// pair forces, or (count) the number of pairs within the cutoff into counters
+void enqueue_pair(sdm_context* c, bool count) {
+    auto with = [&](auto geo) {
+        constexpr bool GEO = decltype(geo)::value;
         switch (c->tune.pair_waves_per_group) {
-            case 2: SDM_LAUNCH_N3(2); break;
-            case 4: SDM_LAUNCH_N3(4); break;
-            default: SDM_LAUNCH_N3(1); break;
+            case 2: launch_pair<2, GEO>(c, count); break;
+            case 4: launch_pair<4, GEO>(c, count); break;
+            default: launch_pair<1, GEO>(c, count); break;
         }
-#undef SDM_LAUNCH_N3
-#undef SDM_LAUNCH_N3_G
-#undef SDM_N3_ARGS
-        return;
-    }
-#define SDM_PAIR_ARGS                                                                       \
-    c->R, c->N, c->Np, c->NB, c->maxj, c->posq_s, c->par_s, c->orig_s, c->slot_of, c->tiles, \
-        c->tmask, c->ntiles, c->bb_lo, c->bb_hi, c->ex_start, c->ex_list, c->max_ex, c->F, c->e_pair,   \
-        c->flags, pc, c->g
-#define SDM_LAUNCH_PAIR(W)                                                                   \
-    do {                                                                                     \
-        dim3 gr((waves + W - 1) / W);                                                        \
-        if (newton) {                                                                        \
-            if (count) k_pair<W, true, true><<<gr, 64 * W, lds, s>>>(SDM_PAIR_ARGS);           \
-            else k_pair<W, false, true><<<gr, 64 * W, lds, s>>>(SDM_PAIR_ARGS);                \
-        } else {                                                                             \
-            if (count) k_pair<W, true, false><<<gr, 64 * W, lds, s>>>(SDM_PAIR_ARGS);          \
-            else k_pair<W, false, false><<<gr, 64 * W, lds, s>>>(SDM_PAIR_ARGS);               \
-        }                                                                                    \
-    } while (0)
-    bool newton = c->tune.pair_newton3 != 0;
-    size_t lds = (size_t)c->tune.pair_waves_per_group * std::max(1, c->max_ex) * 64 * sizeof(int);
-    switch (c->tune.pair_waves_per_group) {
-        case 2: SDM_LAUNCH_PAIR(2); break;
-        case 4: SDM_LAUNCH_PAIR(4); break;
-        default: SDM_LAUNCH_PAIR(1); break;
-    }
-#undef SDM_PAIR_ARGS
-#undef SDM_LAUNCH_PAIR
+    };
+    if (c->g.geo) with(std::true_type());
+    else with(std::false_type());
 }
 
 // A step's Langevin kernel adds the displaced-state forces itself (MixGather) instead of a
@@ -586,14 +520,14 @@ void enqueue_eval(sdm_context* c, bool advance, bool components, bool full, bool
     }
     enqueue_order(c, full, energy);
     const bool tiles_after_fork = mode == 1 || mode == 3 || mode == 4;
-    if (!tiles_after_fork) enqueue_tiles(c, energy);
+    if (!tiles_after_fork) enqueue_tiles(c);
     if (mode != 2) {
         (void)hipEventRecord(c->ev_fork, s);
         (void)hipStreamWaitEvent(s1, c->ev_fork, 0);
         (void)hipStreamWaitEvent(s2, c->ev_fork, 0);
         if (mode == 4) bonded();
     }
-    if (tiles_after_fork) enqueue_tiles(c, energy);
+    if (tiles_after_fork) enqueue_tiles(c);
     if (mode == 2) bonded();
     if (c->ncen + c->nali > 0)
         k_restraints<<<dim3(c->ncen + c->nali, R), 64, 0, s1>>>(
@@ -636,7 +570,7 @@ void enqueue_eval(sdm_context* c, bool advance, bool components, bool full, bool
     }
     if (pe0) (void)hipEventRecord(pe0, s);
     // forces in FP32; the pair energies, when asked for, in FP64 by their own kernel
-    enqueue_pair(c, false, false);
+    enqueue_pair(c, false);
     if (pe1) (void)hipEventRecord(pe1, s);
     if (energy && mode == 2) enqueue_energy64(c, s);
     if (mode != 2) {
@@ -801,7 +735,7 @@ int sdm_create(const sdm_system_desc* sys, int32_t n_replicas, sdm_context** out
     *out = nullptr;
     int N = sys->n_atoms;
     if (N <= 0) return fail(SDM_ERR_INVALID, "n_atoms must be positive");
-    // the grouped pair kernel addresses 32-byte slot records with 32-bit byte offsets
+    // slot records are addressed with 32-bit indices (two per 32-byte record)
     if (N >= (1 << 26)) return fail(SDM_ERR_UNSUPPORTED, "n_atoms must be below 2^26");
     if (n_replicas <= 0) return fail(SDM_ERR_INVALID, "n_replicas must be positive");
     if (!sys->charge || !sys->sigma || !sys->epsilon || !sys->mass || !sys->displacement)
@@ -974,14 +908,16 @@ int sdm_create(const sdm_system_desc* sys, int32_t n_replicas, sdm_context** out
     A(bstart, N + 1); A(bcode, 2 * std::max(1, c->nbond));
     A(astart, N + 1); A(acode, 3 * std::max(1, c->nang));
     if (c->nbond + c->nang > 0) A(Fb, 3 * RNp);
-    A(x64, 3 * RNp); A(v64, 3 * RNp); A(posq_s, RNp); A(par_s, RNp); A(arec, 2 * RNp);
+    A(x64, 3 * RNp); A(v64, 3 * RNp); A(arec, 2 * RNp);
+    A(bref, (size_t)R * NB);
     A(orig_s, RNp);
     A(slot_of, RNp); A(key, RNp); A(bb_lo, (size_t)R * NB); A(bb_hi, (size_t)R * NB);
+    A(cbox, (size_t)R * NB * 16); A(exs, (size_t)RNp * c->max_ex); A(exblocks, (size_t)R * NB);
     A(tiles, (size_t)R * NB * c->maxj); A(tmask, (size_t)R * NB * c->maxj);
     A(xb, RNp); A(dmax, (size_t)R * DISP_STRIDE);
     A(cmap, (size_t)R * NB); A(lig_of, Np);
     A(ntiles, (size_t)R * NB); A(F, 3 * RNp);
-    A(e_pair, (size_t)R * NB * 32); A(e_bond, (size_t)R * c->nbw); A(u_part, (size_t)R * c->LB);
+    A(e_bond, (size_t)R * c->nbw); A(u_part, (size_t)R * c->LB);
     A(e64, (size_t)R * NB * E64_SPLIT); A(rec64, RNp);
     A(cand, (size_t)R * c->maxc); A(ncand, R);
     A(dA, (size_t)R * c->maxc * c->LB * 64); A(dlig, (size_t)R * std::max(1, c->L));
@@ -1838,7 +1774,7 @@ int sdm_count_pairs(sdm_context* c, int64_t* p0, int64_t* pdelta) {
     std::vector<unsigned long long> h(n);
     CHK(download(c, h.data(), c->counters, n));
     for (int r = 0; r < c->R; r++) {
-        p0[r] = (int64_t)((c->tune.pair_group || c->tune.pair_newton3) ? h[r] : h[r] / 2);
+        p0[r] = (int64_t)h[r];
         pdelta[r] = (int64_t)h[c->R + r];
     }
     return SDM_OK;
@@ -1859,7 +1795,7 @@ int sdm_time_pair_kernel(sdm_context* c, int32_t nsteps, double* avg_ms) {
         for (int s = 0; s < nsteps; s++) {
             enqueue_sort(c, take_order(c, false));
             (void)hipEventRecord(ev[2 * s], c->stream);
-            enqueue_pair(c, false, false);
+            enqueue_pair(c, false);
             (void)hipEventRecord(ev[2 * s + 1], c->stream);
         }
         rc = check_launch();
@@ -1963,22 +1899,19 @@ int sdm_autotune(sdm_context* c, int32_t steps, sdm_tuning* chosen) {
         CHK(upload(c, c->flags, fl.data(), c->R));
         return SDM_OK;
     };
-    // pair kernels: block waves without Newton-3, with Newton-3 and 1, 2, 4, 8, 16 or 32 waves
-    // per i-block, grouped waves of 16 and of 8
-    const int kernels[][3] = {{0, 0, 1}, {0, 1, 1}, {0, 1, 2}, {0, 1, 4}, {0, 1, 8},
-                              {0, 1, 16}, {0, 1, 32}, {16, 1, 1}, {8, 1, 1}};
+    // waves per i-block of the pair kernel
+    const int splits[] = {1, 2, 4, 8, 16, 32};
     std::vector<std::pair<double, sdm_tuning>> timed;
     int rc = SDM_OK;
     for (double side : cell_sides)
         for (int w : waves)
-            for (const auto& kn : kernels) {
+            for (int split : splits) {
                 if (rc != SDM_OK) break;
-                if (c->g.geo && (kn[0] != 0 || kn[1] != 1)) continue;  // see sdm_set_tuning
                 sdm_tuning t = c->tune;
                 t.pair_waves_per_group = w;
-                t.pair_group = kn[0];
-                t.pair_newton3 = kn[1];
-                t.pair_split = kn[2];
+                t.pair_group = 0;
+                t.pair_newton3 = 1;
+                t.pair_split = split;
                 t.cell_cells_per_dim = std::max(1, (int)std::floor(L / side));
                 double ms = 0.0;
                 rc = trial(t, steps, ms);
@@ -2020,7 +1953,7 @@ int sdm_autotune(sdm_context* c, int32_t steps, sdm_tuning* chosen) {
     // then the Verlet skin of the tile lists for the chosen configuration (block kernels
     // only): a wider skin keeps the lists longer but the pair kernel evaluates more pairs
     // outside the cutoff.  Two rounds again, ranked by the sum.
-    if (rc == SDM_OK && best.pair_group == 0) {
+    if (rc == SDM_OK) {
         const float skins[] = {0.f, 0.01f, 0.02f, 0.03f, 0.04f};
         constexpr int NS = sizeof(skins) / sizeof(skins[0]);
         double tsk[NS] = {};

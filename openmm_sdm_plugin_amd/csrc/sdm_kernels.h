@@ -3,8 +3,9 @@
 // One step of every replica r of a context (LangevinIntegratorSDM::step,
 // openmmapi/src/LangevinIntegratorSDM.cpp:153-183) is the launch sequence
 //
-//   k_bin -> k_scan -> k_scatter -> k_cellsort -> k_bbox -> k_tiles     spatial sort + tiles
-//   k_pair                 F0: full LJ+RF sweep at x (FP32 math, fixed-point forces)
+//   k_bin -> k_scan -> k_scatter -> k_cellsort -> k_blockorder          spatial sort
+//   k_refresh -> k_tiles   slot records, boxes; tile lists
+//   k_pair                 F0: LJ+RF of every pair at x (FP32 math, fixed-point forces)
 //   k_energy64             U0 on the steps that report energies (FP64 pair sums)
 //   k_bonded               Ub, Fb: harmonic bonds/angles at x (FP64, gathered per atom)
 //   k_ligcand              j-blocks near the displaced atoms at x or at x+d
@@ -143,15 +144,9 @@ __global__ void k_scatter(int N, int Np, int NC, const int* __restrict__ key,
     if (s >= 0 && s < N) orig_s[(size_t)r * Np + s] = i;  // always, with consistent counts
 }
 
-// per cell: order its slots by atom index, then gather the sorted FP32 arrays and clear
-// the slot-ordered force accumulator.
+// per cell: order its slots by atom index
 __global__ void k_cellsort(int N, int Np, int NC, const int* __restrict__ cstart,
-                           int* __restrict__ orig_s, int* __restrict__ slot_of,
-                           const double* __restrict__ x64, const float* __restrict__ qs,
-                           const float* __restrict__ sh, const float* __restrict__ se,
-                           float4* __restrict__ posq_s, float2* __restrict__ par_s,
-                           float4* __restrict__ arec, long long* __restrict__ F, Geom g,
-                           const double4* __restrict__ par64, Rec64* __restrict__ rec) {
+                           int* __restrict__ orig_s) {
     int r = blockIdx.y;
     int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= NC) return;
@@ -167,91 +162,172 @@ __global__ void k_cellsort(int N, int Np, int NC, const int* __restrict__ cstart
         }
         o[b + 1] = v;
     }
+}
+
+// Orders the 64 slots of a block so that its clusters of 8 are compact: the block is split
+// at the median of its longest axis into halves of 32, these into 16 and these into 8 (one
+// wave per block, bitonic sorts of the axis' coordinate, ties by atom index, so that the
+// order is unique).  Writes the final orig_s and slot_of.  In a disordered 22,750-atom box
+// (cells of 0.305 nm) it leaves 8% fewer pairs of clusters within the list radius and 5%
+// fewer with a pair within the cutoff than the order along the curve.
+__global__ __launch_bounds__(64) void k_blockorder(int N, int Np, const double* __restrict__ x64,
+                                                   int* __restrict__ orig_s,
+                                                   int* __restrict__ slot_of, Geom g) {
+    const int r = blockIdx.y, b = blockIdx.x, lane = threadIdx.x;
+    const int sl = b * 64 + lane;
+    int* O = orig_s + (size_t)r * Np;
     const double* X = x64 + (size_t)r * 3 * Np;
-    for (int s = beg; s < end; s++) {
-        int i = o[s];
-        slot_of[(size_t)r * Np + i] = s;
-        double wx = X[i], wy = X[Np + i], wz = X[2 * Np + i];
-        wx -= g.Lx * floor(wx * g.iLx);
-        wy -= g.Ly * floor(wy * g.iLy);
-        wz -= g.Lz * floor(wz * g.iLz);
-        float4 pq = make_float4((float)wx, (float)wy, (float)wz, qs[i]);
-        posq_s[(size_t)r * Np + s] = pq;
-        if (rec) {  // energy evaluations: the FP64 record in the same image
-            double4 pr = par64[i];
-            rec[(size_t)r * Np + s] = Rec64{wx, wy, wz, pr.x, pr.y, pr.z};
+    const bool v = sl < N;
+    int idx = v ? O[sl] : 0x7FFFFFFF;
+    float p[3] = {0.f, 0.f, 0.f};
+    const double* L = &g.Lx;
+    const double* iL = &g.iLx;
+#pragma unroll
+    for (int d = 0; d < 3; d++) {  // relative to the block's first atom, in its image
+        const double w = X[(size_t)d * Np + (v ? idx : O[b * 64])];
+        const double dw = w - __shfl(w, 0, 64);
+        p[d] = (float)(dw - L[d] * rint(dw * iL[d]));
+    }
+#pragma unroll
+    for (int n = 64; n >= 16; n >>= 1) {
+        float ext[3];
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            float lo = idx != 0x7FFFFFFF ? p[d] : 3.0e38f, hi = idx != 0x7FFFFFFF ? p[d] : -3.0e38f;
+            for (int o = n / 2; o > 0; o >>= 1) {
+                lo = fminf(lo, __shfl_xor(lo, o, 64));
+                hi = fmaxf(hi, __shfl_xor(hi, o, 64));
+            }
+            ext[d] = hi - lo;
         }
-        par_s[(size_t)r * Np + s] = make_float2(sh[i], se[i]);
-        // interleaved copy for the grouped pair kernel: one 32-byte record per slot
-        arec[2 * ((size_t)r * Np + s)] = pq;
-        arec[2 * ((size_t)r * Np + s) + 1] = make_float4(sh[i], se[i], 0.f, 0.f);
-        long long* Fr = F + (size_t)r * 3 * Np;  // forces are accumulated in slot order
-        Fr[s] = 0;
-        Fr[Np + s] = 0;
-        Fr[2 * Np + s] = 0;
+        const int ax = ext[0] >= ext[1] && ext[0] >= ext[2] ? 0 : ext[1] >= ext[2] ? 1 : 2;
+        for (int k = 2; k <= n; k <<= 1)
+            for (int j = k >> 1; j > 0; j >>= 1) {
+                const float key = idx == 0x7FFFFFFF ? 3.0e38f : ax == 0 ? p[0] : ax == 1 ? p[1] : p[2];
+                const float ok = __shfl_xor(key, j, 64);
+                const int oi = __shfl_xor(idx, j, 64);
+                const bool less = ok < key || (ok == key && oi < idx);  // the partner's is smaller
+                const bool up = ((lane & (n - 1)) & k) == 0, first = (lane & j) == 0;
+                // (up, first) and (!up, !first) lanes keep the smaller of the two
+                const bool take = (up == first) ? less : !less;
+#pragma unroll
+                for (int d = 0; d < 3; d++) {
+                    const float op = __shfl_xor(p[d], j, 64);
+                    p[d] = take ? op : p[d];
+                }
+                idx = take ? oi : idx;
+            }
+    }
+    if (v) {  // the empty slots of the last block stay last
+        O[sl] = idx;
+        slot_of[(size_t)r * Np + idx] = sl;
     }
 }
 
-// bounding box of each 64-slot block (one wave per block).  After a sort the slot
-// order is new, so the replica's displacement record (dmax, read by k_tiles) is set to a
-// value that makes the next tile-list build unconditional.
-__global__ __launch_bounds__(64) void k_bbox(int N, int Np, int NB,
-                                             const float4* __restrict__ posq_s,
-                                             float4* __restrict__ bb_lo, float4* __restrict__ bb_hi,
-                                             float* __restrict__ dmax) {
-    int r = blockIdx.y, b = blockIdx.x, lane = threadIdx.x;
-    int s = b * 64 + lane;
-    bool v = s < N;
-    float4 p = posq_s[(size_t)r * Np + s];
-    float lx = wave_min(v ? p.x : 3.0e38f), ly = wave_min(v ? p.y : 3.0e38f),
-          lz = wave_min(v ? p.z : 3.0e38f);
-    float hx = wave_max(v ? p.x : -3.0e38f), hy = wave_max(v ? p.y : -3.0e38f),
-          hz = wave_max(v ? p.z : -3.0e38f);
+// min / max over the 8 lanes of each group of 8 (lane ^ 7, lane ^ 2, lane ^ 1 via DPP)
+__device__ __forceinline__ float min8(float v) {
+    v = fminf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xf, 0xf, true)));
+    v = fminf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xf, 0xf, true)));
+    return fminf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xf, 0xf, true)));
+}
+__device__ __forceinline__ float max8(float v) {
+    v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xf, 0xf, true)));
+    v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xf, 0xf, true)));
+    return fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xf, 0xf, true)));
+}
+
+// Boxes of one 64-slot block (one wave, lane = slot, v: the slot holds an atom at p): the
+// block's corners, and per cluster of 8 slots its centre (cbox[0..7]) and half extents
+// (cbox[8..15]; -1e30 for a cluster without atoms, whose gap to any box is then never in
+// range).
+__device__ __forceinline__ void block_boxes(float4 p, bool v, int lane, float4* __restrict__ lo,
+                                            float4* __restrict__ hi, float4* __restrict__ cbox) {
+    float lx = min8(v ? p.x : 3.0e38f), ly = min8(v ? p.y : 3.0e38f), lz = min8(v ? p.z : 3.0e38f);
+    float hx = max8(v ? p.x : -3.0e38f), hy = max8(v ? p.y : -3.0e38f), hz = max8(v ? p.z : -3.0e38f);
+    if ((lane & 7) == 0) {
+        const bool any = lx <= hx;
+        cbox[lane >> 3] = any ? make_float4(0.5f * (lx + hx), 0.5f * (ly + hy), 0.5f * (lz + hz), 0.f)
+                              : make_float4(0.f, 0.f, 0.f, 0.f);
+        cbox[8 + (lane >> 3)] = any ? make_float4(0.5f * (hx - lx), 0.5f * (hy - ly), 0.5f * (hz - lz), 0.f)
+                                    : make_float4(-1.0e30f, -1.0e30f, -1.0e30f, 0.f);
+    }
+#pragma unroll
+    for (int o = 32; o >= 8; o >>= 1) {
+        lx = fminf(lx, __shfl_xor(lx, o, 64));
+        ly = fminf(ly, __shfl_xor(ly, o, 64));
+        lz = fminf(lz, __shfl_xor(lz, o, 64));
+        hx = fmaxf(hx, __shfl_xor(hx, o, 64));
+        hy = fmaxf(hy, __shfl_xor(hy, o, 64));
+        hz = fmaxf(hz, __shfl_xor(hz, o, 64));
+    }
     if (lane == 0) {
-        bb_lo[(size_t)r * NB + b] = make_float4(lx, ly, lz, 0.f);
-        bb_hi[(size_t)r * NB + b] = make_float4(hx, hy, hz, 0.f);
-        if (b == 0) dmax[(size_t)r * DISP_STRIDE] = DISP_STALE;
+        *lo = make_float4(lx, ly, lz, 0.f);
+        *hi = make_float4(hx, hy, hz, 0.f);
     }
 }
 
-// Between full sorts the slot order of the last sort is kept.  One wave per 64-slot
-// block re-gathers its atoms' coordinates from the FP64 positions, each wrapped to the
-// periodic image nearest the block's first atom (itself wrapped into the box), so a
-// block stays compact when one of its atoms crosses a face of the box; then the block's
-// box is recomputed and the slot-ordered force accumulator cleared.  Culling and pair
-// distances take minimum images of box centres or of pairs, so they hold for any image.
-__global__ __launch_bounds__(64) void k_refresh(int N, int Np, int NB,
-                                                const double* __restrict__ x64,
-                                                const int* __restrict__ orig_s,
-                                                const float* __restrict__ qs, Geom g,
-                                                float4* __restrict__ posq_s,
-                                                float4* __restrict__ arec,
-                                                long long* __restrict__ F,
-                                                float4* __restrict__ bb_lo,
-                                                float4* __restrict__ bb_hi,
-                                                const double4* __restrict__ par64,
-                                                Rec64* __restrict__ rec,
-                                                const float4* __restrict__ xb,
-                                                float* __restrict__ dmax) {
+// The slot records of one evaluation.  One wave per 64-slot block gathers its atoms'
+// coordinates from the FP64 positions, each wrapped into the box and then to the periodic
+// image nearest the block's first atom, so a block stays compact when one of its atoms
+// crosses a face of the box; then the boxes of the block and its clusters are
+// computed and the slot-ordered force accumulator cleared.  The FP32 records hold
+// coordinates relative to the block's first atom (bref, FP64), both in whole QUANTUMs
+// (quantize), instead of coordinates in the box, whose FP32 rounding is 2e-7 nm and more.  Culling and pair distances take minimum images of box
+// centres or of pairs, so they hold for any image.
+//   SORT = true (after a sort; the slot order is new): also the records' parameters; the
+// replica's displacement record (dmax, read by k_tiles) is set to a value that makes the
+// next tile-list build unconditional; and the exclusions are written in slot order:
+// exs[block][k][lane], the slot of the k-th partner of the block's atom `lane` (-1: none),
+// and exblocks[block], a 64-bit set that has bit b & 63 for every j-block b that holds a
+// partner (mostly the block and its neighbours, now and then one far along the curve).  The
+// pair and energy kernels then read them with one coalesced load instead of a chain of four
+// (atom, list start, list entry, slot), and only for the tiles that need them.
+//   SORT = false: the order of the last sort is kept; the displacement record of kept lists
+// is updated (xb, dmax).
+constexpr double QUANTUM = 1.0 / 8388608.0;  // 2^-23 nm
+// x in whole QUANTUMs.  Sums and differences of such numbers below 2 nm are exact in FP32, so
+// the separation of two atoms in range, whether it is within the cutoff, and the force have
+// the same bits in whatever blocks and images the atoms lie (the box length between two
+// images is taken in whole QUANTUMs too), at a rounding of at most 6e-8 nm.
+__device__ __forceinline__ double quantize(double x) { return rint(x * 8388608.0) * QUANTUM; }
+
+template <bool SORT>
+__global__ __launch_bounds__(64) void k_refresh(
+    int N, int Np, int NB, const double* __restrict__ x64, const int* __restrict__ orig_s,
+    const float* __restrict__ qs, const float* __restrict__ sh, const float* __restrict__ se,
+    Geom g, float4* __restrict__ arec, double4* __restrict__ bref, long long* __restrict__ F,
+    float4* __restrict__ bb_lo, float4* __restrict__ bb_hi, float4* __restrict__ cbox,
+    const double4* __restrict__ par64, Rec64* __restrict__ rec, const float4* __restrict__ xb,
+    float* __restrict__ dmax, const int* __restrict__ slot_of, const int* __restrict__ ex_start,
+    const int* __restrict__ ex_list, int max_ex, int* __restrict__ exs,
+    unsigned long long* __restrict__ exblocks) {
     int r = blockIdx.y, b = blockIdx.x, lane = threadIdx.x;
     int sl = b * 64 + lane;
     bool v = sl < N;  // slot b * 64 (lane 0) is always below N
     const int* O = orig_s + (size_t)r * Np;
     const double* X = x64 + (size_t)r * 3 * Np;
     int i = O[v ? sl : b * 64];
-    double wx = X[i], wy = X[Np + i], wz = X[2 * Np + i];
-    double rx = __shfl(wx, 0, 64), ry = __shfl(wy, 0, 64), rz = __shfl(wz, 0, 64);
-    rx -= g.Lx * floor(rx * g.iLx);
-    ry -= g.Ly * floor(ry * g.iLy);
-    rz -= g.Lz * floor(rz * g.iLz);
-    wx -= g.Lx * rint((wx - rx) * g.iLx);
-    wy -= g.Ly * rint((wy - ry) * g.iLy);
-    wz -= g.Lz * rint((wz - rz) * g.iLz);
-    float4 p = make_float4((float)wx, (float)wy, (float)wz, qs[i]);
+    double wx = X[i], wy = X[Np + i], wz = X[2 * Np + i];  // wrapped into the box
+    wx -= g.Lx * floor(wx * g.iLx);
+    wy -= g.Ly * floor(wy * g.iLy);
+    wz -= g.Lz * floor(wz * g.iLz);
+    const double rx = __shfl(wx, 0, 64), ry = __shfl(wy, 0, 64), rz = __shfl(wz, 0, 64);
+    // box lengths to the image nearest the first atom
+    const double kx = rint((wx - rx) * g.iLx), ky = rint((wy - ry) * g.iLy),
+                 kz = rint((wz - rz) * g.iLz);
+    const double qx = quantize(wx) - kx * quantize(g.Lx), qy = quantize(wy) - ky * quantize(g.Ly),
+                 qz = quantize(wz) - kz * quantize(g.Lz);
+    wx -= g.Lx * kx;
+    wy -= g.Ly * ky;
+    wz -= g.Lz * kz;
+    const float4 p = make_float4((float)wx, (float)wy, (float)wz, 0.f);
     size_t o = (size_t)r * Np + sl;
+    const size_t bo = (size_t)r * NB + b;
+    const double bx = quantize(rx), by = quantize(ry), bz = quantize(rz);
+    if (lane == 0) bref[bo] = make_double4(bx, by, bz, 0.0);
     if (v) {
-        posq_s[o] = p;
-        arec[2 * o] = p;
+        arec[2 * o] = make_float4((float)(qx - bx), (float)(qy - by), (float)(qz - bz), qs[i]);
+        if (SORT) arec[2 * o + 1] = make_float4(sh[i], se[i], 0.f, 0.f);
         if (rec) {  // energy evaluations: the FP64 record in the same image
             double4 pr = par64[i];
             rec[o] = Rec64{wx, wy, wz, pr.x, pr.y, pr.z};
@@ -261,13 +337,25 @@ __global__ __launch_bounds__(64) void k_refresh(int N, int Np, int NB,
         Fr[Np + sl] = 0;
         Fr[2 * Np + sl] = 0;
     }
-    float lx = wave_min(v ? p.x : 3.0e38f), ly = wave_min(v ? p.y : 3.0e38f),
-          lz = wave_min(v ? p.z : 3.0e38f);
-    float hx = wave_max(v ? p.x : -3.0e38f), hy = wave_max(v ? p.y : -3.0e38f),
-          hz = wave_max(v ? p.z : -3.0e38f);
-    if (lane == 0) {
-        bb_lo[(size_t)r * NB + b] = make_float4(lx, ly, lz, 0.f);
-        bb_hi[(size_t)r * NB + b] = make_float4(hx, hy, hz, 0.f);
+    block_boxes(p, v, lane, bb_lo + bo, bb_hi + bo, cbox + 16 * bo);
+    if (SORT) {
+        if (lane == 0 && b == 0) dmax[(size_t)r * DISP_STRIDE] = DISP_STALE;
+        unsigned long long set = 0ull;
+        int nex = 0, b0 = 0;
+        if (v) {
+            b0 = ex_start[i];
+            nex = ex_start[i + 1] - b0;
+        }
+        int* E = exs + bo * max_ex * 64;
+        for (int k = 0; k < max_ex; k++) {
+            const int es = k < nex ? slot_of[(size_t)r * Np + ex_list[b0 + k]] : -1;
+            E[k * 64 + lane] = es;
+            if (es >= 0) set |= 1ull << ((es >> 6) & 63);
+        }
+#pragma unroll
+        for (int q = 32; q > 0; q >>= 1) set |= __shfl_xor(set, q, 64);
+        if (lane == 0) exblocks[bo] = set;
+        return;
     }
     // kept tile lists (xb: the slot coordinates when they were built): the block's
     // largest squared displacement since, as a minimum image (the block may have moved
@@ -314,191 +402,115 @@ __device__ __forceinline__ int lane_rank(unsigned long long m) {
     return __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
 }
 
-// min / max over the 8 lanes of each group of 8 (lane ^ 7, lane ^ 2, lane ^ 1 via DPP)
-__device__ __forceinline__ float min8(float v) {
-    v = fminf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xf, 0xf, true)));
-    v = fminf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xf, 0xf, true)));
-    return fminf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xf, 0xf, true)));
-}
-__device__ __forceinline__ float max8(float v) {
-    v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xf, 0xf, true)));
-    v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xf, 0xf, true)));
-    return fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xf, 0xf, true)));
+// Which of two blocks lists their tile.  Taking j >= i would give the first blocks of the
+// slot order all of their neighbours and the last ones none; by the parity of i + j every
+// block lists about half of its neighbours, so that i-blocks (and with them the XCDs, which
+// work on consecutive blocks) have equal work.
+__device__ __forceinline__ bool lists_tile(int ib, int jb) {
+    return jb == ib || (jb > ib) == (((ib ^ jb) & 1) != 0);
 }
 
-// tile list of one i-block: every j-block (j >= i for the half list) whose box is within
-// the list radius r_l (r_c + skin + slack, TileRadius) of the i-block's box, ascending,
-// each with a 64-bit mask of the j atoms that lie within r_l of the box of at least one
-// of the block's eight 8-slot groups (atoms outside all of them cannot have a partner
-// within r_l in the i-block; the union of the small boxes is a much tighter region than
-// the block's box).  Half list: in the diagonal tile an atom only counts for groups that
-// start below it.
-// NW waves per i-block: the candidate j-blocks (box test) are listed in LDS, each
-// wave computes the atom masks of every NW-th candidate, and wave 0 compacts the
-// non-empty ones in candidate order.  Results do not depend on NW.
+// tile list of one i-block: every j-block it lists (lists_tile) whose box is within the
+// list radius r_l (r_c + skin + slack, TileRadius) of the i-block's box, ascending, each
+// with a 64-bit mask of the pairs of 8-slot clusters whose boxes lie within r_l: bit
+// 8 jc + ic for cluster jc of the j-block and ic of the i-block.  In the diagonal tile
+// only jc >= ic.  A wave tests the 64 cluster pairs of a candidate at once (lane = bit),
+// about 30 VALU instructions per candidate; the ballot is the mask.
+// NW waves per i-block: in each round wave w takes 64 j-blocks (their box tests on its
+// lanes, then the masks of those in range) and the waves' lists are put one after the other.
+// Results do not depend on NW.
 // Kept lists (tr.reuse_d2 >= 0): the workgroup returns at once while no atom of the
 // replica has moved more than half the skin since the build (dmax); a build stores the
 // block's slot coordinates in xb.
-constexpr int TILE_CAND = 256;  // candidates per round
 template <int NW>  // waves per i-block workgroup
 __global__ __launch_bounds__(64 * NW) void k_tiles(int N, int Np, int NB, int maxj,
-                                               const float4* __restrict__ posq_s,
+                                               const float4* __restrict__ arec,
+                                               const double4* __restrict__ bref,
                                                const float4* __restrict__ bb_lo,
                                                const float4* __restrict__ bb_hi,
+                                               const float4* __restrict__ cbox,
                                                int* __restrict__ tiles,
                                                unsigned long long* __restrict__ tmask,
                                                int* __restrict__ ntiles,
                                                const float* __restrict__ dmax,
                                                float4* __restrict__ xb, TileRadius tr, Geom g,
-                                               int half, int* __restrict__ flags) {
-    __shared__ float4 sub[8][2];
-    __shared__ int cand[TILE_CAND];
-    __shared__ unsigned long long cmk[TILE_CAND];
-    __shared__ int ncand_s, base_s;
-    int r = blockIdx.y, ib = blockIdx.x;
-    int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+                                               int* __restrict__ flags) {
+    __shared__ int nkept[2][NW];
+    const int r = blockIdx.y, ib = blockIdx.x;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const float list_r2 = tr.r2;
     // kept lists: every workgroup of the replica reads the same record (written by the
     // slot refresh or the sort before this launch), so all of them keep or all rebuild
     if (tr.reuse_d2 >= 0.f && dmax[(size_t)r * DISP_STRIDE] <= tr.reuse_d2) return;
     const float4* lo = bb_lo + (size_t)r * NB;
     const float4* hi = bb_hi + (size_t)r * NB;
-    const float4* P = posq_s + (size_t)r * Np;
-    float4 li = lo[ib], hi_i = hi[ib];
-    // the eight group boxes (empty groups past N get a negative extent and never match)
-    if (wave == 0) {
+    const float4* CB = cbox + (size_t)r * NB * 16;
+    const float4 li = lo[ib], hi_i = hi[ib];
+    if (wave == 0 && tr.reuse_d2 >= 0.f) {  // the build coordinates
         int is = ib * 64 + lane;
-        bool v = is < N;
-        float4 p = P[min(is, N - 1)];
-        if (tr.reuse_d2 >= 0.f && v) xb[(size_t)r * Np + is] = p;  // the build coordinates
-        float lx = min8(v ? p.x : 3.0e38f), ly = min8(v ? p.y : 3.0e38f), lz = min8(v ? p.z : 3.0e38f);
-        float hx = max8(v ? p.x : -3.0e38f), hy = max8(v ? p.y : -3.0e38f), hz = max8(v ? p.z : -3.0e38f);
-        if ((lane & 7) == 0) {
-            bool any = lx <= hx;
-            sub[lane >> 3][0] = make_float4(0.5f * (lx + hx), 0.5f * (ly + hy), 0.5f * (lz + hz), 0.f);
-            sub[lane >> 3][1] = any ? make_float4(0.5f * (hx - lx), 0.5f * (hy - ly), 0.5f * (hz - lz), 0.f)
-                                    : make_float4(-1.0e30f, -1.0e30f, -1.0e30f, 0.f);
-        }
+        const double4 o = bref[(size_t)r * NB + ib];
+        const float4 p = arec[2 * ((size_t)r * Np + min(is, N - 1))];
+        if (is < N)
+            xb[(size_t)r * Np + is] =
+                make_float4((float)(o.x + p.x), (float)(o.y + p.y), (float)(o.z + p.z), 0.f);
     }
-    // atom mask of candidate j-block jb2 (lane = atom)
-    auto mask_of = [&](int jb2) {
-        int s = jb2 * 64 + lane;
-        float4 p = P[s];
-        // one periodic shift for the whole tile when it is exact for every pair within
-        // the list radius (TileRadius::oix); otherwise the minimum image per group
-        float4 lj = lo[jb2], hj = hi[jb2];
-        float dcx = 0.5f * (li.x + hi_i.x - lj.x - hj.x);
-        float dcy = 0.5f * (li.y + hi_i.y - lj.y - hj.y);
-        float dcz = 0.5f * (li.z + hi_i.z - lj.z - hj.z);
-        float sx = g.bx * rintf(dcx * g.ibx), sy = g.by * rintf(dcy * g.iby),
-              sz = g.bz * rintf(dcz * g.ibz);
-        bool one_image =
-            fabsf(dcx - sx) + 0.5f * (hi_i.x - li.x + hj.x - lj.x) < tr.oix &&
-            fabsf(dcy - sy) + 0.5f * (hi_i.y - li.y + hj.y - lj.y) < tr.oiy &&
-            fabsf(dcz - sz) + 0.5f * (hi_i.z - li.z + hj.z - lj.z) < tr.oiz;
-        if (one_image) {
-            p.x += sx;
-            p.y += sy;
-            p.z += sz;
-        }
-        // groups whose box is within rc of the j-block's box (lane q tests group q);
-        // only those are tested atom by atom
-        unsigned long long rel;
-        {
-            float4 c = sub[lane & 7][0], h = sub[lane & 7][1];
-            float dx = 0.5f * (lj.x + hj.x) - c.x, dy = 0.5f * (lj.y + hj.y) - c.y,
-                  dz = 0.5f * (lj.z + hj.z) - c.z;
-            if (one_image) {
-                dx += sx;
-                dy += sy;
-                dz += sz;
-            } else {
-                dx -= g.bx * rintf(dx * g.ibx);
-                dy -= g.by * rintf(dy * g.iby);
-                dz -= g.bz * rintf(dz * g.ibz);
-            }
-            float gx = fmaxf(fabsf(dx) - h.x - 0.5f * (hj.x - lj.x), 0.f);
-            float gy = fmaxf(fabsf(dy) - h.y - 0.5f * (hj.y - lj.y), 0.f);
-            float gz = fmaxf(fabsf(dz) - h.z - 0.5f * (hj.z - lj.z), 0.f);
-            rel = __ballot(lane < 8 && h.x >= 0.f && gx * gx + gy * gy + gz * gz < list_r2);
-        }
-        // the atom tests, with the per-pair image only where the tile needs it and the
-        // half-list rule only in the diagonal tile (both uniform: separate loops)
-        auto atom_in = [&](auto mic, auto diagc) {
-            constexpr bool MI = decltype(mic)::value, DIAG = decltype(diagc)::value;
-            bool in = false;
-            unsigned long long rq = rel;
-            while (rq) {
-                int q = __ffsll((long long)rq) - 1;
-                rq &= rq - 1ull;
-                float4 c = sub[q][0], h = sub[q][1];
-                float dx = p.x - c.x, dy = p.y - c.y, dz = p.z - c.z;
-                if (MI) {
-                    dx -= g.bx * rintf(dx * g.ibx);
-                    dy -= g.by * rintf(dy * g.iby);
-                    dz -= g.bz * rintf(dz * g.ibz);
-                }
-                float gx = fmaxf(fabsf(dx) - h.x, 0.f), gy = fmaxf(fabsf(dy) - h.y, 0.f),
-                      gz = fmaxf(fabsf(dz) - h.z, 0.f);
-                bool inq = gx * gx + gy * gy + gz * gz < list_r2;
-                if (DIAG) inq = inq && s > ib * 64 + q * 8;
-                in = in || inq;
-            }
-            return in;
-        };
-        using T = std::true_type;
-        using Fa = std::false_type;
-        bool in;
-        if (half && jb2 == ib) in = one_image ? atom_in(Fa(), T()) : atom_in(T(), T());
-        else in = one_image ? atom_in(Fa(), Fa()) : atom_in(T(), Fa());
-        return __ballot(in && (s < N));
+    // this lane's pair of clusters: ic of the i-block, jc of the candidate
+    const int ic = lane & 7, jc = lane >> 3;
+    const float4 ci = CB[16 * ib + ic], hc = CB[16 * ib + 8 + ic];
+    auto mask_of = [&](int jb, float4 cj, float4 hj) {
+        // the smallest gap over all images is the one at the centres' minimum image
+        float dx = ci.x - cj.x, dy = ci.y - cj.y, dz = ci.z - cj.z;
+        dx -= g.bx * rintf(dx * g.ibx);
+        dy -= g.by * rintf(dy * g.iby);
+        dz -= g.bz * rintf(dz * g.ibz);
+        // a cluster without atoms has half extents of -1e30: its gap is never in range
+        const float gx = fmaxf(fabsf(dx) - (hc.x + hj.x), 0.f),
+                    gy = fmaxf(fabsf(dy) - (hc.y + hj.y), 0.f),
+                    gz = fmaxf(fabsf(dz) - (hc.z + hj.z), 0.f);
+        return __ballot(gx * gx + gy * gy + gz * gz < list_r2 && (jb != ib || jc >= ic));
     };
     int* out = tiles + ((size_t)r * NB + ib) * maxj;
     unsigned long long* mout = tmask + ((size_t)r * NB + ib) * maxj;
-    int count = 0;    // wave 0's running output count
-    int base = half ? (ib & ~63) : 0;
-    while (base < NB) {
-        // list up to TILE_CAND candidates (wave 0), continuing from base
-        if (wave == 0) {
-            int nc = 0;
-            while (base < NB && nc + 64 <= TILE_CAND) {
-                int jb = base + lane;
-                bool ok = false;
-                if (jb < NB && (!half || jb >= ib)) ok = bbox_gap2(li, hi_i, lo[jb], hi[jb], g) < list_r2;
-                unsigned long long m = __ballot(ok);
-                if (ok) cand[nc + lane_rank(m)] = jb;
-                nc += __popcll(m);
-                base += 64;
+    int count = 0;  // tiles of the rounds before (uniform)
+    for (int base = 0, round = 0; base < NB; base += 64 * NW, round ^= 1) {
+        const int jl = base + 64 * wave + lane;  // this lane's j-block
+        bool ok = false;
+        if (jl < NB && lists_tile(ib, jl)) ok = bbox_gap2(li, hi_i, lo[jl], hi[jl], g) < list_r2;
+        unsigned long long near = __ballot(ok), am = 0ull;
+        // the masks of the candidates, each kept by its lane; four at a time, so that their
+        // box loads are in flight together
+        while (near) {
+            int q[4];
+            float4 cj[4], hj[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                q[k] = near ? __builtin_ctzll(near) : (k ? q[k - 1] : 0);
+                near &= near - 1ull;
+                const float4* C = CB + 16 * (base + 64 * wave + q[k]) + jc;
+                cj[k] = C[0];
+                hj[k] = C[8];
             }
-            if (lane == 0) {
-                ncand_s = nc;
-                base_s = base;
-            }
-        }
-        __syncthreads();
-        int nc = ncand_s;
-        base = base_s;  // every wave continues from wave 0's position (uniform loop)
-        for (int c = wave; c < nc; c += NW) {
-            // the candidate is the same for the whole wave: scalar, so that its box
-            // loads and the uniform tests above compile to scalar code and branches
-            unsigned long long am = mask_of(__builtin_amdgcn_readfirstlane(cand[c]));
-            if (lane == 0) cmk[c] = am;
-        }
-        __syncthreads();
-        if (wave == 0) {
-            for (int c0 = 0; c0 < nc; c0 += 64) {
-                int c = c0 + lane;
-                unsigned long long am = c < nc ? cmk[c] : 0ull;
-                unsigned long long keep = __ballot(am != 0ull);
-                int pos = count + lane_rank(keep);
-                if (am != 0ull && pos < maxj) {
-                    out[pos] = cand[c];
-                    mout[pos] = am;
-                }
-                count += __popcll(keep);
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const unsigned long long b = mask_of(base + 64 * wave + q[k], cj[k], hj[k]);
+                if (lane == q[k]) am = b;
             }
         }
-        __syncthreads();
+        const unsigned long long keep = __ballot(am != 0ull);
+        if (lane == 0) nkept[round][wave] = __popcll(keep);
+        __syncthreads();  // one barrier a round: the counts alternate between two rows
+        int pos = count + lane_rank(keep);
+#pragma unroll
+        for (int w = 0; w < NW; w++) {
+            const int n = nkept[round][w];
+            if (w < wave) pos += n;
+            count += n;
+        }
+        if (am != 0ull && pos < maxj) {
+            out[pos] = jl;
+            mout[pos] = am;
+        }
     }
     if (threadIdx.x == 0) {
         ntiles[(size_t)r * NB + ib] = min(count, maxj);
@@ -507,120 +519,33 @@ __global__ __launch_bounds__(64 * NW) void k_tiles(int N, int Np, int NB, int ma
 }
 
 // ---------------------------------------------------------------------------
-// the hot kernel: U0 and F0 over all pairs at x.  One wave per (replica, i-block):
-// lane = i atom (registers), j atoms are wave-uniform (scalar loads) taken from each
-// tile's j mask.
-//   NEWTON = false: full tile list, every ordered pair once, no j forces, energy halved.
-//   NEWTON = true:  half tile list (j-block >= i-block, j > i inside the diagonal tile),
-//                   every pair once; the j forces of 8 j atoms at a time are summed over
-//                   the wave by a reduce-scatter and added with int64 atomics.
-// When one shift is exact for every pair of a tile within the list radius (Geom::oix)
-// the periodic image is that shift for the whole tile (applied to the i coordinates);
-// otherwise each pair takes the minimum image.  Pair energies are accumulated in FP64 per pair and the per-tile FP32 force and
-// reaction-field sums in FP64 in tile order; fixed-point atomics commute, so results are
-// bit-reproducible.
+// The pair kernel: F0 over all pairs at x, each pair once (Newton-3 over the tile lists).
+// One wave per (replica, i-block), or `split` waves per i-block, each taking every
+// split-th tile.  A wave holds the 64 i atoms as eight clusters of 8: lane 8 jl + il keeps
+// atom il of every cluster in registers, and takes one cluster of 8 j atoms at a time,
+// lane 8 jl + il holding j atom jl.  One step is a pair of clusters, 64 pairs on 64 lanes,
+// taken for the bits of the tile's mask (uniform branches).  A step none of whose pairs
+// is within the cutoff ends after the distance test.
+//   i forces: FP32 in the lane (24 registers), added up over the eight lanes that share an
+//     i atom and over to the accumulator after every PAIRS_PER_FLUSH pairs or more (pairs
+//     within the cutoff, so that the sums do not depend on what else the lists hold).
+//   j forces: FP32 over the cluster's steps, added up over the eight lanes that share a j
+//     atom, kept in registers over the tile and added to the slot-ordered int64 accumulator
+//     once per tile with coalesced atomics.
+// The periodic image is one shift per tile when that is exact for every pair within the
+// list radius (Geom::oix), otherwise the minimum image of each pair.  Fixed-point atomics
+// commute, so results are bit-reproducible.
+//
+// What bounds it: VALU issue (89% of the cycles of 22 x 22,750 atoms, 4 waves per SIMD at
+// 127 registers).  A step takes 7 instructions to the distance test and 21 after it.  One
+// lane per i atom against one j atom at a time, the form before, took 37 instructions per 64
+// pairs with 22% of them within the cutoff; pairs of clusters have 30% (40% after the
+// distance test's early end) and no sum over the wave for each j atom.  Measured alone, 22
+// x 22,750 atoms: 532 -> 384 us (297M -> 201M VALU instructions); 8 x 99,920 atoms:
+// 1,054 -> 814 us; one replica of 22,750 atoms: 55 -> 43 us.  Where the i atoms' charges and
+// LJ parameters came from LDS instead (122 registers), or the j forces of four clusters were
+// summed together (as many instructions in all, 30% more code), it was 4% and 14% slower.
 // ---------------------------------------------------------------------------
-struct PairAcc {
-    float fx, fy, fz;  // per-tile force on the lane's i atom
-    float sqr2, sq;    // per-tile sums of qq r^2 and qq (reaction-field energy terms)
-    double e;          // LJ + qq/r energy in FP64 (net energies cancel strongly)
-    float ef;          // the same over the current chunk of 8 pairs, added to e per chunk
-    int cnt;
-};
-
-// one pair (i on the lane, j uniform); returns F/r (0 outside the cutoff or excluded)
-template <bool MINIMG, bool EXCL>
-__device__ __forceinline__ float pair_one(float4 pi, float2 qi, float4 pj, float2 qj,
-                                          bool extra_ok, const Geom& g, PairAcc& a,
-                                          float& dx, float& dy, float& dz) {
-    dx = pi.x - pj.x;
-    dy = pi.y - pj.y;
-    dz = pi.z - pj.z;
-    if (MINIMG) {
-        dx -= g.bx * rintf(dx * g.ibx);
-        dy -= g.by * rintf(dy * g.iby);
-        dz -= g.bz * rintf(dz * g.ibz);
-    }
-    float r2 = dx * dx + dy * dy + dz * dz;
-    bool ok = r2 < g.rc2f;
-    if (EXCL) ok = ok && extra_ok;
-    float ir = __frsqrt_rn(r2);
-    float ir2 = ir * ir;
-    float sig = qi.x + qj.x;
-    float s2 = sig * sig * ir2;
-    float s6 = s2 * s2 * s2;
-    float es6 = (qi.y * qj.y) * s6;
-    float qq = pi.w * pj.w;
-    float fr = es6 * (12.0f * s6 - 6.0f) * ir2 + qq * (ir * ir2 - 2.0f * g.krff);
-    fr = ok ? fr : 0.0f;
-    // E = LJ + qq/r here; the reaction-field terms qq(k_rf r^2 - c_rf) are summed as
-    // sq*r^2 and sq and scaled by k_rf, c_rf in FP64 (their FP32 rounding would bias a
-    // sum over millions of pairs)
-    float ee = ok ? (es6 * (s6 - 1.0f) + qq * ir) : 0.0f;
-    float qqm = ok ? qq : 0.0f;
-    a.fx += fr * dx;
-    a.fy += fr * dy;
-    a.fz += fr * dz;
-    a.e += (double)ee;
-    a.sqr2 += qqm * r2;
-    a.sq += qqm;
-    a.cnt += ok ? 1 : 0;
-    return fr;
-}
-
-// One pair, branch free: the result is computed for every lane and cleared with a bit
-// mask outside the cutoff (a never-taken branch per pair would cost more and would keep
-// the scheduler from overlapping consecutive pairs).  Masked lanes may hold inf or NaN
-// before the mask (r = 0 for an unused slot); the AND yields +0.
-// ENERGY = false: forces only (the energy terms and their sums are left out).  GEO: the
-// geometric sigma rule, qi.x and qj.x holding sigma itself (Geom::geo)
-template <bool ENERGY = true, bool GEO = false>
-__device__ __forceinline__ float pair_masked(float4 pi, float2 qi, float4 pj, float2 qj,
-                                             bool incl, bool minimg, const Geom& g, PairAcc& a,
-                                             float& dx, float& dy, float& dz) {
-    dx = pi.x - pj.x;
-    dy = pi.y - pj.y;
-    dz = pi.z - pj.z;
-    if (minimg) {  // wave-uniform
-        dx -= g.bx * rintf(dx * g.ibx);
-        dy -= g.by * rintf(dy * g.iby);
-        dz -= g.bz * rintf(dz * g.ibz);
-    }
-    float r2 = dx * dx + dy * dy + dz * dz;
-    unsigned m = (incl && r2 < g.rc2f) ? 0xFFFFFFFFu : 0u;
-    float ir = __frsqrt_rn(r2);
-    float ir2 = ir * ir;
-    float s2;
-    if constexpr (GEO) {
-        s2 = (qi.x * qj.x) * ir2;
-    } else {
-        float sig = qi.x + qj.x;
-        s2 = sig * sig * ir2;
-    }
-    float s6 = s2 * s2 * s2;
-    float es6 = (qi.y * qj.y) * s6;
-    float qq = pi.w * pj.w;
-    float fr = es6 * (12.0f * s6 - 6.0f) * ir2 + qq * (ir * ir2 - 2.0f * g.krff);
-    fr = __uint_as_float(__float_as_uint(fr) & m);
-    a.fx += fr * dx;
-    a.fy += fr * dy;
-    a.fz += fr * dz;
-    a.cnt += (int)(m & 1u);
-    // pin the sums here: otherwise the compiler sinks every pair's accumulation to the
-    // end of the chunk and keeps all eight pairs' operands live (VGPR pressure)
-    if (ENERGY) {
-        float ee = es6 * (s6 - 1.0f) + qq * ir;
-        ee = __uint_as_float(__float_as_uint(ee) & m);
-        float qqm = __uint_as_float(__float_as_uint(qq) & m);
-        a.ef += ee;
-        a.sqr2 += qqm * r2;
-        a.sq += qqm;
-        asm volatile("" : "+v"(a.fx), "+v"(a.fy), "+v"(a.fz), "+v"(a.ef), "+v"(a.sqr2), "+v"(a.sq));
-    } else {
-        asm volatile("" : "+v"(a.fx), "+v"(a.fy), "+v"(a.fz));
-    }
-    return fr;
-}
 
 // a + b taken from the DPP partner lane.  bound_ctrl lets the mov fold into the add as
 // its DPP operand; contraction is off so the add is not fused with the product that
@@ -629,6 +554,13 @@ template <int CTRL>
 __device__ __forceinline__ float dpp_add(float a, float b) {
 #pragma clang fp contract(off)
     return a + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(b), CTRL, 0xf, 0xf, true));
+}
+
+// sum over the 8 lanes of each aligned group of 8, on every lane of the group
+__device__ __forceinline__ float sum8(float y) {
+    y = dpp_add<0xB1>(y, y);     // quad_perm [1,0,3,2] = lane ^ 1
+    y = dpp_add<0x4E>(y, y);     // quad_perm [2,3,0,1] = lane ^ 2
+    return dpp_add<0x141>(y, y); // row_half_mirror: lane i <- 7 - i within 8
 }
 
 // Maps workgroup ids so that consecutive (replica, block) work lands on one XCD:
@@ -646,47 +578,13 @@ __device__ __forceinline__ void wait_vmem() {
     __builtin_amdgcn_sched_barrier(0);
 }
 
-__device__ __forceinline__ int next_bit(unsigned long long& m) {
-    int j = m ? __ffsll((long long)m) - 1 : -1;
-    m &= m - 1ull;
-    return j;
-}
-
-// full evaluation: all j of one tile, four at a time so their scalar loads overlap
-template <bool MINIMG, bool EXCL>
-__device__ __forceinline__ void tile_full(const float4* __restrict__ P, const float2* __restrict__ Q,
-                                          int jbeg, unsigned long long am, float4 pi, float2 qi,
-                                          unsigned long long em, const Geom& g, PairAcc& a) {
-    float dx, dy, dz;
-    while (am) {
-        int j0 = next_bit(am), j1 = next_bit(am), j2 = next_bit(am), j3 = next_bit(am);
-        float4 p0 = P[jbeg + j0];
-        float2 q0 = Q[jbeg + j0];
-        float4 p1 = P[jbeg + max(j1, 0)];
-        float2 q1 = Q[jbeg + max(j1, 0)];
-        float4 p2 = P[jbeg + max(j2, 0)];
-        float2 q2 = Q[jbeg + max(j2, 0)];
-        float4 p3 = P[jbeg + max(j3, 0)];
-        float2 q3 = Q[jbeg + max(j3, 0)];
-        pair_one<MINIMG, EXCL>(pi, qi, p0, q0, !((em >> j0) & 1ull), g, a, dx, dy, dz);
-        if (j1 >= 0) pair_one<MINIMG, EXCL>(pi, qi, p1, q1, !((em >> j1) & 1ull), g, a, dx, dy, dz);
-        if (j2 >= 0) pair_one<MINIMG, EXCL>(pi, qi, p2, q2, !((em >> j2) & 1ull), g, a, dx, dy, dz);
-        if (j3 >= 0) pair_one<MINIMG, EXCL>(pi, qi, p3, q3, !((em >> j3) & 1ull), g, a, dx, dy, dz);
-    }
-}
-
-template <int CTRL>
-__device__ __forceinline__ float dpp_f(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
-}
-
-// Sum v[24] (8 j atoms x 3 components, index 3k+c) over the 64 lanes so that lanes
-// 8k..8k+7 end up holding the three components of j atom k.  Three halving stages split
-// the values between lane halves (bit 5: v_permlane32_swap, bit 4: v_permlane16_swap,
-// bit 3: DPP row_ror:8), then a DPP sum over the 8 lanes of each group.  The swaps
-// exchange the upper half of their first operand with the lower half of their second,
-// so r0 + r1 is the pairwise sum of the value each half keeps, with no selects.
-__device__ __forceinline__ void reduce_scatter24(const float (&v)[24], int lane, float (&out)[3]) {
+// Sums v[24] (8 i clusters x 3 components, index 3k+c) over the eight lanes with equal
+// lane & 7 so that lane 8k + il ends up holding the components of cluster k, atom il.
+// Three halving stages split the values between lane halves (bit 5: v_permlane32_swap,
+// bit 4: v_permlane16_swap, bit 3: DPP row_ror:8).  The swaps exchange the upper half of
+// their first operand with the lower half of their second, so r0 + r1 is the pairwise
+// sum of the value each half keeps, with no selects.
+__device__ __forceinline__ void scatter_clusters24(const float (&v)[24], int lane, float (&out)[3]) {
     float w[12], x[6];
 #pragma unroll
     for (int t = 0; t < 12; t++) {
@@ -700,257 +598,76 @@ __device__ __forceinline__ void reduce_scatter24(const float (&v)[24], int lane,
                                                    false, false);
         x[t] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
     }
-    bool b3 = (lane & 8) != 0;
+    const bool b3 = (lane & 8) != 0;
 #pragma unroll
     for (int t = 0; t < 3; t++) {
         float keep = b3 ? x[t + 3] : x[t];
         float send = b3 ? x[t] : x[t + 3];
-        float y = dpp_add<0x128>(keep, send);  // row_ror:8 = lane ^ 8 within 16
-        y = dpp_add<0xB1>(y, y);               // quad_perm [1,0,3,2] = lane ^ 1
-        y = dpp_add<0x4E>(y, y);               // quad_perm [2,3,0,1] = lane ^ 2
-        out[t] = dpp_add<0x141>(y, y);         // row_half_mirror: lane i <- 7 - i within 8
+        out[t] = dpp_add<0x128>(keep, send);  // row_ror:8 = lane ^ 8 within 16
     }
 }
 
-// Sum v[12] (4 j atoms x 3 components, index 3k+c) over the 64 lanes so that lanes
-// 16k..16k+15 end up holding the three components of j atom k: two halving stages
-// (v_permlane32_swap on lane bit 5, v_permlane16_swap on bit 4), then DPP sums over the
-// 16 lanes of each row (row_ror:8, the two quad swaps, row_half_mirror).
-__device__ __forceinline__ void reduce_scatter12(const float (&v)[12], float (&out)[3]) {
-    float w[6];
-#pragma unroll
-    for (int t = 0; t < 6; t++) {
-        auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[t]), __float_as_uint(v[t + 6]),
-                                                   false, false);
-        w[t] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+// pairs per FP32 partial sum of the i forces: about 16 terms per lane and i atom, as
+// many as the eight lanes that share it then add
+constexpr int PAIRS_PER_FLUSH = 8192;
+
+// j atoms of block jb that i atom `lane` must not be paired with in this tile: exclusion
+// partners, in the diagonal tile the atoms up to itself, slots past N; everything for a
+// lane without an atom
+__device__ __forceinline__ unsigned long long tile_exclusions(unsigned long long set,
+                                                              int max_ex,
+                                                              const int* __restrict__ exs,
+                                                              int lane, bool vi, int ib, int jb,
+                                                              int N) {
+    unsigned long long em = 0;
+    if ((set >> (jb & 63)) & 1ull) {
+        for (int k = 0; k < max_ex; k++) {
+            int sl = exs[k * 64 + lane];
+            if ((sl >> 6) == jb) em |= 1ull << (sl & 63);  // -1 (none) is in no block
+        }
     }
-#pragma unroll
-    for (int t = 0; t < 3; t++) {
-        auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(w[t]), __float_as_uint(w[t + 3]),
-                                                   false, false);
-        float y = __uint_as_float(r[0]) + __uint_as_float(r[1]);
-        y = dpp_add<0x128>(y, y);      // row_ror:8 = lane ^ 8 within 16
-        y = dpp_add<0xB1>(y, y);       // quad_perm [1,0,3,2] = lane ^ 1
-        y = dpp_add<0x4E>(y, y);       // quad_perm [2,3,0,1] = lane ^ 2
-        out[t] = dpp_add<0x141>(y, y); // row_half_mirror: lane i <- 7 - i within 8
-    }
+    if (jb == ib) em |= (2ull << lane) - 1ull;
+    if (jb * 64 + 64 > N) em |= ~0ull << (N - jb * 64);  // uniform; N > jb * 64
+    return vi ? em : ~0ull;
 }
 
-// The same for v[6] (2 j atoms): lanes 32k..32k+31 end up holding j atom k.  Each sum
-// pairs lanes in the same order as reduce_scatter24 and reduce_scatter12 (lane ^ 32,
-// ^ 16, ^ 8, ^ 1, ^ 2, half mirror), so a j atom's sum does not depend on the width of
-// the chunk it was taken in.
-__device__ __forceinline__ void reduce_scatter6(const float (&v)[6], float (&out)[3]) {
-#pragma unroll
-    for (int t = 0; t < 3; t++) {
-        auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[t]), __float_as_uint(v[t + 3]),
-                                                   false, false);
-        float w = __uint_as_float(r[0]) + __uint_as_float(r[1]);
-        auto q = __builtin_amdgcn_permlane16_swap(__float_as_uint(w), __float_as_uint(w), false,
-                                                   false);
-        float y = __uint_as_float(q[0]) + __uint_as_float(q[1]);
-        y = dpp_add<0x128>(y, y);      // row_ror:8 = lane ^ 8 within 16
-        y = dpp_add<0xB1>(y, y);       // quad_perm [1,0,3,2] = lane ^ 1
-        y = dpp_add<0x4E>(y, y);       // quad_perm [2,3,0,1] = lane ^ 2
-        out[t] = dpp_add<0x141>(y, y); // row_half_mirror: lane i <- 7 - i within 8
-    }
+// the periodic shift of a whole tile (boxes of the two blocks): (kx, ky, kz) box lengths;
+// returns whether it is exact for every pair within the list radius (Geom::oix)
+__device__ __forceinline__ bool tile_shift(float4 bli, float4 bhi, float4 blj, float4 bhj,
+                                           const Geom& g, float& kx, float& ky, float& kz) {
+    float dcx = 0.5f * (bli.x + bhi.x - blj.x - bhj.x);
+    float dcy = 0.5f * (bli.y + bhi.y - blj.y - bhj.y);
+    float dcz = 0.5f * (bli.z + bhi.z - blj.z - bhj.z);
+    kx = rintf(dcx * g.ibx);
+    ky = rintf(dcy * g.iby);
+    kz = rintf(dcz * g.ibz);
+    return fabsf(dcx - g.bx * kx) + 0.5f * (bhi.x - bli.x + bhj.x - blj.x) < g.oix &&
+           fabsf(dcy - g.by * ky) + 0.5f * (bhi.y - bli.y + bhj.y - blj.y) < g.oiy &&
+           fabsf(dcz - g.bz * kz) + 0.5f * (bhi.z - bli.z + bhj.z - blj.z) < g.oiz;
 }
 
-// Newton-3 evaluation of one tile: j atoms in groups of 8; their forces are scattered
-// to the slot-ordered fixed-point accumulator F (3 planes of Np).  Slots past the last j
-// atom re-read the first one and are masked off.
-template <bool MINIMG, bool EXCL>
-__device__ __forceinline__ void tile_newton(const float4* __restrict__ P, const float2* __restrict__ Q,
-                                            int jbeg, unsigned long long am, float4 pi, float2 qi,
-                                            bool vi, unsigned long long em, const Geom& g,
-                                            PairAcc& a, unsigned long long* __restrict__ Fr,
-                                            int Np, int lane, int& bad) {
-    while (am) {
-        int jj[8];
-#pragma unroll
-        for (int k = 0; k < 8; k++) jj[k] = next_bit(am);
-        float v[24];
-#pragma unroll
-        for (int k = 0; k < 8; k++) {
-            int j = jj[k] < 0 ? jj[0] : jj[k];
-            float4 pj = P[jbeg + j];
-            float2 qj = Q[jbeg + j];
-            bool incl = vi && jj[k] >= 0;
-            if (EXCL) incl = incl && !((em >> j) & 1ull);
-            float dx, dy, dz;
-            float fr = pair_masked(pi, qi, pj, qj, incl, MINIMG, g, a, dx, dy, dz);
-            v[3 * k] = -fr * dx;
-            v[3 * k + 1] = -fr * dy;
-            v[3 * k + 2] = -fr * dz;
-        }
-        float f[3];
-        reduce_scatter24(v, lane, f);
-        a.e += (double)a.ef;  // FP32 over 8 pairs, FP64 beyond
-        a.ef = 0.f;
-        int k = lane >> 3;
-        int mine = jj[0];
-#pragma unroll
-        for (int q = 1; q < 8; q++) mine = (k == q) ? jj[q] : mine;
-        if ((lane & 7) == 0 && mine >= 0) {
-            int s = jbeg + mine;
-            atomicAdd(&Fr[s], fixed_from_float(f[0], &bad));
-            atomicAdd(&Fr[Np + s], fixed_from_float(f[1], &bad));
-            atomicAdd(&Fr[2 * Np + s], fixed_from_float(f[2], &bad));
-        }
-    }
-}
-
-template <int WPW, bool COUNT, bool NEWTON>
-__global__ __launch_bounds__(64 * WPW) void k_pair(
-    int R, int N, int Np, int NB, int maxj, const float4* __restrict__ posq_s,
-    const float2* __restrict__ par_s, const int* __restrict__ orig_s,
-    const int* __restrict__ slot_of, const int* __restrict__ tiles,
-    const unsigned long long* __restrict__ tmask, const int* __restrict__ ntiles,
-    const float4* __restrict__ bb_lo, const float4* __restrict__ bb_hi,
-    const int* __restrict__ ex_start, const int* __restrict__ ex_list, int max_ex,
-    long long* __restrict__ F, double* __restrict__ e_pair, int* __restrict__ flags,
-    unsigned long long* __restrict__ pair_count, Geom g) {
-    extern __shared__ int exs_lds_dyn[];  // [WPW][max_ex][64] exclusion partners' slots
-    // wave-uniform by construction; readfirstlane lets the compiler keep everything
-    // derived from it (replica, block, tile, j index) in scalar registers
-    int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    int w = xcd_linear_id(blockIdx.x, gridDim.x) * WPW + wv;
-    int lane = threadIdx.x & 63;
-    if (w >= R * NB) return;
-    int r = w / NB;
-    int ib = w - r * NB;
-    const float4* P = posq_s + (size_t)r * Np;
-    const float2* Q = par_s + (size_t)r * Np;
-    unsigned long long* Fr = (unsigned long long*)(F + (size_t)r * 3 * Np);
-    int islot = ib * 64 + lane;
-    bool vi = islot < N;
-    float4 pi = P[islot];
-    float2 qi = Q[islot];
-    int nex = 0;
-    if (vi) {
-        int ai = orig_s[(size_t)r * Np + islot];
-        int b0 = ex_start[ai];
-        nex = ex_start[ai + 1] - b0;
-        for (int k = 0; k < nex; k++)
-            exs_lds_dyn[(wv * max_ex + k) * 64 + lane] = slot_of[(size_t)r * Np + ex_list[b0 + k]];
-    }
-    float4 bli = bb_lo[(size_t)r * NB + ib], bhi = bb_hi[(size_t)r * NB + ib];
-    double ax = 0.0, ay = 0.0, az = 0.0, aqr2 = 0.0, aq = 0.0;
-    PairAcc acc;
-    acc.e = 0.0;
-    acc.ef = 0.f;
-    acc.cnt = 0;
-    int bad = 0;
-    const int* tl = tiles + ((size_t)r * NB + ib) * maxj;
-    const unsigned long long* tm = tmask + ((size_t)r * NB + ib) * maxj;
-    int nt = ntiles[(size_t)r * NB + ib];
-    for (int t = 0; t < nt; t++) {
-        int jb = tl[t];
-        unsigned long long am = tm[t];
-        unsigned long long em = 0;
-        for (int k = 0; k < nex; k++) {
-            int sl = exs_lds_dyn[(wv * max_ex + k) * 64 + lane];
-            if ((sl >> 6) == jb) em |= 1ull << (sl & 63);
-        }
-        if (jb == ib) em |= NEWTON ? ((2ull << lane) - 1ull) : (1ull << lane);
-        // one periodic shift for the whole tile when it is exact for every pair within
-        // the list radius (Geom::oix); otherwise the minimum image per pair
-        float4 blj = bb_lo[(size_t)r * NB + jb], bhj = bb_hi[(size_t)r * NB + jb];
-        float dcx = 0.5f * (bli.x + bhi.x - blj.x - bhj.x);
-        float dcy = 0.5f * (bli.y + bhi.y - blj.y - bhj.y);
-        float dcz = 0.5f * (bli.z + bhi.z - blj.z - bhj.z);
-        float sx = g.bx * rintf(dcx * g.ibx), sy = g.by * rintf(dcy * g.iby),
-              sz = g.bz * rintf(dcz * g.ibz);
-        bool one_image =
-            fabsf(dcx - sx) + 0.5f * (bhi.x - bli.x + bhj.x - blj.x) < g.oix &&
-            fabsf(dcy - sy) + 0.5f * (bhi.y - bli.y + bhj.y - blj.y) < g.oiy &&
-            fabsf(dcz - sz) + 0.5f * (bhi.z - bli.z + bhj.z - blj.z) < g.oiz;
-        float4 ps = pi;
-        if (one_image) {
-            ps.x -= sx;
-            ps.y -= sy;
-            ps.z -= sz;
-        }
-        acc.fx = acc.fy = acc.fz = acc.sqr2 = acc.sq = 0.f;
-        bool ex = __ballot(em != 0ull) != 0ull;
-        int jbeg = jb * 64;
-        if (NEWTON) {
-            if (one_image) {
-                if (ex) tile_newton<false, true>(P, Q, jbeg, am, ps, qi, vi, em, g, acc, Fr, Np, lane, bad);
-                else tile_newton<false, false>(P, Q, jbeg, am, ps, qi, vi, em, g, acc, Fr, Np, lane, bad);
-            } else {
-                if (ex) tile_newton<true, true>(P, Q, jbeg, am, ps, qi, vi, em, g, acc, Fr, Np, lane, bad);
-                else tile_newton<true, false>(P, Q, jbeg, am, ps, qi, vi, em, g, acc, Fr, Np, lane, bad);
-            }
-        } else {
-            if (one_image) {
-                if (ex) tile_full<false, true>(P, Q, jbeg, am, ps, qi, em, g, acc);
-                else tile_full<false, false>(P, Q, jbeg, am, ps, qi, em, g, acc);
-            } else {
-                if (ex) tile_full<true, true>(P, Q, jbeg, am, ps, qi, em, g, acc);
-                else tile_full<true, false>(P, Q, jbeg, am, ps, qi, em, g, acc);
-            }
-        }
-        ax += (double)acc.fx;
-        ay += (double)acc.fy;
-        az += (double)acc.fz;
-        aqr2 += (double)acc.sqr2;
-        aq += (double)acc.sq;
-    }
-    if (COUNT) {
-        double c = wave_sum(vi ? (double)acc.cnt : 0.0);
-        if (lane == 0) atomicAdd(&pair_count[r], (unsigned long long)(c + 0.5));
-        return;
-    }
-    if (vi) {  // atomic in both modes: the bonded kernel may run concurrently
-        long long fx = to_fixed(ax, &bad), fy = to_fixed(ay, &bad), fz = to_fixed(az, &bad);
-        atomicAdd(&Fr[islot], (unsigned long long)fx);
-        atomicAdd(&Fr[Np + islot], (unsigned long long)fy);
-        atomicAdd(&Fr[2 * Np + islot], (unsigned long long)fz);
-    }
-    double es = wave_sum(vi ? (acc.e + g.krf * aqr2 - g.crf * aq) : 0.0);
-    if (__ballot(bad) != 0ull && lane == 0) atomicOr(&flags[r], 2);
-    if (lane == 0) e_pair[(size_t)r * NB + ib] = NEWTON ? es : 0.5 * es;
-}
-
-// ---------------------------------------------------------------------------
-// Block kernel, Newton-3, with LDS-staged j tiles.  Same work split as k_pair<.., true>
-// (one wave per i-block, half tile list, j wave-uniform; or `split` waves per i-block,
-// each taking every split-th tile, with their own i-force atomics and energy slot, for
-// batches too small to fill the GPU with one wave per block), but the 64 slot records of
-// each j-block are copied global -> LDS by DMA one tile ahead (no registers, no scalar
-// loads in the pair loop), and the j forces of a tile are kept in LDS (each j atom's
-// sum at its rank in the tile's mask: every j atom falls in exactly one chunk) and
-// added to the global accumulator once per tile with coalesced atomics.
-//   LDS per wave: two 2 KB tile buffers (separate objects, so reading one never waits
-//   for the copy into the other), 768 B of j-force sums, max_ex*256 B of exclusions.
+//   LDS per wave: two 2 KB tile buffers, 512 B of exclusion masks.
 //   vmcnt discipline: the only vector memory operations inside the tile loop are the
-//   next tile's copy and the three flush atomics that end each tile.  Loads and
-//   stores/atomics share vmcnt but need not retire in issue order, so the copy is
-//   waited for with vmcnt(0) before the atomics, not with vmcnt(3) after them.
-//   ENERGY = false: forces only; e_pair is not written.
-// ---------------------------------------------------------------------------
-
-// At least 5 waves per SIMD (at most 96 VGPRs, allocated in granules of 8): the energy
-// variant otherwise takes 97, which leaves room for 4.  The forces-only variant takes
-// 84; held to 80 for 6 waves it spills 24 bytes per lane and runs 3.3% slower.
-template <int WPW, bool COUNT, bool ENERGY, bool GEO = false>
-__global__ __launch_bounds__(64 * WPW) __attribute__((amdgpu_waves_per_eu(5))) void k_pair_n3(
+//   next tile's copy (global -> LDS by DMA), the exclusion loads of the few tiles that have
+//   any, and the three flush atomics that end each tile.  Loads and stores/atomics share
+//   vmcnt but need not retire in issue order, so the copy is waited for with vmcnt(0) before
+//   the atomics, not with vmcnt(3) after them.
+//   GEO: the geometric LJ sigma rule, the records holding sigma itself (Geom::geo).
+template <int WPW, bool COUNT, bool GEO>
+__global__ __launch_bounds__(64 * WPW) __attribute__((amdgpu_waves_per_eu(4))) void k_pair(
     int R, int N, int Np, int NB, int maxj, int split, const float4* __restrict__ arec,
-    const int* __restrict__ orig_s, const int* __restrict__ slot_of, const int* __restrict__ tiles,
-    const unsigned long long* __restrict__ tmask, const int* __restrict__ ntiles,
-    const float4* __restrict__ bb_lo, const float4* __restrict__ bb_hi,
-    const int* __restrict__ ex_start, const int* __restrict__ ex_list, int max_ex,
-    long long* __restrict__ F, double* __restrict__ e_pair, int* __restrict__ flags,
-    unsigned long long* __restrict__ pair_count, Geom g) {
-    // two tile buffers of 64 slot records (2 float4 each) plus 8 zero records: a chunk's
-    // entries past the tile's mask read there or the tile's own finite records
-    __shared__ float4 tile_a[WPW][144], tile_b[WPW][144];
-    __shared__ float facc[WPW][3][64];
-    extern __shared__ int exs_dyn[];
+    const double4* __restrict__ bref, const int* __restrict__ tiles, const unsigned long long* __restrict__ tmask,
+    const int* __restrict__ ntiles, const float4* __restrict__ bb_lo,
+    const float4* __restrict__ bb_hi, const int* __restrict__ exs,
+    const unsigned long long* __restrict__ exblocks, int max_ex, long long* __restrict__ F,
+    int* __restrict__ flags, unsigned long long* __restrict__ pair_count, Geom g) {
+    __shared__ float4 tile_s[WPW][2][128];
+    __shared__ unsigned long long em_s[WPW][64];
+    // wave-uniform by construction; readfirstlane lets the compiler keep everything
+    // derived from it (replica, block, tile, mask) in scalar registers
     int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     int w = xcd_linear_id(blockIdx.x, gridDim.x) * WPW + wv;
-    int lane = threadIdx.x & 63;
+    const int lane = threadIdx.x & 63;
     if (w >= R * NB * split) return;
     // split waves per (replica, i-block), wave `part` taking tiles part, part + split, ..
     const int part = w % split;
@@ -959,55 +676,18 @@ __global__ __launch_bounds__(64 * WPW) __attribute__((amdgpu_waves_per_eu(5))) v
     int ib = rb - r * NB;
     const float4* A = arec + (size_t)r * Np * 2;
     unsigned long long* Fr = (unsigned long long*)(F + (size_t)r * 3 * Np);
-    int* exs = exs_dyn + wv * max_ex * 64;
-    int islot = ib * 64 + lane;
-    bool vi = islot < N;
-    float4 pi = A[2 * islot];
-    float4 qi4 = A[2 * islot + 1];
-    float2 qi = make_float2(qi4.x, qi4.y);
-    int nex = 0;
-    // the range of j-blocks that hold an exclusion partner of one of the wave's i atoms
-    // (bonded partners are close: mostly this block and its neighbours); tiles outside
-    // it skip the exclusion test (wave-uniform)
-    int exlo = NB, exhi = -1;
-    if (vi) {
-        int ai = orig_s[(size_t)r * Np + islot];
-        int b0 = ex_start[ai];
-        nex = ex_start[ai + 1] - b0;
-        for (int k = 0; k < nex; k++) {
-            const int sl = slot_of[(size_t)r * Np + ex_list[b0 + k]];
-            exs[k * 64 + lane] = sl;
-            exlo = min(exlo, sl >> 6);
-            exhi = max(exhi, sl >> 6);
-        }
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        exlo = min(exlo, __shfl_xor(exlo, o, 64));
-        exhi = max(exhi, __shfl_xor(exhi, o, 64));
-    }
-    exlo = __builtin_amdgcn_readfirstlane(exlo);
-    exhi = __builtin_amdgcn_readfirstlane(exhi);
-    float4 bli = bb_lo[(size_t)r * NB + ib], bhi = bb_hi[(size_t)r * NB + ib];
-    if (lane < 16) {
-        tile_a[wv][128 + lane] = make_float4(0.f, 0.f, 0.f, 0.f);
-        tile_b[wv][128 + lane] = make_float4(0.f, 0.f, 0.f, 0.f);
-    }
-    double ax = 0.0, ay = 0.0, az = 0.0, aqr2 = 0.0, aq = 0.0;
-    PairAcc acc;
-    acc.e = 0.0;
-    acc.ef = 0.f;
-    acc.cnt = 0;
-    int bad = 0;
-    const int* tl = tiles + ((size_t)r * NB + ib) * maxj;
-    const unsigned long long* tmk = tmask + ((size_t)r * NB + ib) * maxj;
-    int nt = ntiles[(size_t)r * NB + ib];
+    const int islot = ib * 64 + lane;
+    const bool vi = islot < N;
+    const int il = lane & 7, jl = lane >> 3;
+    const int* tl = tiles + (size_t)rb * maxj;
+    const unsigned long long* tmk = tmask + (size_t)rb * maxj;
+    const float4* lo = bb_lo + (size_t)r * NB;
+    const float4* hi = bb_hi + (size_t)r * NB;
 
-    // copies the 64 slot records (32 B) of j-block jb into tile buffer B: lane L moves
+    // copies the 64 slot records (32 B) of j-block jb into tile buffer b: lane L moves
     // half L&1 of record L>>1 (first instruction) and of record 32 + (L>>1) (second)
-    auto stage = [&](int jb, auto bufc) {
-        constexpr int B = decltype(bufc)::value;
-        float4* dst = B ? tile_b[wv] : tile_a[wv];
+    auto stage = [&](int jb, int b) {
+        float4* dst = tile_s[wv][b];
         const char* src = (const char*)(A + 2 * jb * 64) + lane * 16;
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_global_load_lds((const void*)src,
@@ -1016,666 +696,225 @@ __global__ __launch_bounds__(64 * WPW) __attribute__((amdgpu_waves_per_eu(5))) v
                                          (__attribute__((address_space(3))) void*)(dst + 64), 16, 0, 0);
         __builtin_amdgcn_wave_barrier();
     };
-
-    auto do_tile = [&](int t, auto bufc) {
-        constexpr int B = decltype(bufc)::value;
-        const float4* buf = B ? tile_b[wv] : tile_a[wv];
-        int jb = tl[t];
-        unsigned long long am = tmk[t];
-        const unsigned long long am0 = am;
-        if (t + split < nt) stage(tl[t + split], std::integral_constant<int, 1 - B>());
-        unsigned long long em = 0;
-        if (jb >= exlo && jb <= exhi) {
-            for (int k = 0; k < nex; k++) {
-                int sl = exs[k * 64 + lane];
-                if ((sl >> 6) == jb) em |= 1ull << (sl & 63);
-            }
+    // the wave's next 64 tiles, one per lane, so that no tile waits for its descriptor:
+    // j-block (TILE_MI set where every pair needs its own minimum image), mask, and the
+    // offset (hx, hy, hz) from the i-block's reference to the j-block's, in the periodic
+    // image that the tile's pairs take: x_i - x_j = rel_i - (rel_j + h)
+    constexpr int TILE_MI = 1 << 30;
+    int tj = 0;
+    float hx = 0.f, hy = 0.f, hz = 0.f;
+    unsigned long long tm = 0ull;
+    const int nt = ntiles[rb];
+    if (part >= nt) return;
+    auto load_tiles = [&](int t0) {
+        const int tq = t0 + lane * split;
+        if (tq < nt) {
+            tj = tl[tq];
+            tm = tmk[tq];
         }
-        if (jb == ib) em |= (2ull << lane) - 1ull;
-        // one periodic shift for the whole tile when it is exact for every pair within
-        // the list radius (Geom::oix); otherwise the minimum image per pair
-        float4 blj = bb_lo[(size_t)r * NB + jb], bhj = bb_hi[(size_t)r * NB + jb];
-        float dcx = 0.5f * (bli.x + bhi.x - blj.x - bhj.x);
-        float dcy = 0.5f * (bli.y + bhi.y - blj.y - bhj.y);
-        float dcz = 0.5f * (bli.z + bhi.z - blj.z - bhj.z);
-        float sx = g.bx * rintf(dcx * g.ibx), sy = g.by * rintf(dcy * g.iby),
-              sz = g.bz * rintf(dcz * g.ibz);
-        bool one_image =
-            fabsf(dcx - sx) + 0.5f * (bhi.x - bli.x + bhj.x - blj.x) < g.oix &&
-            fabsf(dcy - sy) + 0.5f * (bhi.y - bli.y + bhj.y - blj.y) < g.oiy &&
-            fabsf(dcz - sz) + 0.5f * (bhi.z - bli.z + bhj.z - blj.z) < g.oiz;
-        float4 ps = pi;
-        if (one_image) {
-            ps.x -= sx;
-            ps.y -= sy;
-            ps.z -= sz;
-        }
-        const bool ex = __ballot(em != 0ull) != 0ull;
-        // the mask's records to the front of the buffer in mask order (entry e = the e-th
-        // set bit), so that a chunk reads its W records at fixed offsets from one address.
-        // Every lane reads its own record before any lane writes (one wave: its LDS
-        // accesses are carried out in order); the records past the mask stay finite.
-        {
-            float4* bw = B ? tile_b[wv] : tile_a[wv];
-            const float4 r0 = bw[2 * lane], r1 = bw[2 * lane + 1];
-            if ((am0 >> lane) & 1ull) {
-                const int rank = lane_rank(am0);
-                bw[2 * rank] = r0;
-                bw[2 * rank + 1] = r1;
-            }
-        }
-        acc.fx = acc.fy = acc.fz = acc.sqr2 = acc.sq = 0.f;
-        // all j atoms of the tile, 8 at a time; MI: per-pair minimum image, EX: the tile
-        // holds excluded pairs (both wave-uniform, compile-time inside the loop).  ent:
-        // entries (j atoms in mask order) taken so far, nvalid: entries of this chunk.
-        int ent = 0, nvalid = 0;
-        auto chunks = [&](auto mic, auto exc) {
-            constexpr bool MI = decltype(mic)::value, EX = decltype(exc)::value;
-            // the next W j atoms of the tile, W = 8, 4 or 2: a chunk costs about 310, 166
-            // and 100 VALU instructions, so the tail of a tile is taken in narrower ones
-            auto chunk = [&](auto wc) {
-                constexpr int W = decltype(wc)::value;
-                constexpr int SH = W == 8 ? 3 : W == 4 ? 4 : 5;  // lanes per j atom: 1 << SH
-                int jj[W];
+    };
+    load_tiles(part);
+    float xi[8], yi[8], zi[8], qi[8], si[8], ei[8], fi[24];
 #pragma unroll
-                for (int k = 0; k < W; k++) jj[k] = next_bit(am);
-                float v[3 * W];
-                const float4* cb = buf + 2 * ent;  // the chunk's records, in entry order
+    for (int k = 0; k < 8; k++) {
+        const float4 a = A[2 * (ib * 64 + 8 * k + il)];
+        const float2 b = *(const float2*)&A[2 * (ib * 64 + 8 * k + il) + 1];
+        xi[k] = a.x;
+        yi[k] = a.y;
+        zi[k] = a.z;
+        qi[k] = a.w;
+        si[k] = b.x;
+        ei[k] = b.y;
+        fi[3 * k] = fi[3 * k + 1] = fi[3 * k + 2] = 0.f;
+    }
+    const float4 bli = lo[ib], bhi = hi[ib];
+    const int* E = exs + (size_t)rb * max_ex * 64;
+    const unsigned long long eset = exblocks[rb];
+    const double4 ri = bref[rb];
+    auto load_shifts = [&](int t0) {
+        if (t0 + lane * split < nt) {
+            float kx, ky, kz;
+            const bool one = tile_shift(bli, bhi, lo[tj], hi[tj], g, kx, ky, kz);
+            const double4 rj = bref[(size_t)r * NB + tj];
+            hx = (float)((rj.x - ri.x) + quantize(g.Lx) * (double)kx);
+            hy = (float)((rj.y - ri.y) + quantize(g.Ly) * (double)ky);
+            hz = (float)((rj.z - ri.z) + quantize(g.Lz) * (double)kz);
+            if (!one) tj |= TILE_MI;
+        }
+    };
+    stage(__builtin_amdgcn_readfirstlane(tj), 0);
+    load_shifts(part);
+    int bad = 0;
+    // adds the i forces of the pairs so far to the accumulator: lane = i atom (atomic: other
+    // waves and the side kernels add to the same accumulator)
+    auto flush_i = [&]() {
+        float f[3];
+        scatter_clusters24(fi, lane, f);
+        if (vi) {
+            atomicAdd(&Fr[islot], fixed_from_float(f[0], &bad));
+            atomicAdd(&Fr[Np + islot], fixed_from_float(f[1], &bad));
+            atomicAdd(&Fr[2 * Np + islot], fixed_from_float(f[2], &bad));
+        }
 #pragma unroll
-                for (int k = 0; k < W; k++) {
-                    float4 pj = cb[2 * k];
-                    float2 qj = *(const float2*)&cb[2 * k + 1];
-                    bool incl = vi && k < nvalid;
-                    if (EX) incl = incl && !((em >> (jj[k] & 63)) & 1ull);
-                    float dx, dy, dz;
-                    float fr =
-                        pair_masked<ENERGY, GEO>(ps, qi, pj, qj, incl, MI, g, acc, dx, dy, dz);
-                    v[3 * k] = -fr * dx;
-                    v[3 * k + 1] = -fr * dy;
-                    v[3 * k + 2] = -fr * dz;
-                }
-                float f[3];
-                if constexpr (W == 8) reduce_scatter24(v, lane, f);
-                else if constexpr (W == 4) reduce_scatter12(v, f);
-                else reduce_scatter6(v, f);
-                if (ENERGY) {
-                    acc.e += (double)acc.ef;  // FP32 over W pairs, FP64 beyond
-                    acc.ef = 0.f;
-                }
-                // Lanes (lane >> SH) << SH hold the sum of entry ent + (lane >> SH): every
-                // j atom of the tile is one entry of one chunk, taken in mask order, so
-                // its sum is written (not added) at its rank in the tile's mask.  Written
-                // out because the compiler would otherwise put an s_waitcnt vmcnt(0) (a
-                // wait for the tile copy in flight) in front of any LDS access it cannot
-                // separate from that copy.
-                const int kq = lane >> SH;
-                if ((lane & ((1 << SH) - 1)) == 0 && kq < nvalid) {
-                    unsigned addr = (unsigned)(size_t)&facc[wv][0][ent + kq];
-                    asm volatile(
-                        "ds_write_b32 %0, %1\n\t"
-                        "ds_write_b32 %0, %2 offset:256\n\t"
-                        "ds_write_b32 %0, %3 offset:512"
-                        :
-                        : "v"(addr), "v"(f[0]), "v"(f[1]), "v"(f[2])
-                        : "memory");
-                }
-            };
-            while (am) {
-                const int n = __popcll(am);
-                if (n >= 7) {
-                    nvalid = min(n, 8);
-                    chunk(std::integral_constant<int, 8>());
-                } else if (n >= 3) {
-                    nvalid = min(n, 4);
-                    chunk(std::integral_constant<int, 4>());
-                } else {
-                    nvalid = n;
-                    chunk(std::integral_constant<int, 2>());
-                }
-                ent += nvalid;
+        for (int k = 0; k < 24; k++) fi[k] = 0.f;
+    };
+    int npair = 0, buf = 0;
+    // lane that holds the sum of j atom `lane` of a tile (cluster lane >> 3 in lanes with
+    // il = that cluster), as a byte address for ds_bpermute
+    const int transpose = 4 * ((lane >> 3) + 8 * (lane & 7));
+    const unsigned rec_lds = (unsigned)(size_t)&tile_s[wv][0][2 * jl];
+    wait_vmem();  // the first tile and the i atoms have arrived
+    for (int t = part, q = 0; t < nt; t += split, q++, buf ^= 1) {
+        const int ql = q & 63;
+        const int jt = __builtin_amdgcn_readlane(tj, ql), jb = jt & ~TILE_MI;
+        const unsigned long long m =
+            (unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(unsigned)tm, ql) |
+            (unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(unsigned)(tm >> 32), ql) << 32;
+        const float sx = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(hx), ql));
+        const float sy = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(hy), ql));
+        const float sz = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(hz), ql));
+        if (t + split < nt) {
+            if (ql == 63) {
+                load_tiles(t + split);
+                load_shifts(t + split);
             }
-        };
-        using T = std::true_type;
-        using Fa = std::false_type;
-        if (one_image) {
-            if (ex) chunks(Fa(), T());
-            else chunks(Fa(), Fa());
-        } else {
-            if (ex) chunks(T(), T());
-            else chunks(T(), Fa());
+            stage(__builtin_amdgcn_readlane(tj, (q + 1) & 63) & ~TILE_MI, buf ^ 1);
         }
-        ax += (double)acc.fx;
-        ay += (double)acc.fy;
-        az += (double)acc.fz;
-        if (ENERGY) {
-            aqr2 += (double)acc.sqr2;
-            aq += (double)acc.sq;
+        if (!COUNT && npair >= PAIRS_PER_FLUSH) {
+            flush_i();
+            npair = 0;
         }
-        // flush the tile's j forces: lane = j atom, which reads its sum at its rank in
-        // the mask (bits of am0 below the lane), coalesced fixed-point atomics
-        float fjx, fjy, fjz;
-        {
-            const int rank = __builtin_amdgcn_mbcnt_hi(
-                (unsigned)(am0 >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)am0, 0u));
-            unsigned addr = (unsigned)(size_t)&facc[wv][0][rank];
-            // early-clobber outputs: the first load's result lands while the other two
-            // still read the address, so no output may share the address register
-            asm volatile(
-                "ds_read_b32 %0, %3\n\t"
-                "ds_read_b32 %1, %3 offset:256\n\t"
-                "ds_read_b32 %2, %3 offset:512\n\t"
-                "s_waitcnt lgkmcnt(0)"
-                : "=&v"(fjx), "=&v"(fjy), "=&v"(fjz)
-                : "v"(addr)
-                : "memory");
+        // pairs of the tile that need more than the offset (uniform): their own minimum
+        // image, or a look at the exclusions and empty slots
+        const bool mi = (jt & TILE_MI) != 0;
+        bool ex = jb == ib || ((eset >> (jb & 63)) & 1ull) || ib * 64 + 64 > N || jb * 64 + 64 > N;
+        if (ex) {
+            const unsigned long long em = tile_exclusions(eset, max_ex, E, lane, vi, ib, jb, N);
+            ex = __ballot(em != 0ull) != 0ull;
+            em_s[wv][lane] = em;
         }
+        const int general = __builtin_amdgcn_readfirstlane(mi || ex ? 1 : 0);
+        float fjx = 0.f, fjy = 0.f, fjz = 0.f;  // sum of cluster il, atom jl
+        unsigned long long rest = m, done = 0ull;
+        do {
+            const int jc8 = __builtin_ctzll(rest) & 56;  // 8 jc
+            const unsigned ics = (unsigned)(m >> jc8) & 0xffu;
+            rest &= ~(0xffull << jc8);
+            // the cluster's records.  Written out because the compiler would otherwise put an
+            // s_waitcnt vmcnt(0) (a wait for the next tile's copy, which goes to the other
+            // half of the same array) in front of the reads.
+            float4 pj;
+            float2 pq;
+            {
+                const unsigned addr = rec_lds + (unsigned)(buf * 2048 + jc8 * 32);
+                asm volatile(
+                    "ds_read_b128 %0, %2\n\t"
+                    "ds_read_b64 %1, %2 offset:16\n\t"
+                    "s_waitcnt lgkmcnt(0)"
+                    : "=&v"(pj), "=&v"(pq)
+                    : "v"(addr)
+                    : "memory");
+            }
+            const float xj = pj.x + sx, yj = pj.y + sy, zj = pj.z + sz;
+            float fx = 0.f, fy = 0.f, fz = 0.f;
+            // opaque to the compiler, which would otherwise carry the zeros through the
+            // branches below as constants and copy the registers at the joins
+            asm volatile("" : "+v"(fx), "+v"(fy), "+v"(fz));
+            const int before = npair;
+#pragma unroll
+            for (int k = 0; k < 8; k++) {
+                if (!(ics & (1u << k))) continue;  // uniform
+                float dx = xi[k] - xj, dy = yi[k] - yj, dz = zi[k] - zj;
+                float r2 = dx * dx + dy * dy + dz * dz;
+                unsigned long long in = __ballot(r2 < g.rc2f);
+                if (general != 0) {
+                    if (mi) {
+                        dx -= g.bx * rintf(dx * g.ibx);
+                        dy -= g.by * rintf(dy * g.iby);
+                        dz -= g.bz * rintf(dz * g.ibz);
+                        r2 = dx * dx + dy * dy + dz * dz;
+                        in = __ballot(r2 < g.rc2f);
+                    }
+                    if (ex) {  // the shift by uniform jc8 and lane jl in two steps
+                        const unsigned long long em = em_s[wv][8 * k + il];
+                        const unsigned eb = (unsigned)(jc8 & 32 ? em >> 32 : em) >> (jc8 & 31);
+                        in &= __ballot(!((eb >> jl) & 1u));
+                    }
+                }
+                npair += __popcll(in);
+                if (COUNT) continue;
+                // lanes outside the cutoff are off; a step without any ends here
+                if (__builtin_amdgcn_inverse_ballot_w64(in)) {
+                    const float ir = __frsqrt_rn(r2);
+                    const float ir2 = ir * ir;
+                    float s2;
+                    if constexpr (GEO) {
+                        s2 = (si[k] * pq.x) * ir2;
+                    } else {
+                        const float sig = si[k] + pq.x;
+                        s2 = sig * sig * ir2;
+                    }
+                    const float s6 = s2 * s2 * s2;
+                    const float es6 = (ei[k] * pq.y) * s6;
+                    const float qq = qi[k] * pj.w;
+                    const float fr =
+                        es6 * (12.0f * s6 - 6.0f) * ir2 + qq * (ir * ir2 - 2.0f * g.krff);
+                    fi[3 * k] += fr * dx;
+                    fi[3 * k + 1] += fr * dy;
+                    fi[3 * k + 2] += fr * dz;
+                    fx -= fr * dx;
+                    fy -= fr * dy;
+                    fz -= fr * dz;
+                }
+            }
+            if (COUNT || npair == before) continue;  // uniform: no pair of the cluster
+            // each j atom of the tile is in exactly one cluster: lanes with il = jc keep it
+            const unsigned long long mine = 0x0101010101010101ull << (jc8 >> 3);
+            done |= 0xffull << jc8;
+            fx = sum8(fx);
+            fy = sum8(fy);
+            fz = sum8(fz);
+            const bool keep = __builtin_amdgcn_inverse_ballot_w64(mine);
+            fjx = keep ? fx : fjx;
+            fjy = keep ? fy : fjy;
+            fjz = keep ? fz : fjz;
+        } while (rest);
+        // flush the tile's j forces: lane = j atom, coalesced fixed-point atomics
+        fjx = __int_as_float(__builtin_amdgcn_ds_bpermute(transpose, __float_as_int(fjx)));
+        fjy = __int_as_float(__builtin_amdgcn_ds_bpermute(transpose, __float_as_int(fjy)));
+        fjz = __int_as_float(__builtin_amdgcn_ds_bpermute(transpose, __float_as_int(fjz)));
         // the next tile's records have landed (and the previous tile's atomics, issued a
         // tile earlier, are done): waited for before this tile's atomics, because a load
         // and later atomics share vmcnt but may retire out of order
         wait_vmem();
-        if (!COUNT && ((am0 >> lane) & 1ull)) {
+        if (!COUNT && __builtin_amdgcn_inverse_ballot_w64(done)) {
             int s = jb * 64 + lane;
             atomicAdd(&Fr[s], fixed_from_float(fjx, &bad));
             atomicAdd(&Fr[Np + s], fixed_from_float(fjy, &bad));
             atomicAdd(&Fr[2 * Np + s], fixed_from_float(fjz, &bad));
         }
-    };
-
-    if (part < nt) stage(tl[part], std::integral_constant<int, 0>());
-    wait_vmem();  // the first tile, this lane's atom and the block boxes have arrived
-    for (int t = part; t < nt; t += 2 * split) {
-        do_tile(t, std::integral_constant<int, 0>());
-        if (t + split < nt) do_tile(t + split, std::integral_constant<int, 1>());
     }
     if (COUNT) {
-        double c = wave_sum(vi ? (double)acc.cnt : 0.0);
-        if (lane == 0) atomicAdd(&pair_count[r], (unsigned long long)(c + 0.5));
+        if (lane == 0) atomicAdd(&pair_count[r], (unsigned long long)npair);
         return;
     }
-    if (vi) {  // atomic: the bonded kernel may run concurrently
-        long long fx = to_fixed(ax, &bad), fy = to_fixed(ay, &bad), fz = to_fixed(az, &bad);
-        atomicAdd(&Fr[islot], (unsigned long long)fx);
-        atomicAdd(&Fr[Np + islot], (unsigned long long)fy);
-        atomicAdd(&Fr[2 * Np + islot], (unsigned long long)fz);
-    }
+    flush_i();
     if (__ballot(bad) != 0ull && lane == 0) atomicOr(&flags[r], 2);
-    if (ENERGY) {
-        double es = wave_sum(vi ? (acc.e + g.krf * aqr2 - g.crf * aq) : 0.0);
-        if (lane == 0) e_pair[((size_t)r * NB + ib) * split + part] = es;
-    }
-}
-
-// ---------------------------------------------------------------------------
-// Grouped pair kernel (Newton-3, each pair once).  One wave per (replica, 64-slot
-// i-block), split into NG = 64/G groups of G consecutive slots.  Every group streams its
-// own j atoms -- those within rc of the GROUP's box rather than the block's -- so far
-// fewer of the evaluated lane pairs lie outside the cutoff (a 16-atom group's box is
-// about half as wide as a 64-atom block's).
-//
-// Candidate j-blocks (j-block >= i-block) are found by the wave from the block boxes,
-// without a tile list; those that need no periodic shift come first, the rest after
-// them.  For each j-block the 64 lanes test its 64 atoms against every group's box and
-// append the slots that pass to that group's ring buffer in LDS (entry = slot | flags).
-// Full chunks of 8 entries per group are consumed as soon as every group has one; at the
-// end, and when a ring would overflow, partial chunks are consumed with per-lane guards.
-//
-// Within a chunk lane L of a group evaluates ring entry k ^ rot(L) in its register slot
-// k.  With that order the j forces are summed over the group's lanes by halving DPP
-// stages that never select: at each stage a lane keeps slots [0, n/2) and adds its
-// partner's slots [n/2, n), which hold the same j atoms.  The lane then owns the force
-// on the j atom of its register slot 0 and adds it with int64 atomics.
-// ---------------------------------------------------------------------------
-constexpr unsigned RING_SLOT = 0x1FFFFFFFu;
-constexpr unsigned RING_EXCL = 1u << 29;    // pair needs j > i and the exclusion test
-constexpr unsigned RING_MINIMG = 1u << 30;  // pair needs the per-pair minimum image
-
-// Ring order of lane gl (0..G-1) of a group.  G = 16: stage partners lane^8 (bit 3),
-// lane^7 (bits 2,1,0), lane^2 (bit 1), then lane^1 sums equal atoms.  G = 8: lane^7,
-// lane^2, lane^1.  rot flips exactly the bit the stage halves on for each partner.
-template <int G>
-__device__ __forceinline__ int group_rot(int gl) {
-    if (G == 16) {
-        int b3 = (gl >> 3) & 1, b2 = (gl >> 2) & 1, b1 = (gl >> 1) & 1;
-        return 4 * b3 + 2 * b2 + (b1 ^ b2);
-    }
-    int b2 = (gl >> 2) & 1, b1 = (gl >> 1) & 1, b0 = gl & 1;
-    return 4 * b2 + 2 * (b1 ^ b2) + (b0 ^ b2);
-}
-
-// v[3k + c]: component c of the force on ring entry k ^ rot(L).  Returns in out[] the
-// group's sum for ring entry rot(L) (register slot 0).
-template <int G>
-__device__ __forceinline__ void group_reduce24(const float (&v)[24], float (&out)[3]) {
-    float w[12], x[6];
-    if (G == 16) {
-#pragma unroll
-        for (int t = 0; t < 12; t++) w[t] = dpp_add<0x128>(v[t], v[t + 12]);  // row_ror:8
-#pragma unroll
-        for (int t = 0; t < 6; t++) x[t] = dpp_add<0x141>(w[t], w[t + 6]);    // half mirror
-#pragma unroll
-        for (int t = 0; t < 3; t++) {
-            float y = dpp_add<0x4E>(x[t], x[t + 3]);                          // lane ^ 2
-            out[t] = dpp_add<0xB1>(y, y);                                     // lane ^ 1
-        }
-    } else {
-#pragma unroll
-        for (int t = 0; t < 12; t++) w[t] = dpp_add<0x141>(v[t], v[t + 12]);
-#pragma unroll
-        for (int t = 0; t < 6; t++) x[t] = dpp_add<0x4E>(w[t], w[t + 6]);
-#pragma unroll
-        for (int t = 0; t < 3; t++) out[t] = dpp_add<0xB1>(x[t], x[t + 3]);
-    }
-}
-
-// min / max over the G lanes of a group (same butterfly as the force sum)
-template <int G>
-__device__ __forceinline__ float group_min(float v) {
-    if (G == 16) v = fminf(v, dpp_f<0x128>(v));
-    v = fminf(v, dpp_f<0x141>(v));
-    v = fminf(v, dpp_f<0x4E>(v));
-    return fminf(v, dpp_f<0xB1>(v));
-}
-template <int G>
-__device__ __forceinline__ float group_max(float v) {
-    if (G == 16) v = fmaxf(v, dpp_f<0x128>(v));
-    v = fmaxf(v, dpp_f<0x141>(v));
-    v = fmaxf(v, dpp_f<0x4E>(v));
-    return fmaxf(v, dpp_f<0xB1>(v));
-}
-
-
-
-// One chunk: 8 ring entries per group.  SRC 0 / 1: every entry is valid and the records
-// were copied to LDS staging buffer `stage` (record of group q, entry k at
-// stage[2 (8q + k)]); SRC 2: the records are loaded from A and bit k of `valid` says
-// whether register slot k holds an entry.  mi (per-pair minimum image) and ex (entries
-// that need the j > i / exclusion test) are wave-uniform.  The pairs run in the order
-// 0,4,2,6,1,5,3,7 so that the first two halving stages of the j-force sum fold in as
-// soon as both of their slots are done (12 live partial sums instead of 24).  The j
-// force of register slot 0's entry is returned in f.
-template <int G, int SRC>
-__device__ __forceinline__ void grp_chunk(const float4* __restrict__ A,
-                                          const float4* __restrict__ stage, const unsigned (&e)[8],
-                                          unsigned valid, bool mi, bool ex, int gi, int rot,
-                                          float4 pi, float2 qi, int islot, bool vi,
-                                          const int* __restrict__ exs, int nex, const Geom& g,
-                                          PairAcc& a, float (&f)[3]) {
-    constexpr bool STAGED = SRC != 2;
-    constexpr int ord[8] = {0, 4, 2, 6, 1, 5, 3, 7};
-    constexpr int S1 = G == 16 ? 0x128 : 0x141;  // row_ror:8 | row_half_mirror
-    constexpr int S2 = G == 16 ? 0x141 : 0x4E;   // row_half_mirror | lane ^ 2
-    constexpr int S3 = G == 16 ? 0x4E : 0xB1;    // lane ^ 2 | lane ^ 1
-    float4 pj[8];
-    float2 qj[8];
-    auto ld = [&](int k) {
-        if (STAGED) {
-            int ix = 2 * (gi * 8 + (k ^ rot));
-            pj[k] = stage[ix];
-            qj[k] = *(const float2*)&stage[ix + 1];
-        } else {
-            // e << 5 = the slot's byte offset (32-byte records; the flag bits shift out)
-            const char* rec = (const char*)A + (e[k] << 5);
-            pj[k] = *(const float4*)rec;
-            qj[k] = *(const float2*)(rec + 16);
-        }
-    };
-    auto pair = [&](int k, float (&v)[3]) {
-        bool incl = vi;
-        if (!STAGED) incl = incl && ((valid >> k) & 1u);
-        if (ex && (e[k] & RING_EXCL)) {
-            int js = (int)(e[k] & RING_SLOT);
-            bool part = js <= islot;
-            for (int x = 0; x < nex; x++) part |= exs[x * 64] == js;
-            incl = incl && !part;
-        }
-        float dx, dy, dz;
-        float fr = pair_masked(pi, qi, pj[k], qj[k], incl, mi, g, a, dx, dy, dz);
-        v[0] = -fr * dx;
-        v[1] = -fr * dy;
-        v[2] = -fr * dz;
-    };
-    // staged records are read two pairs ahead; global ones (rare partial chunks) just
-    // before their pair, which keeps this path's registers within the staged one's
-    constexpr int AHEAD = STAGED ? 2 : 0;
-#pragma unroll
-    for (int t = 0; t < AHEAD; t++) ld(ord[t]);
-    float w[4][3], x[2][3];
-#pragma unroll
-    for (int t = 0; t < 8; t += 2) {
-        float v0[3], v1[3];
-        if (t + AHEAD < 8) ld(ord[t + AHEAD]);
-        __builtin_amdgcn_sched_barrier(0);
-        pair(ord[t], v0);
-        if (t + 1 + AHEAD < 8) ld(ord[t + 1 + AHEAD]);
-        __builtin_amdgcn_sched_barrier(0);
-        pair(ord[t + 1], v1);
-        const int sl = ord[t];  // slot sl pairs with slot sl + 4: 0, 2, 1, 3
-#pragma unroll
-        for (int c = 0; c < 3; c++) w[sl][c] = dpp_add<S1>(v0[c], v1[c]);
-        if (sl == 2)
-#pragma unroll
-            for (int c = 0; c < 3; c++) x[0][c] = dpp_add<S2>(w[0][c], w[2][c]);
-        if (sl == 3)
-#pragma unroll
-            for (int c = 0; c < 3; c++) x[1][c] = dpp_add<S2>(w[1][c], w[3][c]);
-    }
-#pragma unroll
-    for (int c = 0; c < 3; c++) {
-        float y = dpp_add<S3>(x[0][c], x[1][c]);
-        f[c] = G == 16 ? dpp_add<0xB1>(y, y) : y;
-    }
-    a.e += (double)a.ef;  // FP32 over 8 pairs, FP64 beyond
-    a.ef = 0.f;
-}
-
-
-template <int G, int CAP, int WPW, bool COUNT>
-__global__ __launch_bounds__(64 * WPW) void k_pair_grp(
-    int R, int N, int Np, int NB, const float4* __restrict__ arec,
-    const int* __restrict__ orig_s, const int* __restrict__ slot_of,
-    const float4* __restrict__ bb_lo, const float4* __restrict__ bb_hi,
-    const int* __restrict__ ex_start, const int* __restrict__ ex_list, int max_ex,
-    long long* __restrict__ F, double* __restrict__ e_pair, int* __restrict__ flags,
-    unsigned long long* __restrict__ pair_count, float list_r2, Geom g) {
-    constexpr int NG = 64 / G;
-    extern __shared__ unsigned sdm_lds[];
-    // two staging buffers as separate LDS objects: the compiler then knows that reading
-    // one does not have to wait for the copy into the other
-    __shared__ float4 stage_a[WPW][NG * 16], stage_b[WPW][NG * 16];
-    int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    int w = xcd_linear_id(blockIdx.x, gridDim.x) * WPW + wv;
-    int lane = threadIdx.x & 63;
-    if (w >= R * NB) return;
-    int r = w / NB;
-    int ib = w - r * NB;
-    // per wave: rings [NG][CAP] | exclusion partners [max_ex][64] | group boxes [NG][2]
-    unsigned* ring = sdm_lds + wv * (NG * CAP + max_ex * 64 + NG * 8);
-    int* exs = (int*)(ring + NG * CAP);
-    const float4* A = arec + (size_t)r * Np * 2;
-    unsigned long long* Fr = (unsigned long long*)(F + (size_t)r * 3 * Np);
-    const int gi = lane / G, gl = lane % G;
-    const int rot = group_rot<G>(gl);
-    int islot = ib * 64 + lane;
-    bool vi = islot < N;
-    float4 pi = A[2 * islot];
-    float4 qi4 = A[2 * islot + 1];
-    float2 qi = make_float2(qi4.x, qi4.y);
-    int nex = 0;
-    if (vi) {
-        int ai = orig_s[(size_t)r * Np + islot];
-        int b0 = ex_start[ai];
-        nex = ex_start[ai + 1] - b0;
-        for (int k = 0; k < nex; k++) exs[k * 64 + lane] = slot_of[(size_t)r * Np + ex_list[b0 + k]];
-    }
-    // group boxes: every lane knows its own group's, the wave holds all of them uniform
-    float glx = group_min<G>(vi ? pi.x : 3.0e38f), gly = group_min<G>(vi ? pi.y : 3.0e38f),
-          glz = group_min<G>(vi ? pi.z : 3.0e38f);
-    float ghx = group_max<G>(vi ? pi.x : -3.0e38f), ghy = group_max<G>(vi ? pi.y : -3.0e38f),
-          ghz = group_max<G>(vi ? pi.z : -3.0e38f);
-    float gcx = 0.5f * (glx + ghx), gcy = 0.5f * (gly + ghy), gcz = 0.5f * (glz + ghz);
-    float gex = 0.5f * (ghx - glx), gey = 0.5f * (ghy - gly), gez = 0.5f * (ghz - glz);
-    // every group's box in LDS (center, half extent), read back uniformly when appending
-    float4* gbox = (float4*)(exs + max_ex * 64);
-    if (gl == 0) {
-        gbox[2 * gi] = make_float4(gcx, gcy, gcz, 0.f);
-        gbox[2 * gi + 1] = make_float4(gex, gey, gez, 0.f);
-    }
-    __builtin_amdgcn_wave_barrier();
-    // groups with at least one atom (slots are filled in order, so the first lane decides)
-    int ngv = min(NG, (N - ib * 64 + G - 1) / G);
-    float4 bli = bb_lo[(size_t)r * NB + ib], bhi = bb_hi[(size_t)r * NB + ib];
-    // ring head, common to every group and a multiple of 8: a chunk takes 8 entries from
-    // every ring, and a ring with fewer has its tail moved up to the new head
-    int h = 0;
-    int tail[NG];
-#pragma unroll
-    for (int q = 0; q < NG; q++) tail[q] = 0;
-    double ax = 0.0, ay = 0.0, az = 0.0, aqr2 = 0.0, aq = 0.0;
-    PairAcc acc;
-    acc.fx = acc.fy = acc.fz = acc.sqr2 = acc.sq = 0.f;
-    acc.e = 0.0;
-    acc.ef = 0.f;
-    acc.cnt = 0;
-    int bad = 0;
-    int nchunk = 0;
-    const unsigned rot4 = (unsigned)rot * 4u;
-    const bool own_j = G == 8 || (gl & 1) == 0;  // lane that adds its j atom's force
-    // staging: lane L copies half L&1 of record (L>>1) + 32 i of the chunk (DMA i)
-    int dkoff[NG / 4];
-#pragma unroll
-    for (int i = 0; i < NG / 4; i++) {
-        int ri = i * 32 + (lane >> 1);
-        dkoff[i] = (ri >> 3) * CAP + (ri & 7);
-    }
-    int cur = 0;       // staging buffer of the next full chunk
-    bool pre = false;  // its records are already there
-    // copies the records of ring entries hd..hd+7 of every group into staging buffer b
-    // (global -> LDS without registers; completion is waited for with vmcnt)
-    // copies the records of ring entries hd..hd+7 of every group into staging buffer B
-    // (global -> LDS without registers; completion is waited for with vmcnt)
-    auto stage_chunk = [&](int hd, auto bufc) {
-        constexpr int B = decltype(bufc)::value;
-        float4* dst = B ? stage_b[wv] : stage_a[wv];
-        int hb = hd & (CAP - 1);
-        __builtin_amdgcn_wave_barrier();
-#pragma unroll
-        for (int i = 0; i < NG / 4; i++) {
-            unsigned ee = ring[dkoff[i] + hb];
-            const char* src = (const char*)A + ((ee << 5) | ((unsigned)(lane & 1) << 4));
-            __builtin_amdgcn_global_load_lds(
-                (const void*)src, (__attribute__((address_space(3))) void*)(dst + i * 64), 16, 0, 0);
-        }
-        __builtin_amdgcn_wave_barrier();
-    };
-    auto add_j = [&](unsigned e0, const float (&f)[3]) {
-        int s = (int)(e0 & RING_SLOT);
-        atomicAdd(&Fr[s], fixed_from_float(f[0], &bad));
-        atomicAdd(&Fr[Np + s], fixed_from_float(f[1], &bad));
-        atomicAdd(&Fr[2 * Np + s], fixed_from_float(f[2], &bad));
-    };
-    auto after_chunk = [&]() {
-        h += 8;
-#pragma unroll
-        for (int q = 0; q < NG; q++) tail[q] = max(tail[q], h);
-        if ((++nchunk & 3) == 0) {  // FP32 partial sums of 32 pairs go to FP64
-            ax += (double)acc.fx;
-            ay += (double)acc.fy;
-            az += (double)acc.fz;
-            aqr2 += (double)acc.sqr2;
-            aq += (double)acc.sq;
-            acc.fx = acc.fy = acc.fz = acc.sqr2 = acc.sq = 0.f;
-        }
-    };
-    // full chunk from staging buffer B; stages the next one into the other buffer first
-    // when every ring holds it (next_ok), so its copy overlaps this chunk's arithmetic.
-    // B is a compile-time constant so every LDS access names its buffer.
-    auto consume_full = [&](bool next_ok, auto bufc) {
-        constexpr int B = decltype(bufc)::value;
-        if (!pre) {
-            stage_chunk(h, std::integral_constant<int, B>());
-            wait_vmem();
-        }
-        pre = false;
-        if (next_ok) {
-            stage_chunk(h + 8, std::integral_constant<int, 1 - B>());
-            pre = true;
-        }
-        unsigned base4 = (unsigned)(gi * CAP + (h & (CAP - 1))) * 4u;
-        unsigned e[8];
-        unsigned fl = 0;
-#pragma unroll
-        for (int k = 0; k < 8; k++) {
-            e[k] = *(const unsigned*)((const char*)ring + (((unsigned)k * 4u) ^ rot4) + base4);
-            fl |= e[k];
-        }
-        bool mi = __ballot((fl & RING_MINIMG) != 0u) != 0ull;
-        bool ex = __ballot((fl & RING_EXCL) != 0u) != 0ull;
-        float f[3];
-        grp_chunk<G, B>(A, B ? stage_b[wv] : stage_a[wv], e, 0xFFu, mi, ex, gi, rot, pi, qi,
-                        islot, vi, exs + lane, nex, g, acc, f);
-        wait_vmem();  // the next chunk's records have landed; older atomics are done
-        if (own_j) add_j(e[0], f);
-        cur ^= 1;
-        after_chunk();
-    };
-    // partial chunk (fewer than 8 entries in some ring): records loaded directly
-    auto consume_partial = [&]() {
-        pre = false;
-        int t = tail[0];
-#pragma unroll
-        for (int q = 1; q < NG; q++) t = (gi == q) ? tail[q] : t;
-        int n = t - h;
-        unsigned base4 = (unsigned)(gi * CAP + (h & (CAP - 1))) * 4u;
-        unsigned e[8];
-        unsigned valid = 0;
-#pragma unroll
-        for (int k = 0; k < 8; k++) {
-            bool ok = (k ^ rot) < n;
-            unsigned v = *(const unsigned*)((const char*)ring + (((unsigned)k * 4u) ^ rot4) + base4);
-            e[k] = ok ? v : (unsigned)islot;  // unused slot: own record
-            valid |= ok ? (1u << k) : 0u;
-        }
-        float f[3];
-        grp_chunk<G, 2>(A, nullptr, e, valid, true, true, gi, rot, pi, qi, islot, vi, exs + lane, nex, g, acc, f);
-        if (own_j && (valid & 1u)) add_j(e[0], f);
-        after_chunk();
-    };
-    auto min_avail = [&]() {
-        int m = tail[0];
-#pragma unroll
-        for (int q = 1; q < NG; q++) m = min(m, tail[q]);
-        return m - h;
-    };
-    auto max_avail = [&]() {
-        int m = tail[0];
-#pragma unroll
-        for (int q = 1; q < NG; q++) m = max(m, tail[q]);
-        return m - h;
-    };
-
-    // candidate j-blocks of one pass among blocks base..base+63 (pass 0: the plain
-    // difference is the minimum image for every pair of the two boxes; pass 1: the rest)
-    auto candidates = [&](int pass, int base) {
-        int jb = base + lane;
-        bool cand = false;
-        if (jb < NB && jb >= ib) {
-            float4 blj = bb_lo[(size_t)r * NB + jb], bhj = bb_hi[(size_t)r * NB + jb];
-            float dcx = 0.5f * (bli.x + bhi.x - blj.x - bhj.x);
-            float dcy = 0.5f * (bli.y + bhi.y - blj.y - bhj.y);
-            float dcz = 0.5f * (bli.z + bhi.z - blj.z - bhj.z);
-            bool plain = fabsf(dcx) + 0.5f * (bhi.x - bli.x + bhj.x - blj.x) < g.oix &&
-                         fabsf(dcy) + 0.5f * (bhi.y - bli.y + bhj.y - blj.y) < g.oiy &&
-                         fabsf(dcz) + 0.5f * (bhi.z - bli.z + bhj.z - blj.z) < g.oiz;
-            cand = (plain ? 0 : 1) == pass && bbox_gap2(bli, bhi, blj, bhj, g) < list_r2;
-        }
-        return __ballot(cand);
-    };
-    // appends the atoms of j-block jb that lie within rc of each group's box
-    auto append = [&](int jb, int pass) {
-        __builtin_amdgcn_wave_barrier();
-        int s = jb * 64 + lane;
-        bool vj = s < N;
-        float4 pj = A[2 * min(s, N - 1)];
-        bool mine = jb == ib;
-        for (int k = 0; k < nex; k++) mine |= (exs[k * 64 + lane] >> 6) == jb;
-        unsigned fl = (__ballot(mine) != 0ull ? RING_EXCL : 0u) | (pass ? RING_MINIMG : 0u);
-#pragma unroll
-        for (int q = 0; q < NG; q++) {
-            float4 c = gbox[2 * q], h = gbox[2 * q + 1];
-            float dx = pj.x - c.x, dy = pj.y - c.y, dz = pj.z - c.z;
-            if (pass) {
-                dx -= g.bx * rintf(dx * g.ibx);
-                dy -= g.by * rintf(dy * g.iby);
-                dz -= g.bz * rintf(dz * g.ibz);
-            }
-            float ux = fmaxf(fabsf(dx) - h.x, 0.f), uy = fmaxf(fabsf(dy) - h.y, 0.f),
-                  uz = fmaxf(fabsf(dz) - h.z, 0.f);
-            bool in = vj && q < ngv && ux * ux + uy * uy + uz * uz < list_r2;
-            if (jb == ib) in = in && s > ib * 64 + q * G;  // j must follow an i of the group
-            unsigned long long mq = __ballot(in);
-            if (in) ring[q * CAP + ((tail[q] + lane_rank(mq)) & (CAP - 1))] = (unsigned)s | fl;
-            tail[q] += __popcll(mq);
-        }
-        __builtin_amdgcn_wave_barrier();
-    };
-
-    // Fill first (every ring 16 deep, so a full chunk can stage the next one), then full
-    // chunks; partial chunks only when a ring would overflow or no tile is left.
-    int pass = 0, base = ib & ~63;
-    unsigned long long tm = candidates(0, base);
-    bool tiles_left = true;
-    // Everything loaded so far (this lane's atom, the block boxes) has arrived: without
-    // this wait the compiler would place one in the loop at the first use of each such
-    // value, and it would then also wait for the staging copy in flight every chunk.
-    wait_vmem();
-    while (true) {
-        int mn = min_avail(), mx = max_avail();
-        if (tiles_left && mn < 16 && mx <= CAP - 64) {
-            while (tm == 0ull && tiles_left) {
-                base += 64;
-                if (base >= NB) {
-                    if (pass == 1) {
-                        tiles_left = false;
-                        break;
-                    }
-                    pass = 1;
-                    base = ib & ~63;
-                }
-                tm = candidates(pass, base);
-            }
-            if (!tiles_left) continue;
-            int jb = base + __ffsll((long long)tm) - 1;
-            tm &= tm - 1ull;
-            append(jb, pass);
-            continue;
-        }
-        if (mn >= 8) {
-            if (cur == 0) consume_full(mn >= 16, std::integral_constant<int, 0>());
-            else consume_full(mn >= 16, std::integral_constant<int, 1>());
-            continue;
-        }
-        if (mx > 0) {
-            consume_partial();
-            continue;
-        }
-        break;
-    }
-    ax += (double)acc.fx;
-    ay += (double)acc.fy;
-    az += (double)acc.fz;
-    aqr2 += (double)acc.sqr2;
-    aq += (double)acc.sq;
-    if (COUNT) {
-        double c = wave_sum(vi ? (double)acc.cnt : 0.0);
-        if (lane == 0) atomicAdd(&pair_count[r], (unsigned long long)(c + 0.5));
-        return;
-    }
-    if (vi) {
-        long long fx = to_fixed(ax, &bad), fy = to_fixed(ay, &bad), fz = to_fixed(az, &bad);
-        atomicAdd(&Fr[islot], (unsigned long long)fx);
-        atomicAdd(&Fr[Np + islot], (unsigned long long)fy);
-        atomicAdd(&Fr[2 * Np + islot], (unsigned long long)fz);
-    }
-    double es = wave_sum(vi ? (acc.e + g.krf * aqr2 - g.crf * aq) : 0.0);
-    if (__ballot(bad) != 0ull && lane == 0) atomicOr(&flags[r], 2);
-    if (lane == 0) e_pair[(size_t)r * NB + ib] = es;
 }
 
 // ---------------------------------------------------------------------------
 // Pair energies in FP64 (the energy evaluations: U0 and with it U1 = U0 + u and the
-// potential energy).  The force kernels compute in FP32 from FP32 coordinates, whose
+// potential energy).  The force kernel computes in FP32 from FP32 coordinates, whose
 // rounding (an ulp is ~5e-7 nm at 4-8 nm) and arithmetic leave ~2^-24 of the summed pair
 // magnitudes in U0; where U0 is a small net of large terms that exceeds 1e-5 of U0.  This
 // kernel takes the FP64 positions and parameters of every pair with r < rc once, in
 // Newton-3 order over the half tile lists, so U0 is exact to FP64 rounding.
 //
-// One wave per (replica, i-block, part): part p of `split` takes tiles p, p + split, ..
-// Per tile the wave screens the mask's j atoms against its 64 i atoms in FP32 (the FP32
-// slot records, cutoff widened by 1e-4 nm so no pair inside rc is dropped) and queues
-// the surviving (i, j) lane pairs in LDS; every 64 queued pairs are evaluated one per
-// lane in FP64 (minimum image, exact cutoff test, LJ + reaction field), so the FP64 work
-// is spent on the ~25% of screened pairs that lie inside the cutoff.  half = 0: full tile
-// lists (the non-Newton kernel's), of which only tiles with j-block >= i-block are taken.
+// One wave per (replica, i-block, part): part p of `split` takes tiles p, p + split, ..,
+// pair of clusters by pair of clusters as the pair kernel does (lane 8 jl + il: j atom jl,
+// i atom il), all in FP64: vector FP64 issues at the rate of unpacked FP32.  The i records
+// stay in LDS (eight clusters of FP64 records would take 96 registers), the next tile's j
+// records are loaded into registers while the current tile is evaluated.
 // ---------------------------------------------------------------------------
 constexpr int E64_SPLIT = 4;  // waves (parts) per i-block of the FP64 energy kernel
 
@@ -1685,208 +924,109 @@ constexpr int E64_SPLIT = 4;  // waves (parts) per i-block of the FP64 energy ke
 __device__ __forceinline__ void lds_order() { asm volatile("" ::: "memory"); }
 
 __global__ __launch_bounds__(64) void k_energy64(
-    int R, int N, int Np, int NB, int maxj, int split, int half, const float4* __restrict__ arec,
-    const Rec64* __restrict__ rec, const int* __restrict__ orig_s,
-    const int* __restrict__ slot_of, const int* __restrict__ tiles,
-    const unsigned long long* __restrict__ tmask, const int* __restrict__ ntiles,
-    const float4* __restrict__ bb_lo, const float4* __restrict__ bb_hi,
-    const int* __restrict__ ex_start, const int* __restrict__ ex_list, int max_ex,
-    double* __restrict__ e_out, Geom g) {
+    int R, int N, int Np, int NB, int maxj, int split, const Rec64* __restrict__ rec,
+    const int* __restrict__ tiles, const unsigned long long* __restrict__ tmask,
+    const int* __restrict__ ntiles, const float4* __restrict__ bb_lo,
+    const float4* __restrict__ bb_hi, const int* __restrict__ exs,
+    const unsigned long long* __restrict__ exblocks, int max_ex, double* __restrict__ e_out, Geom g) {
     __shared__ Rec64 irec[64], jrec[64];
-    __shared__ float4 jpos[64];
-    __shared__ unsigned short queue[128];
-    extern __shared__ int exs64[];  // [max_ex][64] exclusion partners' slots
+    __shared__ unsigned long long em_s[64];
     const int w = xcd_linear_id(blockIdx.x, gridDim.x);
     const int lane = threadIdx.x;
     if (w >= R * NB * split) return;
     const int part = w % split, rb = w / split;
     const int r = rb / NB, ib = rb - r * NB;
-    const float4* A = arec + (size_t)r * Np * 2;
     const Rec64* RC = rec + (size_t)r * Np;
     const int islot = ib * 64 + lane;
     const bool vi = islot < N;
-    const bool full_block = ib * 64 + 63 < N;  // uniform: every lane holds an atom
-    // this lane's i atom: FP32 record for the screen, FP64 record for the pairs
-    const float4 pi = A[2 * islot];
+    const int il = lane & 7, jl = lane >> 3;
     irec[lane] = RC[vi ? islot : ib * 64];
-    int nex = 0;
-    int exlo = NB, exhi = -1;  // j-blocks holding exclusion partners (as in k_pair_n3)
-    if (vi) {
-        int ai = orig_s[(size_t)r * Np + islot];
-        int b0 = ex_start[ai];
-        nex = ex_start[ai + 1] - b0;
-        for (int k = 0; k < nex; k++) {
-            const int sl = slot_of[(size_t)r * Np + ex_list[b0 + k]];
-            exs64[k * 64 + lane] = sl;
-            exlo = min(exlo, sl >> 6);
-            exhi = max(exhi, sl >> 6);
-        }
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        exlo = min(exlo, __shfl_xor(exlo, o, 64));
-        exhi = max(exhi, __shfl_xor(exhi, o, 64));
-    }
-    exlo = __builtin_amdgcn_readfirstlane(exlo);
-    exhi = __builtin_amdgcn_readfirstlane(exhi);
-    const float rcs = sqrtf(g.rc2f) + 1e-4f;
-    const float rc2s = rcs * rcs;
+    const int* E = exs + (size_t)(r * NB + ib) * max_ex * 64;
+    const unsigned long long eset = exblocks[(size_t)r * NB + ib];
     const float4 bli = bb_lo[(size_t)r * NB + ib], bhi = bb_hi[(size_t)r * NB + ib];
     const int* tl = tiles + ((size_t)r * NB + ib) * maxj;
     const unsigned long long* tmk = tmask + ((size_t)r * NB + ib) * maxj;
     const int nt = ntiles[(size_t)r * NB + ib];
     double e = 0.0;
-    unsigned head = 0, tail = 0;  // queue positions (wave-uniform)
-    // the queued pairs head .. head + n - 1 (n <= 64), one per lane.  one_image: every
-    // pair of the tile takes the shift (sx, sy, sz) (records are in the FP32 records'
-    // images); otherwise the minimum image per pair
-    double sx = 0.0, sy = 0.0, sz = 0.0;
-    bool one_image = true;
-    auto evaluate = [&](unsigned n) {
-        if ((unsigned)lane < n) {
-            unsigned q = queue[(head + lane) & 127u];
-            const Rec64 I = irec[q & 63u], J = jrec[q >> 6];
-            double dx = (I.x - sx) - J.x, dy = (I.y - sy) - J.y, dz = (I.z - sz) - J.z;
-            if (!one_image) {
-                dx = min_image(dx, g.Lx, g.iLx);
-                dy = min_image(dy, g.Ly, g.iLy);
-                dz = min_image(dz, g.Lz, g.iLz);
-            }
-            double r2 = dx * dx + dy * dy + dz * dz;
-            if (r2 < g.rc2) {
-                double ir = rsqrt(r2);
-                double ir2 = ir * ir;
-                double s2;
-                if (g.geo) {  // Geom::geo: the records hold sigma itself
-                    s2 = I.sh * J.sh * ir2;
-                } else {
-                    double sig = I.sh + J.sh;
-                    s2 = sig * sig * ir2;
-                }
-                double s6 = s2 * s2 * s2;
-                double qq = I.qk * J.qk;
-                e += (I.es * J.es) * s6 * (s6 - 1.0) + qq * (ir + g.krf * r2 - g.crf);
-            }
-        }
-        head += n;
-    };
-    // screen of one j atom against the wave's i atoms, queueing the pairs inside the
-    // widened cutoff.  MI: per-pair minimum image (otherwise the tile's shift is in ps);
-    // CHK: some lane is padding or has an exclusion partner in the tile
-    auto screen = [&](int j, float4 pj, float4 ps, unsigned long long em, auto mic, auto chk) {
-        constexpr bool MI = decltype(mic)::value, CHK = decltype(chk)::value;
-        float dx = ps.x - pj.x, dy = ps.y - pj.y, dz = ps.z - pj.z;
-        if (MI) {
-            dx -= g.bx * rintf(dx * g.ibx);
-            dy -= g.by * rintf(dy * g.iby);
-            dz -= g.bz * rintf(dz * g.ibz);
-        }
-        bool in = dx * dx + dy * dy + dz * dz < rc2s;
-        if (CHK) in = in && vi && !((em >> j) & 1ull);
-        const unsigned long long m = __ballot(in);
-        if (in) queue[(tail + (unsigned)lane_rank(m)) & 127u] = (unsigned short)(lane | (j << 6));
-        tail += (unsigned)__popcll(m);
-        if (tail - head >= 64u) {
-            lds_order();  // the queue entries are written
-            evaluate(64u);
-            lds_order();  // and read before they are overwritten
-        }
-    };
-    // the j records of the wave's next tile are loaded into registers while the current
-    // tile is screened and evaluated, and stored to LDS when its turn comes
-    // (plain vector values, not a struct, so that they stay in registers).  This lane's
-    // i record is used here first, so that the loop's waits for it are settled before
-    // the first prefetch is in flight (a wait inside the loop would wait for that too)
-    asm volatile("" ::"v"(pi.x), "v"(pi.y), "v"(pi.z), "v"(pi.w));
-    double2 na = make_double2(0.0, 0.0), nb = na, nc = na;  // a record is 3 x 16 bytes
-    float4 npos = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (part < nt) {
-        const int js = tl[part] * 64 + lane;
+    // the j records of the wave's next tile (a record is 3 x 16 bytes)
+    double2 na = make_double2(0.0, 0.0), nb = na, nc = na;
+    auto prefetch = [&](int jb) {
+        const int js = jb * 64 + lane;
         if (js < N) {
             const double2* src = (const double2*)(RC + js);
             na = src[0];
             nb = src[1];
             nc = src[2];
-            npos = A[2 * js];
         }
-    }
+    };
+    if (part < nt) prefetch(tl[part]);
     for (int t = part; t < nt; t += split) {
         const int jb = tl[t];
-        unsigned long long am = tmk[t];
+        const unsigned long long m = tmk[t];
         lds_order();  // the previous tile's records are no longer read
-        if (jb * 64 + lane < N) {
-            jrec[lane] = Rec64{na.x, na.y, nb.x, nb.y, nc.x, nc.y};
-            jpos[lane] = npos;
-        }
-        if (t + split < nt) {
-            const int js = tl[t + split] * 64 + lane;
-            if (js < N) {
-                const double2* src = (const double2*)(RC + js);
-                na = src[0];
-                nb = src[1];
-                nc = src[2];
-                npos = A[2 * js];
-            }
-        }
-        if (!half && jb < ib) continue;  // full lists: each block pair once
-        unsigned long long em = 0;
-        if (jb >= exlo && jb <= exhi) {
-            for (int k = 0; k < nex; k++) {
-                int sl = exs64[k * 64 + lane];
-                if ((sl >> 6) == jb) em |= 1ull << (sl & 63);
-            }
-        }
-        if (jb == ib) em |= (2ull << lane) - 1ull;  // the diagonal tile: j > i only
-        const bool chk = !full_block || __ballot(em != 0ull) != 0ull;
-        // one periodic shift for the whole tile when it is exact for every pair within
-        // the list radius (Geom::oix), as in the pair kernel
-        const float4 blj = bb_lo[(size_t)r * NB + jb], bhj = bb_hi[(size_t)r * NB + jb];
-        const float dcx = 0.5f * (bli.x + bhi.x - blj.x - bhj.x);
-        const float dcy = 0.5f * (bli.y + bhi.y - blj.y - bhj.y);
-        const float dcz = 0.5f * (bli.z + bhi.z - blj.z - bhj.z);
-        const float kx = rintf(dcx * g.ibx), ky = rintf(dcy * g.iby), kz = rintf(dcz * g.ibz);
-        const float fsx = g.bx * kx, fsy = g.by * ky, fsz = g.bz * kz;
-        one_image = fabsf(dcx - fsx) + 0.5f * (bhi.x - bli.x + bhj.x - blj.x) < g.oix &&
-                    fabsf(dcy - fsy) + 0.5f * (bhi.y - bli.y + bhj.y - blj.y) < g.oiy &&
-                    fabsf(dcz - fsz) + 0.5f * (bhi.z - bli.z + bhj.z - blj.z) < g.oiz;
-        float4 ps = pi;
-        if (one_image) {
-            ps.x -= fsx;
-            ps.y -= fsy;
-            ps.z -= fsz;
-            sx = g.Lx * (double)kx;  // the same shift in FP64 (0 if not periodic)
-            sy = g.Ly * (double)ky;
-            sz = g.Lz * (double)kz;
-        } else {
-            sx = sy = sz = 0.0;
-        }
+        jrec[lane] = Rec64{na.x, na.y, nb.x, nb.y, nc.x, nc.y};
+        if (t + split < nt) prefetch(tl[t + split]);
+        const unsigned long long em = tile_exclusions(eset, max_ex, E, lane, vi, ib, jb, N);
+        const bool ex = __ballot(em != 0ull) != 0ull;
+        if (ex) em_s[lane] = em;
+        float kx, ky, kz;
+        const bool one_image = tile_shift(bli, bhi, bb_lo[(size_t)r * NB + jb],
+                                          bb_hi[(size_t)r * NB + jb], g, kx, ky, kz);
+        const double sx = g.Lx * (double)kx, sy = g.Ly * (double)ky, sz = g.Lz * (double)kz;
         lds_order();  // this tile's records are stored
-        // the mask's j atoms four at a time: their four position reads are in flight
-        // together instead of one LDS round trip per atom
-        auto screen4 = [&](auto mic, auto chk) {
-            while (am) {
-                int jq[4];
-                float4 pq[4];
-#pragma unroll
-                for (int k = 0; k < 4; k++) jq[k] = next_bit(am);
-#pragma unroll
-                for (int k = 0; k < 4; k++) pq[k] = jpos[jq[k] & 63];
-#pragma unroll
-                for (int k = 0; k < 4; k++)
-                    if (jq[k] >= 0) screen(jq[k], pq[k], ps, em, mic, chk);
-            }
+        auto clusters = [&](auto mic, auto exc) {
+            constexpr bool MI = decltype(mic)::value, EX = decltype(exc)::value;
+            unsigned long long rest = m;
+            do {
+                const int jc = __builtin_ctzll(rest) >> 3;
+                unsigned ics = (unsigned)(m >> (8 * jc)) & 0xffu;
+                rest &= ~(0xffull << (8 * jc));
+                Rec64 J = jrec[8 * jc + jl];
+                if (!MI) {
+                    J.x += sx;
+                    J.y += sy;
+                    J.z += sz;
+                }
+                do {
+                    const int k = __builtin_ctz(ics);
+                    ics &= ics - 1u;
+                    const Rec64 I = irec[8 * k + il];
+                    double dx = I.x - J.x, dy = I.y - J.y, dz = I.z - J.z;
+                    if (MI) {
+                        dx = min_image(dx, g.Lx, g.iLx);
+                        dy = min_image(dy, g.Ly, g.iLy);
+                        dz = min_image(dz, g.Lz, g.iLz);
+                    }
+                    const double r2 = dx * dx + dy * dy + dz * dz;
+                    bool ok = r2 < g.rc2;
+                    if (EX) ok = ok && !((em_s[8 * k + il] >> (8 * jc + jl)) & 1ull);
+                    if (__ballot(ok) == 0ull) continue;  // uniform
+                    const double ir = rsqrt(r2);
+                    const double ir2 = ir * ir;
+                    double s2;
+                    if (g.geo) {  // Geom::geo: the records hold sigma itself
+                        s2 = I.sh * J.sh * ir2;
+                    } else {
+                        const double sig = I.sh + J.sh;
+                        s2 = sig * sig * ir2;
+                    }
+                    const double s6 = s2 * s2 * s2;
+                    const double qq = I.qk * J.qk;
+                    const double ee = (I.es * J.es) * s6 * (s6 - 1.0) +
+                                      qq * (ir + g.krf * r2 - g.crf);
+                    e += ok ? ee : 0.0;  // also clears inf or NaN of excluded or empty slots
+                } while (ics);
+            } while (rest);
         };
         using T = std::true_type;
         using Fa = std::false_type;
         if (one_image) {
-            if (chk) screen4(Fa(), T());
-            else screen4(Fa(), Fa());
+            if (ex) clusters(Fa(), T());
+            else clusters(Fa(), Fa());
         } else {
-            if (chk) screen4(T(), T());
-            else screen4(T(), Fa());
+            if (ex) clusters(T(), T());
+            else clusters(T(), Fa());
         }
-        lds_order();
-        evaluate(tail - head);  // the tile's remaining pairs (its j records change next)
     }
     e = wave_sum(e);
     if (lane == 0) e_out[(size_t)rb * split + part] = e;
