@@ -176,6 +176,10 @@ struct sdm_context {
     size_t sel_cap = 0;
     // this device's `scratch` (selection staging of the allocation-free adjoint)
     int32_t* scratch_sel = nullptr;
+    // partials of the adjoint kernels (k_adj): at least one tile of selected atoms of a frame
+    double* adj_part = nullptr;
+    size_t adj_cap = 0;
+    std::vector<int> h_cls;  // displacement class of each atom (0: not displaced)
     sdm_tuning tune{1, 0, 1, 1, 0, 20, 0, 4, 1, 0.f};
     // steps evaluated in the current slot order (0: stale, the next evaluation sorts)
     int since_sort = 0;
@@ -923,6 +927,12 @@ int sdm_create(const sdm_system_desc* sys, int32_t n_replicas, sdm_context** out
     A(dA, (size_t)R * c->maxc * c->LB * 64); A(dlig, (size_t)R * std::max(1, c->L));
     A(mlig, (size_t)R * c->maxc * std::max(1, c->L));
     A(dB, (size_t)R * c->maxc * 64); A(state, R); A(rec, R); A(flags, R);
+    if (c->L > 0) {
+        c->adj_cap = std::max<size_t>(1 << 20, (size_t)((N + ADJ_ATOMS - 1) / ADJ_ATOMS) *
+                                                   std::max(ADJ_PART, (c->L + ADJ_SEL - 1) / ADJ_SEL));
+        A(adj_part, c->adj_cap);
+    }
+    c->h_cls = cls;
     A(uhist, (size_t)R * c->hist_cap); A(counters, 2 * (size_t)R); A(ke_out, R);
 #undef A
     // topology upload
@@ -1982,21 +1992,56 @@ int sdm_autotune(sdm_context* c, int32_t steps, sdm_tuning* chosen) {
 
 }  // extern "C"
 
-// The adjoint's kernels for a selection already staged on the device at d_sel.
+// The adjoint's kernels for a selection already staged on the device at d_sel (h_sel: the
+// same on the host).  Frames go in batches whose partials fit the context's buffer; the
+// results do not depend on the batches.
 static int du_dparams_launch(sdm_context* c, const double* d_frames, int32_t nframes,
-                             const int32_t* d_sel, int32_t nsel, double* d_grad, double* d_u) {
-    if (d_u && c->L > 0)
-        k_u_frames<<<nframes, 256, 0, c->stream>>>(c->N, c->L, c->lig, c->cls, c->cdispl, c->q64,
-                                                   c->sig64, c->eps64, c->ex_start, c->ex_list,
-                                                   d_frames, d_u, c->g);
-    else if (d_u)
-        k_fill_d<<<(nframes + 255) / 256, 256, 0, c->stream>>>(d_u, (size_t)nframes);
-    if (d_grad)
-        k_du_dparams<<<dim3(nsel, nframes), 64, 0, c->stream>>>(
-            c->N, d_sel, nsel, c->cls, c->cdispl, c->q64, c->sig64, c->eps64, c->ex_start,
-            c->ex_list, d_frames, d_grad, c->g);
+                             const int32_t* h_sel, const int32_t* d_sel, int32_t nsel,
+                             double* d_grad, double* d_u) {
+    const int N = c->N, nchunk = (N + ADJ_ATOMS - 1) / ADJ_ATOMS;
+    hipStream_t st = c->stream;
+    if (d_u && c->L > 0) {
+        const int ntile = (c->L + ADJ_SEL - 1) / ADJ_SEL, np = ntile * nchunk;
+        const int fb = (int)std::min<size_t>(32768, std::max<size_t>(1, c->adj_cap / np));
+        for (int f0 = 0; f0 < nframes; f0 += fb) {
+            const int nf = std::min(fb, nframes - f0);
+            k_adj<false><<<dim3(nchunk, nf, ntile), ADJ_ATOMS, 0, st>>>(
+                N, c->L, c->ncls, c->lig, c->L, c->lig, c->cls, c->cdispl, c->q64, c->sig64,
+                c->eps64, c->ex_start, c->ex_list, d_frames + (size_t)f0 * 3 * N, 0,
+                c->adj_part, c->g);
+            k_adj_u<<<nf, 64, 0, st>>>(np, c->adj_part, d_u + f0);
+        }
+    } else if (d_u) {
+        k_fill_d<<<(nframes + 255) / 256, 256, 0, st>>>(d_u, (size_t)nframes);
+    }
+    bool env = false, displaced = false;
+    for (int k = 0; k < nsel && d_grad; k++) (c->h_cls[h_sel[k]] ? displaced : env) = true;
+    if (displaced) {
+        // tiles of the selection per launch, and frames per launch, that fit the buffer
+        const int ntile = (nsel + ADJ_SEL - 1) / ADJ_SEL;
+        const size_t one = (size_t)nchunk * ADJ_PART;
+        const int tb = (int)std::min<size_t>(std::min(ntile, 32768), c->adj_cap / one);
+        const int fb = tb < ntile ? 1 : (int)std::min<size_t>(32768, c->adj_cap / (one * ntile));
+        for (int f0 = 0; f0 < nframes; f0 += fb)
+            for (int t0 = 0; t0 < ntile; t0 += tb) {
+                const int nf = std::min(fb, nframes - f0), nt = std::min(tb, ntile - t0);
+                k_adj<true><<<dim3(nchunk, nf, nt), ADJ_ATOMS, 0, st>>>(
+                    N, c->L, c->ncls, d_sel, nsel, c->lig, c->cls, c->cdispl, c->q64, c->sig64,
+                    c->eps64, c->ex_start, c->ex_list, d_frames + (size_t)f0 * 3 * N, t0,
+                    c->adj_part, c->g);
+                k_adj_grad<<<dim3(3, nf, nt), 256, 0, st>>>(nchunk, d_sel, nsel, c->cls, t0,
+                                                            c->adj_part,
+                                                            d_grad + (size_t)f0 * 3 * nsel);
+            }
+    }
+    if (env)
+        for (int f0 = 0; f0 < nframes; f0 += 32768)
+            k_adj_env<<<dim3(nsel, std::min(32768, nframes - f0)), 64, 0, st>>>(
+                N, c->L, d_sel, nsel, c->lig, c->cls, c->cdispl, c->q64, c->sig64, c->eps64,
+                c->ex_start, c->ex_list, d_frames + (size_t)f0 * 3 * N,
+                d_grad + (size_t)f0 * 3 * nsel, c->g);
     CHK(check_launch());
-    HIPCHK(hipStreamSynchronize(c->stream));
+    HIPCHK(hipStreamSynchronize(st));
     return SDM_OK;
 }
 
@@ -2026,7 +2071,7 @@ int sdm_du_dparams_frames(sdm_context* c, const double* d_frames, int32_t nframe
         }
         HIPCHK(hipMemcpyAsync(c->sel_dev, sel, sizeof(int) * nsel, hipMemcpyHostToDevice, c->stream));
     }
-    return du_dparams_launch(c, d_frames, nframes, c->sel_dev, nsel, d_grad, d_u);
+    return du_dparams_launch(c, d_frames, nframes, sel, c->sel_dev, nsel, d_grad, d_u);
 }
 
 int sdm_du_dparams_frames_noalloc(sdm_context* c, const double* d_frames, int32_t nframes,
@@ -2042,7 +2087,7 @@ int sdm_du_dparams_frames_noalloc(sdm_context* c, const double* d_frames, int32_
     if (d_grad)
         HIPCHK(hipMemcpyAsync(c->scratch_sel, sel, sizeof(int32_t) * nsel,
                               hipMemcpyHostToDevice, c->stream));
-    return du_dparams_launch(c, d_frames, nframes, c->scratch_sel, nsel, d_grad, d_u);
+    return du_dparams_launch(c, d_frames, nframes, sel, c->scratch_sel, nsel, d_grad, d_u);
 }
 
 void registerPlatforms(void) {}

@@ -2558,6 +2558,21 @@ __global__ __launch_bounds__(256) void k_kinetic(
 // ---------------------------------------------------------------------------
 // adjoint (parameter gradients of u over many frames).  Frames are [F][N][3] doubles in
 // atom order; pair terms are recomputed from the positions, never stored.
+//
+// k_adj: one workgroup per (256 atoms of a frame, frame, 64 selected atoms).  Its atoms
+// within reach of a displaced class (its box at x or at x+d, FP64, any image) are listed in
+// LDS with their parameters, in atom order; then lanes = selected atoms and the listed
+// atoms are taken one after the other (LDS broadcasts), so every selected atom's sums have
+// one owner and no cross-lane reduction: the parts of the list that the workgroup's waves
+// (or, for 32 selected atoms or fewer, parts of waves) take are added in order.  One partial
+// per workgroup goes to the context's buffer and k_adj_u / k_adj_grad add the frame's
+// partials in order: bit-reproducible, whatever number of frames fits the buffer.
+//   GRAD = false: u (selected = the displaced atoms; pairs of two displaced atoms once).
+//   GRAD = true: du/d(q, sigma, eps) of the selected atoms that are displaced.
+// What bounds it: FP64 issue on the listed pairs.  One workgroup per frame over all (displaced
+// atom, atom) pairs with an integer division each left 3/4 of the GPU idle and took 8.1 ms
+// for u and 0.60 ms for the gradient (a wave per selected atom and frame over all atoms) for
+// 64 frames of 22,750 atoms with 50 displaced; 481 and 80 us for 3,000 atoms with 30.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ void load_frame_atom(const double* __restrict__ X, int a, double& x,
                                                 double& y, double& z) {
@@ -2566,95 +2581,268 @@ __device__ __forceinline__ void load_frame_atom(const double* __restrict__ X, in
     z = X[3 * a + 2];
 }
 
-// u of every frame: one workgroup per frame, pairs (displaced atom i, atom j) with
-// d_i != d_j, displaced-displaced pairs once
-__global__ __launch_bounds__(256) void k_u_frames(
-    int N, int L, const int* __restrict__ lig, const int* __restrict__ cls,
-    const double* __restrict__ cdispl, const double* __restrict__ q64,
-    const double* __restrict__ sig64, const double* __restrict__ eps64,
-    const int* __restrict__ ex_start, const int* __restrict__ ex_list,
-    const double* __restrict__ frames, double* __restrict__ u_out, Geom g) {
-    __shared__ double red[256];
-    int f = blockIdx.x, t = threadIdx.x;
-    const double* X = frames + (size_t)f * 3 * N;
-    double acc = 0.0;
-    for (long long idx = t; idx < (long long)L * N; idx += 256) {
-        int i = lig[idx / N];
-        int j = (int)(idx % N);
-        int ci = cls[i], cj = cls[j];
-        if (ci == cj || (cj != 0 && j < i)) continue;
-        if (excluded(ex_start, ex_list, i, j)) continue;
-        Atom64 I, J;
-        load_frame_atom(X, i, I.x, I.y, I.z);
-        load_frame_atom(X, j, J.x, J.y, J.z);
-        I.dx = cdispl[3 * ci]; I.dy = cdispl[3 * ci + 1]; I.dz = cdispl[3 * ci + 2];
-        J.dx = cdispl[3 * cj]; J.dy = cdispl[3 * cj + 1]; J.dz = cdispl[3 * cj + 2];
-        I.qk = q64[i]; I.sig = sig64[i]; I.se = sqrt(eps64[i]);
-        J.qk = q64[j]; J.sig = sig64[j]; J.se = sqrt(eps64[j]);
-        double fx = 0, fy = 0, fz = 0;
-        int iny;
-        acc += delta_pair(I, J, g, fx, fy, fz, &iny);
-    }
-    red[t] = acc;
-    __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if (t < o) red[t] += red[t + o];
-        __syncthreads();
-    }
-    if (t == 0) u_out[f] = red[0];
-}
+constexpr int ADJ_ATOMS = 256;  // atoms (and threads) per workgroup
+constexpr int ADJ_SEL = 64;     // selected atoms per workgroup
+constexpr int ADJ_PART = 3 * ADJ_SEL;  // doubles of a workgroup's gradient partial
 
-// du/d(q_s, sigma_s, eps_s) for selected atom s in frame f: one wave per (s, f)
-__global__ __launch_bounds__(64) void k_du_dparams(
-    int N, const int* __restrict__ sel, int nsel, const int* __restrict__ cls,
-    const double* __restrict__ cdispl, const double* __restrict__ q64,
-    const double* __restrict__ sig64, const double* __restrict__ eps64,
-    const int* __restrict__ ex_start, const int* __restrict__ ex_list,
-    const double* __restrict__ frames, double* __restrict__ grad, Geom g) {
-    int k = blockIdx.x, f = blockIdx.y, lane = threadIdx.x;
-    int s = sel[k];
-    const double* X = frames + (size_t)f * 3 * N;
-    int cs = cls[s];
-    double xs, ys, zs;
-    load_frame_atom(X, s, xs, ys, zs);
-    const double ske = sqrt(SDM_ONE_4PI_EPS0);
-    double dq = 0.0, dsig = 0.0, deps = 0.0;
-    for (int j = lane; j < N; j += 64) {
-        int cj = cls[j];
-        if (cj == cs || excluded(ex_start, ex_list, s, j)) continue;
-        double xj, yj, zj;
-        load_frame_atom(X, j, xj, yj, zj);
-        double sig = g.geo ? sqrt(sig64[s] * sig64[j]) : 0.5 * (sig64[s] + sig64[j]);
-        double eps = sqrt(eps64[s] * eps64[j]);
-        // d sigma_sj / d sigma_s: 1/2, or sigma_j / (2 sigma_sj) for the geometric rule
-        // (zero with sigma_sj = 0, where the LJ terms vanish)
-        const double dsds = g.geo ? (sig > 0.0 ? sig64[j] / (2.0 * sig) : 0.0) : 0.5;
-        const bool lj = !g.geo || sig > 0.0;
-        for (int geo = 0; geo < 2; geo++) {  // geo 0: at x (sign -), geo 1: at x+d (sign +)
-            double dx = min_image((xs + (geo ? cdispl[3 * cs] : 0.0)) - (xj + (geo ? cdispl[3 * cj] : 0.0)), g.Lx, g.iLx);
-            double dy = min_image((ys + (geo ? cdispl[3 * cs + 1] : 0.0)) - (yj + (geo ? cdispl[3 * cj + 1] : 0.0)), g.Ly, g.iLy);
-            double dz = min_image((zs + (geo ? cdispl[3 * cs + 2] : 0.0)) - (zj + (geo ? cdispl[3 * cj + 2] : 0.0)), g.Lz, g.iLz);
-            double r2 = dx * dx + dy * dy + dz * dz;
-            if (!(r2 < g.rc2)) continue;
-            double sgn = geo ? 1.0 : -1.0;
-            double ir = 1.0 / sqrt(r2);
-            double s2 = sig * sig / r2;
-            double s6 = s2 * s2 * s2;
-            double s12 = s6 * s6;
-            // q64 holds q*sqrt(k_e): d(k_e q_s q_j f)/dq_s = sqrt(k_e) * q64[j] * f
-            dq += sgn * ske * q64[j] * (ir + g.krf * r2 - g.crf);
-            if (lj) dsig += sgn * dsds * 4.0 * eps * (12.0 * s12 - 6.0 * s6) / sig;
-            if (eps > 0.0) deps += sgn * 4.0 * (s12 - s6) * eps64[j] / (2.0 * eps);
+// what the two geometries of one pair (I displaced by I.d, J by J.d) add to the sums
+struct AdjSums {
+    double u, q, s, e;
+};
+
+template <bool GRAD>
+__device__ __forceinline__ void adj_pair(const Atom64& I, const Atom64& J, const Geom& g, AdjSums& a) {
+    double ex = min_image(I.x - J.x, g.Lx, g.iLx), ey = min_image(I.y - J.y, g.Ly, g.iLy),
+           ez = min_image(I.z - J.z, g.Lz, g.iLz);
+    const double r0 = ex * ex + ey * ey + ez * ez;
+    ex = min_image((I.x + I.dx) - (J.x + J.dx), g.Lx, g.iLx);
+    ey = min_image((I.y + I.dy) - (J.y + J.dy), g.Ly, g.iLy);
+    ez = min_image((I.z + I.dz) - (J.z + J.dz), g.Lz, g.iLz);
+    const double r1 = ex * ex + ey * ey + ez * ez;
+    if (!(r0 < g.rc2) && !(r1 < g.rc2)) return;
+    const double sig = g.geo ? sqrt(I.sig * J.sig) : 0.5 * (I.sig + J.sig);
+    const double sig2 = sig * sig;
+    double c = 0.0, A = 0.0, B = 0.0;  // sums over the geometries, x with sign -
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+        const double r2 = t ? r1 : r0, sgn = t ? 1.0 : -1.0;
+        if (r2 < g.rc2) {
+            const double ir = rsqrt(r2);
+            const double s2 = sig2 * (ir * ir);
+            const double s6 = s2 * s2 * s2;
+            c += sgn * (ir + g.krf * r2 - g.crf);
+            B += sgn * (s6 * (s6 - 1.0));
+            if (GRAD) A += sgn * (s6 * (12.0 * s6 - 6.0));
         }
     }
-    dq = wave_sum(dq);
-    dsig = wave_sum(dsig);
-    deps = wave_sum(deps);
+    if (GRAD) {
+        a.q += J.qk * c;
+        a.e += J.se * B;
+        // d sigma_ij / d sigma_i / sigma_ij: 1 / (2 sigma_ij), or 1 / (2 sigma_i) for the
+        // geometric rule (the terms vanish with sigma_ij = 0)
+        if (sig > 0.0) a.s += J.se * A / (g.geo ? I.sig : sig);
+    } else {
+        a.u += 4.0 * I.se * J.se * B + I.qk * J.qk * c;
+    }
+}
+
+template <bool GRAD>
+__global__ __launch_bounds__(ADJ_ATOMS) void k_adj(
+    int N, int L, int ncls, const int* __restrict__ sel, int nsel, const int* __restrict__ lig,
+    const int* __restrict__ cls, const double* __restrict__ cdispl,
+    const double* __restrict__ q64, const double* __restrict__ sig64,
+    const double* __restrict__ eps64, const int* __restrict__ ex_start,
+    const int* __restrict__ ex_list, const double* __restrict__ frames, int tile0,
+    double* __restrict__ part, Geom g) {
+    constexpr int NW = ADJ_ATOMS / 64;
+    __shared__ double box[SDM_MAX_CLASSES][6];  // per class: centre and half extent
+    __shared__ double jx[ADJ_ATOMS], jy[ADJ_ATOMS], jz[ADJ_ATOMS], jq[ADJ_ATOMS], js[ADJ_ATOMS],
+        je[ADJ_ATOMS];
+    __shared__ int jc[ADJ_ATOMS], ji[ADJ_ATOMS];
+    __shared__ double red[GRAD ? 3 : 1][ADJ_ATOMS];
+    __shared__ int wcount[NW];
+    const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+    const int chunk = blockIdx.x, f = blockIdx.y, tile = tile0 + blockIdx.z;
+    const double* X = frames + (size_t)f * 3 * N;
+    for (int k = 1 + wv; k <= ncls; k += NW) {
+        double v[6] = {1e300, 1e300, 1e300, -1e300, -1e300, -1e300};
+        for (int li = lane; li < L; li += 64) {
+            const int a = lig[li];
+            if (cls[a] != k) continue;
+            for (int d = 0; d < 3; d++) {
+                v[d] = fmin(v[d], X[3 * a + d]);
+                v[3 + d] = fmax(v[3 + d], X[3 * a + d]);
+            }
+        }
+        for (int d = 0; d < 3; d++) {
+            const double lo = wave_min_d(v[d]), hi = wave_max_d(v[3 + d]);
+            if (lane == 0) {
+                box[k - 1][d] = 0.5 * (lo + hi);
+                box[k - 1][3 + d] = 0.5 * (hi - lo);
+            }
+        }
+    }
+    __syncthreads();
+    // the chunk's atoms that can have a partner
+    const int j = chunk * ADJ_ATOMS + t;
+    bool near = false;
+    double xj = 0.0, yj = 0.0, zj = 0.0;
+    int cj = 0;
+    if (j < N) {
+        load_frame_atom(X, j, xj, yj, zj);
+        cj = cls[j];
+        const double reach = sqrt(g.rc2) + 1e-6, reach2 = reach * reach;
+        const double* dj = cdispl + 3 * cj;
+        for (int k = 1; k <= ncls; k++) {
+            if (k == cj) continue;
+            const double* dk = cdispl + 3 * k;
+            const double* b = box[k - 1];
+            for (int geo = 0; geo < 2; geo++) {  // at x, at x + d
+                const double dx = xj - b[0] + (geo ? dj[0] - dk[0] : 0.0),
+                             dy = yj - b[1] + (geo ? dj[1] - dk[1] : 0.0),
+                             dz = zj - b[2] + (geo ? dj[2] - dk[2] : 0.0);
+                const double gx = fmax(fabs(min_image(dx, g.Lx, g.iLx)) - b[3], 0.0),
+                             gy = fmax(fabs(min_image(dy, g.Ly, g.iLy)) - b[4], 0.0),
+                             gz = fmax(fabs(min_image(dz, g.Lz, g.iLz)) - b[5], 0.0);
+                near = near || !(gx * gx + gy * gy + gz * gz >= reach2);
+            }
+        }
+    }
+    const unsigned long long m = __ballot(near);
+    if (lane == 0) wcount[wv] = __popcll(m);
+    __syncthreads();
+    int n = 0, pos = lane_rank(m);
+    for (int w = 0; w < NW; w++) {
+        if (w < wv) pos += wcount[w];
+        n += wcount[w];
+    }
+    if (near) {
+        jx[pos] = xj;
+        jy[pos] = yj;
+        jz[pos] = zj;
+        jq[pos] = q64[j];
+        js[pos] = sig64[j];
+        je[pos] = sqrt(eps64[j]);
+        jc[pos] = cj;
+        ji[pos] = j;
+    }
+    __syncthreads();
+    // lanes = selected atoms; the list in 256 / W parts
+    const int ns = min(ADJ_SEL, nsel - tile * ADJ_SEL);
+    const int W = ns <= 16 ? 16 : ns <= 32 ? 32 : 64;
+    const int k = t & (W - 1), p = t / W, parts = ADJ_ATOMS / W;
+    AdjSums a{0.0, 0.0, 0.0, 0.0};
+    double ise = 0.0, ses = 0.0;
+    if (k < ns && n > 0) {
+        const int i = sel[tile * ADJ_SEL + k];
+        const int ci = cls[i];
+        if (ci != 0) {
+            Atom64 I;
+            load_frame_atom(X, i, I.x, I.y, I.z);
+            I.dx = cdispl[3 * ci];
+            I.dy = cdispl[3 * ci + 1];
+            I.dz = cdispl[3 * ci + 2];
+            I.qk = q64[i];
+            I.sig = sig64[i];
+            I.se = sqrt(eps64[i]);
+            const int e0 = ex_start[i], e1 = ex_start[i + 1];
+            // exclusions across classes are rare: only atoms that have one search their list
+            bool exI = false;
+            for (int q = e0; q < e1; q++) exI = exI || cls[ex_list[q]] != ci;
+            for (int e = p; e < n; e += parts) {
+                const int cq = jc[e], jj = ji[e];
+                if (cq == ci || (!GRAD && cq != 0 && jj < i)) continue;
+                if (exI && excluded(ex_start, ex_list, i, jj)) continue;
+                Atom64 J;
+                J.x = jx[e];
+                J.y = jy[e];
+                J.z = jz[e];
+                J.dx = cdispl[3 * cq];
+                J.dy = cdispl[3 * cq + 1];
+                J.dz = cdispl[3 * cq + 2];
+                J.qk = jq[e];
+                J.sig = js[e];
+                J.se = je[e];
+                adj_pair<GRAD>(I, J, g, a);
+            }
+            ses = I.se;
+            ise = I.se > 0.0 ? 1.0 / I.se : 0.0;
+        }
+    }
+    if (GRAD) {
+        red[0][t] = sqrt(SDM_ONE_4PI_EPS0) * a.q;  // q64 holds q sqrt(k_e)
+        red[1][t] = 2.0 * ses * a.s;
+        red[2][t] = 2.0 * ise * a.e;
+        __syncthreads();
+        if (p == 0) {
+            double* o = part + (((size_t)f * gridDim.z + blockIdx.z) * gridDim.x + chunk) * ADJ_PART;
+            for (int c = 0; c < 3; c++) {
+                double v = 0.0;
+                for (int q = 0; q < parts; q++) v += red[c][q * W + k];
+                o[c * ADJ_SEL + k] = v;
+            }
+        }
+    } else {
+        red[0][t] = a.u;
+        __syncthreads();
+        for (int o = ADJ_ATOMS / 2; o > 0; o >>= 1) {
+            if (t < o) red[0][t] += red[0][t + o];
+            __syncthreads();
+        }
+        if (t == 0) part[((size_t)f * gridDim.z + blockIdx.z) * gridDim.x + chunk] = red[0][0];
+    }
+}
+
+// u of frame f: its np partials in order (one wave per frame, a lane's in stride 64)
+__global__ __launch_bounds__(64) void k_adj_u(int np, const double* __restrict__ part,
+                                              double* __restrict__ u_out) {
+    const int f = blockIdx.x;
+    double v = 0.0;
+    for (int k = threadIdx.x; k < np; k += 64) v += part[(size_t)f * np + k];
+    v = wave_sum(v);
+    if (threadIdx.x == 0) u_out[f] = v;
+}
+
+// one component of the gradient of 64 selected atoms in a frame: the chunks' partials in
+// four interleaved runs, added in order; atoms that are not displaced are left to k_adj_env
+__global__ __launch_bounds__(256) void k_adj_grad(int nchunk, const int* __restrict__ sel, int nsel,
+                                                  const int* __restrict__ cls, int tile0,
+                                                  const double* __restrict__ part,
+                                                  double* __restrict__ grad) {
+    __shared__ double red[4][64];
+    const int c = blockIdx.x, f = blockIdx.y, k = threadIdx.x & 63, p = threadIdx.x >> 6;
+    const double* P = part + ((size_t)f * gridDim.z + blockIdx.z) * nchunk * ADJ_PART + c * ADJ_SEL + k;
+    const int s = (tile0 + blockIdx.z) * ADJ_SEL + k;
+    const bool mine = s < nsel && cls[sel[s]] != 0;
+    double v = 0.0;
+    if (mine)
+#pragma unroll 4
+        for (int q = p; q < nchunk; q += 4) v += P[(size_t)q * ADJ_PART];
+    red[p][k] = v;
+    __syncthreads();
+    if (p == 0 && mine)
+        grad[((size_t)f * nsel + s) * 3 + c] = ((red[0][k] + red[1][k]) + red[2][k]) + red[3][k];
+}
+
+// du/d(q, sigma, eps) of a selected atom that is not displaced: its partners are the
+// displaced atoms.  One wave per (selected atom, frame)
+__global__ __launch_bounds__(64) void k_adj_env(
+    int N, int L, const int* __restrict__ sel, int nsel, const int* __restrict__ lig,
+    const int* __restrict__ cls, const double* __restrict__ cdispl,
+    const double* __restrict__ q64, const double* __restrict__ sig64,
+    const double* __restrict__ eps64, const int* __restrict__ ex_start,
+    const int* __restrict__ ex_list, const double* __restrict__ frames,
+    double* __restrict__ grad, Geom g) {
+    const int k = blockIdx.x, f = blockIdx.y, lane = threadIdx.x;
+    const int s = sel[k];
+    if (cls[s] != 0) return;
+    const double* X = frames + (size_t)f * 3 * N;
+    Atom64 I;
+    load_frame_atom(X, s, I.x, I.y, I.z);
+    I.dx = I.dy = I.dz = 0.0;
+    I.qk = q64[s];
+    I.sig = sig64[s];
+    I.se = sqrt(eps64[s]);
+    AdjSums a{0.0, 0.0, 0.0, 0.0};
+    for (int li = lane; li < L; li += 64) {
+        const int j = lig[li], cj = cls[j];
+        if (excluded(ex_start, ex_list, s, j)) continue;
+        Atom64 J;
+        load_frame_atom(X, j, J.x, J.y, J.z);
+        J.dx = cdispl[3 * cj];
+        J.dy = cdispl[3 * cj + 1];
+        J.dz = cdispl[3 * cj + 2];
+        J.qk = q64[j];
+        J.sig = sig64[j];
+        J.se = sqrt(eps64[j]);
+        adj_pair<true>(I, J, g, a);
+    }
+    const double dq = wave_sum(a.q), ds = wave_sum(a.s), de = wave_sum(a.e);
     if (lane == 0) {
         double* o = grad + ((size_t)f * nsel + k) * 3;
-        o[0] = dq;
-        o[1] = dsig;
-        o[2] = deps;
+        o[0] = sqrt(SDM_ONE_4PI_EPS0) * dq;
+        o[1] = 2.0 * I.se * ds;
+        o[2] = I.se > 0.0 ? 2.0 / I.se * de : 0.0;
     }
 }
 
