@@ -163,7 +163,9 @@ typedef struct {
                                      over the FP64 positions (their own kernel); the
                                      forces are FP32 pair arithmetic. */
     int32_t pair_split;           /* with pair_newton3 1 and pair_group 0: 1, 2, 4 (the
-                                     default), 8, 16 or 32 waves per i-block, each taking every
+                                     default), 8, 16 or 32 waves per i-block (at least:
+                                     systems of fewer than 512 blocks of 64 atoms get more,
+                                     except with 1), each taking every
                                      pair_split-th tile, so that short tile lists do not
                                      leave the GPU waiting on long ones and small batches
                                      fill it.

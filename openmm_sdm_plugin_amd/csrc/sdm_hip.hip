@@ -109,10 +109,9 @@ struct sdm_context {
     double* Fb = nullptr;  // [R][3][Np] FP64 bonded forces, atom order
     // per replica
     double *x64 = nullptr, *v64 = nullptr;
-    float4* arec = nullptr;  // [R][Np][2] slot records of the pair kernel, coordinates
-                             // relative to the block's reference
-    double4* bref = nullptr; // [R][NB] the blocks' references (first atom)
+    float4* arec = nullptr;  // [R][Np][2] slot records of the pair kernel
     int *orig_s = nullptr, *slot_of = nullptr, *key = nullptr;
+    int* bfirst = nullptr;   // [R][NB] atom that a kept block's images are taken about
     int *ccount = nullptr, *cstart = nullptr, *cfill = nullptr;
     float4 *bb_lo = nullptr, *bb_hi = nullptr;
     int* exs = nullptr;      // [R][NB][max_ex][64] exclusion partners in slot order (k_bbox)
@@ -128,7 +127,7 @@ struct sdm_context {
                             // or stale after a sort (k_bbox)
     long long* F = nullptr;
     double *e_bond = nullptr, *u_part = nullptr;
-    double* e64 = nullptr;  // [R][NB * E64_SPLIT] FP64 pair-energy slots
+    double* e64 = nullptr;  // FP64 pair-energy slots, one per wave of k_energy64
     // SDMUtils restraints (group 1): centroid and alignment terms, their group atoms and
     // normalized weights, and one energy slot per (replica, restraint)
     DevCentroid* rcen = nullptr;
@@ -379,9 +378,9 @@ void enqueue_order(sdm_context* c, bool full, bool energy = false) {
     Rec64* rec = energy ? c->rec64 : nullptr;
 #define SDM_REFRESH(SORT)                                                                      \
     k_refresh<SORT><<<dim3(c->NB, R), 64, 0, s>>>(                                             \
-        N, Np, c->NB, c->x64, c->orig_s, c->qs, c->sh, c->se, c->g, c->arec, c->bref, c->F,    \
+        N, Np, c->NB, c->x64, c->orig_s, c->qs, c->sh, c->se, c->g, c->arec, c->F,             \
         c->bb_lo, c->bb_hi, c->cbox, c->par64, rec, lists_kept(c) ? c->xb : nullptr, c->dmax,  \
-        c->slot_of, c->ex_start, c->ex_list, c->max_ex, c->exs, c->exblocks)
+        c->slot_of, c->bfirst, c->ex_start, c->ex_list, c->max_ex, c->exs, c->exblocks)
     if (!full) {
         SDM_REFRESH(false);
         return;
@@ -391,7 +390,8 @@ void enqueue_order(sdm_context* c, bool full, bool energy = false) {
     k_scan<<<R, 1024, 0, s>>>(c->NC, c->ccount, c->cstart, c->cfill);
     k_scatter<<<g2(N, 256, R), 256, 0, s>>>(N, Np, c->NC, c->key, c->cstart, c->cfill, c->orig_s);
     k_cellsort<<<g2(c->NC, 128, R), 128, 0, s>>>(N, Np, c->NC, c->cstart, c->orig_s);
-    k_blockorder<<<dim3(c->NB, R), 64, 0, s>>>(N, Np, c->x64, c->orig_s, c->slot_of, c->g);
+    k_blockorder<<<dim3(c->NB, R), 64, 0, s>>>(N, Np, c->x64, c->orig_s, c->slot_of,
+                                                c->bfirst, c->g);
     SDM_REFRESH(true);
 #undef SDM_REFRESH
 }
@@ -423,7 +423,7 @@ void enqueue_tiles(sdm_context* c) {
     // replicas -1% with 8).
 #define SDM_TILES(NW)                                                                         \
     k_tiles<NW><<<dim3(c->NB, c->R), 64 * NW, 0, c->stream>>>(                                \
-        c->N, c->Np, c->NB, c->maxj, c->arec, c->bref, c->bb_lo, c->bb_hi, c->cbox, c->tiles,  \
+        c->N, c->Np, c->NB, c->maxj, c->arec, c->bb_lo, c->bb_hi, c->cbox, c->tiles,          \
         c->tmask, c->ntiles, c->dmax, c->xb, tr, c->g, c->flags)
     if (few_blocks(c)) SDM_TILES(8);
     else SDM_TILES(4);
@@ -436,27 +436,42 @@ void enqueue_sort(sdm_context* c, bool full) {
     enqueue_tiles(c);
 }
 
-// FP64 pair energies into e64 (needs the tile lists and FP64 records of this evaluation)
-void enqueue_energy64(sdm_context* c, hipStream_t st) {
-    unsigned waves = (unsigned)(c->R * c->NB * E64_SPLIT);
-    k_energy64<<<waves, 64, 0, st>>>(c->R, c->N, c->Np, c->NB, c->maxj, E64_SPLIT, c->rec64,
-                                     c->tiles, c->tmask, c->ntiles, c->bb_lo, c->bb_hi, c->exs,
-                                     c->exblocks, c->max_ex, c->e64, c->g);
+// Waves per i-block by the number of blocks of one replica: systems of few blocks have short
+// tile lists but leave most of the GPU idle with few waves.  The number of replicas does not
+// enter, so that a replica in a batch gives the bits of the same replica alone.  Pair kernel
+// measured alone (us), waves 4 / 8 / 16 / 32 per block: 3 blocks 19 / 19 / 19 / 19 (a tile is
+// what it waits for; in 4 parts: 11), 47 blocks 41 / 29 / 23 / 19 and 20 replicas of them 63 /
+// 60 / 57 / 59, 174 blocks 48 / 36 / 30 / 31, 350 blocks 54 / 43 / 40 / 41 and 4 replicas of
+// them 94 / 85 / 86 / 108, 22 replicas of 356 blocks 405 / 406 / 445 / -.
+TileShare block_share(const sdm_context* c) {
+    return {c->NB < 256 ? 16 : c->NB < 512 ? 8 : 4, c->NB <= 16 ? 4 : c->NB <= 32 ? 2 : 1};
 }
 
-// waves per i-block of the pair kernel (tuning.pair_split; 1 where tuning asks for the full
-// tile lists or the grouped form, for which pair_split has no meaning)
-int pair_waves(const sdm_context* c) {
-    return c->tune.pair_group == 0 && c->tune.pair_newton3 ? c->tune.pair_split : 1;
+// FP64 pair energies into e64 (needs the tile lists and FP64 records of this evaluation)
+void enqueue_energy64(sdm_context* c, hipStream_t st) {
+    const TileShare sh = block_share(c);
+    k_energy64<<<(unsigned)(c->R * c->NB * sh.waves()), 64, 0, st>>>(
+        c->R, c->N, c->Np, c->NB, c->maxj, sh, c->rec64, c->tiles, c->tmask, c->ntiles,
+        c->bb_lo, c->bb_hi, c->exs, c->exblocks, c->max_ex, c->e64, c->g);
+}
+
+// Waves of the pair kernel: tuning.pair_split, or more where block_share has more (one
+// where tuning asks for one, or for the full tile lists or the grouped form, for which
+// pair_split has no meaning).
+TileShare pair_share(const sdm_context* c) {
+    const int split = c->tune.pair_group == 0 && c->tune.pair_newton3 ? c->tune.pair_split : 1;
+    const TileShare sh = block_share(c);
+    return split == 1 ? TileShare{1, 1} : TileShare{std::max(split, sh.split), sh.sub};
 }
 
 template <int W, bool GEO>
 void launch_pair(sdm_context* c, bool count) {
-    const int split = pair_waves(c), waves = c->R * c->NB * split;
+    const TileShare sh = pair_share(c);
+    const int waves = c->R * c->NB * sh.waves();
     const dim3 gr((waves + W - 1) / W);
 #define SDM_PAIR(COUNT)                                                                       \
     k_pair<W, COUNT, GEO><<<gr, 64 * W, 0, c->stream>>>(                                      \
-        c->R, c->N, c->Np, c->NB, c->maxj, split, c->arec, c->bref, c->tiles, c->tmask,       \
+        c->R, c->N, c->Np, c->NB, c->maxj, sh, c->arec, c->tiles, c->tmask,                \
         c->ntiles, c->bb_lo, c->bb_hi, c->exs, c->exblocks, c->max_ex, c->F, c->flags, c->counters, c->g)
     if (count) SDM_PAIR(true);
     else SDM_PAIR(false);
@@ -585,7 +600,8 @@ void enqueue_eval(sdm_context* c, bool advance, bool components, bool full, bool
         (void)hipEventRecord(c->ev_join[1], s2);
         (void)hipStreamWaitEvent(s, c->ev_join[1], 0);
     }
-    k_scalar<<<R, 256, 0, s>>>(c->NB * E64_SPLIT, c->nbw, c->LB, c->e64, c->e_bond, c->u_part, c->state,
+    k_scalar<<<R, 256, 0, s>>>(c->NB * block_share(c).waves(), c->nbw, c->LB, c->e64,
+                               c->e_bond, c->u_part, c->state,
                                c->rec, c->flags, advance ? 1 : 0, energy ? 1 : 0,
                                c->hist_every, c->hist_cap, c->uhist, c->e_rest,
                                c->ncen + c->nali, c->e_t1, c->e_t2, c->ntb, c->dmax);
@@ -913,8 +929,7 @@ int sdm_create(const sdm_system_desc* sys, int32_t n_replicas, sdm_context** out
     A(astart, N + 1); A(acode, 3 * std::max(1, c->nang));
     if (c->nbond + c->nang > 0) A(Fb, 3 * RNp);
     A(x64, 3 * RNp); A(v64, 3 * RNp); A(arec, 2 * RNp);
-    A(bref, (size_t)R * NB);
-    A(orig_s, RNp);
+    A(orig_s, RNp); A(bfirst, (size_t)R * NB);
     A(slot_of, RNp); A(key, RNp); A(bb_lo, (size_t)R * NB); A(bb_hi, (size_t)R * NB);
     A(cbox, (size_t)R * NB * 16); A(exs, (size_t)RNp * c->max_ex); A(exblocks, (size_t)R * NB);
     A(tiles, (size_t)R * NB * c->maxj); A(tmask, (size_t)R * NB * c->maxj);
@@ -922,7 +937,7 @@ int sdm_create(const sdm_system_desc* sys, int32_t n_replicas, sdm_context** out
     A(cmap, (size_t)R * NB); A(lig_of, Np);
     A(ntiles, (size_t)R * NB); A(F, 3 * RNp);
     A(e_bond, (size_t)R * c->nbw); A(u_part, (size_t)R * c->LB);
-    A(e64, (size_t)R * NB * E64_SPLIT); A(rec64, RNp);
+    A(e64, (size_t)R * NB * block_share(c).waves()); A(rec64, RNp);
     A(cand, (size_t)R * c->maxc); A(ncand, R);
     A(dA, (size_t)R * c->maxc * c->LB * 64); A(dlig, (size_t)R * std::max(1, c->L));
     A(mlig, (size_t)R * c->maxc * std::max(1, c->L));

@@ -167,18 +167,22 @@ __global__ void k_cellsort(int N, int Np, int NC, const int* __restrict__ cstart
 // Orders the 64 slots of a block so that its clusters of 8 are compact: the block is split
 // at the median of its longest axis into halves of 32, these into 16 and these into 8 (one
 // wave per block, bitonic sorts of the axis' coordinate, ties by atom index, so that the
-// order is unique).  Writes the final orig_s and slot_of.  In a disordered 22,750-atom box
+// order is unique).  Writes the final orig_s and slot_of, and the atom that the periodic
+// images of the block's atoms are taken about until the next sort (bfirst, the first along
+// the curve).  In a disordered 22,750-atom box
 // (cells of 0.305 nm) it leaves 8% fewer pairs of clusters within the list radius and 5%
 // fewer with a pair within the cutoff than the order along the curve.
 __global__ __launch_bounds__(64) void k_blockorder(int N, int Np, const double* __restrict__ x64,
                                                    int* __restrict__ orig_s,
-                                                   int* __restrict__ slot_of, Geom g) {
+                                                   int* __restrict__ slot_of,
+                                                   int* __restrict__ bfirst, Geom g) {
     const int r = blockIdx.y, b = blockIdx.x, lane = threadIdx.x;
     const int sl = b * 64 + lane;
     int* O = orig_s + (size_t)r * Np;
     const double* X = x64 + (size_t)r * 3 * Np;
     const bool v = sl < N;
     int idx = v ? O[sl] : 0x7FFFFFFF;
+    if (lane == 0) bfirst[(size_t)r * gridDim.x + b] = idx;  // slot b * 64 is always below N
     float p[3] = {0.f, 0.f, 0.f};
     const double* L = &g.Lx;
     const double* iL = &g.iLx;
@@ -267,13 +271,11 @@ __device__ __forceinline__ void block_boxes(float4 p, bool v, int lane, float4* 
 }
 
 // The slot records of one evaluation.  One wave per 64-slot block gathers its atoms'
-// coordinates from the FP64 positions, each wrapped into the box and then to the periodic
-// image nearest the block's first atom, so a block stays compact when one of its atoms
-// crosses a face of the box; then the boxes of the block and its clusters are
-// computed and the slot-ordered force accumulator cleared.  The FP32 records hold
-// coordinates relative to the block's first atom (bref, FP64), both in whole QUANTUMs
-// (quantize), instead of coordinates in the box, whose FP32 rounding is 2e-7 nm and more.  Culling and pair distances take minimum images of box
-// centres or of pairs, so they hold for any image.
+// coordinates from the FP64 positions, wrapped into the box after a sort and then taken in
+// the periodic image nearest the block's atom bfirst, so a block stays compact when one of
+// its atoms crosses a face of the box; then the boxes of the block and its clusters are
+// computed and the slot-ordered force accumulator cleared.  Culling and pair distances take
+// minimum images of box centres or of pairs, so they hold for any image.
 //   SORT = true (after a sort; the slot order is new): also the records' parameters; the
 // replica's displacement record (dmax, read by k_tiles) is set to a value that makes the
 // next tile-list build unconditional; and the exclusions are written in slot order:
@@ -284,21 +286,15 @@ __device__ __forceinline__ void block_boxes(float4 p, bool v, int lane, float4* 
 // (atom, list start, list entry, slot), and only for the tiles that need them.
 //   SORT = false: the order of the last sort is kept; the displacement record of kept lists
 // is updated (xb, dmax).
-constexpr double QUANTUM = 1.0 / 8388608.0;  // 2^-23 nm
-// x in whole QUANTUMs.  Sums and differences of such numbers below 2 nm are exact in FP32, so
-// the separation of two atoms in range, whether it is within the cutoff, and the force have
-// the same bits in whatever blocks and images the atoms lie (the box length between two
-// images is taken in whole QUANTUMs too), at a rounding of at most 6e-8 nm.
-__device__ __forceinline__ double quantize(double x) { return rint(x * 8388608.0) * QUANTUM; }
-
 template <bool SORT>
 __global__ __launch_bounds__(64) void k_refresh(
     int N, int Np, int NB, const double* __restrict__ x64, const int* __restrict__ orig_s,
     const float* __restrict__ qs, const float* __restrict__ sh, const float* __restrict__ se,
-    Geom g, float4* __restrict__ arec, double4* __restrict__ bref, long long* __restrict__ F,
+    Geom g, float4* __restrict__ arec, long long* __restrict__ F,
     float4* __restrict__ bb_lo, float4* __restrict__ bb_hi, float4* __restrict__ cbox,
     const double4* __restrict__ par64, Rec64* __restrict__ rec, const float4* __restrict__ xb,
-    float* __restrict__ dmax, const int* __restrict__ slot_of, const int* __restrict__ ex_start,
+    float* __restrict__ dmax, const int* __restrict__ slot_of, const int* __restrict__ bfirst,
+    const int* __restrict__ ex_start,
     const int* __restrict__ ex_list, int max_ex, int* __restrict__ exs,
     unsigned long long* __restrict__ exblocks) {
     int r = blockIdx.y, b = blockIdx.x, lane = threadIdx.x;
@@ -307,26 +303,26 @@ __global__ __launch_bounds__(64) void k_refresh(
     const int* O = orig_s + (size_t)r * Np;
     const double* X = x64 + (size_t)r * 3 * Np;
     int i = O[v ? sl : b * 64];
-    double wx = X[i], wy = X[Np + i], wz = X[2 * Np + i];  // wrapped into the box
-    wx -= g.Lx * floor(wx * g.iLx);
-    wy -= g.Ly * floor(wy * g.iLy);
-    wz -= g.Lz * floor(wz * g.iLz);
-    const double rx = __shfl(wx, 0, 64), ry = __shfl(wy, 0, 64), rz = __shfl(wz, 0, 64);
-    // box lengths to the image nearest the first atom
-    const double kx = rint((wx - rx) * g.iLx), ky = rint((wy - ry) * g.iLy),
-                 kz = rint((wz - rz) * g.iLz);
-    const double qx = quantize(wx) - kx * quantize(g.Lx), qy = quantize(wy) - ky * quantize(g.Ly),
-                 qz = quantize(wz) - kz * quantize(g.Lz);
-    wx -= g.Lx * kx;
-    wy -= g.Ly * ky;
-    wz -= g.Lz * kz;
-    const float4 p = make_float4((float)wx, (float)wy, (float)wz, 0.f);
+    double wx = X[i], wy = X[Np + i], wz = X[2 * Np + i];
+    if (SORT) {
+        wx -= g.Lx * floor(wx * g.iLx);
+        wy -= g.Ly * floor(wy * g.iLy);
+        wz -= g.Lz * floor(wz * g.iLz);
+    } else {
+        const int f = bfirst[(size_t)r * NB + b];
+        double rx = X[f], ry = X[Np + f], rz = X[2 * Np + f];
+        rx -= g.Lx * floor(rx * g.iLx);
+        ry -= g.Ly * floor(ry * g.iLy);
+        rz -= g.Lz * floor(rz * g.iLz);
+        wx -= g.Lx * rint((wx - rx) * g.iLx);
+        wy -= g.Ly * rint((wy - ry) * g.iLy);
+        wz -= g.Lz * rint((wz - rz) * g.iLz);
+    }
+    const float4 p = make_float4((float)wx, (float)wy, (float)wz, qs[i]);
     size_t o = (size_t)r * Np + sl;
     const size_t bo = (size_t)r * NB + b;
-    const double bx = quantize(rx), by = quantize(ry), bz = quantize(rz);
-    if (lane == 0) bref[bo] = make_double4(bx, by, bz, 0.0);
     if (v) {
-        arec[2 * o] = make_float4((float)(qx - bx), (float)(qy - by), (float)(qz - bz), qs[i]);
+        arec[2 * o] = p;
         if (SORT) arec[2 * o + 1] = make_float4(sh[i], se[i], 0.f, 0.f);
         if (rec) {  // energy evaluations: the FP64 record in the same image
             double4 pr = par64[i];
@@ -425,7 +421,6 @@ __device__ __forceinline__ bool lists_tile(int ib, int jb) {
 template <int NW>  // waves per i-block workgroup
 __global__ __launch_bounds__(64 * NW) void k_tiles(int N, int Np, int NB, int maxj,
                                                const float4* __restrict__ arec,
-                                               const double4* __restrict__ bref,
                                                const float4* __restrict__ bb_lo,
                                                const float4* __restrict__ bb_hi,
                                                const float4* __restrict__ cbox,
@@ -449,11 +444,7 @@ __global__ __launch_bounds__(64 * NW) void k_tiles(int N, int Np, int NB, int ma
     const float4 li = lo[ib], hi_i = hi[ib];
     if (wave == 0 && tr.reuse_d2 >= 0.f) {  // the build coordinates
         int is = ib * 64 + lane;
-        const double4 o = bref[(size_t)r * NB + ib];
-        const float4 p = arec[2 * ((size_t)r * Np + min(is, N - 1))];
-        if (is < N)
-            xb[(size_t)r * Np + is] =
-                make_float4((float)(o.x + p.x), (float)(o.y + p.y), (float)(o.z + p.z), 0.f);
+        if (is < N) xb[(size_t)r * Np + is] = arec[2 * ((size_t)r * Np + is)];
     }
     // this lane's pair of clusters: ic of the i-block, jc of the candidate
     const int ic = lane & 7, jc = lane >> 3;
@@ -520,10 +511,9 @@ __global__ __launch_bounds__(64 * NW) void k_tiles(int N, int Np, int NB, int ma
 
 // ---------------------------------------------------------------------------
 // The pair kernel: F0 over all pairs at x, each pair once (Newton-3 over the tile lists).
-// One wave per (replica, i-block), or `split` waves per i-block, each taking every
-// split-th tile.  A wave holds the 64 i atoms as eight clusters of 8: lane 8 jl + il keeps
-// atom il of every cluster in registers, and takes one cluster of 8 j atoms at a time,
-// lane 8 jl + il holding j atom jl.  One step is a pair of clusters, 64 pairs on 64 lanes,
+// Each i-block has one wave or several (TileShare).  A wave holds the 64 i atoms as eight
+// clusters of 8: lane 8 jl + il keeps atom il of every cluster in registers, and takes one
+// cluster of 8 j atoms at a time, lane 8 jl + il holding j atom jl.  One step is a pair of clusters, 64 pairs on 64 lanes,
 // taken for the bits of the tile's mask (uniform branches).  A step none of whose pairs
 // is within the cutoff ends after the distance test.
 //   i forces: FP32 in the lane (24 registers), added up over the eight lanes that share an
@@ -533,16 +523,20 @@ __global__ __launch_bounds__(64 * NW) void k_tiles(int N, int Np, int NB, int ma
 //     atom, kept in registers over the tile and added to the slot-ordered int64 accumulator
 //     once per tile with coalesced atomics.
 // The periodic image is one shift per tile when that is exact for every pair within the
-// list radius (Geom::oix), otherwise the minimum image of each pair.  Fixed-point atomics
-// commute, so results are bit-reproducible.
+// list radius (Geom::oix), otherwise the minimum image of each pair.  The shift is taken off
+// the lower block's atoms, the i atoms (read from LDS again when it changes) or the j atoms,
+// because a separation in FP32 (2e-7 nm) decides what is within the cutoff, where the
+// reaction-field force ends with a step: coordinates relative to the block, with the shift in
+// the j atoms' offset, took 5% less time but rounded otherwise than the box's coordinates.
+// Fixed-point atomics commute, so results are bit-reproducible.
 //
 // What bounds it: VALU issue (89% of the cycles of 22 x 22,750 atoms, 4 waves per SIMD at
-// 127 registers).  A step takes 7 instructions to the distance test and 21 after it.  One
+// 123 registers).  A step takes 7 instructions to the distance test and 21 after it.  One
 // lane per i atom against one j atom at a time, the form before, took 37 instructions per 64
 // pairs with 22% of them within the cutoff; pairs of clusters have 30% (40% after the
 // distance test's early end) and no sum over the wave for each j atom.  Measured alone, 22
-// x 22,750 atoms: 532 -> 384 us (297M -> 201M VALU instructions); 8 x 99,920 atoms:
-// 1,054 -> 814 us; one replica of 22,750 atoms: 55 -> 43 us.  Where the i atoms' charges and
+// x 22,750 atoms: 532 -> 405 us (297M -> 201M VALU instructions); 8 x 99,920 atoms:
+// 1,054 -> 850 us; one replica of 22,750 atoms: 55 -> 44 us.  Where the i atoms' charges and
 // LJ parameters came from LDS instead (122 registers), or the j forces of four clusters were
 // summed together (as many instructions in all, 30% more code), it was 4% and 14% slower.
 // ---------------------------------------------------------------------------
@@ -609,7 +603,21 @@ __device__ __forceinline__ void scatter_clusters24(const float (&v)[24], int lan
 
 // pairs per FP32 partial sum of the i forces: about 16 terms per lane and i atom, as
 // many as the eight lanes that share it then add
-constexpr int PAIRS_PER_FLUSH = 8192;
+constexpr int PAIRS_PER_FLUSH = 4096;
+
+// How the tiles of an i-block are shared out: `split` waves take every split-th tile, and
+// with sub = 2, 4 or 8 each of them is sub waves that take the j clusters jc = part mod sub
+// of its tiles.
+struct TileShare {
+    int split, sub;
+    __host__ __device__ int waves() const { return split * sub; }
+};
+// the bits of a tile's mask that part `sp` of `sub` takes
+__device__ __forceinline__ unsigned long long sub_mask(int sub, int sp) {
+    const unsigned long long m = sub == 8 ? 0xffull : sub == 4 ? 0x000000ff000000ffull
+                                 : sub == 2 ? 0x00ff00ff00ff00ffull : ~0ull;
+    return m << (8 * sp);
+}
 
 // j atoms of block jb that i atom `lane` must not be paired with in this tile: exclusion
 // partners, in the diagonal tile the atoms up to itself, slots past N; everything for a
@@ -646,7 +654,7 @@ __device__ __forceinline__ bool tile_shift(float4 bli, float4 bhi, float4 blj, f
            fabsf(dcz - g.bz * kz) + 0.5f * (bhi.z - bli.z + bhj.z - blj.z) < g.oiz;
 }
 
-//   LDS per wave: two 2 KB tile buffers, 512 B of exclusion masks.
+//   LDS per wave: two 2 KB tile buffers, 512 B of exclusion masks, 768 B of i coordinates.
 //   vmcnt discipline: the only vector memory operations inside the tile loop are the
 //   next tile's copy (global -> LDS by DMA), the exclusion loads of the few tiles that have
 //   any, and the three flush atomics that end each tile.  Loads and stores/atomics share
@@ -655,23 +663,26 @@ __device__ __forceinline__ bool tile_shift(float4 bli, float4 bhi, float4 blj, f
 //   GEO: the geometric LJ sigma rule, the records holding sigma itself (Geom::geo).
 template <int WPW, bool COUNT, bool GEO>
 __global__ __launch_bounds__(64 * WPW) __attribute__((amdgpu_waves_per_eu(4))) void k_pair(
-    int R, int N, int Np, int NB, int maxj, int split, const float4* __restrict__ arec,
-    const double4* __restrict__ bref, const int* __restrict__ tiles, const unsigned long long* __restrict__ tmask,
+    int R, int N, int Np, int NB, int maxj, TileShare share, const float4* __restrict__ arec,
+    const int* __restrict__ tiles, const unsigned long long* __restrict__ tmask,
     const int* __restrict__ ntiles, const float4* __restrict__ bb_lo,
     const float4* __restrict__ bb_hi, const int* __restrict__ exs,
     const unsigned long long* __restrict__ exblocks, int max_ex, long long* __restrict__ F,
     int* __restrict__ flags, unsigned long long* __restrict__ pair_count, Geom g) {
     __shared__ float4 tile_s[WPW][2][128];
     __shared__ unsigned long long em_s[WPW][64];
+    __shared__ float xi_s[WPW][3][64];
     // wave-uniform by construction; readfirstlane lets the compiler keep everything
     // derived from it (replica, block, tile, mask) in scalar registers
     int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     int w = xcd_linear_id(blockIdx.x, gridDim.x) * WPW + wv;
     const int lane = threadIdx.x & 63;
-    if (w >= R * NB * split) return;
-    // split waves per (replica, i-block), wave `part` taking tiles part, part + split, ..
-    const int part = w % split;
-    const int rb = w / split;
+    const int split = share.split, waves = share.waves();
+    if (w >= R * NB * waves) return;
+    // waves per (replica, i-block): tiles part, part + split, .., clusters of smask
+    const int rb = w / waves;
+    const int part = (w - rb * waves) / share.sub;
+    const unsigned long long smask = sub_mask(share.sub, (w - rb * waves) % share.sub);
     int r = rb / NB;
     int ib = rb - r * NB;
     const float4* A = arec + (size_t)r * Np * 2;
@@ -698,8 +709,9 @@ __global__ __launch_bounds__(64 * WPW) __attribute__((amdgpu_waves_per_eu(4))) v
     };
     // the wave's next 64 tiles, one per lane, so that no tile waits for its descriptor:
     // j-block (TILE_MI set where every pair needs its own minimum image), mask, and the
-    // offset (hx, hy, hz) from the i-block's reference to the j-block's, in the periodic
-    // image that the tile's pairs take: x_i - x_j = rel_i - (rel_j + h)
+    // shift (hx, hy, hz) of the periodic image that the tile's pairs take, which is taken off
+    // the atoms of the lower block whichever of the two lists the tile, so that the rounding
+    // of a separation (and what is within the cutoff) does not depend on that
     constexpr int TILE_MI = 1 << 30;
     int tj = 0;
     float hx = 0.f, hy = 0.f, hz = 0.f;
@@ -710,7 +722,7 @@ __global__ __launch_bounds__(64 * WPW) __attribute__((amdgpu_waves_per_eu(4))) v
         const int tq = t0 + lane * split;
         if (tq < nt) {
             tj = tl[tq];
-            tm = tmk[tq];
+            tm = tmk[tq] & smask;
         }
     };
     load_tiles(part);
@@ -727,18 +739,26 @@ __global__ __launch_bounds__(64 * WPW) __attribute__((amdgpu_waves_per_eu(4))) v
         ei[k] = b.y;
         fi[3 * k] = fi[3 * k + 1] = fi[3 * k + 2] = 0.f;
     }
-    const float4 bli = lo[ib], bhi = hi[ib];
+    if (vi) {  // i coordinates as stored, for tiles that shift them
+        const float4 a = A[2 * islot];
+        xi_s[wv][0][lane] = a.x;
+        xi_s[wv][1][lane] = a.y;
+        xi_s[wv][2][lane] = a.z;
+    }
+    int ox = 0, oy = 0, oz = 0;  // what xi, yi, zi are shifted by now (bits of the floats)
     const int* E = exs + (size_t)rb * max_ex * 64;
     const unsigned long long eset = exblocks[rb];
-    const double4 ri = bref[rb];
     auto load_shifts = [&](int t0) {
         if (t0 + lane * split < nt) {
-            float kx, ky, kz;
-            const bool one = tile_shift(bli, bhi, lo[tj], hi[tj], g, kx, ky, kz);
-            const double4 rj = bref[(size_t)r * NB + tj];
-            hx = (float)((rj.x - ri.x) + quantize(g.Lx) * (double)kx);
-            hy = (float)((rj.y - ri.y) + quantize(g.Ly) * (double)ky);
-            hz = (float)((rj.z - ri.z) + quantize(g.Lz) * (double)kz);
+            // the i-block's box is read here each time (opaque index): kept in registers
+            // over the tile loop it made it spill
+            int ibo = ib;
+            asm volatile("" : "+s"(ibo));
+            const int lower = min(ibo, tj), upper = max(ibo, tj);
+            const bool one = tile_shift(lo[lower], hi[lower], lo[upper], hi[upper], g, hx, hy, hz);
+            hx = one ? g.bx * hx : 0.f;
+            hy = one ? g.by * hy : 0.f;
+            hz = one ? g.bz * hz : 0.f;
             if (!one) tj |= TILE_MI;
         }
     };
@@ -770,9 +790,24 @@ __global__ __launch_bounds__(64 * WPW) __attribute__((amdgpu_waves_per_eu(4))) v
         const unsigned long long m =
             (unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(unsigned)tm, ql) |
             (unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(unsigned)(tm >> 32), ql) << 32;
-        const float sx = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(hx), ql));
-        const float sy = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(hy), ql));
-        const float sz = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(hz), ql));
+        // the shift (bits of the floats) of the i atoms, or else of each j atom as it is read
+        const bool up = jb > ib;
+        const int sx = __builtin_amdgcn_readlane(__float_as_int(hx), ql),
+                  sy = __builtin_amdgcn_readlane(__float_as_int(hy), ql),
+                  sz = __builtin_amdgcn_readlane(__float_as_int(hz), ql);
+        const float ux = __int_as_float(up ? 0 : sx), uy = __int_as_float(up ? 0 : sy),
+                    uz = __int_as_float(up ? 0 : sz);
+        if ((up ? sx : 0) != ox || (up ? sy : 0) != oy || (up ? sz : 0) != oz) {
+            ox = up ? sx : 0;
+            oy = up ? sy : 0;
+            oz = up ? sz : 0;
+#pragma unroll
+            for (int k = 0; k < 8; k++) {
+                xi[k] = xi_s[wv][0][8 * k + il] - __int_as_float(ox);
+                yi[k] = xi_s[wv][1][8 * k + il] - __int_as_float(oy);
+                zi[k] = xi_s[wv][2][8 * k + il] - __int_as_float(oz);
+            }
+        }
         if (t + split < nt) {
             if (ql == 63) {
                 load_tiles(t + split);
@@ -784,7 +819,7 @@ __global__ __launch_bounds__(64 * WPW) __attribute__((amdgpu_waves_per_eu(4))) v
             flush_i();
             npair = 0;
         }
-        // pairs of the tile that need more than the offset (uniform): their own minimum
+        // pairs of the tile that need more than the shift (uniform): their own minimum
         // image, or a look at the exclusions and empty slots
         const bool mi = (jt & TILE_MI) != 0;
         bool ex = jb == ib || ((eset >> (jb & 63)) & 1ull) || ib * 64 + 64 > N || jb * 64 + 64 > N;
@@ -796,7 +831,7 @@ __global__ __launch_bounds__(64 * WPW) __attribute__((amdgpu_waves_per_eu(4))) v
         const int general = __builtin_amdgcn_readfirstlane(mi || ex ? 1 : 0);
         float fjx = 0.f, fjy = 0.f, fjz = 0.f;  // sum of cluster il, atom jl
         unsigned long long rest = m, done = 0ull;
-        do {
+        if (rest) do {
             const int jc8 = __builtin_ctzll(rest) & 56;  // 8 jc
             const unsigned ics = (unsigned)(m >> jc8) & 0xffu;
             rest &= ~(0xffull << jc8);
@@ -815,7 +850,7 @@ __global__ __launch_bounds__(64 * WPW) __attribute__((amdgpu_waves_per_eu(4))) v
                     : "v"(addr)
                     : "memory");
             }
-            const float xj = pj.x + sx, yj = pj.y + sy, zj = pj.z + sz;
+            const float xj = pj.x - ux, yj = pj.y - uy, zj = pj.z - uz;
             float fx = 0.f, fy = 0.f, fz = 0.f;
             // opaque to the compiler, which would otherwise carry the zeros through the
             // branches below as constants and copy the registers at the joins
@@ -910,21 +945,19 @@ __global__ __launch_bounds__(64 * WPW) __attribute__((amdgpu_waves_per_eu(4))) v
 // kernel takes the FP64 positions and parameters of every pair with r < rc once, in
 // Newton-3 order over the half tile lists, so U0 is exact to FP64 rounding.
 //
-// One wave per (replica, i-block, part): part p of `split` takes tiles p, p + split, ..,
-// pair of clusters by pair of clusters as the pair kernel does (lane 8 jl + il: j atom jl,
-// i atom il), all in FP64: vector FP64 issues at the rate of unpacked FP32.  The i records
+// Waves per (replica, i-block) and their shares of the tiles as in the pair kernel
+// (TileShare), pair of clusters by pair of clusters as the pair kernel does (lane 8 jl + il:
+// j atom jl, i atom il), all in FP64: vector FP64 issues at the rate of unpacked FP32.  The i records
 // stay in LDS (eight clusters of FP64 records would take 96 registers), the next tile's j
 // records are loaded into registers while the current tile is evaluated.
 // ---------------------------------------------------------------------------
-constexpr int E64_SPLIT = 4;  // waves (parts) per i-block of the FP64 energy kernel
-
 // Orders the LDS accesses of a one-wave workgroup around this point.  A wave's LDS
 // instructions are carried out in issue order, so a compiler barrier is enough: unlike
 // __syncthreads() it does not wait for the wave's global loads in flight.
 __device__ __forceinline__ void lds_order() { asm volatile("" ::: "memory"); }
 
 __global__ __launch_bounds__(64) void k_energy64(
-    int R, int N, int Np, int NB, int maxj, int split, const Rec64* __restrict__ rec,
+    int R, int N, int Np, int NB, int maxj, TileShare share, const Rec64* __restrict__ rec,
     const int* __restrict__ tiles, const unsigned long long* __restrict__ tmask,
     const int* __restrict__ ntiles, const float4* __restrict__ bb_lo,
     const float4* __restrict__ bb_hi, const int* __restrict__ exs,
@@ -933,8 +966,10 @@ __global__ __launch_bounds__(64) void k_energy64(
     __shared__ unsigned long long em_s[64];
     const int w = xcd_linear_id(blockIdx.x, gridDim.x);
     const int lane = threadIdx.x;
-    if (w >= R * NB * split) return;
-    const int part = w % split, rb = w / split;
+    const int split = share.split, waves = share.waves();
+    if (w >= R * NB * waves) return;
+    const int rb = w / waves, part = (w - rb * waves) / share.sub;
+    const unsigned long long smask = sub_mask(share.sub, (w - rb * waves) % share.sub);
     const int r = rb / NB, ib = rb - r * NB;
     const Rec64* RC = rec + (size_t)r * Np;
     const int islot = ib * 64 + lane;
@@ -962,7 +997,7 @@ __global__ __launch_bounds__(64) void k_energy64(
     if (part < nt) prefetch(tl[part]);
     for (int t = part; t < nt; t += split) {
         const int jb = tl[t];
-        const unsigned long long m = tmk[t];
+        const unsigned long long m = tmk[t] & smask;
         lds_order();  // the previous tile's records are no longer read
         jrec[lane] = Rec64{na.x, na.y, nb.x, nb.y, nc.x, nc.y};
         if (t + split < nt) prefetch(tl[t + split]);
@@ -977,7 +1012,7 @@ __global__ __launch_bounds__(64) void k_energy64(
         auto clusters = [&](auto mic, auto exc) {
             constexpr bool MI = decltype(mic)::value, EX = decltype(exc)::value;
             unsigned long long rest = m;
-            do {
+            while (rest) {
                 const int jc = __builtin_ctzll(rest) >> 3;
                 unsigned ics = (unsigned)(m >> (8 * jc)) & 0xffu;
                 rest &= ~(0xffull << (8 * jc));
@@ -1016,7 +1051,7 @@ __global__ __launch_bounds__(64) void k_energy64(
                                       qq * (ir + g.krf * r2 - g.crf);
                     e += ok ? ee : 0.0;  // also clears inf or NaN of excluded or empty slots
                 } while (ics);
-            } while (rest);
+            }
         };
         using T = std::true_type;
         using Fa = std::false_type;
@@ -1029,7 +1064,7 @@ __global__ __launch_bounds__(64) void k_energy64(
         }
     }
     e = wave_sum(e);
-    if (lane == 0) e_out[(size_t)rb * split + part] = e;
+    if (lane == 0) e_out[w] = e;
 }
 
 // ---------------------------------------------------------------------------
