@@ -144,7 +144,7 @@ struct sdm_context {
     double *e_t1 = nullptr, *e_t2 = nullptr;
     // constraints: clusters (atoms, and constraints as local index pairs with squared
     // lengths), the per-atom flag and the displacement scratch of the Langevin update
-    int ncl = 0;
+    int ncl = 0, cl_atoms_max = 0;  // clusters; atoms of the largest
     int *cl_start = nullptr, *cl_atoms = nullptr, *con_start = nullptr, *con_ij = nullptr;
     int* cflag = nullptr;
     double *con_d2 = nullptr, *dxs = nullptr;
@@ -629,7 +629,7 @@ void enqueue_step(sdm_context* c, bool full, bool energy, hipEvent_t pe0 = nullp
                                                            c->slot_of, c->cflag, c->dxs, mg,
                                                            c->flags);
     if (c->ncl > 0)
-        k_constrain<<<g2(c->ncl, 256, c->R), 256, 0, c->stream>>>(
+        k_constrain<<<g2(c->ncl, 64, c->R), 64, c->cl_atoms_max * SHAKE_LDS, c->stream>>>(
             c->Np, c->ncl, c->cl_start, c->cl_atoms, c->con_start, c->con_ij, c->con_d2,
             c->con_tol, c->invm, c->dxs, c->x64, c->v64, c->rec, c->flags);
     if (c->nvs > 0)  // the sites placed from their parents' new positions
@@ -1116,10 +1116,12 @@ static int set_constraints(sdm_context* c, const sdm_forcefield_terms* t) {
     for (int k = 0; k < nc; k++) cons[root_cl[find(t->constraint_atoms[2 * k])]].push_back(k);
     std::vector<int> con_start{0}, con_ij;
     std::vector<double> con_d2;
+    size_t largest = 0;
     for (size_t q = 0; q < members.size(); q++) {
         if ((int)members[q].size() > SHAKE_MAX_ATOMS || (int)cons[q].size() > SHAKE_MAX_CONS)
             return fail(SDM_ERR_UNSUPPORTED, "a constraint cluster has more than 16 atoms or "
                                              "32 constraints");
+        largest = std::max(largest, members[q].size());
         for (int a : members[q]) cl_atoms.push_back(a);
         cl_start.push_back((int)cl_atoms.size());
         for (int k : cons[q]) {
@@ -1153,6 +1155,7 @@ static int set_constraints(sdm_context* c, const sdm_forcefield_terms* t) {
     CHK(upload(c, c->con_d2, con_d2.data(), con_d2.size()));
     CHK(upload(c, c->cflag, flag.data(), c->N));
     c->ncl = (int)members.size();
+    c->cl_atoms_max = (int)largest;
     return SDM_OK;
 }
 

@@ -2460,58 +2460,124 @@ __global__ __launch_bounds__(1024) void k_cm_remove(int N, int Np, int every,
 // constraint in turn moves its two atoms along their bond vector before the step, in
 // inverse proportion to their masses, until every |r_ij|^2 is within tol of d_ij^2.
 // Then x = x', v = (x' - x)/dt.  Sets flag 8 if a cluster does not converge.
+//
+// What bounds it is the chain of constraints of one cluster (each needs the positions the
+// one before left), a few dozen FP64 divisions long.  A rigid three-site molecule
+// (constraints 0-1, 0-2, 1-2) is worked on in registers; other clusters keep their atoms in
+// LDS ([atom][value][lane], no bank conflicts), since arrays indexed by the constraint
+// lists would lie in scratch memory.  990 rigid waters: 67 us with the arrays in scratch and
+// 256 threads per workgroup, 9 us so.
 constexpr int SHAKE_MAX_ATOMS = 16, SHAKE_MAX_CONS = 32, SHAKE_MAX_ITER = 500;
-__global__ __launch_bounds__(256) void k_constrain(
+constexpr int SHAKE_LDS = 7 * 64 * sizeof(double);  // bytes of LDS per atom of the largest cluster
+
+// one constraint: moves atoms i and j along ro, their separation before the step; returns
+// whether it was within the tolerance
+__device__ __forceinline__ bool shake(const double (&ro)[3], double (&xi)[3], double (&xj)[3],
+                                      double mi, double mj, double d2, double tol) {
+    double rn[3];
+#pragma unroll
+    for (int d = 0; d < 3; d++) rn[d] = xi[d] - xj[d];
+    const double diff = d2 - dot3(rn, rn);
+    const double g = diff / (2.0 * (mi + mj) * dot3(ro, rn));
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        xi[d] += g * mi * ro[d];
+        xj[d] -= g * mj * ro[d];
+    }
+    return !(fabs(diff) > tol * d2);
+}
+
+__global__ __launch_bounds__(64) void k_constrain(
     int Np, int ncl, const int* __restrict__ cl_start, const int* __restrict__ cl_atoms,
     const int* __restrict__ con_start, const int* __restrict__ con_ij,
     const double* __restrict__ con_d2, double tol, const double* __restrict__ invm,
     const double* __restrict__ dxs, double* __restrict__ x64, double* __restrict__ v64,
     const DevRecord* __restrict__ rec, int* __restrict__ flags) {
-    int r = blockIdx.y, q = blockIdx.x * blockDim.x + threadIdx.x;
+    extern __shared__ double atoms_s[];  // atom k, value f of lane: [(7 k + f) * 64 + lane]
+    const int r = blockIdx.y, lane = threadIdx.x, q = blockIdx.x * 64 + lane;
     if (q >= ncl) return;
     double* X = x64 + (size_t)r * 3 * Np;
     double* V = v64 + (size_t)r * 3 * Np;
     const double* D = dxs + (size_t)r * 3 * Np;
-    int a0 = cl_start[q], na = cl_start[q + 1] - a0;
-    int c0 = con_start[q], nc = con_start[q + 1] - c0;
-    double xo[SHAKE_MAX_ATOMS][3], xn[SHAKE_MAX_ATOMS][3], im[SHAKE_MAX_ATOMS];
-    for (int k = 0; k < na; k++) {
-        int a = cl_atoms[a0 + k];
-        im[k] = invm[a];
-        for (int d = 0; d < 3; d++) {
-            xo[k][d] = X[d * Np + a];
-            xn[k][d] = xo[k][d] + D[d * Np + a];
-        }
-    }
+    const int a0 = cl_start[q], na = cl_start[q + 1] - a0;
+    const int c0 = con_start[q], nc = con_start[q + 1] - c0;
+    const int* ij = con_ij + 2 * c0;
+    const double inv = 1.0 / rec[r].dt;
     bool done = false;
-    for (int it = 0; it < SHAKE_MAX_ITER && !done; it++) {
-        done = true;
-        for (int k = 0; k < nc; k++) {
-            int i = con_ij[2 * (c0 + k)], j = con_ij[2 * (c0 + k) + 1];
-            double d2 = con_d2[c0 + k];
-            double ro[3], rn[3];
+    if (na == 3 && nc == 3 && ij[0] == 0 && ij[1] == 1 && ij[2] == 0 && ij[3] == 2 && ij[4] == 1 &&
+        ij[5] == 2) {
+        double xo[3][3], xn[3][3], im[3], ro[3][3];
+        int a[3];
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            a[k] = cl_atoms[a0 + k];
+            im[k] = invm[a[k]];
+#pragma unroll
             for (int d = 0; d < 3; d++) {
-                ro[d] = xo[i][d] - xo[j][d];
-                rn[d] = xn[i][d] - xn[j][d];
+                xo[k][d] = X[d * Np + a[k]];
+                xn[k][d] = xo[k][d] + D[d * Np + a[k]];
             }
-            double diff = d2 - dot3(rn, rn);
-            if (fabs(diff) > tol * d2) done = false;
-            double g = diff / (2.0 * (im[i] + im[j]) * dot3(ro, rn));
+        }
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            ro[0][d] = xo[0][d] - xo[1][d];
+            ro[1][d] = xo[0][d] - xo[2][d];
+            ro[2][d] = xo[1][d] - xo[2][d];
+        }
+        const double d01 = con_d2[c0], d02 = con_d2[c0 + 1], d12 = con_d2[c0 + 2];
+        for (int it = 0; it < SHAKE_MAX_ITER && !done; it++) {
+            done = shake(ro[0], xn[0], xn[1], im[0], im[1], d01, tol);
+            done &= shake(ro[1], xn[0], xn[2], im[0], im[2], d02, tol);
+            done &= shake(ro[2], xn[1], xn[2], im[1], im[2], d12, tol);
+        }
+#pragma unroll
+        for (int k = 0; k < 3; k++)
+#pragma unroll
             for (int d = 0; d < 3; d++) {
-                xn[i][d] += g * im[i] * ro[d];
-                xn[j][d] -= g * im[j] * ro[d];
+                V[d * Np + a[k]] = inv * (xn[k][d] - xo[k][d]);
+                X[d * Np + a[k]] = xn[k][d];
+            }
+    } else {
+        // values 0-2: position before the step, 3-5: new position, 6: inverse mass
+        auto at = [&](int k, int f) -> double& { return atoms_s[(7 * k + f) * 64 + lane]; };
+        for (int k = 0; k < na; k++) {
+            const int a = cl_atoms[a0 + k];
+            for (int d = 0; d < 3; d++) {
+                const double x = X[d * Np + a];
+                at(k, d) = x;
+                at(k, 3 + d) = x + D[d * Np + a];
+            }
+            at(k, 6) = invm[a];
+        }
+        for (int it = 0; it < SHAKE_MAX_ITER && !done; it++) {
+            done = true;
+            for (int k = 0; k < nc; k++) {
+                const int i = ij[2 * k], j = ij[2 * k + 1];
+                double ro[3], xi[3], xj[3];
+#pragma unroll
+                for (int d = 0; d < 3; d++) {
+                    ro[d] = at(i, d) - at(j, d);
+                    xi[d] = at(i, 3 + d);
+                    xj[d] = at(j, 3 + d);
+                }
+                done &= shake(ro, xi, xj, at(i, 6), at(j, 6), con_d2[c0 + k], tol);
+#pragma unroll
+                for (int d = 0; d < 3; d++) {
+                    at(i, 3 + d) = xi[d];
+                    at(j, 3 + d) = xj[d];
+                }
+            }
+        }
+        for (int k = 0; k < na; k++) {
+            const int a = cl_atoms[a0 + k];
+            for (int d = 0; d < 3; d++) {
+                const double x = at(k, 3 + d);
+                V[d * Np + a] = inv * (x - at(k, d));
+                X[d * Np + a] = x;
             }
         }
     }
     if (!done) atomicOr(&flags[r], 8);
-    double inv = 1.0 / rec[r].dt;
-    for (int k = 0; k < na; k++) {
-        int a = cl_atoms[a0 + k];
-        for (int d = 0; d < 3; d++) {
-            V[d * Np + a] = inv * (xn[k][d] - xo[k][d]);
-            X[d * Np + a] = xn[k][d];
-        }
-    }
 }
 
 // Kinetic energy 0.5 sum m v^2 of every replica (one workgroup per replica), with the

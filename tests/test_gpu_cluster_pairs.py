@@ -4,8 +4,8 @@ waves per block, where each pair takes its own minimum image (box of about two c
 without periodic images, and with the geometric sigma rule; against the FP64 oracle.
 
 Tolerances: U0 is an FP64 sum (1e-10 of the summed magnitudes' scale, as pair energies of
-opposite sign cancel); forces are FP32 pair arithmetic on coordinates rounded to 6e-8 nm:
-|dF/F| <= 13 * 6e-8 / 0.1 nm for the steepest term of the closest pairs, plus a few FP32
+opposite sign cancel); forces are FP32 pair arithmetic on coordinates rounded to 1.2e-7 nm at most:
+|dF/F| <= 13 * 1.2e-7 / 0.1 nm for the steepest term of the closest pairs, plus a few FP32
 roundings, so 2e-5 of the RMS force; the pair count is exact except for pairs whose distance
 is within FP32 rounding of the cutoff."""
 import numpy as np
