@@ -171,19 +171,15 @@ typedef struct {
                                      fill it.
                                      Results differ only in rounding: each wave's i forces
                                      are summed on their own before they are added up. */
-    int32_t side_fork;            /* where the restraints, force-field terms and the
-                                     displaced-state chain run: 0 on two side streams
-                                     forked after the tile lists (beside the pair kernel),
-                                     1 (the default) forked after the slot order (beside
-                                     the tile-list build as well), 2 on the main stream
-                                     between the tile lists and the pair kernel, 3 as 1
-                                     but with the displaced-state chain joined back
-                                     before the pair kernel (beside the tile lists only),
-                                     4 as 1 but with the bonds and angles forked with the
-                                     rest.  With 0, 1 and 3 the bonds and angles start
-                                     with the step on a side stream (beside the spatial
-                                     sort, one more fork event per step); with 2 they
-                                     run with the rest.  Same results. */
+    int32_t side_fork;            /* where the restraints and force-field terms run: 0 on a
+                                     side stream forked after the tile lists (beside the
+                                     forces), 1 (the default), 3 and 4 forked after the
+                                     slot order (beside the tile-list build as well), 2 on
+                                     the main stream between the tile lists and the
+                                     forces.  Pair energies of large batches run on the
+                                     side stream as well, except with 2.  Bonds, angles
+                                     and the displaced-state pairs run with the pair
+                                     forces in one launch.  Same results. */
     float list_skin;              /* Verlet skin of the tile lists in nm, 0 to
                                      SDM_MAX_LIST_SKIN (pair_group 0 only; 0, the
                                      default, builds them on every evaluation).  Lists
@@ -422,7 +418,7 @@ int sdm_time_pair_kernel(sdm_context* ctx, int32_t nsteps, double* avg_ms);
 /* Launch-configuration search (project-written autotuner): times each candidate (waves
    per workgroup and per i-block of the pair kernel, sort grid) on the context's own replicas
    for `steps` steps, then times the three fastest, each with and without graph replay
-   and with each of the five placements of the side work (side_fork), for 3 x `steps`
+   and with the placements of the side work that differ (side_fork), for 3 x `steps`
    steps in two rounds, and keeps the one with the smallest total; it then times that one
    with list_skin 0, 0.01, 0.02, 0.03 and 0.04 nm the same way.  The state the context had before the call is restored. */
 int sdm_autotune(sdm_context* ctx, int32_t steps, sdm_tuning* chosen);

@@ -75,11 +75,8 @@ int resolve_scratch(int device, int32_t** out) {
 struct sdm_context {
     int device = 0;
     hipStream_t stream = nullptr;
-    // side streams of the step's fork/join: bonded terms and the displaced-state chain
-    // run concurrently with the pair kernel
-    hipStream_t side[2] = {nullptr, nullptr};
-    hipEvent_t ev_fork0 = nullptr, ev_fork = nullptr, ev_join[2] = {nullptr, nullptr};
-    hipEvent_t ev_tiles = nullptr;  // the tile lists are built (energy evaluations)
+    hipStream_t side = nullptr;  // restraints and force-field terms, beside the forces
+    hipEvent_t ev_fork = nullptr, ev_join = nullptr;
     int N = 0, Np = 0, NB = 0, R = 0, L = 0, LB = 0, ncls = 0;
     // 0: CutoffNonPeriodic (no images; the sort grid spans reg_lo .. reg_hi, the union of
     // the positions' bounding boxes over the replicas, widened by GRID_MARGIN)
@@ -103,7 +100,7 @@ struct sdm_context {
     double *bond_r0 = nullptr, *bond_k = nullptr;
     int* ang_atoms = nullptr;
     double *ang_t0 = nullptr, *ang_k = nullptr;
-    // per-atom lists of the bonds and angles each atom belongs to (k_bonded's gather):
+    // per-atom lists of the bonds and angles each atom belongs to (bonded_wave's gather):
     // entries (term << 1 | role) and (term << 2 | role) in term order
     int *bstart = nullptr, *bcode = nullptr, *astart = nullptr, *acode = nullptr;
     double* Fb = nullptr;  // [R][3][Np] FP64 bonded forces, atom order
@@ -119,7 +116,7 @@ struct sdm_context {
     float4* cbox = nullptr;  // [R][NB][16] centres and half extents of the 8-slot clusters
     int *tiles = nullptr, *ntiles = nullptr;
     unsigned long long* tmask = nullptr;
-    int* cmap = nullptr;    // [R][NB] block -> candidate index of k_ligcand (-1: none)
+    int* cmap = nullptr;    // [R][NB] block -> candidate index (-1: none)
     int* lig_of = nullptr;  // [Np] atom -> index in lig (-1: environment)
     float4* xb = nullptr;   // [R][Np] slot coordinates when the tile lists were built
     float* dmax = nullptr;  // [R][DISP_STRIDE] (first float used) largest squared
@@ -127,7 +124,7 @@ struct sdm_context {
                             // or stale after a sort (k_bbox)
     long long* F = nullptr;
     double *e_bond = nullptr, *u_part = nullptr;
-    double* e64 = nullptr;  // FP64 pair-energy slots, one per wave of k_energy64
+    double* e64 = nullptr;  // FP64 pair-energy slots, one per wave of energy64_wave
     // SDMUtils restraints (group 1): centroid and alignment terms, their group atoms and
     // normalized weights, and one energy slot per (replica, restraint)
     DevCentroid* rcen = nullptr;
@@ -152,9 +149,6 @@ struct sdm_context {
     int cm_every = 0;  // centre-of-mass motion removal interval (0: never)
     int *cand = nullptr, *ncand = nullptr;
     double4 *dA = nullptr, *dlig = nullptr, *dB = nullptr;
-    // [R][maxc][L] 64-bit lists: the undisplaced slots of candidate block c that displaced
-    // atom li pairs with (k_denv's screen, read by k_dlig)
-    unsigned long long* mlig = nullptr;
     DevState* state = nullptr;
     DevRecord* rec = nullptr;
     int* flags = nullptr;
@@ -413,18 +407,20 @@ TileRadius tile_radius(const sdm_context* c) {
     return tr;
 }
 
-// tile lists of the pair and energy kernels.  With a skin, k_tiles keeps a replica's lists
+// tile lists of the pairs and pair energies, candidate blocks of the displaced atoms.  With a skin, k_tiles keeps a replica's lists
 // while its atoms have moved less than half the skin since they were built.
 void enqueue_tiles(sdm_context* c) {
     const TileRadius tr = tile_radius(c);
+    const LigCand lc{c->L > 0 ? 1 : 0, c->L, c->ncls, c->maxc, c->list_r2, c->lig, c->cls,
+                     c->cdispl, c->x64, c->cand, c->ncand, c->cmap};
     // One workgroup per (replica, i-block).  Its time is the serial path through it, so
     // when the workgroups do not fill the GPU (fewer than 8 per CU) each gets 8 waves for
     // the candidate masks, otherwise 4 (measured: one replica of 22,750 atoms +6%, 22
     // replicas -1% with 8).
 #define SDM_TILES(NW)                                                                         \
-    k_tiles<NW><<<dim3(c->NB, c->R), 64 * NW, 0, c->stream>>>(                                \
+    k_tiles<NW><<<dim3(c->NB + lc.groups, c->R), 64 * NW, 0, c->stream>>>(                    \
         c->N, c->Np, c->NB, c->maxj, c->arec, c->bb_lo, c->bb_hi, c->cbox, c->tiles,          \
-        c->tmask, c->ntiles, c->dmax, c->xb, tr, c->g, c->flags)
+        c->tmask, c->ntiles, c->dmax, c->xb, tr, c->g, c->flags, lc)
     if (few_blocks(c)) SDM_TILES(8);
     else SDM_TILES(4);
 #undef SDM_TILES
@@ -447,14 +443,6 @@ TileShare block_share(const sdm_context* c) {
     return {c->NB < 256 ? 16 : c->NB < 512 ? 8 : 4, c->NB <= 16 ? 4 : c->NB <= 32 ? 2 : 1};
 }
 
-// FP64 pair energies into e64 (needs the tile lists and FP64 records of this evaluation)
-void enqueue_energy64(sdm_context* c, hipStream_t st) {
-    const TileShare sh = block_share(c);
-    k_energy64<<<(unsigned)(c->R * c->NB * sh.waves()), 64, 0, st>>>(
-        c->R, c->N, c->Np, c->NB, c->maxj, sh, c->rec64, c->tiles, c->tmask, c->ntiles,
-        c->bb_lo, c->bb_hi, c->exs, c->exblocks, c->max_ex, c->e64, c->g);
-}
-
 // Waves of the pair kernel: tuning.pair_split, or more where block_share has more (one
 // where tuning asks for one, or for the full tile lists or the grouped form, for which
 // pair_split has no meaning).
@@ -464,32 +452,64 @@ TileShare pair_share(const sdm_context* c) {
     return split == 1 ? TileShare{1, 1} : TileShare{std::max(split, sh.split), sh.sub};
 }
 
-template <int W, bool GEO>
-void launch_pair(sdm_context* c, bool count) {
-    const TileShare sh = pair_share(c);
-    const int waves = c->R * c->NB * sh.waves();
-    const dim3 gr((waves + W - 1) / W);
-#define SDM_PAIR(COUNT)                                                                       \
-    k_pair<W, COUNT, GEO><<<gr, 64 * W, 0, c->stream>>>(                                      \
-        c->R, c->N, c->Np, c->NB, c->maxj, sh, c->arec, c->tiles, c->tmask,                \
-        c->ntiles, c->bb_lo, c->bb_hi, c->exs, c->exblocks, c->max_ex, c->F, c->flags, c->counters, c->g)
-    if (count) SDM_PAIR(true);
-    else SDM_PAIR(false);
-#undef SDM_PAIR
+// Whether the pairs alone run for several generations of waves (4,096 are resident): 20 x
+// 2,976 atoms have 15,000 waves, 22 x 22,750 and 8 x 99,920 atoms 31,000 and 50,000.
+bool many_waves(const sdm_context* c) {
+    return (long long)c->R * c->NB * pair_share(c).waves() >= 6 * 4096;
 }
 
-// pair forces, or (count) the number of pairs within the cutoff into counters
-void enqueue_pair(sdm_context* c, bool count) {
+// parts of the displaced-state forces on a candidate block (env_force)
+int displaced_parts(const sdm_context* c) { return many_waves(c) ? 1 : DISP_WAVES; }
+
+// what a launch of k_forces does
+enum ForceParts { PAIRS = 1, DISPLACED = 2, BONDED = 4, ENERGY = 8 };
+
+template <int W, bool COUNT, bool GEO>
+void launch_forces(sdm_context* c, int parts) {
+    // workgroups of W waves for n waves, a multiple of 8 (k_forces)
+    auto groups = [](int part, int n) { return part ? ((n + W - 1) / W + 7) / 8 * 8 : 0; };
+    const TileShare sh = pair_share(c), esh = block_share(c);
+    // A wave per group of displaced atoms where the launch is short, one for all groups of a
+    // candidate block where it is long: fewer waves then wait for their atoms while others
+    // could compute (22 x 22,750 atoms, 10 steps: 6.45 -> 6.33 ms, and 6.15 ms with the
+    // Langevin kernel then reading one part of the forces on a candidate block, not eight)
+    const int pair_waves = c->R * c->NB * sh.waves();
+    const int subs = DISP_WAVES / displaced_parts(c);
+    const int disp = std::min(c->maxc, DISP_BLOCKS) * displaced_parts(c);
+    const ForceGroups fg{groups(c->L > 0 ? parts & DISPLACED : 0, c->R * disp),
+                         groups(parts & ENERGY, c->R * c->NB * esh.waves()),
+                         groups(parts & PAIRS, pair_waves), disp, subs};
+    const int bonded = groups(c->nbond + c->nang > 0 ? parts & BONDED : 0, c->R * c->nbw);
+    k_forces<W, COUNT, GEO><<<fg.displaced + fg.energy + fg.pairs + bonded, 64 * W, 0, c->stream>>>(
+        fg, c->R, c->N, c->Np, c->NB, c->maxj, sh, c->arec, c->tiles, c->tmask, c->ntiles,
+        c->bb_lo, c->bb_hi, c->exs, c->exblocks, c->max_ex, c->F, c->flags, c->counters, esh,
+        c->rec64, c->e64, c->nbw, c->bstart, c->bcode, c->astart, c->acode, c->bond_atoms,
+        c->bond_r0, c->bond_k, c->ang_atoms, c->ang_t0, c->ang_k, c->x64, c->Fb, c->e_bond, c->L,
+        c->LB, c->lig, c->lb_start, c->lb_count, c->cls, c->cdispl, c->q64, c->sig64, c->eps64,
+        c->ex_start, c->ex_list, c->orig_s, c->cand, c->ncand, c->maxc, c->dA, c->dB, c->g);
+}
+
+void enqueue_forces(sdm_context* c, int parts) {
     auto with = [&](auto geo) {
         constexpr bool GEO = decltype(geo)::value;
         switch (c->tune.pair_waves_per_group) {
-            case 2: launch_pair<2, GEO>(c, count); break;
-            case 4: launch_pair<4, GEO>(c, count); break;
-            default: launch_pair<1, GEO>(c, count); break;
+            case 2: launch_forces<2, false, GEO>(c, parts); break;
+            case 4: launch_forces<4, false, GEO>(c, parts); break;
+            default: launch_forces<1, false, GEO>(c, parts); break;
         }
     };
     if (c->g.geo) with(std::true_type());
     else with(std::false_type());
+}
+
+// u and F1-F0 on the displaced atoms from k_forces' partials (or, with counters, the pairs
+// among them added to the count)
+void enqueue_delta(sdm_context* c, unsigned long long* counters) {
+    if (c->L > 0)
+        k_deltaA_red<DRED_WAVES><<<dim3(c->LB, c->R), 64 * DRED_WAVES, 0, c->stream>>>(
+            c->Np, c->L, c->LB, c->lig, c->lb_start, c->lb_count, c->cls, c->cdispl, c->q64,
+            c->sig64, c->eps64, c->ex_start, c->ex_list, c->x64, c->ncand, c->maxc, c->dA,
+            c->dlig, c->u_part, c->g, counters);
 }
 
 // A step's Langevin kernel adds the displaced-state forces itself (MixGather) instead of a
@@ -501,53 +521,31 @@ bool mix_in_langevin(const sdm_context* c, bool advance) {
     return advance && c->L > 0 && c->nvs == 0;
 }
 
-// evaluation of one step (everything before the Langevin update).  After the slot order
-// and the tile lists the work forks: the pair kernel on the main stream, the bonded terms
-// and the displaced-state chain on two side streams; they join before the scalar stage.
-// (Forking before the tile lists, which the side work does not need, was measured
-// slower on 22 replicas, where the side kernels then slow the tile builder, which is on
-// the critical path, and no faster on one.)  pe0/pe1 (optional) are recorded around the
-// pair kernel.
-void enqueue_eval(sdm_context* c, bool advance, bool components, bool full, bool energy,
-                  hipEvent_t pe0 = nullptr, hipEvent_t pe1 = nullptr) {
-    // tuning.side_fork: the side work (restraints, force-field terms, the displaced-state
-    // chain) needs the slot order, block boxes and cleared accumulator, not the tile
-    // lists.  0: it forks onto the two side streams after the tile lists, 1: before them,
-    // 2: it runs on the main stream between the tile lists and the pair kernel (no fork;
-    // while the pair kernel fills the GPU, side kernels beside it wait for free wave
-    // slots and can outlast it), 3: as 1, but the displaced-state chain joins the main
-    // stream before the pair kernel (it runs beside the tile lists only), 4: as 1, but the
-    // bonded terms fork with the rest (no event at the start of the step).  The bonded
-    // terms need only the positions and write their own FP64 array: with 0, 1 and 3 they
-    // start with the step, beside the sort (measured: 22 replicas 0.7% faster than 4; one
-    // replica 1.6% slower replayed from a graph, 4% launched directly).
+// Evaluation of one step (everything before the Langevin update): slot order, tile lists
+// with the candidate blocks, all forces, the sums on the displaced atoms, the scalar stage,
+// one launch each on the main stream.  Restraints and force-field terms, where there are
+// any, run beside them on the side stream, and so do the pair energies where the pairs run
+// for long (many_waves).  Measured, energies in k_forces against on the side stream: 5 steps
+// of 22 x 22,750 atoms with energies 5.32 against 5.01 ms, but one evaluation of 22,750 atoms
+// 0.40 against 0.44 ms.
+void enqueue_eval(sdm_context* c, bool advance, bool components, bool full, bool energy) {
+    // tuning.side_fork: restraints and force-field terms need the slot order and cleared
+    // accumulator, not the tile lists.  0: they start after the tile lists, 1, 3 and 4:
+    // before them, 2: there is no side stream, everything runs on the main one.
     const int mode = c->tune.side_fork;
-    hipStream_t s = c->stream;
-    hipStream_t s1 = mode == 2 ? s : c->side[0], s2 = mode == 2 ? s : c->side[1];
-    int N = c->N, Np = c->Np, R = c->R;
-    auto bonded = [&]() {
-        if (c->nbond + c->nang > 0)
-            k_bonded<<<dim3(c->nbw, R), 256, 0, s1>>>(
-                N, Np, c->bstart, c->bcode, c->astart, c->acode, c->bond_atoms, c->bond_r0,
-                c->bond_k, c->ang_atoms, c->ang_t0, c->ang_k, c->x64, c->Fb, c->e_bond,
-                c->nbw, c->flags);
-    };
-    if (mode != 2 && mode != 4) {
-        (void)hipEventRecord(c->ev_fork0, s);
-        (void)hipStreamWaitEvent(s1, c->ev_fork0, 0);
-        bonded();
-    }
-    enqueue_order(c, full, energy);
-    const bool tiles_after_fork = mode == 1 || mode == 3 || mode == 4;
-    if (!tiles_after_fork) enqueue_tiles(c);
-    if (mode != 2) {
+    const bool terms = mode != 2 && c->ncen + c->nali + c->nterm > 0;
+    const bool apart = mode != 2 && energy && many_waves(c);
+    hipStream_t s = c->stream, s1 = mode == 2 ? s : c->side;
+    const int N = c->N, Np = c->Np, R = c->R;
+    auto fork = [&](bool yes) {
+        if (!yes) return;
         (void)hipEventRecord(c->ev_fork, s);
         (void)hipStreamWaitEvent(s1, c->ev_fork, 0);
-        (void)hipStreamWaitEvent(s2, c->ev_fork, 0);
-        if (mode == 4) bonded();
-    }
-    if (tiles_after_fork) enqueue_tiles(c);
-    if (mode == 2) bonded();
+    };
+    enqueue_order(c, full, energy);
+    fork(terms && mode != 0);
+    enqueue_tiles(c);
+    fork((terms && mode == 0) || apart);
     if (c->ncen + c->nali > 0)
         k_restraints<<<dim3(c->ncen + c->nali, R), 64, 0, s1>>>(
             Np, c->ncen, c->ncen + c->nali, c->rcen, c->rali, c->ratom, c->rw, c->x64,
@@ -558,47 +556,17 @@ void enqueue_eval(sdm_context* c, bool advance, bool components, bool full, bool
             Np, c->terms, c->x64, components ? nullptr : c->slot_of,
             components ? c->Fb_sep : c->F, c->slot_of, c->F, c->e_t1, c->e_t2, c->ntb, c->g,
             c->flags);
-    if (c->L > 0) {
-        k_ligcand<<<R, LIGCAND_THREADS, 0, s2>>>(Np, c->NB, c->L, c->ncls, c->lig, c->cls, c->cdispl, c->x64,
-                                    c->bb_lo, c->bb_hi, c->maxc, c->cand, c->ncand, c->list_r2,
-                                    c->g, c->flags, c->cmap);
-        k_denv<DPAIR_WAVES><<<dim3(c->maxc, R), 64 * DPAIR_WAVES, 0, s2>>>(
-            N, Np, c->L, c->LB, c->lig, c->lb_start, c->lb_count, c->cls, c->cdispl, c->q64,
-            c->sig64, c->eps64, c->ex_start, c->ex_list, c->x64, c->orig_s, c->cand, c->ncand,
-            c->maxc, c->mlig, c->dB, c->g);
-        k_dlig<DPAIR_WAVES><<<dim3(c->maxc, c->LB, R), 64 * DPAIR_WAVES, 0, s2>>>(
-            N, Np, c->L, c->LB, c->lig, c->lb_start, c->lb_count, c->cls, c->cdispl, c->q64,
-            c->sig64, c->eps64, c->x64, c->orig_s, c->cand, c->ncand, c->maxc, c->mlig, c->dA,
-            c->g, nullptr);
-        k_deltaA_red<DRED_WAVES><<<dim3(c->LB, R), 64 * DRED_WAVES, 0, s2>>>(
-            Np, c->L, c->LB, c->lig, c->lb_start, c->lb_count, c->cls, c->cdispl, c->q64,
-            c->sig64, c->eps64, c->ex_start, c->ex_list, c->x64, c->ncand, c->maxc, c->dA,
-            c->dlig, c->u_part, c->g, nullptr);
+    if (apart) {
+        const TileShare sh = block_share(c);
+        k_energy64<<<(unsigned)(R * c->NB * sh.waves()), 64, 0, s1>>>(
+            R, N, Np, c->NB, c->maxj, sh, c->rec64, c->tiles, c->tmask, c->ntiles, c->bb_lo,
+            c->bb_hi, c->exs, c->exblocks, c->max_ex, c->e64, c->g);
     }
-    // the FP64 pair energies need the tile lists and this evaluation's FP64 records, not
-    // the pair forces: they run beside the pair kernel on the first side stream, which
-    // joins before the scalar stage
-    if (energy && mode != 2) {
-        (void)hipEventRecord(c->ev_tiles, s);
-        (void)hipStreamWaitEvent(s1, c->ev_tiles, 0);
-        enqueue_energy64(c, s1);
-    }
-    if (mode == 3) {
-        (void)hipEventRecord(c->ev_join[1], s2);
-        (void)hipStreamWaitEvent(s, c->ev_join[1], 0);
-    }
-    if (pe0) (void)hipEventRecord(pe0, s);
-    // forces in FP32; the pair energies, when asked for, in FP64 by their own kernel
-    enqueue_pair(c, false);
-    if (pe1) (void)hipEventRecord(pe1, s);
-    if (energy && mode == 2) enqueue_energy64(c, s);
-    if (mode != 2) {
-        (void)hipEventRecord(c->ev_join[0], s1);
-        (void)hipStreamWaitEvent(s, c->ev_join[0], 0);
-    }
-    if (mode == 0 || mode == 1 || mode == 4) {
-        (void)hipEventRecord(c->ev_join[1], s2);
-        (void)hipStreamWaitEvent(s, c->ev_join[1], 0);
+    enqueue_forces(c, PAIRS | DISPLACED | BONDED | (energy && !apart ? ENERGY : 0));
+    enqueue_delta(c, nullptr);
+    if (terms || apart) {
+        (void)hipEventRecord(c->ev_join, s1);
+        (void)hipStreamWaitEvent(s, c->ev_join, 0);
     }
     k_scalar<<<R, 256, 0, s>>>(c->NB * block_share(c).waves(), c->nbw, c->LB, c->e64,
                                c->e_bond, c->u_part, c->state,
@@ -607,13 +575,12 @@ void enqueue_eval(sdm_context* c, bool advance, bool components, bool full, bool
                                c->ncen + c->nali, c->e_t1, c->e_t2, c->ntb, c->dmax);
     if (c->L > 0 && !components && !mix_in_langevin(c, advance))
         k_mix<<<dim3(c->maxc + c->LB, R), 64, 0, s>>>(N, Np, c->L, c->maxc, c->lig, c->cls,
-                                                       c->orig_s, c->cand, c->ncand, c->dB,
-                                                       c->dlig, c->rec, c->slot_of, c->F, c->flags);
+                                                       c->orig_s, c->cand, c->ncand,
+                                                       displaced_parts(c), c->dB, c->dlig, c->rec, c->slot_of, c->F, c->flags);
 }
 
-void enqueue_step(sdm_context* c, bool full, bool energy, hipEvent_t pe0 = nullptr,
-                  hipEvent_t pe1 = nullptr) {
-    enqueue_eval(c, true, false, full, energy, pe0, pe1);
+void enqueue_step(sdm_context* c, bool full, bool energy) {
+    enqueue_eval(c, true, false, full, energy);
     if (c->cm_every > 0)
         k_cm_remove<<<c->R, 1024, 0, c->stream>>>(c->N, c->Np, c->cm_every, c->mass, c->v64,
                                                    c->state);
@@ -623,7 +590,7 @@ void enqueue_step(sdm_context* c, bool full, bool energy, hipEvent_t pe0 = nullp
             c->flags);
     MixGather mg{};
     if (mix_in_langevin(c, true))
-        mg = MixGather{c->lig_of, c->cmap, c->dB, c->dlig, c->NB, c->maxc, c->L};
+        mg = MixGather{c->lig_of, c->cmap, c->dB, c->dlig, c->NB, c->maxc, c->L, displaced_parts(c)};
     k_langevin<<<g2(c->N, 256, c->R), 256, 0, c->stream>>>(c->N, c->Np, c->invm, c->F, c->Fb,
                                                            c->x64, c->v64, c->rec, c->state,
                                                            c->slot_of, c->cflag, c->dxs, mg,
@@ -852,13 +819,9 @@ int sdm_create(const sdm_system_desc* sys, int32_t n_replicas, sdm_context** out
     if (hipGetDevice(&c->device) != hipSuccess) return bail(fail(SDM_ERR_HIP, "no HIP device"));
     if ((rc = resolve_scratch(c->device, &c->scratch_sel)) != SDM_OK) return bail(rc);
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
-        hipStreamCreateWithFlags(&c->side[0], hipStreamNonBlocking) != hipSuccess ||
-        hipStreamCreateWithFlags(&c->side[1], hipStreamNonBlocking) != hipSuccess ||
-        hipEventCreateWithFlags(&c->ev_fork0, hipEventDisableTiming) != hipSuccess ||
+        hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking) != hipSuccess ||
         hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&c->ev_join[0], hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&c->ev_join[1], hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&c->ev_tiles, hipEventDisableTiming) != hipSuccess)
+        hipEventCreateWithFlags(&c->ev_join, hipEventDisableTiming) != hipSuccess)
         return bail(fail(SDM_ERR_HIP, "hipStreamCreate/hipEventCreate failed"));
     c->N = N;
     c->max_ex = max_ex;
@@ -870,7 +833,7 @@ int sdm_create(const sdm_system_desc* sys, int32_t n_replicas, sdm_context** out
     c->ncls = (int)cd.size() / 3 - 1;
     c->nbond = sys->n_bonds;
     c->nang = sys->n_angles;
-    c->nbw = std::max(1, (N + 255) / 256);
+    c->nbw = c->NB;  // a wave of 64 atoms each
     c->maxj = tile_capacity(sys, c->NB);
     c->maxc = std::min(c->NB, 256 * std::max(1, c->ncls) + 64);
     Geom& g = c->g;
@@ -940,8 +903,7 @@ int sdm_create(const sdm_system_desc* sys, int32_t n_replicas, sdm_context** out
     A(e64, (size_t)R * NB * block_share(c).waves()); A(rec64, RNp);
     A(cand, (size_t)R * c->maxc); A(ncand, R);
     A(dA, (size_t)R * c->maxc * c->LB * 64); A(dlig, (size_t)R * std::max(1, c->L));
-    A(mlig, (size_t)R * c->maxc * std::max(1, c->L));
-    A(dB, (size_t)R * c->maxc * 64); A(state, R); A(rec, R); A(flags, R);
+    A(dB, (size_t)R * c->maxc * DISP_WAVES * 64); A(state, R); A(rec, R); A(flags, R);
     if (c->L > 0) {
         c->adj_cap = std::max<size_t>(1 << 20, (size_t)((N + ADJ_ATOMS - 1) / ADJ_ATOMS) *
                                                    std::max(ADJ_PART, (c->L + ADJ_SEL - 1) / ADJ_SEL));
@@ -1026,10 +988,9 @@ int sdm_destroy(sdm_context* c) {
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     drop_graph(c);
     for (void* p : c->allocs) (void)hipFree(p);
-    for (hipEvent_t e : {c->ev_fork0, c->ev_fork, c->ev_join[0], c->ev_join[1], c->ev_tiles})
+    for (hipEvent_t e : {c->ev_fork, c->ev_join})
         if (e) (void)hipEventDestroy(e);
-    for (hipStream_t st : {c->side[0], c->side[1]})
-        if (st) (void)hipStreamDestroy(st);
+    if (c->side) (void)hipStreamDestroy(c->side);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
     return SDM_OK;
@@ -1542,8 +1503,8 @@ int sdm_compute_components(sdm_context* c) {
     enqueue_eval(c, false, true, take_order(c, false), true);
     if (c->L > 0)
         k_scatter_dF<<<dim3(c->maxc + c->LB, c->R), 64, 0, c->stream>>>(
-            c->N, c->Np, c->L, c->maxc, c->lig, c->cls, c->orig_s, c->cand, c->ncand, c->dB,
-            c->dlig, c->dFd);
+            c->N, c->Np, c->L, c->maxc, c->lig, c->cls, c->orig_s, c->cand, c->ncand,
+            displaced_parts(c), c->dB, c->dlig, c->dFd);
     CHK(check_launch());
     HIPCHK(hipStreamSynchronize(c->stream));
     c->components_valid = true;
@@ -1780,24 +1741,9 @@ int sdm_count_pairs(sdm_context* c, int64_t* p0, int64_t* pdelta) {
     hipStream_t s = c->stream;
     k_fill_u64<<<1, 256, 0, s>>>(c->counters, n);
     enqueue_sort(c, take_order(c, false));
-    enqueue_pair(c, true);
-    if (c->L > 0) {
-        k_ligcand<<<c->R, LIGCAND_THREADS, 0, s>>>(c->Np, c->NB, c->L, c->ncls, c->lig, c->cls, c->cdispl,
-                                      c->x64, c->bb_lo, c->bb_hi, c->maxc, c->cand, c->ncand,
-                                      c->list_r2, c->g, c->flags, c->cmap);
-        k_denv<DPAIR_WAVES><<<dim3(c->maxc, c->R), 64 * DPAIR_WAVES, 0, s>>>(
-            c->N, c->Np, c->L, c->LB, c->lig, c->lb_start, c->lb_count, c->cls, c->cdispl,
-            c->q64, c->sig64, c->eps64, c->ex_start, c->ex_list, c->x64, c->orig_s, c->cand,
-            c->ncand, c->maxc, c->mlig, c->dB, c->g);
-        k_dlig<DPAIR_WAVES><<<dim3(c->maxc, c->LB, c->R), 64 * DPAIR_WAVES, 0, s>>>(
-            c->N, c->Np, c->L, c->LB, c->lig, c->lb_start, c->lb_count, c->cls, c->cdispl,
-            c->q64, c->sig64, c->eps64, c->x64, c->orig_s, c->cand, c->ncand, c->maxc, c->mlig,
-            c->dA, c->g, c->counters + c->R);
-        k_deltaA_red<DRED_WAVES><<<dim3(c->LB, c->R), 64 * DRED_WAVES, 0, s>>>(
-            c->Np, c->L, c->LB, c->lig, c->lb_start, c->lb_count, c->cls, c->cdispl, c->q64,
-            c->sig64, c->eps64, c->ex_start, c->ex_list, c->x64, c->ncand, c->maxc, c->dA,
-            c->dlig, c->u_part, c->g, c->counters + c->R);
-    }
+    if (c->g.geo) launch_forces<1, true, true>(c, PAIRS | DISPLACED);
+    else launch_forces<1, true, false>(c, PAIRS | DISPLACED);
+    enqueue_delta(c, c->counters + c->R);
     CHK(check_launch());
     std::vector<unsigned long long> h(n);
     CHK(download(c, h.data(), c->counters, n));
@@ -1823,7 +1769,7 @@ int sdm_time_pair_kernel(sdm_context* c, int32_t nsteps, double* avg_ms) {
         for (int s = 0; s < nsteps; s++) {
             enqueue_sort(c, take_order(c, false));
             (void)hipEventRecord(ev[2 * s], c->stream);
-            enqueue_pair(c, false);
+            enqueue_forces(c, PAIRS);
             (void)hipEventRecord(ev[2 * s + 1], c->stream);
         }
         rc = check_launch();
@@ -1947,23 +1893,22 @@ int sdm_autotune(sdm_context* c, int32_t steps, sdm_tuning* chosen) {
             }
     // the three fastest again with trials three times as long (configurations within a
     // few percent of each other are not told apart reliably by short trials), each with
-    // the side work forked before or after the tile lists, and with the step replayed
-    // from a captured graph and launched kernel by kernel: which is
-    // faster depends on the size of the step, and it changes the ranking of the other
-    // settings (graph replay of the three-stream step was measured slower than direct
-    // launches at 22 x 22,750 atoms, where 8 waves per i-block won under replay and 4
-    // under direct launches)
+    // the placements of the side work, and with the step replayed from a captured graph and
+    // launched kernel by kernel: which is faster depends on the size of the step
     // Each finalist is timed in two rounds over all of them and ranked by the sum, so
     // that a slow moment of the GPU during one trial does not decide between settings
     // that differ by a few percent.
     std::stable_sort(timed.begin(), timed.end(),
                      [](const auto& p, const auto& q) { return p.first < q.first; });
     std::vector<sdm_tuning> finalists;
+    const bool terms = c->ncen + c->nali + c->nterm > 0;
     for (size_t k = 0; k < timed.size() && k < 3; k++)
         for (int variant = 0; variant < 10; variant++) {
             sdm_tuning t = timed[k].second;
             t.use_graph = variant & 1;
             t.side_fork = variant >> 1;
+            // without restraints and force-field terms 0, 1, 3 and 4 are the same step
+            if (!terms && t.side_fork != 1 && t.side_fork != 2) continue;
             finalists.push_back(t);
         }
     std::vector<double> total(finalists.size(), 0.0);

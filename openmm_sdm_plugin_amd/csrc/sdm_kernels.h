@@ -5,12 +5,12 @@
 //
 //   k_bin -> k_scan -> k_scatter -> k_cellsort -> k_blockorder          spatial sort
 //   k_refresh -> k_tiles   slot records, boxes; tile lists
-//   k_pair                 F0: LJ+RF of every pair at x (FP32 math, fixed-point forces)
-//   k_energy64             U0 on the steps that report energies (FP64 pair sums)
-//   k_bonded               Ub, Fb: harmonic bonds/angles at x (FP64, gathered per atom)
-//   k_ligcand              j-blocks near the displaced atoms at x or at x+d
-//   k_denv                 screened pair lists; F1-F0 on the surrounding atoms (FP64)
-//   k_dlig, k_deltaA_red   u and F1-F0 on displaced atoms (FP64, pairs with d_i != d_j)
+//                          and the j-blocks near the displaced atoms at x or at x+d
+//   k_forces               F0: LJ+RF of every pair at x (FP32 math, fixed-point forces)
+//                          U0 on the steps that report energies (FP64 pair sums)
+//                          Ub, Fb: harmonic bonds/angles at x (FP64, gathered per atom)
+//                          u and F1-F0 (FP64, pairs with d_i != d_j)
+//   k_deltaA_red           the sums of u and F1-F0 on displaced atoms
 //   k_scalar               SoftCoreF, bias W/W', PotEnergy, noneq schedule/work, sp
 //   k_mix                  F += sp (F1 - F0)
 //   k_langevin             leapfrog Langevin update, Philox noise (FP64)
@@ -406,6 +406,86 @@ __device__ __forceinline__ bool lists_tile(int ib, int jb) {
     return jb == ib || (jb > ib) == (((ib ^ jb) & 1) != 0);
 }
 
+// candidate j-blocks: within rc of a displaced class's box at x or at x+d_k.  One
+// workgroup of NW waves per replica (they share the class boxes' reductions and the scan
+// over the blocks, so the replica's serial chain is short); candidates are written in
+// ascending block order.
+template <int NW>
+__device__ __forceinline__ void lig_candidates(
+    int r, int Np, int NB, int L, int ncls, const int* __restrict__ lig, const int* __restrict__ cls,
+    const double* __restrict__ cdispl, const double* __restrict__ x64,
+    const float4* __restrict__ bb_lo, const float4* __restrict__ bb_hi, int maxc,
+    int* __restrict__ cand, int* __restrict__ ncand, float list_r2, const Geom& g,
+    int* __restrict__ flags, int* __restrict__ cmap) {
+    __shared__ float4 blo[2 * SDM_MAX_CLASSES], bhi[2 * SDM_MAX_CLASSES];
+    __shared__ double red[6][NW];
+    __shared__ int wcount[NW];
+    const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+    const double* X = x64 + (size_t)r * 3 * Np;
+    for (int k = 1; k <= ncls; k++) {
+        double v[6] = {1e300, 1e300, 1e300, -1e300, -1e300, -1e300};
+        for (int li = t; li < L; li += 64 * NW) {
+            int a = lig[li];
+            if (cls[a] != k) continue;
+            for (int d = 0; d < 3; d++) {
+                double x = X[d * Np + a];
+                v[d] = fmin(v[d], x);
+                v[3 + d] = fmax(v[3 + d], x);
+            }
+        }
+        for (int d = 0; d < 3; d++) {
+            v[d] = wave_min_d(v[d]);
+            v[3 + d] = wave_max_d(v[3 + d]);
+        }
+        if (lane == 0)
+            for (int q = 0; q < 6; q++) red[q][wv] = v[q];
+        __syncthreads();
+        if (t == 0) {
+            for (int w = 1; w < NW; w++)
+                for (int d = 0; d < 3; d++) {
+                    v[d] = fmin(v[d], red[d][w]);
+                    v[3 + d] = fmax(v[3 + d], red[3 + d][w]);
+                }
+            const double* dk = cdispl + 3 * k;
+            blo[2 * (k - 1)] = make_float4((float)v[0], (float)v[1], (float)v[2], 0.f);
+            bhi[2 * (k - 1)] = make_float4((float)v[3], (float)v[4], (float)v[5], 0.f);
+            blo[2 * (k - 1) + 1] = make_float4((float)(v[0] + dk[0]), (float)(v[1] + dk[1]),
+                                               (float)(v[2] + dk[2]), 0.f);
+            bhi[2 * (k - 1) + 1] = make_float4((float)(v[3] + dk[0]), (float)(v[4] + dk[1]),
+                                               (float)(v[5] + dk[2]), 0.f);
+        }
+        __syncthreads();  // red is reused by the next class
+    }
+    const float4* lo = bb_lo + (size_t)r * NB;
+    const float4* hi = bb_hi + (size_t)r * NB;
+    int* out = cand + (size_t)r * maxc;
+    int count = 0;  // candidates before this round (uniform)
+    for (int base = 0; base < NB; base += 64 * NW) {
+        int jb = base + t;
+        bool ok = false;
+        if (jb < NB) {
+            float4 lj = lo[jb], hj = hi[jb];
+            for (int k = 0; k < 2 * ncls; k++) ok = ok || (bbox_gap2(blo[k], bhi[k], lj, hj, g) < list_r2);
+        }
+        unsigned long long m = __ballot(ok);
+        if (lane == 0) wcount[wv] = __popcll(m);
+        __syncthreads();
+        int before = count;
+        for (int w = 0; w < wv; w++) before += wcount[w];
+        int pos = before + lane_rank(m);
+        if (ok && pos < maxc) out[pos] = jb;
+        // block -> candidate index (-1: none), for the Langevin kernel's gather of the
+        // displaced-state forces
+        if (cmap && jb < NB) cmap[(size_t)r * NB + jb] = (ok && pos < maxc) ? pos : -1;
+        for (int w = 0; w < NW; w++) count += wcount[w];
+        __syncthreads();  // wcount is rewritten next round
+    }
+    if (t == 0) {
+        ncand[r] = min(count, maxc);
+        if (count > maxc) atomicOr(&flags[r], 4);
+    }
+}
+
 // tile list of one i-block: every j-block it lists (lists_tile) whose box is within the
 // list radius r_l (r_c + skin + slack, TileRadius) of the i-block's box, ascending, each
 // with a 64-bit mask of the pairs of 8-slot clusters whose boxes lie within r_l: bit
@@ -418,6 +498,16 @@ __device__ __forceinline__ bool lists_tile(int ib, int jb) {
 // Kept lists (tr.reuse_d2 >= 0): the workgroup returns at once while no atom of the
 // replica has moved more than half the skin since the build (dmax); a build stores the
 // block's slot coordinates in xb.
+// The first workgroup of a replica with displaced atoms finds the candidate blocks
+// (LigCand::groups is 1) instead: both need the boxes only, and a launch of its own would
+// take as long as this one.
+struct LigCand {
+    int groups, L, ncls, maxc;
+    float r2;
+    const int *lig, *cls;
+    const double *cdispl, *x64;
+    int *cand, *ncand, *cmap;
+};
 template <int NW>  // waves per i-block workgroup
 __global__ __launch_bounds__(64 * NW) void k_tiles(int N, int Np, int NB, int maxj,
                                                const float4* __restrict__ arec,
@@ -429,9 +519,14 @@ __global__ __launch_bounds__(64 * NW) void k_tiles(int N, int Np, int NB, int ma
                                                int* __restrict__ ntiles,
                                                const float* __restrict__ dmax,
                                                float4* __restrict__ xb, TileRadius tr, Geom g,
-                                               int* __restrict__ flags) {
+                                               int* __restrict__ flags, LigCand lc) {
     __shared__ int nkept[2][NW];
-    const int r = blockIdx.y, ib = blockIdx.x;
+    const int r = blockIdx.y, ib = (int)blockIdx.x - lc.groups;
+    if (ib < 0) {
+        lig_candidates<NW>(r, Np, NB, lc.L, lc.ncls, lc.lig, lc.cls, lc.cdispl, lc.x64, bb_lo,
+                           bb_hi, lc.maxc, lc.cand, lc.ncand, lc.r2, g, flags, lc.cmap);
+        return;
+    }
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const float list_r2 = tr.r2;
@@ -557,6 +652,19 @@ __device__ __forceinline__ float sum8(float y) {
     return dpp_add<0x141>(y, y); // row_half_mirror: lane i <- 7 - i within 8
 }
 
+template <int CTRL>
+__device__ __forceinline__ double dpp_d(double v) {
+    const long long b = __double_as_longlong(v);
+    const unsigned lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, true);
+    const unsigned hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
+    return __longlong_as_double((long long)((unsigned long long)hi << 32 | lo));
+}
+__device__ __forceinline__ double sum8(double y) {
+    y += dpp_d<0xB1>(y);
+    y += dpp_d<0x4E>(y);
+    return y + dpp_d<0x141>(y);
+}
+
 // Maps workgroup ids so that consecutive (replica, block) work lands on one XCD:
 // workgroups are dispatched to the 8 XCDs round-robin, each XCD has its own L2.
 __device__ __forceinline__ int xcd_linear_id(int id, int n) {
@@ -661,22 +769,16 @@ __device__ __forceinline__ bool tile_shift(float4 bli, float4 bhi, float4 blj, f
 //   vmcnt but need not retire in issue order, so the copy is waited for with vmcnt(0) before
 //   the atomics, not with vmcnt(3) after them.
 //   GEO: the geometric LJ sigma rule, the records holding sigma itself (Geom::geo).
-template <int WPW, bool COUNT, bool GEO>
-__global__ __launch_bounds__(64 * WPW) __attribute__((amdgpu_waves_per_eu(4))) void k_pair(
-    int R, int N, int Np, int NB, int maxj, TileShare share, const float4* __restrict__ arec,
+//   w: the wave among those of all replicas and i-blocks; tile_s, em_s, xi_s: its LDS.
+template <bool COUNT, bool GEO>
+__device__ __forceinline__ void pair_wave(
+    int w, int lane, float4* tile_s, unsigned long long* em_s, float* xi_s, int R, int N, int Np,
+    int NB, int maxj, TileShare share, const float4* __restrict__ arec,
     const int* __restrict__ tiles, const unsigned long long* __restrict__ tmask,
     const int* __restrict__ ntiles, const float4* __restrict__ bb_lo,
     const float4* __restrict__ bb_hi, const int* __restrict__ exs,
     const unsigned long long* __restrict__ exblocks, int max_ex, long long* __restrict__ F,
-    int* __restrict__ flags, unsigned long long* __restrict__ pair_count, Geom g) {
-    __shared__ float4 tile_s[WPW][2][128];
-    __shared__ unsigned long long em_s[WPW][64];
-    __shared__ float xi_s[WPW][3][64];
-    // wave-uniform by construction; readfirstlane lets the compiler keep everything
-    // derived from it (replica, block, tile, mask) in scalar registers
-    int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    int w = xcd_linear_id(blockIdx.x, gridDim.x) * WPW + wv;
-    const int lane = threadIdx.x & 63;
+    int* __restrict__ flags, unsigned long long* __restrict__ pair_count, const Geom& g) {
     const int split = share.split, waves = share.waves();
     if (w >= R * NB * waves) return;
     // waves per (replica, i-block): tiles part, part + split, .., clusters of smask
@@ -698,7 +800,7 @@ __global__ __launch_bounds__(64 * WPW) __attribute__((amdgpu_waves_per_eu(4))) v
     // copies the 64 slot records (32 B) of j-block jb into tile buffer b: lane L moves
     // half L&1 of record L>>1 (first instruction) and of record 32 + (L>>1) (second)
     auto stage = [&](int jb, int b) {
-        float4* dst = tile_s[wv][b];
+        float4* dst = tile_s + 128 * b;
         const char* src = (const char*)(A + 2 * jb * 64) + lane * 16;
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_global_load_lds((const void*)src,
@@ -741,9 +843,9 @@ __global__ __launch_bounds__(64 * WPW) __attribute__((amdgpu_waves_per_eu(4))) v
     }
     if (vi) {  // i coordinates as stored, for tiles that shift them
         const float4 a = A[2 * islot];
-        xi_s[wv][0][lane] = a.x;
-        xi_s[wv][1][lane] = a.y;
-        xi_s[wv][2][lane] = a.z;
+        xi_s[lane] = a.x;
+        xi_s[64 + lane] = a.y;
+        xi_s[128 + lane] = a.z;
     }
     int ox = 0, oy = 0, oz = 0;  // what xi, yi, zi are shifted by now (bits of the floats)
     const int* E = exs + (size_t)rb * max_ex * 64;
@@ -782,7 +884,7 @@ __global__ __launch_bounds__(64 * WPW) __attribute__((amdgpu_waves_per_eu(4))) v
     // lane that holds the sum of j atom `lane` of a tile (cluster lane >> 3 in lanes with
     // il = that cluster), as a byte address for ds_bpermute
     const int transpose = 4 * ((lane >> 3) + 8 * (lane & 7));
-    const unsigned rec_lds = (unsigned)(size_t)&tile_s[wv][0][2 * jl];
+    const unsigned rec_lds = (unsigned)(size_t)&tile_s[2 * jl];
     wait_vmem();  // the first tile and the i atoms have arrived
     for (int t = part, q = 0; t < nt; t += split, q++, buf ^= 1) {
         const int ql = q & 63;
@@ -803,9 +905,9 @@ __global__ __launch_bounds__(64 * WPW) __attribute__((amdgpu_waves_per_eu(4))) v
             oz = up ? sz : 0;
 #pragma unroll
             for (int k = 0; k < 8; k++) {
-                xi[k] = xi_s[wv][0][8 * k + il] - __int_as_float(ox);
-                yi[k] = xi_s[wv][1][8 * k + il] - __int_as_float(oy);
-                zi[k] = xi_s[wv][2][8 * k + il] - __int_as_float(oz);
+                xi[k] = xi_s[8 * k + il] - __int_as_float(ox);
+                yi[k] = xi_s[64 + 8 * k + il] - __int_as_float(oy);
+                zi[k] = xi_s[128 + 8 * k + il] - __int_as_float(oz);
             }
         }
         if (t + split < nt) {
@@ -826,7 +928,7 @@ __global__ __launch_bounds__(64 * WPW) __attribute__((amdgpu_waves_per_eu(4))) v
         if (ex) {
             const unsigned long long em = tile_exclusions(eset, max_ex, E, lane, vi, ib, jb, N);
             ex = __ballot(em != 0ull) != 0ull;
-            em_s[wv][lane] = em;
+            em_s[lane] = em;
         }
         const int general = __builtin_amdgcn_readfirstlane(mi || ex ? 1 : 0);
         float fjx = 0.f, fjy = 0.f, fjz = 0.f;  // sum of cluster il, atom jl
@@ -871,7 +973,7 @@ __global__ __launch_bounds__(64 * WPW) __attribute__((amdgpu_waves_per_eu(4))) v
                         in = __ballot(r2 < g.rc2f);
                     }
                     if (ex) {  // the shift by uniform jc8 and lane jl in two steps
-                        const unsigned long long em = em_s[wv][8 * k + il];
+                        const unsigned long long em = em_s[8 * k + il];
                         const unsigned eb = (unsigned)(jc8 & 32 ? em >> 32 : em) >> (jc8 & 31);
                         in &= __ballot(!((eb >> jl) & 1u));
                     }
@@ -956,16 +1058,15 @@ __global__ __launch_bounds__(64 * WPW) __attribute__((amdgpu_waves_per_eu(4))) v
 // __syncthreads() it does not wait for the wave's global loads in flight.
 __device__ __forceinline__ void lds_order() { asm volatile("" ::: "memory"); }
 
-__global__ __launch_bounds__(64) void k_energy64(
-    int R, int N, int Np, int NB, int maxj, TileShare share, const Rec64* __restrict__ rec,
+//   irec, jrec, em_s: the wave's LDS
+__device__ __forceinline__ void energy64_wave(
+    int w, int lane, Rec64* irec, Rec64* jrec, unsigned long long* em_s, int R, int N, int Np,
+    int NB, int maxj, TileShare share, const Rec64* __restrict__ rec,
     const int* __restrict__ tiles, const unsigned long long* __restrict__ tmask,
     const int* __restrict__ ntiles, const float4* __restrict__ bb_lo,
     const float4* __restrict__ bb_hi, const int* __restrict__ exs,
-    const unsigned long long* __restrict__ exblocks, int max_ex, double* __restrict__ e_out, Geom g) {
-    __shared__ Rec64 irec[64], jrec[64];
-    __shared__ unsigned long long em_s[64];
-    const int w = xcd_linear_id(blockIdx.x, gridDim.x);
-    const int lane = threadIdx.x;
+    const unsigned long long* __restrict__ exblocks, int max_ex, double* __restrict__ e_out,
+    const Geom& g) {
     const int split = share.split, waves = share.waves();
     if (w >= R * NB * waves) return;
     const int rb = w / waves, part = (w - rb * waves) / share.sub;
@@ -1077,17 +1178,17 @@ __global__ __launch_bounds__(64) void k_energy64(
 // [astart[i], astart[i+1]).  The forces go to Fb (FP64, atom order, [R][3][Np]), which
 // the integrator adds to the fixed-point accumulator.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_bonded(
-    int N, int Np, const int* __restrict__ bstart, const int* __restrict__ bcode,
-    const int* __restrict__ astart, const int* __restrict__ acode,
-    const int* __restrict__ bond_atoms, const double* __restrict__ bond_r0,
-    const double* __restrict__ bond_k, const int* __restrict__ ang_atoms,
-    const double* __restrict__ ang_t0, const double* __restrict__ ang_k,
-    const double* __restrict__ x64, double* __restrict__ Fb, double* __restrict__ e_bond,
-    int nbw, int* __restrict__ flags) {
-    __shared__ double red[256];
-    int r = blockIdx.y;
-    int i = blockIdx.x * 256 + threadIdx.x;
+//   One wave takes 64 atoms of one replica (w: replica, then block of 64 atoms).
+__device__ __forceinline__ void bonded_wave(
+    int w, int lane, int R, int N, int Np, int nbw, const int* __restrict__ bstart,
+    const int* __restrict__ bcode, const int* __restrict__ astart,
+    const int* __restrict__ acode, const int* __restrict__ bond_atoms,
+    const double* __restrict__ bond_r0, const double* __restrict__ bond_k,
+    const int* __restrict__ ang_atoms, const double* __restrict__ ang_t0,
+    const double* __restrict__ ang_k, const double* __restrict__ x64, double* __restrict__ Fb,
+    double* __restrict__ e_bond, int* __restrict__ flags) {
+    if (w >= R * nbw) return;
+    const int r = w / nbw, i = (w - r * nbw) * 64 + lane;
     const double* X = x64 + (size_t)r * 3 * Np;
     double e = 0.0;
     if (i < N) {
@@ -1143,13 +1244,8 @@ __global__ __launch_bounds__(256) void k_bonded(
         }
         if (bad) atomicOr(&flags[r], 2);
     }
-    red[threadIdx.x] = e;
-    __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if (threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) e_bond[(size_t)r * nbw + blockIdx.x] = red[0];
+    e = wave_sum(e);
+    if (lane == 0) e_bond[w] = e;
 }
 
 // ---------------------------------------------------------------------------
@@ -1567,87 +1663,6 @@ __global__ __launch_bounds__(256) void k_terms(int Np, DevTerms T, const double*
 // displaced-state passes (FP64)
 // ---------------------------------------------------------------------------
 
-// candidate j-blocks: within rc of a displaced class's box at x or at x+d_k.  One
-// 256-thread workgroup per replica (4 waves share the class boxes' reductions and the
-// scan over the blocks, so the replica's serial chain is short); candidates are written
-// in ascending block order.
-constexpr int LIGCAND_THREADS = 256;
-__global__ __launch_bounds__(LIGCAND_THREADS) void k_ligcand(
-    int Np, int NB, int L, int ncls, const int* __restrict__ lig, const int* __restrict__ cls,
-    const double* __restrict__ cdispl, const double* __restrict__ x64,
-    const float4* __restrict__ bb_lo, const float4* __restrict__ bb_hi, int maxc,
-    int* __restrict__ cand, int* __restrict__ ncand, float list_r2, Geom g,
-    int* __restrict__ flags, int* __restrict__ cmap) {
-    constexpr int NW = LIGCAND_THREADS / 64;
-    __shared__ float4 blo[2 * SDM_MAX_CLASSES], bhi[2 * SDM_MAX_CLASSES];
-    __shared__ double red[6][NW];
-    __shared__ int wcount[NW];
-    const int r = blockIdx.x, t = threadIdx.x, lane = t & 63, wv = t >> 6;
-    const double* X = x64 + (size_t)r * 3 * Np;
-    for (int k = 1; k <= ncls; k++) {
-        double v[6] = {1e300, 1e300, 1e300, -1e300, -1e300, -1e300};
-        for (int li = t; li < L; li += LIGCAND_THREADS) {
-            int a = lig[li];
-            if (cls[a] != k) continue;
-            for (int d = 0; d < 3; d++) {
-                double x = X[d * Np + a];
-                v[d] = fmin(v[d], x);
-                v[3 + d] = fmax(v[3 + d], x);
-            }
-        }
-        for (int d = 0; d < 3; d++) {
-            v[d] = wave_min_d(v[d]);
-            v[3 + d] = wave_max_d(v[3 + d]);
-        }
-        if (lane == 0)
-            for (int q = 0; q < 6; q++) red[q][wv] = v[q];
-        __syncthreads();
-        if (t == 0) {
-            for (int w = 1; w < NW; w++)
-                for (int d = 0; d < 3; d++) {
-                    v[d] = fmin(v[d], red[d][w]);
-                    v[3 + d] = fmax(v[3 + d], red[3 + d][w]);
-                }
-            const double* dk = cdispl + 3 * k;
-            blo[2 * (k - 1)] = make_float4((float)v[0], (float)v[1], (float)v[2], 0.f);
-            bhi[2 * (k - 1)] = make_float4((float)v[3], (float)v[4], (float)v[5], 0.f);
-            blo[2 * (k - 1) + 1] = make_float4((float)(v[0] + dk[0]), (float)(v[1] + dk[1]),
-                                               (float)(v[2] + dk[2]), 0.f);
-            bhi[2 * (k - 1) + 1] = make_float4((float)(v[3] + dk[0]), (float)(v[4] + dk[1]),
-                                               (float)(v[5] + dk[2]), 0.f);
-        }
-        __syncthreads();  // red is reused by the next class
-    }
-    const float4* lo = bb_lo + (size_t)r * NB;
-    const float4* hi = bb_hi + (size_t)r * NB;
-    int* out = cand + (size_t)r * maxc;
-    int count = 0;  // candidates before this round (uniform)
-    for (int base = 0; base < NB; base += LIGCAND_THREADS) {
-        int jb = base + t;
-        bool ok = false;
-        if (jb < NB) {
-            float4 lj = lo[jb], hj = hi[jb];
-            for (int k = 0; k < 2 * ncls; k++) ok = ok || (bbox_gap2(blo[k], bhi[k], lj, hj, g) < list_r2);
-        }
-        unsigned long long m = __ballot(ok);
-        if (lane == 0) wcount[wv] = __popcll(m);
-        __syncthreads();
-        int before = count;
-        for (int w = 0; w < wv; w++) before += wcount[w];
-        int pos = before + lane_rank(m);
-        if (ok && pos < maxc) out[pos] = jb;
-        // block -> candidate index (-1: none), for the Langevin kernel's gather of the
-        // displaced-state forces
-        if (cmap && jb < NB) cmap[(size_t)r * NB + jb] = (ok && pos < maxc) ? pos : -1;
-        for (int w = 0; w < NW; w++) count += wcount[w];
-        __syncthreads();  // wcount is rewritten next round
-    }
-    if (t == 0) {
-        ncand[r] = min(count, maxc);
-        if (count > maxc) atomicOr(&flags[r], 4);
-    }
-}
-
 __device__ __forceinline__ bool excluded(const int* __restrict__ ex_start,
                                          const int* __restrict__ ex_list, int a, int b) {
     for (int k = ex_start[a]; k < ex_start[a + 1]; k++)
@@ -1712,24 +1727,18 @@ struct AtomTile64 {
     int cls[64], idx[64];
 };
 
-__device__ __forceinline__ void stage_atom(AtomTile64& T, int t, const double* __restrict__ X,
-                                           int Np, int a, const int* __restrict__ cls,
-                                           const double* __restrict__ cdispl,
-                                           const double* __restrict__ q,
-                                           const double* __restrict__ sig,
-                                           const double* __restrict__ eps) {
-    int k = cls[a];
-    T.x[t] = X[a];
-    T.y[t] = X[Np + a];
-    T.z[t] = X[2 * Np + a];
-    T.dx[t] = cdispl[3 * k];
-    T.dy[t] = cdispl[3 * k + 1];
-    T.dz[t] = cdispl[3 * k + 2];
-    T.q[t] = q[a];
-    T.sig[t] = sig[a];
-    T.se[t] = sqrt(eps[a]);
-    T.cls[t] = k;
-    T.idx[t] = a;
+__device__ __forceinline__ void stage_atom(AtomTile64& T, int t, const Atom64& A) {
+    T.x[t] = A.x;
+    T.y[t] = A.y;
+    T.z[t] = A.z;
+    T.dx[t] = A.dx;
+    T.dy[t] = A.dy;
+    T.dz[t] = A.dz;
+    T.q[t] = A.qk;
+    T.sig[t] = A.sig;
+    T.se[t] = A.se;
+    T.cls[t] = A.cls;
+    T.idx[t] = A.idx;
 }
 
 __device__ __forceinline__ Atom64 tile_atom(const AtomTile64& T, int t) {
@@ -1762,172 +1771,267 @@ __device__ __forceinline__ bool excl_with(const int* __restrict__ ex_start,
 }
 
 // The displaced-state pairs: every (displaced atom i, undisplaced atom j) within the
-// cutoff at x or at x+d, evaluated in FP64 at both geometries (delta_pair).  Two passes
-// evaluate each such pair once from each side, so that every sum has one owner lane and
-// a fixed order (no atomics):
-//   k_denv  lanes = the 64 slots of candidate block c.  An FP32 screen of the block's
-//           undisplaced atoms against every displaced atom (at x and at x+d, with a
-//           margin that covers FP32 rounding) gives each lane its 64-bit list of partners
-//           per ligand block, whose pairs it then evaluates: F1-F0 on the undisplaced
-//           atom (dB).  The screen's ballot per displaced atom is the same list seen
-//           from the other side; it goes to mlig[r][c][li].
-//   k_dlig  lanes = the displaced atoms of ligand block lb, one candidate block per
-//           workgroup: each lane evaluates the pairs of its mlig bits, giving u and F1-F0
-//           on the displaced atom, one partial per candidate block (dA), added in block
-//           order by k_deltaA_red.
-// A few blocks near the displaced atoms hold most pairs, so both spread a block's pairs
-// over DW waves (wave w takes the partners with index = w mod DW, ascending) and add
-// the waves' partials in wave order.  Excluded pairs are left out of the lists (only
-// atoms with an exclusion across the displaced/undisplaced boundary search their
-// exclusion list).
+// cutoff at x or at x+d, evaluated once in FP64 at both geometries (delta_pair); every sum
+// has one owner and a fixed order (no atomics).  A wave takes eight displaced atoms of each
+// ligand block, one of DISP_WAVES groups, and the 64 slots of candidate block c, a cluster
+// of 8 slots at a time (lane 8 q + k: displaced atom k, slot q of the cluster):
+//   An FP32 screen (at x and at x+d, with a margin that covers FP32 rounding) finds the
+//   clusters with a pair in range.
+//   u and F1-F0 on the displaced atoms are summed in the lane over the clusters and then
+//   over the eight lanes of an atom; one partial per candidate block (dA), added in block
+//   order by k_deltaA_red.
+//   F1-F0 on the slots is summed over the eight displaced atoms at each step, and lane
+//   8 q + k keeps it for cluster k; one part per wave (dB, env_force).
+// Excluded pairs are left out (only atoms with an exclusion across the displaced/undisplaced
+// boundary search their exclusion list).
+//
+// What bounds it is the chain of loads and of up to 8 steps of FP64 pairs of one wave (a few
+// blocks near the displaced atoms hold most pairs) and, with many replicas, FP64 issue.  With
+// lanes = slots and lanes = displaced atoms in turn, each lane walking its list of partners,
+// every pair was evaluated twice and most lanes waited for the longest list: as a part of
+// k_forces it added 58 us to 22 x 22,750 atoms, so 26 us.
 constexpr float DSCREEN_MARGIN = 1e-3f;  // nm; FP32 position rounding is below 1e-6 nm
-constexpr int DPAIR_WAVES = 4;
+constexpr int DISP_WAVES = 8;            // groups of eight displaced atoms of a ligand block
+// candidate blocks of a replica that have waves of their own; further ones take turns
+constexpr int DISP_BLOCKS = 64;
 
-template <int DW>
-__global__ __launch_bounds__(64 * DW) void k_denv(
-    int N, int Np, int L, int LB, const int* __restrict__ lig,
-    const int* __restrict__ lb_start, const int* __restrict__ lb_count,
-    const int* __restrict__ cls, const double* __restrict__ cdispl,
-    const double* __restrict__ q64, const double* __restrict__ sig64,
-    const double* __restrict__ eps64, const int* __restrict__ ex_start,
-    const int* __restrict__ ex_list, const double* __restrict__ x64,
-    const int* __restrict__ orig_s, const int* __restrict__ cand, const int* __restrict__ ncand,
-    int maxc, unsigned long long* __restrict__ mlig, double4* __restrict__ dB, Geom g) {
-    int c = blockIdx.x, r = blockIdx.y, lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    if (c >= ncand[r]) return;  // uniform over the workgroup
-    const double* X = x64 + (size_t)r * 3 * Np;
-    int s = cand[(size_t)r * maxc + c] * 64 + lane;
-    bool v = s < N;
-    int b = v ? orig_s[(size_t)r * Np + s] : 0;
-    Atom64 J = load_atom64(X, Np, b, cls, cdispl, q64, sig64, eps64);
-    bool env = v && J.cls == 0;
-    bool exJ = env && excl_with(ex_start, ex_list, cls, b, true);
-    const float jx = (float)J.x, jy = (float)J.y, jz = (float)J.z;
-    const float rs = (float)sqrt(g.rc2) + DSCREEN_MARGIN, rs2 = rs * rs;
-    __shared__ AtomTile64 T;
-    __shared__ float4 P0[64], P1[64];  // the ligand block at x and at x+d, FP32
-    __shared__ double4 part[DW][64];
-    unsigned long long* ML = mlig + ((size_t)r * maxc + c) * L;
-    double fx = 0.0, fy = 0.0, fz = 0.0;
-    for (int lb = 0; lb < LB; lb++) {
-        const int base = lb_start[lb], n = lb_count[lb];
-        __syncthreads();  // the previous ligand block has been read
-        if ((int)threadIdx.x < n) {
-            int a = lig[base + threadIdx.x];
-            stage_atom(T, threadIdx.x, X, Np, a, cls, cdispl, q64, sig64, eps64);
-            const double* d = cdispl + 3 * cls[a];
-            double x = X[a], y = X[Np + a], z = X[2 * Np + a];
-            P0[threadIdx.x] = make_float4((float)x, (float)y, (float)z, 0.f);
-            P1[threadIdx.x] =
-                make_float4((float)(x + d[0]), (float)(y + d[1]), (float)(z + d[2]), 0.f);
-        }
-        __syncthreads();
-        unsigned long long mine = 0ull, col = 0ull;
-        for (int k = wv; k < n; k += DW) {
-            float4 p0 = P0[k], p1 = P1[k];
-            float dx = jx - p0.x, dy = jy - p0.y, dz = jz - p0.z;
-            dx -= g.bx * rintf(dx * g.ibx);
-            dy -= g.by * rintf(dy * g.iby);
-            dz -= g.bz * rintf(dz * g.ibz);
-            float ex = jx - p1.x, ey = jy - p1.y, ez = jz - p1.z;
-            ex -= g.bx * rintf(ex * g.ibx);
-            ey -= g.by * rintf(ey * g.iby);
-            ez -= g.bz * rintf(ez * g.ibz);
-            bool in = env && (dx * dx + dy * dy + dz * dz < rs2 || ex * ex + ey * ey + ez * ez < rs2);
-            if (exJ && in) in = !excluded(ex_start, ex_list, b, T.idx[k]);
-            unsigned long long bal = __ballot(in);
-            if (lane == k) col = bal;
-            mine |= (unsigned long long)in << k;
-        }
-        if (lane < n && lane % DW == wv) ML[base + lane] = col;
-        while (mine) {  // this lane's partners of this wave, ascending
-            int k = __ffsll((long long)mine) - 1;
-            mine &= mine - 1ull;
-            Atom64 I = tile_atom(T, k);
-            int iny;
-            delta_pair(J, I, g, fx, fy, fz, &iny);
-        }
+// the slots of one wave's candidate block
+struct EnvTile {
+    double x[64], y[64], z[64], q[64], sig[64], se[64];
+    int idx[64];
+};
+
+// F1-F0 on slot `lane` of candidate block cb (r * maxc + c): its waves' parts in order
+__device__ __forceinline__ double4 env_force(const double4* __restrict__ dB, int parts, size_t cb,
+                                             int lane) {
+    const double4* p = dB + cb * parts * 64 + lane;
+    double4 t = p[0];
+    for (int w = 1; w < parts; w++) {
+        const double4 q = p[64 * w];
+        t.x += q.x;
+        t.y += q.y;
+        t.z += q.z;
     }
-    part[wv][lane] = make_double4(fx, fy, fz, 0.0);
-    __syncthreads();
-    if (wv == 0) {
-        double4 t = part[0][lane];
-        for (int w = 1; w < DW; w++) {
-            t.x += part[w][lane].x;
-            t.y += part[w][lane].y;
-            t.z += part[w][lane].z;
+    return t;
+}
+
+//   w: replica, then candidate block and group, of which a wave takes `subs` in turn; waves:
+//   those of one replica; E: LDS.
+//   COUNT: adds the pairs within the cutoff at x+d to pair_count instead.
+template <bool COUNT>
+__device__ __forceinline__ void displaced_wave(
+    int w, int waves, int subs, int lane, EnvTile& E, int R, int N, int Np, int L, int LB,
+    const int* __restrict__ lig, const int* __restrict__ lb_start,
+    const int* __restrict__ lb_count, const int* __restrict__ cls,
+    const double* __restrict__ cdispl, const double* __restrict__ q64,
+    const double* __restrict__ sig64, const double* __restrict__ eps64,
+    const int* __restrict__ ex_start, const int* __restrict__ ex_list,
+    const double* __restrict__ x64, const int* __restrict__ orig_s,
+    const int* __restrict__ cand, const int* __restrict__ ncand, int maxc,
+    double4* __restrict__ dA, double4* __restrict__ dB,
+    unsigned long long* __restrict__ pair_count, const Geom& g) {
+    const int r = w / waves;
+    if (r >= R) return;
+    const int nc = ncand[r], parts = DISP_WAVES / subs, sub0 = (w - r * waves) % parts * subs;
+    const int kk = lane & 7, q = lane >> 3;
+    const double* X = x64 + (size_t)r * 3 * Np;
+    const float rs = (float)sqrt(g.rc2) + DSCREEN_MARGIN, rs2 = rs * rs;
+    for (int c = (w - r * waves) / parts; c < nc; c += waves / parts) {
+        const size_t cb = (size_t)r * maxc + c;
+        const int s = cand[cb] * 64 + lane;
+        const bool v = s < N;
+        const int b = v ? orig_s[(size_t)r * Np + s] : 0;
+        const bool env = v && cls[b] == 0;
+        lds_order();  // the previous block's atoms have been read
+        E.x[lane] = X[b];
+        E.y[lane] = X[Np + b];
+        E.z[lane] = X[2 * Np + b];
+        E.q[lane] = q64[b];
+        E.sig[lane] = sig64[b];
+        E.se[lane] = sqrt(eps64[b]);
+        E.idx[lane] = b;
+        const unsigned long long envm = __ballot(env);
+        const unsigned long long exm =
+            __ballot(env && excl_with(ex_start, ex_list, cls, b, true));
+        lds_order();
+        // the groups' sums are added in order here as in env_force, so that results do not
+        // depend on how many of them a wave takes
+        double tx = 0.0, ty = 0.0, tz = 0.0;
+        for (int sub = sub0; sub < sub0 + subs; sub++) {
+            double fx = 0.0, fy = 0.0, fz = 0.0;  // on slot 8 kk + q
+            for (int lb = 0; lb < LB; lb++) {
+                const int base = lb_start[lb], n = lb_count[lb], k = 8 * sub + kk;
+                if (8 * sub >= n) continue;  // uniform
+                const Atom64 I = load_atom64(X, Np, lig[base + min(k, n - 1)], cls, cdispl, q64, sig64,
+                                             eps64);
+                const float ix = (float)I.x, iy = (float)I.y, iz = (float)I.z;
+                const float jx = (float)(I.x + I.dx), jy = (float)(I.y + I.dy),
+                            jz = (float)(I.z + I.dz);
+                double gx = 0.0, gy = 0.0, gz = 0.0, du = 0.0;
+                int cnt = 0;
+                for (int jc = 0; jc < 8; jc++) {
+                    if (((envm >> (8 * jc)) & 0xffull) == 0ull) continue;  // uniform
+                    const int t = 8 * jc + q;
+                    Atom64 J;
+                    J.x = E.x[t];
+                    J.y = E.y[t];
+                    J.z = E.z[t];
+                    const float x = (float)J.x, y = (float)J.y, z = (float)J.z;
+                    float dx = x - ix, dy = y - iy, dz = z - iz;
+                    dx -= g.bx * rintf(dx * g.ibx);
+                    dy -= g.by * rintf(dy * g.iby);
+                    dz -= g.bz * rintf(dz * g.ibz);
+                    float ex = x - jx, ey = y - jy, ez = z - jz;
+                    ex -= g.bx * rintf(ex * g.ibx);
+                    ey -= g.by * rintf(ey * g.iby);
+                    ez -= g.bz * rintf(ez * g.ibz);
+                    bool in = k < n && ((envm >> t) & 1ull) &&
+                              (dx * dx + dy * dy + dz * dz < rs2 || ex * ex + ey * ey + ez * ez < rs2);
+                    if (((exm >> t) & 1ull) && in) in = !excluded(ex_start, ex_list, E.idx[t], I.idx);
+                    if (__ballot(in) == 0ull) continue;  // uniform
+                    double px = 0.0, py = 0.0, pz = 0.0;
+                    if (in) {
+                        J.dx = J.dy = J.dz = -0.0;  // x + -0.0 is x
+                        J.qk = E.q[t];
+                        J.sig = E.sig[t];
+                        J.se = E.se[t];
+                        int iny;
+                        du += delta_pair(I, J, g, px, py, pz, &iny);
+                        cnt += iny;
+                    }
+                    gx += px;
+                    gy += py;
+                    gz += pz;
+                    if (COUNT) continue;
+                    px = sum8(px);
+                    py = sum8(py);
+                    pz = sum8(pz);
+                    const bool keep = kk == jc;
+                    fx -= keep ? px : 0.0;
+                    fy -= keep ? py : 0.0;
+                    fz -= keep ? pz : 0.0;
+                }
+                if (COUNT) {
+                    const double sc = wave_sum((double)cnt);
+                    if (lane == 0 && sc > 0.0) atomicAdd(&pair_count[r], (unsigned long long)(sc + 0.5));
+                    continue;
+                }
+    #pragma unroll
+                for (int o = 8; o < 64; o <<= 1) {
+                    gx += __shfl_xor(gx, o, 64);
+                    gy += __shfl_xor(gy, o, 64);
+                    gz += __shfl_xor(gz, o, 64);
+                    du += __shfl_xor(du, o, 64);
+                }
+                if (q == 0 && k < n) dA[(cb * LB + lb) * 64 + k] = make_double4(gx, gy, gz, du);
+            }
+            tx = sub == sub0 ? fx : tx + fx;
+            ty = sub == sub0 ? fy : ty + fy;
+            tz = sub == sub0 ? fz : tz + fz;
         }
-        dB[((size_t)r * maxc + c) * 64 + lane] = t;
+        if (!COUNT)
+            dB[(cb * parts + sub0 / subs) * 64 + 8 * kk + q] = make_double4(tx, ty, tz, 0.0);
     }
 }
 
-template <int DW>
-__global__ __launch_bounds__(64 * DW) void k_dlig(
-    int N, int Np, int L, int LB, const int* __restrict__ lig,
-    const int* __restrict__ lb_start, const int* __restrict__ lb_count,
-    const int* __restrict__ cls, const double* __restrict__ cdispl,
-    const double* __restrict__ q64, const double* __restrict__ sig64,
-    const double* __restrict__ eps64, const double* __restrict__ x64,
-    const int* __restrict__ orig_s, const int* __restrict__ cand, const int* __restrict__ ncand,
-    int maxc, const unsigned long long* __restrict__ mlig, double4* __restrict__ dA, Geom g,
-    unsigned long long* __restrict__ pair_count) {
-    int c = blockIdx.x, lb = blockIdx.y, r = blockIdx.z;
-    int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    if (c >= ncand[r]) return;  // uniform; k_deltaA_red reads only the blocks below ncand
-    const double* X = x64 + (size_t)r * 3 * Np;
-    int li = lb_start[lb] + lane;
-    bool v = lane < lb_count[lb];
-    // this wave's partners: slots = wv mod DW
-    unsigned long long sel = 0ull;
-    for (int k = wv; k < 64; k += DW) sel |= 1ull << k;
-    unsigned long long m = v ? (mlig[((size_t)r * maxc + c) * L + li] & sel) : 0ull;
-    __shared__ AtomTile64 T;
-    __shared__ double4 part[DW][64];
-    __shared__ int any_s;
-    if (threadIdx.x == 0) any_s = 0;
-    __syncthreads();
-    const bool wany = __ballot(m != 0ull) != 0ull;
-    if (lane == 0 && wany) any_s = 1;
-    __syncthreads();
-    const bool any = any_s != 0;  // uniform over the workgroup
-    double du = 0.0, fx = 0.0, fy = 0.0, fz = 0.0;
-    int cnt = 0;
-    if (any) {
-        int s = cand[(size_t)r * maxc + c] * 64 + lane;
-        if (wv == 0 && s < N)
-            stage_atom(T, lane, X, Np, orig_s[(size_t)r * Np + s], cls, cdispl, q64, sig64, eps64);
-        Atom64 I = load_atom64(X, Np, v ? lig[li] : lig[lb_start[lb]], cls, cdispl, q64, sig64,
-                               eps64);
-        __syncthreads();
-        while (m) {  // this lane's partners of this wave, ascending slot
-            int k = __ffsll((long long)m) - 1;
-            m &= m - 1ull;
-            Atom64 J = tile_atom(T, k);
-            int iny;
-            du += delta_pair(I, J, g, fx, fy, fz, &iny);
-            cnt += iny;
-        }
-    }
-    if (pair_count) {
-        double sc = wave_sum((double)cnt);
-        if (lane == 0 && any) atomicAdd(&pair_count[r], (unsigned long long)(sc + 0.5));
+// The forces of one evaluation in one launch: workgroups of one wave (WPW, by tuning) take
+// first the displaced-state pairs (the longest chain of dependent loads), then the FP64 pair
+// energies where they are asked for, the pairs, and the bonded terms (short waves that wait
+// for memory, which fill the slots that the last pairs leave: 22 x 22,750 atoms, 10 steps
+// 6.03 ms so, 6.12 ms with them in front).  The parts need the slot records, tile lists and
+// candidates only and write to different places (or by integer atomics), so they run side by
+// side without the streams and events that separate launches would take: a dependency
+// between queues costs 4 to 12 us, and a step had five of them.  Each count is a multiple
+// of 8 workgroups, so that every part spreads over the XCDs alike.  Measured, separate
+// launches on three streams against this: 10 steps of 150 atoms without a box 0.89 -> 0.43 ms,
+// 20 steps of 22,750 atoms 2.24 -> 1.95 ms; 22 replicas of them, 10 steps, 6.14 -> 6.03 ms.
+//   COUNT: pairs within the cutoff (pair_count) and displaced-state pairs (pair_count + R).
+struct ForceGroups {
+    int displaced, energy, pairs;  // workgroups of each part; the rest are the bonded terms'
+    int displaced_waves;           // waves per replica, and groups of displaced atoms per wave
+    int displaced_subs;
+};
+
+template <int WPW, bool COUNT, bool GEO>
+__global__ __launch_bounds__(64 * WPW) __attribute__((amdgpu_waves_per_eu(4))) void k_forces(
+    ForceGroups fg, int R, int N, int Np, int NB, int maxj, TileShare share,
+    const float4* __restrict__ arec, const int* __restrict__ tiles,
+    const unsigned long long* __restrict__ tmask, const int* __restrict__ ntiles,
+    const float4* __restrict__ bb_lo, const float4* __restrict__ bb_hi,
+    const int* __restrict__ exs, const unsigned long long* __restrict__ exblocks, int max_ex,
+    long long* __restrict__ F, int* __restrict__ flags,
+    unsigned long long* __restrict__ pair_count, TileShare eshare,
+    const Rec64* __restrict__ rec, double* __restrict__ e64, int nbw,
+    const int* __restrict__ bstart, const int* __restrict__ bcode,
+    const int* __restrict__ astart, const int* __restrict__ acode,
+    const int* __restrict__ bond_atoms, const double* __restrict__ bond_r0,
+    const double* __restrict__ bond_k, const int* __restrict__ ang_atoms,
+    const double* __restrict__ ang_t0, const double* __restrict__ ang_k,
+    const double* __restrict__ x64, double* __restrict__ Fb, double* __restrict__ e_bond,
+    int L, int LB, const int* __restrict__ lig, const int* __restrict__ lb_start,
+    const int* __restrict__ lb_count, const int* __restrict__ cls,
+    const double* __restrict__ cdispl, const double* __restrict__ q64,
+    const double* __restrict__ sig64, const double* __restrict__ eps64,
+    const int* __restrict__ ex_start, const int* __restrict__ ex_list,
+    const int* __restrict__ orig_s, const int* __restrict__ cand,
+    const int* __restrict__ ncand, int maxc, double4* __restrict__ dA,
+    double4* __restrict__ dB, Geom g) {
+    // one wave's LDS: the pairs' two tiles, or the energies' records, or the displaced atoms
+    constexpr int LDS16 = 2 * 64 * sizeof(Rec64) / 16;
+    static_assert(LDS16 >= 256 && 16 * LDS16 >= sizeof(EnvTile), "LDS");
+    __shared__ float4 wave_s[WPW][LDS16];
+    __shared__ unsigned long long em_s[WPW][64];
+    __shared__ float xi_s[WPW][192];
+    // wave-uniform by construction; readfirstlane lets the compiler keep everything
+    // derived from it (replica, block, tile, mask) in scalar registers
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    int b = blockIdx.x;
+    if (b < fg.displaced) {
+        displaced_wave<COUNT>(b * WPW + wv, fg.displaced_waves, fg.displaced_subs, lane,
+                              *(EnvTile*)wave_s[wv], R, N, Np, L, LB, lig, lb_start, lb_count, cls, cdispl, q64, sig64, eps64,
+                              ex_start, ex_list, x64, orig_s, cand, ncand, maxc, dA, dB,
+                              pair_count + R, g);
         return;
     }
-    part[wv][lane] = make_double4(fx, fy, fz, du);
-    __syncthreads();
-    if (wv == 0) {
-        double4 t = part[0][lane];
-        for (int w = 1; w < DW; w++) {
-            t.x += part[w][lane].x;
-            t.y += part[w][lane].y;
-            t.z += part[w][lane].z;
-            t.w += part[w][lane].w;
-        }
-        dA[(((size_t)r * maxc + c) * LB + lb) * 64 + lane] = t;
+    b -= fg.displaced;
+    if (!COUNT && b < fg.energy) {
+        Rec64* irec = (Rec64*)wave_s[wv];
+        energy64_wave(xcd_linear_id(b, fg.energy) * WPW + wv, lane, irec, irec + 64, em_s[wv], R,
+                      N, Np, NB, maxj, eshare, rec, tiles, tmask, ntiles, bb_lo, bb_hi, exs,
+                      exblocks, max_ex, e64, g);
+        return;
     }
+    b -= fg.energy;
+    if (b < fg.pairs) {
+        pair_wave<COUNT, GEO>(xcd_linear_id(b, fg.pairs) * WPW + wv, lane, wave_s[wv], em_s[wv],
+                              xi_s[wv], R, N, Np, NB, maxj, share, arec, tiles, tmask, ntiles,
+                              bb_lo, bb_hi, exs, exblocks, max_ex, F, flags, pair_count, g);
+        return;
+    }
+    b -= fg.pairs;
+    if (!COUNT)
+        bonded_wave(b * WPW + wv, lane, R, N, Np, nbw, bstart, bcode, astart, acode, bond_atoms,
+                    bond_r0, bond_k, ang_atoms, ang_t0, ang_k, x64, Fb, e_bond, flags);
 }
 
-// per displaced atom: the block partials of k_dlig in order, plus pairs with displaced
+// The FP64 pair energies alone, beside the forces on another stream, for long launches: in
+// k_forces they have its 4 waves per SIMD, here 6, and other waves to run with.
+__global__ __launch_bounds__(64) void k_energy64(
+    int R, int N, int Np, int NB, int maxj, TileShare share, const Rec64* __restrict__ rec,
+    const int* __restrict__ tiles, const unsigned long long* __restrict__ tmask,
+    const int* __restrict__ ntiles, const float4* __restrict__ bb_lo,
+    const float4* __restrict__ bb_hi, const int* __restrict__ exs,
+    const unsigned long long* __restrict__ exblocks, int max_ex, double* __restrict__ e_out,
+    Geom g) {
+    __shared__ Rec64 irec[64], jrec[64];
+    __shared__ unsigned long long em_s[64];
+    energy64_wave(xcd_linear_id(blockIdx.x, gridDim.x), threadIdx.x, irec, jrec, em_s, R, N, Np,
+                  NB, maxj, share, rec, tiles, tmask, ntiles, bb_lo, bb_hi, exs, exblocks, max_ex,
+                  e_out, g);
+}
+
+// per displaced atom: the block partials of displaced_wave in order, plus pairs with displaced
 // atoms of a different class (D x D); writes dlig and the ligand block's u.
 template <int RW>
 __global__ __launch_bounds__(64 * RW) void k_deltaA_red(
@@ -1963,8 +2067,8 @@ __global__ __launch_bounds__(64 * RW) void k_deltaA_red(
         int n = min(64, L - base);
         __syncthreads();  // the previous chunk has been read
         if ((int)threadIdx.x < n)
-            stage_atom(T, threadIdx.x, X, Np, lig[base + threadIdx.x], cls, cdispl, q64, sig64,
-                       eps64);
+            stage_atom(T, threadIdx.x, load_atom64(X, Np, lig[base + threadIdx.x], cls, cdispl, q64,
+                                                   sig64, eps64));
         __syncthreads();
         for (int k = wv; k < n; k += RW) {
             Atom64 J = tile_atom(T, k);
@@ -2174,7 +2278,7 @@ __global__ __launch_bounds__(64) void k_mix(int N, int Np, int L, int maxc,
                                             const int* __restrict__ lig, const int* __restrict__ cls,
                                             const int* __restrict__ orig_s,
                                             const int* __restrict__ cand, const int* __restrict__ ncand,
-                                            const double4* __restrict__ dB,
+                                            int parts, const double4* __restrict__ dB,
                                             const double4* __restrict__ dlig,
                                             const DevRecord* __restrict__ rec,
                                             const int* __restrict__ slot_of,
@@ -2191,7 +2295,7 @@ __global__ __launch_bounds__(64) void k_mix(int N, int Np, int L, int maxc,
         if (s >= N) return;
         int b = orig_s[(size_t)r * Np + s];
         if (cls[b] != 0) return;
-        double4 d = dB[((size_t)r * maxc + c) * 64 + lane];
+        const double4 d = env_force(dB, parts, (size_t)r * maxc + c, lane);
         Fr[s] += to_fixed(sp * d.x, &bad);
         Fr[Np + s] += to_fixed(sp * d.y, &bad);
         Fr[2 * Np + s] += to_fixed(sp * d.z, &bad);
@@ -2221,7 +2325,7 @@ struct MixGather {
     const int* cmap;
     const double4* dB;
     const double4* dlig;
-    int NB, maxc, L;
+    int NB, maxc, L, parts;
 };
 
 __global__ __launch_bounds__(256) void k_langevin(int N, int Np, const double* __restrict__ invm,
@@ -2241,15 +2345,10 @@ __global__ __launch_bounds__(256) void k_langevin(int N, int Np, const double* _
     if (mg.lig_of) {
         const int li = mg.lig_of[i];
         const int sl = slot_of[(size_t)r * Np + i];
-        const double4* dp = nullptr;
-        if (li >= 0) {
-            dp = mg.dlig + (size_t)r * mg.L + li;
-        } else {
-            const int cb = mg.cmap[(size_t)r * mg.NB + (sl >> 6)];
-            if (cb >= 0) dp = mg.dB + ((size_t)r * mg.maxc + cb) * 64 + (sl & 63);
-        }
-        if (dp) {
-            const double4 d = *dp;
+        const int cb = li >= 0 ? 0 : mg.cmap[(size_t)r * mg.NB + (sl >> 6)];
+        if (cb >= 0) {
+            const double4 d = li >= 0 ? mg.dlig[(size_t)r * mg.L + li]
+                                      : env_force(mg.dB, mg.parts, (size_t)r * mg.maxc + cb, sl & 63);
             const double sp = Rr.sp;
             long long* Fm = F + (size_t)r * 3 * Np;
             int bad = 0;
@@ -2850,7 +2949,7 @@ __global__ __launch_bounds__(ADJ_ATOMS) void k_adj(
             ise = I.se > 0.0 ? 1.0 / I.se : 0.0;
         }
     }
-    if (GRAD) {
+    if constexpr (GRAD) {
         red[0][t] = sqrt(SDM_ONE_4PI_EPS0) * a.q;  // q64 holds q sqrt(k_e)
         red[1][t] = 2.0 * ses * a.s;
         red[2][t] = 2.0 * ise * a.e;
@@ -2970,7 +3069,7 @@ __global__ __launch_bounds__(64) void k_scatter_dF(int N, int Np, int L, int max
                                                    const int* __restrict__ orig_s,
                                                    const int* __restrict__ cand,
                                                    const int* __restrict__ ncand,
-                                                   const double4* __restrict__ dB,
+                                                   int parts, const double4* __restrict__ dB,
                                                    const double4* __restrict__ dlig,
                                                    double* __restrict__ dF) {
     int r = blockIdx.y, lane = threadIdx.x;
@@ -2982,7 +3081,7 @@ __global__ __launch_bounds__(64) void k_scatter_dF(int N, int Np, int L, int max
         if (s >= N) return;
         int b = orig_s[(size_t)r * Np + s];
         if (cls[b] != 0) return;
-        double4 d = dB[((size_t)r * maxc + c) * 64 + lane];
+        const double4 d = env_force(dB, parts, (size_t)r * maxc + c, lane);
         D[b] = d.x;
         D[Np + b] = d.y;
         D[2 * Np + b] = d.z;
