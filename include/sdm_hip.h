@@ -163,13 +163,13 @@ typedef struct {
                                      over the FP64 positions (their own kernel); the
                                      forces are FP32 pair arithmetic. */
     int32_t pair_split;           /* with pair_newton3 1 and pair_group 0: 1, 2, 4 (the
-                                     default), 8, 16 or 32 waves per i-block (at least:
-                                     systems of fewer than 512 blocks of 64 atoms get more,
-                                     except with 1), each taking every
-                                     pair_split-th tile, so that short tile lists do not
-                                     leave the GPU waiting on long ones and small batches
-                                     fill it.
-                                     Results differ only in rounding: each wave's i forces
+                                     default), 8, 16 or 32 parts that the tile list of an
+                                     i-block is shared out in (at least: except with 1
+                                     there are no fewer than 4, and more in systems of
+                                     fewer than 512 blocks of 64 atoms), each for a wave of
+                                     its own or several for one, so that the GPU does not
+                                     wait on long lists and small batches fill it.
+                                     Results differ only in rounding: each part's i forces
                                      are summed on their own before they are added up. */
     int32_t side_fork;            /* where the restraints and force-field terms run: 0 on a
                                      side stream forked after the tile lists (beside the

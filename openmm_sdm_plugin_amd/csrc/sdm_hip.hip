@@ -114,8 +114,9 @@ struct sdm_context {
     int* exs = nullptr;      // [R][NB][max_ex][64] exclusion partners in slot order (k_bbox)
     unsigned long long* exblocks = nullptr;  // [R][NB] set of the j-blocks that hold any
     float4* cbox = nullptr;  // [R][NB][16] centres and half extents of the 8-slot clusters
-    int *tiles = nullptr, *ntiles = nullptr;
+    int* tiles = nullptr;
     unsigned long long* tmask = nullptr;
+    int2 *tbounds = nullptr, *ebounds = nullptr;  // [R][NB][TILE_BOUNDS] shares of the waves
     int* cmap = nullptr;    // [R][NB] block -> candidate index (-1: none)
     int* lig_of = nullptr;  // [Np] atom -> index in lig (-1: environment)
     float4* xb = nullptr;   // [R][Np] slot coordinates when the tile lists were built
@@ -407,6 +408,28 @@ TileRadius tile_radius(const sdm_context* c) {
     return tr;
 }
 
+// Parts of an i-block's tiles (share_tiles) by the number of blocks of one replica: systems
+// of few blocks have short tile lists but leave most of the GPU idle with few waves; each
+// part costs about 3 us of a wave (loads, and the sums of the i forces) in large launches.
+// The number of replicas does not enter, so that a replica in a batch gives the bits of the
+// same replica alone.  Measured (us), 8 / 10 / 12 / 16 parts of 356 blocks: 20 steps of one
+// replica 1,953 / 1,874 / 1,900 / -, pair kernel of 22 replicas 379 / 392 / 402 / 426.  16 / 32
+// parts: 47 blocks 17.9 / 15.1 but 20 replicas of them 61 / 88, 174 blocks 22 / 31.
+int block_parts(const sdm_context* c) {
+    return c->NB <= 16 ? 64 : c->NB <= 32 ? 32 : c->NB < 256 ? 16 : c->NB < TILE_SLOPE_BLOCKS ? 10 : 4;
+}
+
+// Parts of the pair kernel: tuning.pair_split, or more where block_parts has more (one where
+// tuning asks for one, or for the full tile lists or the grouped form, for which pair_split
+// has no meaning).
+int pair_parts(const sdm_context* c) {
+    const int split = c->tune.pair_group == 0 && c->tune.pair_newton3 ? c->tune.pair_split : 1;
+    return split == 1 ? 1 : std::max(split, block_parts(c));
+}
+
+// whether the tile lists hold the tiles' shifts (pack_tile)
+int packed_tiles(const sdm_context* c) { return !lists_kept(c) && c->NB <= TILE_BLOCK; }
+
 // tile lists of the pairs and pair energies, candidate blocks of the displaced atoms.  With a skin, k_tiles keeps a replica's lists
 // while its atoms have moved less than half the skin since they were built.
 void enqueue_tiles(sdm_context* c) {
@@ -420,7 +443,8 @@ void enqueue_tiles(sdm_context* c) {
 #define SDM_TILES(NW)                                                                         \
     k_tiles<NW><<<dim3(c->NB + lc.groups, c->R), 64 * NW, 0, c->stream>>>(                    \
         c->N, c->Np, c->NB, c->maxj, c->arec, c->bb_lo, c->bb_hi, c->cbox, c->tiles,          \
-        c->tmask, c->ntiles, c->dmax, c->xb, tr, c->g, c->flags, lc)
+        c->tmask, c->dmax, c->xb, tr, c->g, c->flags, lc,                                     \
+        packed_tiles(c), pair_parts(c), block_parts(c), c->tbounds, c->ebounds)
     if (few_blocks(c)) SDM_TILES(8);
     else SDM_TILES(4);
 #undef SDM_TILES
@@ -432,30 +456,10 @@ void enqueue_sort(sdm_context* c, bool full) {
     enqueue_tiles(c);
 }
 
-// Waves per i-block by the number of blocks of one replica: systems of few blocks have short
-// tile lists but leave most of the GPU idle with few waves.  The number of replicas does not
-// enter, so that a replica in a batch gives the bits of the same replica alone.  Pair kernel
-// measured alone (us), waves 4 / 8 / 16 / 32 per block: 3 blocks 19 / 19 / 19 / 19 (a tile is
-// what it waits for; in 4 parts: 11), 47 blocks 41 / 29 / 23 / 19 and 20 replicas of them 63 /
-// 60 / 57 / 59, 174 blocks 48 / 36 / 30 / 31, 350 blocks 54 / 43 / 40 / 41 and 4 replicas of
-// them 94 / 85 / 86 / 108, 22 replicas of 356 blocks 405 / 406 / 445 / -.
-TileShare block_share(const sdm_context* c) {
-    return {c->NB < 256 ? 16 : c->NB < 512 ? 8 : 4, c->NB <= 16 ? 4 : c->NB <= 32 ? 2 : 1};
-}
-
-// Waves of the pair kernel: tuning.pair_split, or more where block_share has more (one
-// where tuning asks for one, or for the full tile lists or the grouped form, for which
-// pair_split has no meaning).
-TileShare pair_share(const sdm_context* c) {
-    const int split = c->tune.pair_group == 0 && c->tune.pair_newton3 ? c->tune.pair_split : 1;
-    const TileShare sh = block_share(c);
-    return split == 1 ? TileShare{1, 1} : TileShare{std::max(split, sh.split), sh.sub};
-}
-
 // Whether the pairs alone run for several generations of waves (4,096 are resident): 20 x
-// 2,976 atoms have 15,000 waves, 22 x 22,750 and 8 x 99,920 atoms 31,000 and 50,000.
+// 2,976 atoms have 15,000 parts, 22 x 22,750 and 8 x 99,920 atoms 78,000 and 50,000.
 bool many_waves(const sdm_context* c) {
-    return (long long)c->R * c->NB * pair_share(c).waves() >= 6 * 4096;
+    return (long long)c->R * c->NB * pair_parts(c) >= 6 * 4096;
 }
 
 // parts of the displaced-state forces on a candidate block (env_force)
@@ -468,21 +472,22 @@ template <int W, bool COUNT, bool GEO>
 void launch_forces(sdm_context* c, int parts) {
     // workgroups of W waves for n waves, a multiple of 8 (k_forces)
     auto groups = [](int part, int n) { return part ? ((n + W - 1) / W + 7) / 8 * 8 : 0; };
-    const TileShare sh = pair_share(c), esh = block_share(c);
+    const int pparts = pair_parts(c), ewaves = block_parts(c);  // energies: one wave per part
+    const int waves = many_waves(c) && c->NB < TILE_SLOPE_BLOCKS ? std::max(1, (3 * pparts + 3) / 7) : pparts;
     // A wave per group of displaced atoms where the launch is short, one for all groups of a
     // candidate block where it is long: fewer waves then wait for their atoms while others
     // could compute (22 x 22,750 atoms, 10 steps: 6.45 -> 6.33 ms, and 6.15 ms with the
     // Langevin kernel then reading one part of the forces on a candidate block, not eight)
-    const int pair_waves = c->R * c->NB * sh.waves();
     const int subs = DISP_WAVES / displaced_parts(c);
     const int disp = std::min(c->maxc, DISP_BLOCKS) * displaced_parts(c);
     const ForceGroups fg{groups(c->L > 0 ? parts & DISPLACED : 0, c->R * disp),
-                         groups(parts & ENERGY, c->R * c->NB * esh.waves()),
-                         groups(parts & PAIRS, pair_waves), disp, subs};
+                         groups(parts & ENERGY, (c->R * c->NB + 7) / 8 * 8 * ewaves),
+                         groups(parts & PAIRS, (c->R * c->NB + 7) / 8 * 8 * waves), disp, subs};
     const int bonded = groups(c->nbond + c->nang > 0 ? parts & BONDED : 0, c->R * c->nbw);
     k_forces<W, COUNT, GEO><<<fg.displaced + fg.energy + fg.pairs + bonded, 64 * W, 0, c->stream>>>(
-        fg, c->R, c->N, c->Np, c->NB, c->maxj, sh, c->arec, c->tiles, c->tmask, c->ntiles,
-        c->bb_lo, c->bb_hi, c->exs, c->exblocks, c->max_ex, c->F, c->flags, c->counters, esh,
+        fg, c->R, c->N, c->Np, c->NB, c->maxj, waves, pparts, packed_tiles(c), c->arec, c->tiles, c->tmask, c->tbounds,
+        c->bb_lo, c->bb_hi, c->exs, c->exblocks, c->max_ex, c->F, c->flags, c->counters, ewaves,
+        ewaves == pparts ? c->tbounds : c->ebounds,
         c->rec64, c->e64, c->nbw, c->bstart, c->bcode, c->astart, c->acode, c->bond_atoms,
         c->bond_r0, c->bond_k, c->ang_atoms, c->ang_t0, c->ang_k, c->x64, c->Fb, c->e_bond, c->L,
         c->LB, c->lig, c->lb_start, c->lb_count, c->cls, c->cdispl, c->q64, c->sig64, c->eps64,
@@ -557,9 +562,10 @@ void enqueue_eval(sdm_context* c, bool advance, bool components, bool full, bool
             components ? c->Fb_sep : c->F, c->slot_of, c->F, c->e_t1, c->e_t2, c->ntb, c->g,
             c->flags);
     if (apart) {
-        const TileShare sh = block_share(c);
-        k_energy64<<<(unsigned)(R * c->NB * sh.waves()), 64, 0, s1>>>(
-            R, N, Np, c->NB, c->maxj, sh, c->rec64, c->tiles, c->tmask, c->ntiles, c->bb_lo,
+        const int waves = block_parts(c);
+        k_energy64<<<(unsigned)((R * c->NB + 7) / 8 * 8 * waves), 64, 0, s1>>>(
+            R, N, Np, c->NB, c->maxj, waves, packed_tiles(c), c->rec64, c->tiles, c->tmask,
+            waves == pair_parts(c) ? c->tbounds : c->ebounds, c->bb_lo,
             c->bb_hi, c->exs, c->exblocks, c->max_ex, c->e64, c->g);
     }
     enqueue_forces(c, PAIRS | DISPLACED | BONDED | (energy && !apart ? ENERGY : 0));
@@ -568,7 +574,7 @@ void enqueue_eval(sdm_context* c, bool advance, bool components, bool full, bool
         (void)hipEventRecord(c->ev_join, s1);
         (void)hipStreamWaitEvent(s, c->ev_join, 0);
     }
-    k_scalar<<<R, 256, 0, s>>>(c->NB * block_share(c).waves(), c->nbw, c->LB, c->e64,
+    k_scalar<<<R, 256, 0, s>>>(c->NB * block_parts(c), c->nbw, c->LB, c->e64,
                                c->e_bond, c->u_part, c->state,
                                c->rec, c->flags, advance ? 1 : 0, energy ? 1 : 0,
                                c->hist_every, c->hist_cap, c->uhist, c->e_rest,
@@ -898,9 +904,10 @@ int sdm_create(const sdm_system_desc* sys, int32_t n_replicas, sdm_context** out
     A(tiles, (size_t)R * NB * c->maxj); A(tmask, (size_t)R * NB * c->maxj);
     A(xb, RNp); A(dmax, (size_t)R * DISP_STRIDE);
     A(cmap, (size_t)R * NB); A(lig_of, Np);
-    A(ntiles, (size_t)R * NB); A(F, 3 * RNp);
+    A(tbounds, (size_t)R * NB * TILE_BOUNDS);
+    A(ebounds, (size_t)R * NB * TILE_BOUNDS); A(F, 3 * RNp);
     A(e_bond, (size_t)R * c->nbw); A(u_part, (size_t)R * c->LB);
-    A(e64, (size_t)R * NB * block_share(c).waves()); A(rec64, RNp);
+    A(e64, (size_t)R * NB * block_parts(c)); A(rec64, RNp);
     A(cand, (size_t)R * c->maxc); A(ncand, R);
     A(dA, (size_t)R * c->maxc * c->LB * 64); A(dlig, (size_t)R * std::max(1, c->L));
     A(dB, (size_t)R * c->maxc * DISP_WAVES * 64); A(state, R); A(rec, R); A(flags, R);

@@ -486,6 +486,94 @@ __device__ __forceinline__ void lig_candidates(
     }
 }
 
+// How the tiles of an i-block are shared out: in parts of the steps (bits of the masks) of
+// its tile list, in list order, a tile counting TILE_UNITS steps more for its records, shift
+// and j forces.  A tile may be cut between two parts, but not within an eighth of a part (at
+// most 16 steps) of its ends.  The tile kernel finds the bounds, once for all waves of the
+// block: bounds[p] = (tile, steps of it that belong to the parts before p).
+// Parts are equal where one replica's waves are all resident at once (its longest wave is
+// what the launch waits for), and become smaller, to a tenth of the mean, from
+// TILE_SLOPE_BLOCKS blocks on, where waves start as others end: equal waves run in
+// generations, in step, and the last one leaves the GPU partly idle.
+// Tiles hold 1 to 64 steps: dealt out whole, every 8th tile to one of 8 waves, the longest
+// wave of 22,750 atoms took 50 us and the median one 25.  Measured, the pair kernel alone
+// (us): 186 atoms 9.9 -> 8.6, 2,976 atoms 28 -> 20 and 20 replicas of them 70 -> 60, 8 x
+// 99,920 atoms 855 -> 790 (877 with equal parts), 22 x 22,750 atoms 403 -> 392.
+constexpr int TILE_UNITS = 6, TILE_SLOPE_BLOCKS = 512;
+constexpr int MAX_TILE_PARTS = 64, TILE_BOUNDS = MAX_TILE_PARTS + 1;
+
+// inclusive sum over the lanes up to this one
+__device__ __forceinline__ int wave_scan(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);  // row_shr:1, 2, 4, 8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, true);  // row_bcast:15
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, true);  // row_bcast:31
+    return v;
+}
+
+// one wave: the bounds of `waves` (at most 64) parts of a list of nt tiles with masks tmk.
+// Lanes are tiles for the sums in front of them and then parts, which look for their tile.
+__device__ __forceinline__ void share_tiles(const unsigned long long* tmk, int nt, int lane,
+                                            int parts, bool slope,
+                                            int2* __restrict__ bounds) {
+    auto steps = [&](int t) { return t < nt ? __popcll(tmk[t]) : 0; };
+    auto units = [](int n) { return n ? n + TILE_UNITS : 0; };
+    int n = steps(lane), end = wave_scan(units(n));
+    int total = __builtin_amdgcn_readlane(end, 63);
+    for (int t = 64; t < nt; t += 64)
+        total += __builtin_amdgcn_readlane(wave_scan(units(steps(t + lane))), 63);
+    const int snap = min(16, total / parts / 8);
+    const double f = (double)lane / parts;
+    const int at = (int)(total * (slope ? f * (1.9 - 0.9 * f) : f));
+    int2 bound = make_int2(0, 0);
+    for (int t = 0, before = 0; t < nt; t += 64) {
+        if (t > 0) {
+            n = steps(t + lane);
+            end = before + wave_scan(units(n));
+        }
+        int q = 0;  // tiles of these that end at or before `at`
+#pragma unroll
+        for (int h = 32; h > 0; h >>= 1) q += __shfl(end, q + h - 1, 64) <= at ? h : 0;
+        const int qn = __shfl(n, q, 64), qe = __shfl(end, q, 64);
+        if (at >= before && q < 64 && at < qe) {
+            int a = max(at - (qe - qn), 0);
+            if (min(a, qn - a) <= snap) a = a <= qn - a ? 0 : qn;
+            bound = a < qn ? make_int2(t + q, a) : make_int2(t + q + 1, 0);
+        }
+        before = __builtin_amdgcn_readlane(end, 63);
+    }
+    if (lane < parts) bounds[lane] = bound;
+    if (lane == 0) bounds[parts] = make_int2(nt, 0);
+}
+
+// the periodic shift of a whole tile (boxes of the two blocks): (kx, ky, kz) box lengths;
+// returns whether it is exact for every pair within the list radius (Geom::oix)
+__device__ __forceinline__ bool tile_shift(float4 bli, float4 bhi, float4 blj, float4 bhj,
+                                           const Geom& g, float& kx, float& ky, float& kz) {
+    float dcx = 0.5f * (bli.x + bhi.x - blj.x - bhj.x);
+    float dcy = 0.5f * (bli.y + bhi.y - blj.y - bhj.y);
+    float dcz = 0.5f * (bli.z + bhi.z - blj.z - bhj.z);
+    kx = rintf(dcx * g.ibx);
+    ky = rintf(dcy * g.iby);
+    kz = rintf(dcz * g.ibz);
+    return fabsf(dcx - g.bx * kx) + 0.5f * (bhi.x - bli.x + bhj.x - blj.x) < g.oix &&
+           fabsf(dcy - g.by * ky) + 0.5f * (bhi.y - bli.y + bhj.y - blj.y) < g.oiy &&
+           fabsf(dcz - g.bz * kz) + 0.5f * (bhi.z - bli.z + bhj.z - blj.z) < g.oiz;
+}
+
+// An entry of a tile list: the j-block and, where the lists are built for this evaluation
+// (not kept from an earlier one, after which blocks may have moved to another image), the
+// shift of tile_shift: box lengths by dimension, or that each pair takes its own image.
+constexpr int TILE_BLOCK = (1 << 21) - 1, TILE_MI = 1 << 30;
+__device__ __forceinline__ int pack_tile(int jb, bool one, float kx, float ky, float kz) {
+    return jb | (one ? ((int)kx + 4) << 21 | ((int)ky + 4) << 24 | ((int)kz + 4) << 27 : TILE_MI);
+}
+__device__ __forceinline__ float tile_images(int entry, int d) {
+    return entry & TILE_MI ? 0.f : (float)(((entry >> (21 + 3 * d)) & 7) - 4);
+}
+
 // tile list of one i-block: every j-block it lists (lists_tile) whose box is within the
 // list radius r_l (r_c + skin + slack, TileRadius) of the i-block's box, ascending, each
 // with a 64-bit mask of the pairs of 8-slot clusters whose boxes lie within r_l: bit
@@ -497,7 +585,8 @@ __device__ __forceinline__ void lig_candidates(
 // Results do not depend on NW.
 // Kept lists (tr.reuse_d2 >= 0): the workgroup returns at once while no atom of the
 // replica has moved more than half the skin since the build (dmax); a build stores the
-// block's slot coordinates in xb.
+// block's slot coordinates in xb.  Last, the list is shared out among the waves of the pairs
+// (waves, bounds) and, if they are not as many, of the pair energies (ewaves, ebounds).
 // The first workgroup of a replica with displaced atoms finds the candidate blocks
 // (LigCand::groups is 1) instead: both need the boxes only, and a launch of its own would
 // take as long as this one.
@@ -516,10 +605,12 @@ __global__ __launch_bounds__(64 * NW) void k_tiles(int N, int Np, int NB, int ma
                                                const float4* __restrict__ cbox,
                                                int* __restrict__ tiles,
                                                unsigned long long* __restrict__ tmask,
-                                               int* __restrict__ ntiles,
                                                const float* __restrict__ dmax,
                                                float4* __restrict__ xb, TileRadius tr, Geom g,
-                                               int* __restrict__ flags, LigCand lc) {
+                                               int* __restrict__ flags, LigCand lc,
+                                               int packed, int waves, int ewaves,
+                                               int2* __restrict__ bounds,
+                                               int2* __restrict__ ebounds) {
     __shared__ int nkept[2][NW];
     const int r = blockIdx.y, ib = (int)blockIdx.x - lc.groups;
     if (ib < 0) {
@@ -594,26 +685,35 @@ __global__ __launch_bounds__(64 * NW) void k_tiles(int N, int Np, int NB, int ma
             count += n;
         }
         if (am != 0ull && pos < maxj) {
-            out[pos] = jl;
+            int entry = jl;
+            if (packed) {
+                const int lower = min(ib, jl), upper = max(ib, jl);
+                float kx, ky, kz;
+                const bool one = tile_shift(lo[lower], hi[lower], lo[upper], hi[upper], g, kx, ky, kz);
+                entry = pack_tile(jl, one, kx, ky, kz);
+            }
+            out[pos] = entry;
             mout[pos] = am;
         }
     }
-    if (threadIdx.x == 0) {
-        ntiles[(size_t)r * NB + ib] = min(count, maxj);
-        if (count > maxj) atomicOr(&flags[r], 4);
-    }
+    if (threadIdx.x == 0 && count > maxj) atomicOr(&flags[r], 4);
+    __syncthreads();  // the list is complete
+    const size_t rb = (size_t)r * NB + ib;
+    if (wave == 0) share_tiles(mout, min(count, maxj), lane, waves, NB >= TILE_SLOPE_BLOCKS, bounds + rb * TILE_BOUNDS);
+    if (wave == 1 && ewaves != waves)
+        share_tiles(mout, min(count, maxj), lane, ewaves, NB >= TILE_SLOPE_BLOCKS, ebounds + rb * TILE_BOUNDS);
 }
 
 // ---------------------------------------------------------------------------
 // The pair kernel: F0 over all pairs at x, each pair once (Newton-3 over the tile lists).
-// Each i-block has one wave or several (TileShare).  A wave holds the 64 i atoms as eight
+// Each i-block has one wave or several (TilePart).  A wave holds the 64 i atoms as eight
 // clusters of 8: lane 8 jl + il keeps atom il of every cluster in registers, and takes one
-// cluster of 8 j atoms at a time, lane 8 jl + il holding j atom jl.  One step is a pair of clusters, 64 pairs on 64 lanes,
-// taken for the bits of the tile's mask (uniform branches).  A step none of whose pairs
-// is within the cutoff ends after the distance test.
+// cluster of 8 j atoms at a time, lane 8 jl + il holding j atom jl.  One step is a pair of
+// clusters, 64 pairs on 64 lanes, taken for the bits of the tile's mask (uniform branches).
+// A step none of whose pairs is within the cutoff ends after the distance test.
 //   i forces: FP32 in the lane (24 registers), added up over the eight lanes that share an
-//     i atom and over to the accumulator after every PAIRS_PER_FLUSH pairs or more (pairs
-//     within the cutoff, so that the sums do not depend on what else the lists hold).
+//     i atom and over to the accumulator at the end of each part and after every
+//     PAIRS_PER_FLUSH pairs or more (pairs within the cutoff).
 //   j forces: FP32 over the cluster's steps, added up over the eight lanes that share a j
 //     atom, kept in registers over the tile and added to the slot-ordered int64 accumulator
 //     once per tile with coalesced atomics.
@@ -631,7 +731,8 @@ __global__ __launch_bounds__(64 * NW) void k_tiles(int N, int Np, int NB, int ma
 // pairs with 22% of them within the cutoff; pairs of clusters have 30% (40% after the
 // distance test's early end) and no sum over the wave for each j atom.  Measured alone, 22
 // x 22,750 atoms: 532 -> 405 us (297M -> 201M VALU instructions); 8 x 99,920 atoms:
-// 1,054 -> 850 us; one replica of 22,750 atoms: 55 -> 44 us.  Where the i atoms' charges and
+// 1,054 -> 850 us; one replica of 22,750 atoms: 55 -> 44 us (before the tiles were shared out
+// in parts, share_tiles).  Where the i atoms' charges and
 // LJ parameters came from LDS instead (122 registers), or the j forces of four clusters were
 // summed together (as many instructions in all, 30% more code), it was 4% and 14% slower.
 // ---------------------------------------------------------------------------
@@ -665,12 +766,18 @@ __device__ __forceinline__ double sum8(double y) {
     return y + dpp_d<0x141>(y);
 }
 
-// Maps workgroup ids so that consecutive (replica, block) work lands on one XCD:
-// workgroups are dispatched to the 8 XCDs round-robin, each XCD has its own L2.
-__device__ __forceinline__ int xcd_linear_id(int id, int n) {
-    int per = n >> 3, rem = n & 7, x = id & 7, q = id >> 3;
-    return x * per + min(x, rem) + q;
-}
+// Which part of which (replica, i-block) of n a wave takes: workgroup ids go to the 8 XCDs
+// round-robin and each XCD has its own L2, so an XCD gets an eighth of consecutive blocks,
+// first part 0 of all of them, then part 1, ..: parts become smaller (share_tiles), so the
+// launch ends with short waves.
+struct BlockWave {
+    int rb, part;
+    __device__ __forceinline__ BlockWave(int group, int waves_per_group, int wv, int n) {
+        const int per = (n + 7) >> 3, q = (group >> 3) * waves_per_group + wv;
+        part = q / per;
+        rb = (group & 7) * per + q - part * per;
+    }
+};
 
 // s_waitcnt vmcnt(0) alone (expcnt and lgkmcnt at their no-wait maxima).  The
 // scheduling barrier keeps the arithmetic before it from being moved past the wait.
@@ -713,18 +820,47 @@ __device__ __forceinline__ void scatter_clusters24(const float (&v)[24], int lan
 // many as the eight lanes that share it then add
 constexpr int PAIRS_PER_FLUSH = 4096;
 
-// How the tiles of an i-block are shared out: `split` waves take every split-th tile, and
-// with sub = 2, 4 or 8 each of them is sub waves that take the j clusters jc = part mod sub
-// of its tiles.
-struct TileShare {
-    int split, sub;
-    __host__ __device__ int waves() const { return split * sub; }
+// m without its r lowest bits
+__device__ __forceinline__ unsigned long long drop_bits(unsigned long long m, int r) {
+    int p = 0, left = r;
+#pragma unroll
+    for (int h = 32; h > 0; h >>= 1) {
+        const int c = __popcll((m >> p) & ((1ull << h) - 1ull));
+        p += left >= c ? h : 0;
+        left -= left >= c ? c : 0;
+    }
+    return left > 0 ? 0ull : m & (~0ull << p);
+}
+
+// One part of an i-block's tile list: tiles first..last (none: last < first), of the first
+// one without its `skip` lowest steps, of the last one only the `upto` lowest
+struct TilePart {
+    int first, last, skip, upto;
+    __device__ __forceinline__ TilePart(const int2* __restrict__ bounds, int rb, int part) {
+        const int2 a = bounds[(size_t)rb * TILE_BOUNDS + part],
+                   b = bounds[(size_t)rb * TILE_BOUNDS + part + 1];
+        first = a.x;
+        skip = a.y;
+        last = b.y > 0 ? b.x : b.x - 1;
+        upto = b.y > 0 ? b.y : 64;
+        if (first == last && upto <= skip) last = -1;
+    }
+    __device__ __forceinline__ bool empty() const { return last < first; }
+    // the part's bits of tile t's mask m
+    __device__ __forceinline__ unsigned long long take(int t, unsigned long long m) const {
+        unsigned long long k = m;
+        if (t == last && upto < 64) k &= ~drop_bits(m, upto);
+        if (t == first && skip > 0) k &= drop_bits(m, skip);
+        return k;
+    }
 };
-// the bits of a tile's mask that part `sp` of `sub` takes
-__device__ __forceinline__ unsigned long long sub_mask(int sub, int sp) {
-    const unsigned long long m = sub == 8 ? 0xffull : sub == 4 ? 0x000000ff000000ffull
-                                 : sub == 2 ? 0x00ff00ff00ff00ffull : ~0ull;
-    return m << (8 * sp);
+
+// The parts of a block that wave j of `waves` takes, from part_of(j) to part_of(j + 1): one
+// each, or (waves < parts) first more and then fewer.  Where the waves are many, an i-block's
+// atoms are then loaded for several parts at a time and the launch still ends with short waves
+// (22 x 22,750 atoms, parts taken one by one 429 us, so 402, with 12 parts).
+__device__ __forceinline__ int part_of(int j, int waves, int parts) {
+    return waves == parts ? j : parts * j * (2 * waves - j) / (waves * waves);
 }
 
 // j atoms of block jb that i atom `lane` must not be paired with in this tile: exclusion
@@ -747,21 +883,6 @@ __device__ __forceinline__ unsigned long long tile_exclusions(unsigned long long
     return vi ? em : ~0ull;
 }
 
-// the periodic shift of a whole tile (boxes of the two blocks): (kx, ky, kz) box lengths;
-// returns whether it is exact for every pair within the list radius (Geom::oix)
-__device__ __forceinline__ bool tile_shift(float4 bli, float4 bhi, float4 blj, float4 bhj,
-                                           const Geom& g, float& kx, float& ky, float& kz) {
-    float dcx = 0.5f * (bli.x + bhi.x - blj.x - bhj.x);
-    float dcy = 0.5f * (bli.y + bhi.y - blj.y - bhj.y);
-    float dcz = 0.5f * (bli.z + bhi.z - blj.z - bhj.z);
-    kx = rintf(dcx * g.ibx);
-    ky = rintf(dcy * g.iby);
-    kz = rintf(dcz * g.ibz);
-    return fabsf(dcx - g.bx * kx) + 0.5f * (bhi.x - bli.x + bhj.x - blj.x) < g.oix &&
-           fabsf(dcy - g.by * ky) + 0.5f * (bhi.y - bli.y + bhj.y - blj.y) < g.oiy &&
-           fabsf(dcz - g.bz * kz) + 0.5f * (bhi.z - bli.z + bhj.z - blj.z) < g.oiz;
-}
-
 //   LDS per wave: two 2 KB tile buffers, 512 B of exclusion masks, 768 B of i coordinates.
 //   vmcnt discipline: the only vector memory operations inside the tile loop are the
 //   next tile's copy (global -> LDS by DMA), the exclusion loads of the few tiles that have
@@ -769,22 +890,17 @@ __device__ __forceinline__ bool tile_shift(float4 bli, float4 bhi, float4 blj, f
 //   vmcnt but need not retire in issue order, so the copy is waited for with vmcnt(0) before
 //   the atomics, not with vmcnt(3) after them.
 //   GEO: the geometric LJ sigma rule, the records holding sigma itself (Geom::geo).
-//   w: the wave among those of all replicas and i-blocks; tile_s, em_s, xi_s: its LDS.
+//   rb: replica and i-block, of whose tile list the wave takes the parts from `part` up to
+//   part_end; tile_s, em_s, xi_s: its LDS.
 template <bool COUNT, bool GEO>
 __device__ __forceinline__ void pair_wave(
-    int w, int lane, float4* tile_s, unsigned long long* em_s, float* xi_s, int R, int N, int Np,
-    int NB, int maxj, TileShare share, const float4* __restrict__ arec,
+    int rb, int part, int part_end, int lane, float4* tile_s, unsigned long long* em_s, float* xi_s, int R, int N, int Np,
+    int NB, int maxj, int packed, const float4* __restrict__ arec,
     const int* __restrict__ tiles, const unsigned long long* __restrict__ tmask,
-    const int* __restrict__ ntiles, const float4* __restrict__ bb_lo,
+    const int2* __restrict__ bounds, const float4* __restrict__ bb_lo,
     const float4* __restrict__ bb_hi, const int* __restrict__ exs,
     const unsigned long long* __restrict__ exblocks, int max_ex, long long* __restrict__ F,
     int* __restrict__ flags, unsigned long long* __restrict__ pair_count, const Geom& g) {
-    const int split = share.split, waves = share.waves();
-    if (w >= R * NB * waves) return;
-    // waves per (replica, i-block): tiles part, part + split, .., clusters of smask
-    const int rb = w / waves;
-    const int part = (w - rb * waves) / share.sub;
-    const unsigned long long smask = sub_mask(share.sub, (w - rb * waves) % share.sub);
     int r = rb / NB;
     int ib = rb - r * NB;
     const float4* A = arec + (size_t)r * Np * 2;
@@ -792,8 +908,6 @@ __device__ __forceinline__ void pair_wave(
     const int islot = ib * 64 + lane;
     const bool vi = islot < N;
     const int il = lane & 7, jl = lane >> 3;
-    const int* tl = tiles + (size_t)rb * maxj;
-    const unsigned long long* tmk = tmask + (size_t)rb * maxj;
     const float4* lo = bb_lo + (size_t)r * NB;
     const float4* hi = bb_hi + (size_t)r * NB;
 
@@ -809,25 +923,28 @@ __device__ __forceinline__ void pair_wave(
                                          (__attribute__((address_space(3))) void*)(dst + 64), 16, 0, 0);
         __builtin_amdgcn_wave_barrier();
     };
-    // the wave's next 64 tiles, one per lane, so that no tile waits for its descriptor:
-    // j-block (TILE_MI set where every pair needs its own minimum image), mask, and the
-    // shift (hx, hy, hz) of the periodic image that the tile's pairs take, which is taken off
-    // the atoms of the lower block whichever of the two lists the tile, so that the rounding
-    // of a separation (and what is within the cutoff) does not depend on that
-    constexpr int TILE_MI = 1 << 30;
+    // 64 tiles of the list at a time, one per lane, so that no tile waits for its descriptor:
+    // j-block (TILE_MI set where every pair needs its own minimum image), this wave's bits
+    // of the mask, and the shift (hx, hy, hz) of the periodic image that the tile's pairs
+    // take, which is taken off the atoms of the lower block whichever of the two lists the
+    // tile, so that the rounding of a separation (and what is within the cutoff) does not
+    // depend on that
     int tj = 0;
     float hx = 0.f, hy = 0.f, hz = 0.f;
     unsigned long long tm = 0ull;
-    const int nt = ntiles[rb];
-    if (part >= nt) return;
-    auto load_tiles = [&](int t0) {
-        const int tq = t0 + lane * split;
-        if (tq < nt) {
-            tj = tl[tq];
-            tm = tmk[tq] & smask;
+    auto load_tiles = [&](int t) {
+        if (t < maxj) {
+            tj = tiles[(size_t)rb * maxj + t];
+            tm = tmask[(size_t)rb * maxj + t];
         }
     };
-    load_tiles(part);
+    load_tiles(lane);  // mostly the whole list, in flight with the bounds
+    if (part == part_end) return;  // more waves than the falling sizes need
+    TilePart at(bounds, rb, part);
+    while (at.empty()) {
+        if (++part == part_end) return;
+        at = TilePart(bounds, rb, part);
+    }
     float xi[8], yi[8], zi[8], qi[8], si[8], ei[8], fi[24];
 #pragma unroll
     for (int k = 0; k < 8; k++) {
@@ -850,22 +967,29 @@ __device__ __forceinline__ void pair_wave(
     int ox = 0, oy = 0, oz = 0;  // what xi, yi, zi are shifted by now (bits of the floats)
     const int* E = exs + (size_t)rb * max_ex * 64;
     const unsigned long long eset = exblocks[rb];
-    auto load_shifts = [&](int t0) {
-        if (t0 + lane * split < nt) {
-            // the i-block's box is read here each time (opaque index): kept in registers
-            // over the tile loop it made it spill
-            int ibo = ib;
-            asm volatile("" : "+s"(ibo));
-            const int lower = min(ibo, tj), upper = max(ibo, tj);
-            const bool one = tile_shift(lo[lower], hi[lower], lo[upper], hi[upper], g, hx, hy, hz);
-            hx = one ? g.bx * hx : 0.f;
-            hy = one ? g.by * hy : 0.f;
-            hz = one ? g.bz * hz : 0.f;
-            if (!one) tj |= TILE_MI;
+    auto load_shifts = [&]() {
+        if (packed) {
+            hx = g.bx * tile_images(tj, 0);
+            hy = g.by * tile_images(tj, 1);
+            hz = g.bz * tile_images(tj, 2);
+            return;
         }
+        // the i-block's box is read here each time (opaque index): kept in registers
+        // over the tile loop it made it spill
+        int ibo = ib;
+        asm volatile("" : "+s"(ibo));
+        tj = min(tj & TILE_BLOCK, NB - 1);  // past the list's end: anything
+        const int lower = min(ibo, tj), upper = max(ibo, tj);
+        const bool one = tile_shift(lo[lower], hi[lower], lo[upper], hi[upper], g, hx, hy, hz);
+        hx = one ? g.bx * hx : 0.f;
+        hy = one ? g.by * hy : 0.f;
+        hz = one ? g.bz * hz : 0.f;
+        if (!one) tj |= TILE_MI;
     };
-    stage(__builtin_amdgcn_readfirstlane(tj), 0);
-    load_shifts(part);
+    int t = at.first;
+    if (t >= 64) load_tiles((t & ~63) + lane);
+    stage(__builtin_amdgcn_readlane(tj, t & 63) & TILE_BLOCK, 0);
+    load_shifts();
     int bad = 0;
     // adds the i forces of the pairs so far to the accumulator: lane = i atom (atomic: other
     // waves and the side kernels add to the same accumulator)
@@ -886,12 +1010,12 @@ __device__ __forceinline__ void pair_wave(
     const int transpose = 4 * ((lane >> 3) + 8 * (lane & 7));
     const unsigned rec_lds = (unsigned)(size_t)&tile_s[2 * jl];
     wait_vmem();  // the first tile and the i atoms have arrived
-    for (int t = part, q = 0; t < nt; t += split, q++, buf ^= 1) {
-        const int ql = q & 63;
-        const int jt = __builtin_amdgcn_readlane(tj, ql), jb = jt & ~TILE_MI;
-        const unsigned long long m =
-            (unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(unsigned)tm, ql) |
-            (unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(unsigned)(tm >> 32), ql) << 32;
+    while (true) {
+        const int ql = t & 63;
+        const int jt = __builtin_amdgcn_readlane(tj, ql), jb = jt & TILE_BLOCK;
+        const unsigned long long m = at.take(
+            t, (unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(unsigned)tm, ql) |
+                   (unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(unsigned)(tm >> 32), ql) << 32);
         // the shift (bits of the floats) of the i atoms, or else of each j atom as it is read
         const bool up = jb > ib;
         const int sx = __builtin_amdgcn_readlane(__float_as_int(hx), ql),
@@ -910,12 +1034,25 @@ __device__ __forceinline__ void pair_wave(
                 zi[k] = xi_s[128 + 8 * k + il] - __int_as_float(oz);
             }
         }
-        if (t + split < nt) {
-            if (ql == 63) {
-                load_tiles(t + split);
-                load_shifts(t + split);
+        // the next tile, of this part or of the wave's next one (which may begin with the rest
+        // of this tile)
+        const bool part_ends = t == at.last;
+        int next = t + 1;
+        if (part_ends) {
+            next = -1;
+            while (++part < part_end) {
+                at = TilePart(bounds, rb, part);
+                if (at.empty()) continue;
+                next = at.first;
+                break;
             }
-            stage(__builtin_amdgcn_readlane(tj, (q + 1) & 63) & ~TILE_MI, buf ^ 1);
+        }
+        if (next > t) {
+            if (next >> 6 != t >> 6) {
+                load_tiles((next & ~63) + lane);
+                load_shifts();
+            }
+            stage(__builtin_amdgcn_readlane(tj, next & 63) & TILE_BLOCK, buf ^ 1);
         }
         if (!COUNT && npair >= PAIRS_PER_FLUSH) {
             flush_i();
@@ -933,7 +1070,7 @@ __device__ __forceinline__ void pair_wave(
         const int general = __builtin_amdgcn_readfirstlane(mi || ex ? 1 : 0);
         float fjx = 0.f, fjy = 0.f, fjz = 0.f;  // sum of cluster il, atom jl
         unsigned long long rest = m, done = 0ull;
-        if (rest) do {
+        do {
             const int jc8 = __builtin_ctzll(rest) & 56;  // 8 jc
             const unsigned ics = (unsigned)(m >> jc8) & 0xffu;
             rest &= ~(0xffull << jc8);
@@ -1030,12 +1167,20 @@ __device__ __forceinline__ void pair_wave(
             atomicAdd(&Fr[Np + s], fixed_from_float(fjy, &bad));
             atomicAdd(&Fr[2 * Np + s], fixed_from_float(fjz, &bad));
         }
+        // the i forces of each part are added up by themselves, so that results do not depend
+        // on how many parts a wave takes
+        if (!COUNT && part_ends) {
+            flush_i();
+            npair = 0;
+        }
+        if (next < 0) break;
+        buf ^= next > t ? 1 : 0;
+        t = next;
     }
     if (COUNT) {
         if (lane == 0) atomicAdd(&pair_count[r], (unsigned long long)npair);
         return;
     }
-    flush_i();
     if (__ballot(bad) != 0ull && lane == 0) atomicOr(&flags[r], 2);
 }
 
@@ -1048,7 +1193,7 @@ __device__ __forceinline__ void pair_wave(
 // Newton-3 order over the half tile lists, so U0 is exact to FP64 rounding.
 //
 // Waves per (replica, i-block) and their shares of the tiles as in the pair kernel
-// (TileShare), pair of clusters by pair of clusters as the pair kernel does (lane 8 jl + il:
+// (TilePart), pair of clusters by pair of clusters as the pair kernel does (lane 8 jl + il:
 // j atom jl, i atom il), all in FP64: vector FP64 issues at the rate of unpacked FP32.  The i records
 // stay in LDS (eight clusters of FP64 records would take 96 registers), the next tile's j
 // records are loaded into registers while the current tile is evaluated.
@@ -1060,17 +1205,13 @@ __device__ __forceinline__ void lds_order() { asm volatile("" ::: "memory"); }
 
 //   irec, jrec, em_s: the wave's LDS
 __device__ __forceinline__ void energy64_wave(
-    int w, int lane, Rec64* irec, Rec64* jrec, unsigned long long* em_s, int R, int N, int Np,
-    int NB, int maxj, TileShare share, const Rec64* __restrict__ rec,
+    int rb, int part, int lane, Rec64* irec, Rec64* jrec, unsigned long long* em_s, int R, int N, int Np,
+    int NB, int maxj, int waves, int packed, const Rec64* __restrict__ rec,
     const int* __restrict__ tiles, const unsigned long long* __restrict__ tmask,
-    const int* __restrict__ ntiles, const float4* __restrict__ bb_lo,
+    const int2* __restrict__ bounds, const float4* __restrict__ bb_lo,
     const float4* __restrict__ bb_hi, const int* __restrict__ exs,
     const unsigned long long* __restrict__ exblocks, int max_ex, double* __restrict__ e_out,
     const Geom& g) {
-    const int split = share.split, waves = share.waves();
-    if (w >= R * NB * waves) return;
-    const int rb = w / waves, part = (w - rb * waves) / share.sub;
-    const unsigned long long smask = sub_mask(share.sub, (w - rb * waves) % share.sub);
     const int r = rb / NB, ib = rb - r * NB;
     const Rec64* RC = rec + (size_t)r * Np;
     const int islot = ib * 64 + lane;
@@ -1082,7 +1223,6 @@ __device__ __forceinline__ void energy64_wave(
     const float4 bli = bb_lo[(size_t)r * NB + ib], bhi = bb_hi[(size_t)r * NB + ib];
     const int* tl = tiles + ((size_t)r * NB + ib) * maxj;
     const unsigned long long* tmk = tmask + ((size_t)r * NB + ib) * maxj;
-    const int nt = ntiles[(size_t)r * NB + ib];
     double e = 0.0;
     // the j records of the wave's next tile (a record is 3 x 16 bytes)
     double2 na = make_double2(0.0, 0.0), nb = na, nc = na;
@@ -1095,19 +1235,29 @@ __device__ __forceinline__ void energy64_wave(
             nc = src[2];
         }
     };
-    if (part < nt) prefetch(tl[part]);
-    for (int t = part; t < nt; t += split) {
-        const int jb = tl[t];
-        const unsigned long long m = tmk[t] & smask;
+    const TilePart steps(bounds, rb, part);
+    if (steps.first <= steps.last) prefetch(tl[steps.first] & TILE_BLOCK);
+    for (int t = steps.first; t <= steps.last; t++) {
+        const int entry = tl[t], jb = entry & TILE_BLOCK;
+        const unsigned long long m = steps.take(t, tmk[t]);
         lds_order();  // the previous tile's records are no longer read
         jrec[lane] = Rec64{na.x, na.y, nb.x, nb.y, nc.x, nc.y};
-        if (t + split < nt) prefetch(tl[t + split]);
+        if (t < steps.last) prefetch(tl[t + 1] & TILE_BLOCK);
         const unsigned long long em = tile_exclusions(eset, max_ex, E, lane, vi, ib, jb, N);
         const bool ex = __ballot(em != 0ull) != 0ull;
         if (ex) em_s[lane] = em;
         float kx, ky, kz;
-        const bool one_image = tile_shift(bli, bhi, bb_lo[(size_t)r * NB + jb],
-                                          bb_hi[(size_t)r * NB + jb], g, kx, ky, kz);
+        bool one_image;
+        if (packed) {  // of the lower block's atoms
+            const float up = jb > ib ? 1.f : -1.f;
+            kx = up * tile_images(entry, 0);
+            ky = up * tile_images(entry, 1);
+            kz = up * tile_images(entry, 2);
+            one_image = !(entry & TILE_MI);
+        } else {
+            one_image = tile_shift(bli, bhi, bb_lo[(size_t)r * NB + jb], bb_hi[(size_t)r * NB + jb],
+                                   g, kx, ky, kz);
+        }
         const double sx = g.Lx * (double)kx, sy = g.Ly * (double)ky, sz = g.Lz * (double)kz;
         lds_order();  // this tile's records are stored
         auto clusters = [&](auto mic, auto exc) {
@@ -1165,7 +1315,7 @@ __device__ __forceinline__ void energy64_wave(
         }
     }
     e = wave_sum(e);
-    if (lane == 0) e_out[w] = e;
+    if (lane == 0) e_out[rb * waves + part] = e;
 }
 
 // ---------------------------------------------------------------------------
@@ -1954,13 +2104,13 @@ struct ForceGroups {
 
 template <int WPW, bool COUNT, bool GEO>
 __global__ __launch_bounds__(64 * WPW) __attribute__((amdgpu_waves_per_eu(4))) void k_forces(
-    ForceGroups fg, int R, int N, int Np, int NB, int maxj, TileShare share,
+    ForceGroups fg, int R, int N, int Np, int NB, int maxj, int waves, int parts, int packed,
     const float4* __restrict__ arec, const int* __restrict__ tiles,
-    const unsigned long long* __restrict__ tmask, const int* __restrict__ ntiles,
+    const unsigned long long* __restrict__ tmask, const int2* __restrict__ bounds,
     const float4* __restrict__ bb_lo, const float4* __restrict__ bb_hi,
     const int* __restrict__ exs, const unsigned long long* __restrict__ exblocks, int max_ex,
     long long* __restrict__ F, int* __restrict__ flags,
-    unsigned long long* __restrict__ pair_count, TileShare eshare,
+    unsigned long long* __restrict__ pair_count, int ewaves, const int2* __restrict__ ebounds,
     const Rec64* __restrict__ rec, double* __restrict__ e64, int nbw,
     const int* __restrict__ bstart, const int* __restrict__ bcode,
     const int* __restrict__ astart, const int* __restrict__ acode,
@@ -1997,16 +2147,21 @@ __global__ __launch_bounds__(64 * WPW) __attribute__((amdgpu_waves_per_eu(4))) v
     b -= fg.displaced;
     if (!COUNT && b < fg.energy) {
         Rec64* irec = (Rec64*)wave_s[wv];
-        energy64_wave(xcd_linear_id(b, fg.energy) * WPW + wv, lane, irec, irec + 64, em_s[wv], R,
-                      N, Np, NB, maxj, eshare, rec, tiles, tmask, ntiles, bb_lo, bb_hi, exs,
-                      exblocks, max_ex, e64, g);
+        const BlockWave bw(b, WPW, wv, R * NB);
+        if (bw.part < ewaves && bw.rb < R * NB)
+            energy64_wave(bw.rb, bw.part, lane, irec, irec + 64, em_s[wv], R, N, Np, NB, maxj,
+                          ewaves, packed, rec, tiles, tmask, ebounds, bb_lo, bb_hi, exs, exblocks,
+                          max_ex, e64, g);
         return;
     }
     b -= fg.energy;
     if (b < fg.pairs) {
-        pair_wave<COUNT, GEO>(xcd_linear_id(b, fg.pairs) * WPW + wv, lane, wave_s[wv], em_s[wv],
-                              xi_s[wv], R, N, Np, NB, maxj, share, arec, tiles, tmask, ntiles,
-                              bb_lo, bb_hi, exs, exblocks, max_ex, F, flags, pair_count, g);
+        const BlockWave bw(b, WPW, wv, R * NB);
+        if (bw.part < waves && bw.rb < R * NB)
+            pair_wave<COUNT, GEO>(bw.rb, part_of(bw.part, waves, parts),
+                                  part_of(bw.part + 1, waves, parts), lane, wave_s[wv],
+                                  em_s[wv], xi_s[wv], R, N, Np, NB, maxj, packed, arec, tiles, tmask, bounds, bb_lo,
+                                  bb_hi, exs, exblocks, max_ex, F, flags, pair_count, g);
         return;
     }
     b -= fg.pairs;
@@ -2018,17 +2173,18 @@ __global__ __launch_bounds__(64 * WPW) __attribute__((amdgpu_waves_per_eu(4))) v
 // The FP64 pair energies alone, beside the forces on another stream, for long launches: in
 // k_forces they have its 4 waves per SIMD, here 6, and other waves to run with.
 __global__ __launch_bounds__(64) void k_energy64(
-    int R, int N, int Np, int NB, int maxj, TileShare share, const Rec64* __restrict__ rec,
+    int R, int N, int Np, int NB, int maxj, int waves, int packed, const Rec64* __restrict__ rec,
     const int* __restrict__ tiles, const unsigned long long* __restrict__ tmask,
-    const int* __restrict__ ntiles, const float4* __restrict__ bb_lo,
+    const int2* __restrict__ bounds, const float4* __restrict__ bb_lo,
     const float4* __restrict__ bb_hi, const int* __restrict__ exs,
     const unsigned long long* __restrict__ exblocks, int max_ex, double* __restrict__ e_out,
     Geom g) {
     __shared__ Rec64 irec[64], jrec[64];
     __shared__ unsigned long long em_s[64];
-    energy64_wave(xcd_linear_id(blockIdx.x, gridDim.x), threadIdx.x, irec, jrec, em_s, R, N, Np,
-                  NB, maxj, share, rec, tiles, tmask, ntiles, bb_lo, bb_hi, exs, exblocks, max_ex,
-                  e_out, g);
+    const BlockWave bw(blockIdx.x, 1, 0, R * NB);
+    if (bw.part < waves && bw.rb < R * NB)
+        energy64_wave(bw.rb, bw.part, threadIdx.x, irec, jrec, em_s, R, N, Np, NB, maxj, waves,
+                      packed, rec, tiles, tmask, bounds, bb_lo, bb_hi, exs, exblocks, max_ex, e_out, g);
 }
 
 // per displaced atom: the block partials of displaced_wave in order, plus pairs with displaced

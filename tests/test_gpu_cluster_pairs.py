@@ -56,3 +56,25 @@ def test_image_modes(hip_device, cutoff, periodic, geometric, cells):
     print(f"case n={s.n} cutoff={cutoff} periodic={periodic} geo={geometric} cells={cells}", flush=True)
     # a coarse sort grid gives blocks as wide as the box
     _check(s, dict(cell_cells_per_dim=cells, pair_split=2))
+
+
+@pytest.mark.parametrize("skin", [0.0, 0.02])
+@pytest.mark.parametrize("waters,box", [(60, 1.9), (700, 3.3), (11000, 7.0)])
+def test_parts_take_every_pair_once(hip_device, waters, box, skin):
+    """However the tiles of a block are shared out, also in parts of falling size (from 512
+    blocks on): the same pairs, the same energy to FP64 rounding, and forces that differ by
+    FP32 sums in another order (some hundred terms, 1e-6 of the RMS force)."""
+    s = systems.make_small(waters, 6, box=box, cutoff=0.8, frame=2)
+    ref = None
+    for split in (1, 2, 16, 32):
+        print(f"case n={s.n} split={split} skin={skin}", flush=True)
+        ctx = _native.NativeContext(s, 1)
+        ctx.set_tuning(pair_split=split, list_skin=skin)
+        ctx.set_params(0, systems.params_config1())
+        ctx.set_positions(0, s.positions)
+        ctx.compute_components()
+        got = (int(ctx.count_pairs()[0][0]), ctx.energies()[0]["U0"], ctx.forces(0, _native.FORCE_STATE1))
+        ref = ref or got
+        assert got[0] == ref[0] and abs(got[1] - ref[1]) <= 1e-12 * max(abs(ref[1]), 1e3 * s.n)
+        rms = np.sqrt(np.mean(ref[2] ** 2))
+        assert np.sqrt(np.mean((got[2] - ref[2]) ** 2)) <= 1e-6 * rms

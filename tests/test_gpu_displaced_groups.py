@@ -21,9 +21,9 @@ def _run(s, replicas):
         ctx.set_positions(r, s.positions)
     ctx.compute_components()
     e = ctx.energies()
-    dF = [ctx.forces(r, _native.FORCE_STATE2) - ctx.forces(r, _native.FORCE_STATE1)
-          for r in (0, replicas - 1)]
-    return ctx, e, dF
+    F = [ctx.forces(r, _native.FORCE_STATE1) for r in (0, replicas - 1)]
+    dF = [ctx.forces(r, _native.FORCE_STATE2) - F[k] for k, r in enumerate((0, replicas - 1))]
+    return ctx, e, dF, F
 
 
 @pytest.mark.parametrize("displaced", [1, 7, 8, 9, 63, 64, 65, 131])
@@ -35,16 +35,17 @@ def test_groups_and_batches(hip_device, displaced):
     s.displacement[:displaced] = d
     print(f"case n={s.n} displaced={displaced}", flush=True)
     _, u, _, dF, _, nd = O.sdm_direct(O.Topology(s), s.positions)
-    ctx, e, got = _run(s, 1)
+    ctx, e, got, F = _run(s, 1)
     assert e[0]["flags"] == 0
     assert abs(e[0]["u"] - u) <= 1e-10 * max(1e3, 1e3 * abs(u))
     # forces are read back as differences of two FP64 sums with fixed-point parts (2^-32)
     assert np.max(np.abs(got[0] - dF)) <= 1e-9 * (1.0 + np.max(np.abs(dF))) + 4 * 2.0 ** -32
     assert int(ctx.count_pairs()[1][0]) == nd
     nb = (s.n + 63) // 64
-    _, eb, gb = _run(s, 25000 // (64 * nb) + 1)
+    _, eb, gb, Fb = _run(s, 25000 // (64 * nb) + 1)
     for k in ("u", "U0", "Ub", "pot_energy"):
         assert eb[0][k] == eb[-1][k]
+    assert np.array_equal(Fb[0], F[0]) and np.array_equal(Fb[1], F[0])
     assert eb[0]["u"] == e[0]["u"] and np.array_equal(gb[0], got[0]) and np.array_equal(gb[1], got[0])
 
 
@@ -53,7 +54,7 @@ def test_more_candidate_blocks_than_waves(hip_device):
     s.cutoff, s.periodic = 15.0, False  # every block is a candidate
     print(f"case n={s.n}", flush=True)
     _, u, _, dF, _, nd = O.sdm_direct(O.Topology(s), s.positions)
-    ctx, e, got = _run(s, 1)
+    ctx, e, got, _ = _run(s, 1)
     assert e[0]["flags"] == 0
     assert abs(e[0]["u"] - u) <= 1e-10 * max(1e3, 1e3 * abs(u))
     assert np.max(np.abs(got[0] - dF)) <= 1e-9 * (1.0 + np.max(np.abs(dF))) + 4 * 2.0 ** -32
