@@ -446,7 +446,7 @@ void enqueue_tiles(sdm_context* c) {
         c->tmask, c->dmax, c->xb, tr, c->g, c->flags, lc,                                     \
         packed_tiles(c), pair_parts(c), block_parts(c), c->tbounds, c->ebounds)
     if (few_blocks(c)) SDM_TILES(8);
-    else SDM_TILES(4);
+    else SDM_TILES(2);
 #undef SDM_TILES
 }
 

@@ -513,12 +513,17 @@ __device__ __forceinline__ int wave_scan(int v) {
     return v;
 }
 
-// one wave: the bounds of `waves` (at most 64) parts of a list of nt tiles with masks tmk.
-// Lanes are tiles for the sums in front of them and then parts, which look for their tile.
-__device__ __forceinline__ void share_tiles(const unsigned long long* tmk, int nt, int lane,
+// one wave: the bounds of `parts` (at most 64) parts of a list of nt tiles with masks tmk,
+// whose numbers of steps are in nstep for the first SHARE_LDS ones.  Lanes are tiles for the
+// sums in front of them and then parts, which look for their tile.
+constexpr int SHARE_LDS = 256;
+__device__ __forceinline__ void share_tiles(const unsigned char* nstep,
+                                            const unsigned long long* tmk, int nt, int lane,
                                             int parts, bool slope,
                                             int2* __restrict__ bounds) {
-    auto steps = [&](int t) { return t < nt ? __popcll(tmk[t]) : 0; };
+    auto steps = [&](int t) {
+        return t >= nt ? 0 : t < SHARE_LDS ? (int)nstep[t] : __popcll(tmk[t]);
+    };
     auto units = [](int n) { return n ? n + TILE_UNITS : 0; };
     int n = steps(lane), end = wave_scan(units(n));
     int total = __builtin_amdgcn_readlane(end, 63);
@@ -598,7 +603,7 @@ struct LigCand {
     int *cand, *ncand, *cmap;
 };
 template <int NW>  // waves per i-block workgroup
-__global__ __launch_bounds__(64 * NW) void k_tiles(int N, int Np, int NB, int maxj,
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(8))) void k_tiles(int N, int Np, int NB, int maxj,
                                                const float4* __restrict__ arec,
                                                const float4* __restrict__ bb_lo,
                                                const float4* __restrict__ bb_hi,
@@ -612,6 +617,7 @@ __global__ __launch_bounds__(64 * NW) void k_tiles(int N, int Np, int NB, int ma
                                                int2* __restrict__ bounds,
                                                int2* __restrict__ ebounds) {
     __shared__ int nkept[2][NW];
+    __shared__ unsigned char nstep[SHARE_LDS];
     const int r = blockIdx.y, ib = (int)blockIdx.x - lc.groups;
     if (ib < 0) {
         lig_candidates<NW>(r, Np, NB, lc.L, lc.ncls, lc.lig, lc.cls, lc.cdispl, lc.x64, bb_lo,
@@ -694,14 +700,15 @@ __global__ __launch_bounds__(64 * NW) void k_tiles(int N, int Np, int NB, int ma
             }
             out[pos] = entry;
             mout[pos] = am;
+            if (pos < SHARE_LDS) nstep[pos] = (unsigned char)__popcll(am);
         }
     }
     if (threadIdx.x == 0 && count > maxj) atomicOr(&flags[r], 4);
     __syncthreads();  // the list is complete
     const size_t rb = (size_t)r * NB + ib;
-    if (wave == 0) share_tiles(mout, min(count, maxj), lane, waves, NB >= TILE_SLOPE_BLOCKS, bounds + rb * TILE_BOUNDS);
-    if (wave == 1 && ewaves != waves)
-        share_tiles(mout, min(count, maxj), lane, ewaves, NB >= TILE_SLOPE_BLOCKS, ebounds + rb * TILE_BOUNDS);
+    if (wave == 0) share_tiles(nstep, mout, min(count, maxj), lane, waves, NB >= TILE_SLOPE_BLOCKS, bounds + rb * TILE_BOUNDS);
+    if (wave == NW - 1 && ewaves != waves)
+        share_tiles(nstep, mout, min(count, maxj), lane, ewaves, NB >= TILE_SLOPE_BLOCKS, ebounds + rb * TILE_BOUNDS);
 }
 
 // ---------------------------------------------------------------------------
