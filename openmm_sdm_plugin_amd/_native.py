@@ -7,6 +7,7 @@ from __future__ import annotations
 
 import ctypes as C
 import os
+import struct
 
 import numpy as np
 
@@ -68,6 +69,11 @@ class sdm_energies(C.Structure):
         ("work", C.c_double), ("time", C.c_double), ("step", C.c_int64), ("flags", C.c_int32),
         ("pad", C.c_int32),
     ]
+
+
+_ENERGY_NAMES = [n for n, _ in sdm_energies._fields_]
+_ENERGY_STRUCT = struct.Struct("@17dqii")
+assert _ENERGY_STRUCT.size == C.sizeof(sdm_energies)
 
 
 class sdm_tuning(C.Structure):
@@ -434,7 +440,7 @@ class NativeContext:
     def energies(self):
         out = (sdm_energies * self.R)()
         check(self._lib.sdm_get_energies(self.h, out))
-        return [dict((n, getattr(e, n)) for n, _ in sdm_energies._fields_) for e in out]
+        return [dict(zip(_ENERGY_NAMES, e)) for e in _ENERGY_STRUCT.iter_unpack(out)]
 
     def clear_flags(self):
         check(self._lib.sdm_clear_flags(self.h))

@@ -68,9 +68,13 @@ class AdjointModel:
         self.eps = np.asarray(system.epsilon, dtype=np.float64).copy()
 
     def upload(self, q_sel, sig_sel, eps_sel):
-        self.q[self.sel] = q_sel.detach().double().cpu().numpy()
-        self.sig[self.sel] = sig_sel.detach().double().cpu().numpy()
-        self.eps[self.sel] = eps_sel.detach().double().cpu().numpy()
+        sel = [t.detach().double() for t in (q_sel, sig_sel, eps_sel)]
+        if all(t.is_cuda and t.dim() == 1 and t.shape == sel[0].shape and t.device == sel[0].device
+               for t in sel):
+            sel = torch.stack(sel).cpu().numpy()  # one copy and one wait for the three
+        else:
+            sel = [t.cpu().numpy() for t in sel]
+        self.q[self.sel], self.sig[self.sel], self.eps[self.sel] = sel
         self.native.set_nonbonded_params(self.q, self.sig, self.eps)
 
     def mean_W_and_u(self, q_sel, sig_sel, eps_sel, alpha, u0, w0, frames):

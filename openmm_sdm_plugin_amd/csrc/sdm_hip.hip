@@ -6,6 +6,7 @@
 #include "sdm_hip.h"
 
 #include <algorithm>
+#include <cfloat>
 #include <cmath>
 #include <cstddef>
 #include <cstring>
@@ -182,6 +183,12 @@ struct sdm_context {
     hipGraphExec_t gexec[2][2] = {};
     bool components_valid = false;
     std::vector<void*> allocs;
+    // pinned host memory (IO_SLOTS slots for data on its way to the device, in turn, and one
+    // for data on its way back), of io_cap bytes each; 0: none (very large systems)
+    char* io = nullptr;
+    size_t io_cap = 0;
+    int io_next = 0;
+    hipEvent_t io_done[2] = {nullptr, nullptr};  // the slot has been read
 };
 
 namespace {
@@ -193,11 +200,11 @@ int dalloc(sdm_context* c, T** p, size_t n) {
     hipError_t e = hipMalloc(&q, n * sizeof(T));
     if (e != hipSuccess)
         return fail(SDM_ERR_HIP, std::string("hipMalloc: ") + hipGetErrorString(e));
-    // zero-filled on the context's own stream and waited for: the legacy null stream is
-    // not ordered with the context's non-blocking streams, and a reused allocation holds
-    // stale values (counters that must start at zero would give out-of-range offsets)
+    // zero-filled on the context's own stream, on which (or after which) everything that uses
+    // it runs: the legacy null stream is not ordered with the context's non-blocking streams,
+    // and a reused allocation holds stale values (counters that must start at zero would
+    // give out-of-range offsets)
     e = hipMemsetAsync(q, 0, n * sizeof(T), c->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     if (e != hipSuccess)
         return fail(SDM_ERR_HIP, std::string("hipMemsetAsync: ") + hipGetErrorString(e));
     c->allocs.push_back(q);
@@ -205,19 +212,60 @@ int dalloc(sdm_context* c, T** p, size_t n) {
     return SDM_OK;
 }
 
+// Host data goes through pinned memory that kernels read or write, in stream order
+// (k_words).
+constexpr int IO_SLOTS = 2;
+constexpr size_t IO_MAX = (size_t)64 << 20;  // bytes of pinned memory per slot at most
+
+// the next slot for data on its way to the device, free again
+int io_slot(sdm_context* c, int* slot) {
+    *slot = c->io_next;
+    c->io_next = (c->io_next + 1) % IO_SLOTS;
+    HIPCHK(hipEventSynchronize(c->io_done[*slot]));
+    return SDM_OK;
+}
+char* io_ptr(sdm_context* c, int slot) { return c->io + (size_t)slot * c->io_cap; }
+
 template <class T>
 int upload(sdm_context* c, T* dst, const T* src, size_t n) {
+    static_assert(sizeof(T) % 4 == 0, "words");
     if (n == 0) return SDM_OK;
-    HIPCHK(hipMemcpyAsync(dst, src, n * sizeof(T), hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
+    if (n * sizeof(T) > c->io_cap) {
+        HIPCHK(hipMemcpyAsync(dst, src, n * sizeof(T), hipMemcpyHostToDevice, c->stream));
+        HIPCHK(hipStreamSynchronize(c->stream));
+        return SDM_OK;
+    }
+    int slot;
+    CHK(io_slot(c, &slot));
+    std::memcpy(io_ptr(c, slot), src, n * sizeof(T));
+    const size_t words = n * (sizeof(T) / 4);
+    k_words<<<(unsigned)((words + 255) / 256), 256, 0, c->stream>>>(
+        (const unsigned*)io_ptr(c, slot), words, nullptr, 0, (unsigned*)dst);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipEventRecord(c->io_done[slot], c->stream));
     return SDM_OK;
 }
 
-template <class T>
-int download(sdm_context* c, T* dst, const T* src, size_t n) {
-    if (n == 0) return SDM_OK;
-    HIPCHK(hipMemcpyAsync(dst, src, n * sizeof(T), hipMemcpyDeviceToHost, c->stream));
+// a (and b) to the host, waited for
+template <class T, class U = int>
+int download(sdm_context* c, T* dst, const T* src, size_t n, U* dst2 = nullptr,
+             const U* src2 = nullptr, size_t n2 = 0) {
+    static_assert(sizeof(T) % 4 == 0 && sizeof(U) % 4 == 0, "words");
+    const size_t na = n * (sizeof(T) / 4), nb = n2 * (sizeof(U) / 4);
+    if (na + nb == 0) return SDM_OK;
+    if (4 * (na + nb) > c->io_cap) {
+        if (na) HIPCHK(hipMemcpyAsync(dst, src, 4 * na, hipMemcpyDeviceToHost, c->stream));
+        if (nb) HIPCHK(hipMemcpyAsync(dst2, src2, 4 * nb, hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(hipStreamSynchronize(c->stream));
+        return SDM_OK;
+    }
+    char* out = io_ptr(c, IO_SLOTS);
+    k_words<<<(unsigned)((na + nb + 255) / 256), 256, 0, c->stream>>>(
+        (const unsigned*)src, na, (const unsigned*)src2, nb, (unsigned*)out);
+    HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(c->stream));
+    if (na) std::memcpy(dst, out, 4 * na);
+    if (nb) std::memcpy(dst2, out + 4 * na, 4 * nb);
     return SDM_OK;
 }
 
@@ -689,30 +737,38 @@ int tile_capacity(const sdm_system_desc* sys, int NB) {
 }
 
 int upload_nb_params(sdm_context* c, const double* q, const double* sig, const double* eps) {
-    int N = c->N, Np = c->Np;
-    std::vector<float> qs(Np, 0.f), sh(Np, 0.f), se(Np, 0.f);
-    std::vector<double> q64(Np, 0.0), s64(Np, 0.0), e64(Np, 0.0);
-    std::vector<double4> p64(Np, double4{0.0, 0.0, 0.0, 0.0});
-    double sk = std::sqrt(SDM_ONE_4PI_EPS0);
-    for (int i = 0; i < N; i++) {
-        if (!(sig[i] >= 0) || !(eps[i] >= 0) || !std::isfinite(q[i]))
-            return fail(SDM_ERR_INVALID, "nonbonded parameters must be finite, sigma/epsilon >= 0");
-        qs[i] = (float)(q[i] * sk);
-        const double sh64 = c->g.geo ? sig[i] : 0.5 * sig[i];  // the entry each rule combines
-        sh[i] = (float)sh64;
-        se[i] = (float)(2.0 * std::sqrt(eps[i]));
-        q64[i] = q[i] * sk;
-        s64[i] = sig[i];
-        e64[i] = eps[i];
-        p64[i] = double4{q[i] * sk, sh64, 2.0 * std::sqrt(eps[i]), 0.0};
+    const size_t N = (size_t)c->N;
+    bool bad = false;
+    for (size_t i = 0; i < N; i++)
+        bad |= !(sig[i] >= 0) | !(eps[i] >= 0) | !(std::fabs(q[i]) <= DBL_MAX);
+    if (bad)
+        return fail(SDM_ERR_INVALID, "nonbonded parameters must be finite, sigma/epsilon >= 0");
+    const double* src = nullptr;
+    int slot = -1;
+    double* tmp = nullptr;
+    if (3 * N * sizeof(double) <= c->io_cap) {
+        CHK(io_slot(c, &slot));
+        double* io = (double*)io_ptr(c, slot);
+        std::memcpy(io, q, N * sizeof(double));
+        std::memcpy(io + N, sig, N * sizeof(double));
+        std::memcpy(io + 2 * N, eps, N * sizeof(double));
+        src = io;
+    } else {
+        CHK(dalloc(c, &tmp, 3 * N));
+        int rc = upload(c, tmp, q, N);
+        if (rc == SDM_OK) rc = upload(c, tmp + N, sig, N);
+        if (rc == SDM_OK) rc = upload(c, tmp + 2 * N, eps, N);
+        if (rc != SDM_OK) {
+            dfree(c, tmp);
+            return rc;
+        }
+        src = tmp;
     }
-    CHK(upload(c, c->qs, qs.data(), Np));
-    CHK(upload(c, c->sh, sh.data(), Np));
-    CHK(upload(c, c->se, se.data(), Np));
-    CHK(upload(c, c->q64, q64.data(), Np));
-    CHK(upload(c, c->sig64, s64.data(), Np));
-    CHK(upload(c, c->eps64, e64.data(), Np));
-    CHK(upload(c, c->par64, p64.data(), Np));
+    k_nb_params<<<g2(c->N, 256, 1), 256, 0, c->stream>>>(c->N, c->g.geo, src, c->qs, c->sh, c->se,
+                                                         c->q64, c->sig64, c->eps64, c->par64);
+    HIPCHK(hipGetLastError());
+    if (slot >= 0) HIPCHK(hipEventRecord(c->io_done[slot], c->stream));
+    dfree(c, tmp);
     return SDM_OK;
 }
 
@@ -829,6 +885,18 @@ int sdm_create(const sdm_system_desc* sys, int32_t n_replicas, sdm_context** out
         hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&c->ev_join, hipEventDisableTiming) != hipSuccess)
         return bail(fail(SDM_ERR_HIP, "hipStreamCreate/hipEventCreate failed"));
+    for (hipEvent_t& e : c->io_done)
+        if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess)
+            return bail(fail(SDM_ERR_HIP, "hipEventCreate failed"));
+    // a slot holds three FP64 arrays of the atoms, and the records of the replicas
+    const size_t io_cap = std::max((size_t)3 * ((N + 63) / 64 * 64) * sizeof(double),
+                                   (size_t)n_replicas * (sizeof(DevRecord) + sizeof(int)));
+    if (io_cap <= IO_MAX) {
+        if (hipHostMalloc((void**)&c->io, (IO_SLOTS + 1) * io_cap, hipHostMallocDefault) != hipSuccess)
+            return bail(fail(SDM_ERR_HIP, "hipHostMalloc failed"));
+        c->io_cap = io_cap;
+        std::memset(c->io, 0, (IO_SLOTS + 1) * io_cap);  // maps its pages (1 us each)
+    }
     c->N = N;
     c->max_ex = max_ex;
     c->Np = (N + 63) / 64 * 64;
@@ -986,6 +1054,8 @@ int sdm_create(const sdm_system_desc* sys, int32_t n_replicas, sdm_context** out
         if ((rc = upload(c, c->state, st.data(), R))) return bail(rc);
     }
     if ((rc = setup_cells(c, 0)) != SDM_OK) return bail(rc);
+    if (hipStreamSynchronize(c->stream) != hipSuccess)  // nothing of this is left to the first step
+        return bail(fail(SDM_ERR_HIP, "hipStreamSynchronize failed"));
     *out = c;
     return SDM_OK;
 }
@@ -997,6 +1067,9 @@ int sdm_destroy(sdm_context* c) {
     for (void* p : c->allocs) (void)hipFree(p);
     for (hipEvent_t e : {c->ev_fork, c->ev_join})
         if (e) (void)hipEventDestroy(e);
+    for (hipEvent_t e : c->io_done)
+        if (e) (void)hipEventDestroy(e);
+    if (c->io) (void)hipHostFree(c->io);
     if (c->side) (void)hipStreamDestroy(c->side);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
@@ -1014,18 +1087,14 @@ int sdm_set_params(sdm_context* c, int32_t replica, const sdm_params* p) {
     CHK(check_replica(c, replica, true));
     CHK(validate_params(p));
     int r0 = replica < 0 ? 0 : replica, r1 = replica < 0 ? c->R : replica + 1;
-    for (int r = r0; r < r1; r++)
-        HIPCHK(hipMemcpyAsync(&c->state[r], p, sizeof(sdm_params), hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
+    for (int r = r0; r < r1; r++) CHK(upload(c, reinterpret_cast<sdm_params*>(&c->state[r]), p, 1));
     return SDM_OK;
 }
 
 int sdm_get_params(sdm_context* c, int32_t replica, sdm_params* p) {
     CHK(check_replica(c, replica, false));
     if (!p) return fail(SDM_ERR_INVALID, "null output");
-    HIPCHK(hipMemcpyAsync(p, &c->state[replica], sizeof(sdm_params), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    return SDM_OK;
+    return download(c, p, reinterpret_cast<const sdm_params*>(&c->state[replica]), 1);
 }
 
 int sdm_set_time(sdm_context* c, int32_t replica, double time, int64_t step) {
@@ -1340,23 +1409,43 @@ int sdm_set_restraints(sdm_context* c, const sdm_centroid_restraint* cr, int32_t
 static int set_vec(sdm_context* c, double* base, int32_t r, const double* xyz) {
     CHK(check_replica(c, r, false));
     if (!xyz) return fail(SDM_ERR_INVALID, "null array");
-    std::vector<double> soa(3 * (size_t)c->Np, 0.0);
-    for (int i = 0; i < c->N; i++)
-        for (int d = 0; d < 3; d++) {
-            double v = xyz[3 * i + d];
-            if (!std::isfinite(v)) return fail(SDM_ERR_INVALID, "non-finite coordinate");
-            soa[(size_t)d * c->Np + i] = v;
-        }
-    return upload(c, base + (size_t)r * 3 * c->Np, soa.data(), soa.size());
+    const size_t n3 = 3 * (size_t)c->N;
+    bool bad = false;
+    for (size_t k = 0; k < n3; k++) bad |= !(std::fabs(xyz[k]) <= DBL_MAX);
+    if (bad) return fail(SDM_ERR_INVALID, "non-finite coordinate");
+    double* dst = base + (size_t)r * 3 * c->Np;
+    if (n3 * sizeof(double) > c->io_cap) {
+        std::vector<double> soa(3 * (size_t)c->Np, 0.0);
+        for (int i = 0; i < c->N; i++)
+            for (int d = 0; d < 3; d++) soa[(size_t)d * c->Np + i] = xyz[3 * (size_t)i + d];
+        return upload(c, dst, soa.data(), soa.size());
+    }
+    int slot;
+    CHK(io_slot(c, &slot));
+    std::memcpy(io_ptr(c, slot), xyz, n3 * sizeof(double));
+    k_aos_to_soa<<<g2(3 * c->N, 256, 1), 256, 0, c->stream>>>(c->N, c->Np,
+                                                              (const double*)io_ptr(c, slot), dst);
+    CHK(check_launch());
+    HIPCHK(hipEventRecord(c->io_done[slot], c->stream));
+    return SDM_OK;
 }
-
 static int get_vec(sdm_context* c, const double* base, int32_t r, double* xyz) {
     CHK(check_replica(c, r, false));
     if (!xyz) return fail(SDM_ERR_INVALID, "null array");
-    std::vector<double> soa(3 * (size_t)c->Np);
-    CHK(download(c, soa.data(), base + (size_t)r * 3 * c->Np, soa.size()));
-    for (int i = 0; i < c->N; i++)
-        for (int d = 0; d < 3; d++) xyz[3 * i + d] = soa[(size_t)d * c->Np + i];
+    const double* src = base + (size_t)r * 3 * c->Np;
+    const size_t n3 = 3 * (size_t)c->N;
+    if (n3 * sizeof(double) > c->io_cap) {
+        std::vector<double> soa(3 * (size_t)c->Np);
+        CHK(download(c, soa.data(), src, soa.size()));
+        for (int i = 0; i < c->N; i++)
+            for (int d = 0; d < 3; d++) xyz[3 * (size_t)i + d] = soa[(size_t)d * c->Np + i];
+        return SDM_OK;
+    }
+    double* out = (double*)io_ptr(c, IO_SLOTS);
+    k_soa_to_aos<<<g2(3 * c->N, 256, 1), 256, 0, c->stream>>>(c->N, c->Np, src, out);
+    CHK(check_launch());
+    HIPCHK(hipStreamSynchronize(c->stream));
+    std::memcpy(xyz, out, n3 * sizeof(double));
     return SDM_OK;
 }
 
@@ -1384,12 +1473,6 @@ int sdm_get_velocities(sdm_context* c, int32_t r, double* xyz) { return get_vec(
 }  // extern "C"
 
 namespace sdm {
-// [R][N][3] <-> [R][3][Np]
-__global__ void k_aos_to_soa(int N, int Np, const double* __restrict__ in, double* __restrict__ out) {
-    int r = blockIdx.y, i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= N) return;
-    for (int d = 0; d < 3; d++) out[((size_t)r * 3 + d) * Np + i] = in[((size_t)r * N + i) * 3 + d];
-}
 // per replica: lo (3) and hi (3) of the FP64 positions (one workgroup per replica)
 __global__ __launch_bounds__(256) void k_extent(int N, int Np, const double* __restrict__ x64,
                                                 double* __restrict__ out) {
@@ -1412,11 +1495,6 @@ __global__ __launch_bounds__(256) void k_extent(int N, int Np, const double* __r
     }
     if (t < 6) out[(size_t)r * 6 + t] = red[t][0];
 }
-__global__ void k_soa_to_aos(int N, int Np, const double* __restrict__ in, double* __restrict__ out) {
-    int r = blockIdx.y, i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= N) return;
-    for (int d = 0; d < 3; d++) out[((size_t)r * N + i) * 3 + d] = in[((size_t)r * 3 + d) * Np + i];
-}
 }  // namespace sdm
 
 extern "C" {
@@ -1424,7 +1502,7 @@ extern "C" {
 int sdm_set_positions_device(sdm_context* c, const double* d_xyz) {
     if (!c || !d_xyz) return fail(SDM_ERR_INVALID, "null argument");
     c->since_sort = 0;
-    k_aos_to_soa<<<g2(c->N, 256, c->R), 256, 0, c->stream>>>(c->N, c->Np, d_xyz, c->x64);
+    k_aos_to_soa<<<g2(3 * c->N, 256, c->R), 256, 0, c->stream>>>(c->N, c->Np, d_xyz, c->x64);
     CHK(check_launch());
     HIPCHK(hipStreamSynchronize(c->stream));
     if (c->periodic) return SDM_OK;
@@ -1441,7 +1519,7 @@ int sdm_set_positions_device(sdm_context* c, const double* d_xyz) {
 
 int sdm_get_positions_device(sdm_context* c, double* d_xyz) {
     if (!c || !d_xyz) return fail(SDM_ERR_INVALID, "null argument");
-    k_soa_to_aos<<<g2(c->N, 256, c->R), 256, 0, c->stream>>>(c->N, c->Np, c->x64, d_xyz);
+    k_soa_to_aos<<<g2(3 * c->N, 256, c->R), 256, 0, c->stream>>>(c->N, c->Np, c->x64, d_xyz);
     CHK(check_launch());
     HIPCHK(hipStreamSynchronize(c->stream));
     return SDM_OK;
@@ -1478,8 +1556,7 @@ int sdm_get_energies(sdm_context* c, sdm_energies* out) {
     if (!c || !out) return fail(SDM_ERR_INVALID, "null argument");
     std::vector<DevRecord> rec(c->R);
     std::vector<int> fl(c->R);
-    CHK(download(c, rec.data(), c->rec, c->R));
-    CHK(download(c, fl.data(), c->flags, c->R));
+    CHK(download(c, rec.data(), c->rec, c->R, fl.data(), c->flags, c->R));
     for (int r = 0; r < c->R; r++) {
         sdm_energies& e = out[r];
         const DevRecord& d = rec[r];
@@ -1638,12 +1715,6 @@ int sdm_get_forces(sdm_context* c, int32_t r, int32_t which, double* out) {
     if (which < 0 || which > 3) return fail(SDM_ERR_INVALID, "unknown force component");
     int Np = c->Np, N = c->N;
     size_t off = (size_t)r * 3 * Np;
-    std::vector<long long> f(3 * (size_t)Np);
-    std::vector<int> slot(Np);
-    std::vector<double> fbond(3 * (size_t)Np, 0.0);  // FP64 bonds and angles, atom order
-    CHK(download(c, f.data(), c->F + off, f.size()));
-    CHK(download(c, slot.data(), c->slot_of + (size_t)r * Np, Np));
-    if (c->Fb) CHK(download(c, fbond.data(), c->Fb + off, fbond.size()));
     // forces on virtual sites are reported moved to their parents, as the step uses them
     auto sites = [&]() -> int {
         if (c->nvs == 0) return SDM_OK;
@@ -1652,6 +1723,22 @@ int sdm_get_forces(sdm_context* c, int32_t r, int32_t which, double* out) {
         vsite_distribute_host(c, x, out);
         return SDM_OK;
     };
+    const size_t n3 = 3 * (size_t)N;
+    if (which == SDM_FORCE_HYBRID && !c->components_valid && n3 * sizeof(double) <= c->io_cap) {
+        double* io = (double*)io_ptr(c, IO_SLOTS);
+        k_hybrid_forces<<<g2(3 * N, 256, 1), 256, 0, c->stream>>>(
+            N, Np, c->F + off, c->slot_of + (size_t)r * Np, c->Fb ? c->Fb + off : nullptr, io);
+        CHK(check_launch());
+        HIPCHK(hipStreamSynchronize(c->stream));
+        std::memcpy(out, io, n3 * sizeof(double));
+        return sites();
+    }
+    std::vector<long long> f(3 * (size_t)Np);
+    std::vector<int> slot(Np);
+    std::vector<double> fbond(3 * (size_t)Np, 0.0);  // FP64 bonds and angles, atom order
+    CHK(download(c, f.data(), c->F + off, f.size()));
+    CHK(download(c, slot.data(), c->slot_of + (size_t)r * Np, Np));
+    if (c->Fb) CHK(download(c, fbond.data(), c->Fb + off, fbond.size()));
     if (which == SDM_FORCE_HYBRID && !c->components_valid) {
         for (int i = 0; i < N; i++)
             for (int d = 0; d < 3; d++)

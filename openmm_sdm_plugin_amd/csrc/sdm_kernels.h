@@ -603,7 +603,7 @@ struct LigCand {
     int *cand, *ncand, *cmap;
 };
 template <int NW>  // waves per i-block workgroup
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(8))) void k_tiles(int N, int Np, int NB, int maxj,
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_num_vgpr(64))) void k_tiles(int N, int Np, int NB, int maxj,
                                                const float4* __restrict__ arec,
                                                const float4* __restrict__ bb_lo,
                                                const float4* __restrict__ bb_hi,
@@ -3257,6 +3257,60 @@ __global__ __launch_bounds__(64) void k_scatter_dF(int N, int Np, int L, int max
         D[Np + a] = d.y;
         D[2 * Np + a] = d.z;
     }
+}
+
+// ---------------------------------------------------------------------------
+// Data between the host and the device.  These read or write pinned host memory as well as
+// device memory, with consecutive threads on consecutive words of it, so that no copy
+// command waits between the kernels of the stream: bounded by the host link and the
+// launch.  Copies of pageable memory with a wait each, against these: 22,750 atoms
+// set, evaluated and their forces read 380 -> 244 us, 20 replicas of 2,976 atoms 616 -> 427
+// us, a step of 186 atoms read back 132 -> 89 us.
+// ---------------------------------------------------------------------------
+// [R][N][3] -> [R][3][Np] and back
+__global__ void k_aos_to_soa(int N, int Np, const double* __restrict__ in, double* __restrict__ out) {
+    const int r = blockIdx.y, k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= 3 * N) return;
+    out[((size_t)r * 3 + k % 3) * Np + k / 3] = in[(size_t)r * 3 * N + k];
+}
+__global__ void k_soa_to_aos(int N, int Np, const double* __restrict__ in, double* __restrict__ out) {
+    const int r = blockIdx.y, k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= 3 * N) return;
+    out[(size_t)r * 3 * N + k] = in[((size_t)r * 3 + k % 3) * Np + k / 3];
+}
+// words of a and then of b
+__global__ void k_words(const unsigned* __restrict__ a, size_t na, const unsigned* __restrict__ b,
+                        size_t nb, unsigned* __restrict__ dst) {
+    const size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < na) dst[k] = a[k];
+    else if (k < na + nb) dst[k] = b[k - na];
+}
+// hybrid forces of one replica [N][3]: the fixed-point accumulator (slot order) and, where
+// there are any, the bonded forces (atom order)
+__global__ void k_hybrid_forces(int N, int Np, const long long* __restrict__ F,
+                                const int* __restrict__ slot_of, const double* __restrict__ Fb,
+                                double* __restrict__ out) {
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= 3 * N) return;
+    const int i = k / 3, d = k - 3 * i;
+    out[k] = (double)F[(size_t)d * Np + slot_of[i]] / SDM_FIX_SCALE + (Fb ? Fb[(size_t)d * Np + i] : 0.0);
+}
+// the forms of the nonbonded parameters (charges, sigmas, epsilons: [3][N]) that the kernels read
+__global__ void k_nb_params(int N, int geo, const double* __restrict__ p, float* __restrict__ qs,
+                            float* __restrict__ sh, float* __restrict__ se,
+                            double* __restrict__ q64, double* __restrict__ sig64,
+                            double* __restrict__ eps64, double4* __restrict__ par64) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= N) return;
+    const double q = p[i] * sqrt(SDM_ONE_4PI_EPS0), sig = p[N + i], eps = p[2 * (size_t)N + i];
+    const double s = geo ? sig : 0.5 * sig, e = 2.0 * sqrt(eps);  // the entry each rule combines
+    qs[i] = (float)q;
+    sh[i] = (float)s;
+    se[i] = (float)e;
+    q64[i] = q;
+    sig64[i] = sig;
+    eps64[i] = eps;
+    par64[i] = make_double4(q, s, e, 0.0);
 }
 
 }  // namespace sdm
