@@ -92,6 +92,7 @@ struct sdm_context {
     double *q64 = nullptr, *sig64 = nullptr, *eps64 = nullptr, *invm = nullptr, *mass = nullptr;
     double4* par64 = nullptr;  // [Np] (q sqrt(k_e), sigma/2, 2 sqrt(eps), 0): FP64 energies
     Rec64* rec64 = nullptr;    // [R][Np] slot-ordered FP64 records of the energy kernel
+    int* ex_cross = nullptr;  // [Np] 1: excluded from a displaced atom of another class
     int *ex_start = nullptr, *ex_list = nullptr, *cls = nullptr, *lig = nullptr, *cellrank = nullptr;
     // blocks of the displaced-atom list: entries lb_start[b] .. + lb_count[b] (<= 64),
     // all of one displacement class, so a block's bounding box covers one group of atoms
@@ -539,7 +540,7 @@ void launch_forces(sdm_context* c, int parts) {
         c->rec64, c->e64, c->nbw, c->bstart, c->bcode, c->astart, c->acode, c->bond_atoms,
         c->bond_r0, c->bond_k, c->ang_atoms, c->ang_t0, c->ang_k, c->x64, c->Fb, c->e_bond, c->L,
         c->LB, c->lig, c->lb_start, c->lb_count, c->cls, c->cdispl, c->q64, c->sig64, c->eps64,
-        c->ex_start, c->ex_list, c->orig_s, c->cand, c->ncand, c->maxc, c->dA, c->dB, c->g);
+        c->ex_start, c->ex_list, c->ex_cross, c->orig_s, c->cand, c->ncand, c->maxc, c->dA, c->dB, c->g);
 }
 
 void enqueue_forces(sdm_context* c, int parts) {
@@ -560,8 +561,8 @@ void enqueue_forces(sdm_context* c, int parts) {
 void enqueue_delta(sdm_context* c, unsigned long long* counters) {
     if (c->L > 0)
         k_deltaA_red<DRED_WAVES><<<dim3(c->LB, c->R), 64 * DRED_WAVES, 0, c->stream>>>(
-            c->Np, c->L, c->LB, c->lig, c->lb_start, c->lb_count, c->cls, c->cdispl, c->q64,
-            c->sig64, c->eps64, c->ex_start, c->ex_list, c->x64, c->ncand, c->maxc, c->dA,
+            c->Np, c->L, c->LB, c->ncls, c->lig, c->lb_start, c->lb_count, c->cls, c->cdispl, c->q64,
+            c->sig64, c->eps64, c->ex_start, c->ex_list, c->ex_cross, c->x64, c->ncand, c->maxc, c->dA,
             c->dlig, c->u_part, c->g, counters);
 }
 
@@ -617,16 +618,22 @@ void enqueue_eval(sdm_context* c, bool advance, bool components, bool full, bool
             c->bb_hi, c->exs, c->exblocks, c->max_ex, c->e64, c->g);
     }
     enqueue_forces(c, PAIRS | DISPLACED | BONDED | (energy && !apart ? ENERGY : 0));
-    enqueue_delta(c, nullptr);
+    const bool sums = c->L > 0 && c->LB <= DRED_FUSED;  // in k_scalar
+    if (!sums) enqueue_delta(c, nullptr);
     if (terms || apart) {
         (void)hipEventRecord(c->ev_join, s1);
         (void)hipStreamWaitEvent(s, c->ev_join, 0);
     }
-    k_scalar<<<R, 256, 0, s>>>(c->NB * block_parts(c), c->nbw, c->LB, c->e64,
-                               c->e_bond, c->u_part, c->state,
-                               c->rec, c->flags, advance ? 1 : 0, energy ? 1 : 0,
-                               c->hist_every, c->hist_cap, c->uhist, c->e_rest,
-                               c->ncen + c->nali, c->e_t1, c->e_t2, c->ntb, c->dmax);
+    auto scalar = [&](auto kernel) {
+        kernel<<<R, 64 * DRED_WAVES, 0, s>>>(
+            c->NB * block_parts(c), c->nbw, c->LB, c->e64, c->e_bond, c->u_part, c->state, c->rec,
+            c->flags, advance ? 1 : 0, energy ? 1 : 0, c->hist_every, c->hist_cap, c->uhist,
+            c->e_rest, c->ncen + c->nali, c->e_t1, c->e_t2, c->ntb, c->dmax, Np, c->L, c->ncls, c->lig,
+            c->lb_start, c->lb_count, c->cls, c->cdispl, c->q64, c->sig64, c->eps64, c->ex_start,
+            c->ex_list, c->ex_cross, c->x64, c->ncand, c->maxc, c->dA, c->dlig, c->g);
+    };
+    if (sums) scalar(k_scalar<true>);
+    else scalar(k_scalar<false>);
     if (c->L > 0 && !components && !mix_in_langevin(c, advance))
         k_mix<<<dim3(c->maxc + c->LB, R), 64, 0, s>>>(N, Np, c->L, c->maxc, c->lig, c->cls,
                                                        c->orig_s, c->cand, c->ncand,
@@ -957,6 +964,7 @@ int sdm_create(const sdm_system_desc* sys, int32_t n_replicas, sdm_context** out
     if ((rc = dalloc(c, &c->ptr, (n))) != SDM_OK) return bail(rc)
     A(qs, Np); A(sh, Np); A(se, Np); A(q64, Np); A(sig64, Np); A(eps64, Np); A(par64, Np);
     A(invm, Np); A(mass, Np); A(ex_start, N_ + 1); A(ex_list, elist.size());
+    A(ex_cross, Np);
     A(cls, Np); A(lig, std::max(1, c->L)); A(cdispl, cd.size());
     A(lb_start, lbs.size()); A(lb_count, lbn.size());
     A(bond_atoms, 2 * std::max(1, c->nbond)); A(bond_r0, std::max(1, c->nbond));
@@ -997,12 +1005,17 @@ int sdm_create(const sdm_system_desc* sys, int32_t n_replicas, sdm_context** out
         }
         std::vector<int> clsp(Np, 0);
         std::copy(cls.begin(), cls.end(), clsp.begin());
+        std::vector<int> cross(Np, 0);
+        for (int i = 0; i < N; i++)
+            for (int k = ecount[i]; k < ecount[i + 1]; k++)
+                if (cls[elist[k]] != 0 && cls[elist[k]] != cls[i]) cross[i] = 1;
         std::vector<int> orig_pad(RNp, -1);
         if ((rc = upload(c, c->invm, im.data(), Np)) ||
             (rc = upload(c, c->mass, m.data(), Np)) ||
             (rc = upload(c, c->ex_start, ecount.data(), N + 1)) ||
             (rc = upload(c, c->ex_list, elist.data(), elist.size())) ||
             (rc = upload(c, c->cls, clsp.data(), Np)) ||
+            (rc = upload(c, c->ex_cross, cross.data(), Np)) ||
             (rc = upload(c, c->cdispl, cd.data(), cd.size())) ||
             (rc = upload(c, c->orig_s, orig_pad.data(), RNp)))
             return bail(rc);

@@ -101,36 +101,60 @@ __global__ void k_bin(int N, int Np, const double* __restrict__ x64, int* __rest
     atomicAdd(&ccount[(size_t)r * NC + k], 1);
 }
 
+// inclusive sum over the lanes up to this one
+__device__ __forceinline__ int wave_scan(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);  // row_shr:1, 2, 4, 8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, true);  // row_bcast:15
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, true);  // row_bcast:31
+    return v;
+}
+
 // exclusive scan of the cell counts, one 1024-thread workgroup per replica; clears the
-// counters for the next step.
+// counters for the next step.  8 x 1024 cells at a time, coalesced and in flight together,
+// with two barriers: the launch is one workgroup's latency, 19.6 us for 8,000 cells with a
+// run of cells per thread and a barrier per doubling, 3.8 us so.
 __global__ __launch_bounds__(1024) void k_scan(int NC, int* __restrict__ ccount,
                                                int* __restrict__ cstart, int* __restrict__ cfill) {
-    __shared__ int part[1024];
-    int r = blockIdx.x;
-    int t = threadIdx.x;
-    int per = (NC + 1023) / 1024;
-    int beg = min(t * per, NC), end = min(beg + per, NC);
+    __shared__ int sums[2][128];  // of chunk k and wave w: [16 k + w], alternating
+    const int r = blockIdx.x, t = threadIdx.x, lane = t & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
     int* cnt = ccount + (size_t)r * NC;
-    int s = 0;
-    for (int c = beg; c < end; c++) s += cnt[c];
-    part[t] = s;
-    __syncthreads();
-    for (int o = 1; o < 1024; o <<= 1) {
-        int v = (t >= o) ? part[t - o] : 0;
-        __syncthreads();
-        part[t] += v;
-        __syncthreads();
-    }
-    int run = part[t] - s;
     int* st = cstart + (size_t)r * (NC + 1);
     int* fl = cfill + (size_t)r * NC;
-    for (int c = beg; c < end; c++) {
-        st[c] = run;
-        run += cnt[c];
-        cnt[c] = 0;
-        fl[c] = 0;
+    int before = 0;  // cells of the rounds before
+    for (int base = 0, row = 0; base < NC; base += 8192, row ^= 1) {
+        int v[8], end[8];
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            const int c = base + 1024 * k + t;
+            v[k] = c < NC ? cnt[c] : 0;
+        }
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            end[k] = wave_scan(v[k]);
+            if (lane == 63) sums[row][16 * k + wv] = end[k];
+        }
+        __syncthreads();
+        // every wave finds the sums in front of its parts
+        const int a = sums[row][lane], b = sums[row][64 + lane];
+        const int ea = wave_scan(a), ta = __builtin_amdgcn_readlane(ea, 63);
+        const int eb = wave_scan(b) + ta;
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            const int q = 16 * k + wv, x = k < 4 ? ea - a : eb - b;
+            const int c = base + 1024 * k + t;
+            if (c < NC) {
+                st[c] = before + __builtin_amdgcn_readlane(x, q & 63) + end[k] - v[k];
+                cnt[c] = 0;
+                fl[c] = 0;
+            }
+        }
+        before += __builtin_amdgcn_readlane(eb, 63);
     }
-    if (t == 1023) st[NC] = part[1023];
+    if (t == 0) st[NC] = before;
 }
 
 __global__ void k_scatter(int N, int Np, int NC, const int* __restrict__ key,
@@ -501,17 +525,6 @@ __device__ __forceinline__ void lig_candidates(
 // 99,920 atoms 855 -> 790 (877 with equal parts), 22 x 22,750 atoms 403 -> 392.
 constexpr int TILE_UNITS = 6, TILE_SLOPE_BLOCKS = 512;
 constexpr int MAX_TILE_PARTS = 64, TILE_BOUNDS = MAX_TILE_PARTS + 1;
-
-// inclusive sum over the lanes up to this one
-__device__ __forceinline__ int wave_scan(int v) {
-    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);  // row_shr:1, 2, 4, 8
-    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, true);  // row_bcast:15
-    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, true);  // row_bcast:31
-    return v;
-}
 
 // one wave: the bounds of `parts` (at most 64) parts of a list of nt tiles with masks tmk,
 // whose numbers of steps are in nstep for the first SHARE_LDS ones.  Lanes are tiles for the
@@ -1914,19 +1927,6 @@ __device__ __forceinline__ Atom64 tile_atom(const AtomTile64& T, int t) {
     return A;
 }
 
-// whether atom a has an exclusion partner that is displaced (want_displaced) or not.
-// Exclusions across the boundary of the displaced set are rare (a bond from the ligand
-// to the receptor), so only atoms that have one search their list per pair.
-__device__ __forceinline__ bool excl_with(const int* __restrict__ ex_start,
-                                          const int* __restrict__ ex_list,
-                                          const int* __restrict__ cls, int a,
-                                          bool want_displaced) {
-    bool any = false;
-    for (int k = ex_start[a]; k < ex_start[a + 1]; k++)
-        any = any || ((cls[ex_list[k]] != 0) == want_displaced);
-    return any;
-}
-
 // The displaced-state pairs: every (displaced atom i, undisplaced atom j) within the
 // cutoff at x or at x+d, evaluated once in FP64 at both geometries (delta_pair); every sum
 // has one owner and a fixed order (no atomics).  A wave takes eight displaced atoms of each
@@ -1939,8 +1939,9 @@ __device__ __forceinline__ bool excl_with(const int* __restrict__ ex_start,
 //   order by k_deltaA_red.
 //   F1-F0 on the slots is summed over the eight displaced atoms at each step, and lane
 //   8 q + k keeps it for cluster k; one part per wave (dB, env_force).
-// Excluded pairs are left out (only atoms with an exclusion across the displaced/undisplaced
-// boundary search their exclusion list).
+// Excluded pairs are left out: exclusions with a displaced atom of another class (or of an
+// undisplaced atom with a displaced one: a bond from the ligand to the receptor) are rare, so
+// only atoms that have one (ex_cross) search their list per pair.
 //
 // What bounds it is the chain of loads and of up to 8 steps of FP64 pairs of one wave (a few
 // blocks near the displaced atoms hold most pairs) and, with many replicas, FP64 issue.  With
@@ -1982,7 +1983,7 @@ __device__ __forceinline__ void displaced_wave(
     const int* __restrict__ lb_count, const int* __restrict__ cls,
     const double* __restrict__ cdispl, const double* __restrict__ q64,
     const double* __restrict__ sig64, const double* __restrict__ eps64,
-    const int* __restrict__ ex_start, const int* __restrict__ ex_list,
+    const int* __restrict__ ex_start, const int* __restrict__ ex_list, const int* __restrict__ ex_cross,
     const double* __restrict__ x64, const int* __restrict__ orig_s,
     const int* __restrict__ cand, const int* __restrict__ ncand, int maxc,
     double4* __restrict__ dA, double4* __restrict__ dB,
@@ -2009,7 +2010,7 @@ __device__ __forceinline__ void displaced_wave(
         E.idx[lane] = b;
         const unsigned long long envm = __ballot(env);
         const unsigned long long exm =
-            __ballot(env && excl_with(ex_start, ex_list, cls, b, true));
+            __ballot(env && ex_cross[b] != 0);
         lds_order();
         // the groups' sums are added in order here as in env_force, so that results do not
         // depend on how many of them a wave takes
@@ -2129,7 +2130,7 @@ __global__ __launch_bounds__(64 * WPW) __attribute__((amdgpu_waves_per_eu(4))) v
     const int* __restrict__ lb_count, const int* __restrict__ cls,
     const double* __restrict__ cdispl, const double* __restrict__ q64,
     const double* __restrict__ sig64, const double* __restrict__ eps64,
-    const int* __restrict__ ex_start, const int* __restrict__ ex_list,
+    const int* __restrict__ ex_start, const int* __restrict__ ex_list, const int* __restrict__ ex_cross,
     const int* __restrict__ orig_s, const int* __restrict__ cand,
     const int* __restrict__ ncand, int maxc, double4* __restrict__ dA,
     double4* __restrict__ dB, Geom g) {
@@ -2147,7 +2148,7 @@ __global__ __launch_bounds__(64 * WPW) __attribute__((amdgpu_waves_per_eu(4))) v
     if (b < fg.displaced) {
         displaced_wave<COUNT>(b * WPW + wv, fg.displaced_waves, fg.displaced_subs, lane,
                               *(EnvTile*)wave_s[wv], R, N, Np, L, LB, lig, lb_start, lb_count, cls, cdispl, q64, sig64, eps64,
-                              ex_start, ex_list, x64, orig_s, cand, ncand, maxc, dA, dB,
+                              ex_start, ex_list, ex_cross, x64, orig_s, cand, ncand, maxc, dA, dB,
                               pair_count + R, g);
         return;
     }
@@ -2194,21 +2195,22 @@ __global__ __launch_bounds__(64) void k_energy64(
                       packed, rec, tiles, tmask, bounds, bb_lo, bb_hi, exs, exblocks, max_ex, e_out, g);
 }
 
-// per displaced atom: the block partials of displaced_wave in order, plus pairs with displaced
-// atoms of a different class (D x D); writes dlig and the ligand block's u.
+// per displaced atom of ligand block lb: the block partials of displaced_wave, plus pairs with
+// displaced atoms of a different class (D x D); writes dlig and returns the ligand block's u
+// (in the first wave).  A workgroup of RW waves.
 template <int RW>
-__global__ __launch_bounds__(64 * RW) void k_deltaA_red(
-    int Np, int L, int LB, const int* __restrict__ lig, const int* __restrict__ lb_start,
-    const int* __restrict__ lb_count, const int* __restrict__ cls,
-    const double* __restrict__ cdispl, const double* __restrict__ q64,
-    const double* __restrict__ sig64, const double* __restrict__ eps64,
-    const int* __restrict__ ex_start, const int* __restrict__ ex_list,
-    const double* __restrict__ x64, const int* __restrict__ ncand, int maxc,
-    const double4* __restrict__ dA, double4* __restrict__ dlig, double* __restrict__ u_part,
-    Geom g, unsigned long long* __restrict__ pair_count) {
+__device__ __forceinline__ double delta_sums(
+    int lb, int r, int Np, int L, int LB, int ncls, const int* __restrict__ lig,
+    const int* __restrict__ lb_start, const int* __restrict__ lb_count,
+    const int* __restrict__ cls, const double* __restrict__ cdispl,
+    const double* __restrict__ q64, const double* __restrict__ sig64,
+    const double* __restrict__ eps64, const int* __restrict__ ex_start,
+    const int* __restrict__ ex_list, const int* __restrict__ ex_cross, const double* __restrict__ x64,
+    const int* __restrict__ ncand, int maxc, const double4* __restrict__ dA,
+    double4* __restrict__ dlig, const Geom& g, unsigned long long* __restrict__ pair_count) {
     // RW waves: wave w adds the partials of blocks w, w + RW, .. and the D x D pairs of
     // displaced atoms w, w + RW, ..; the waves' sums are added in wave order
-    int lb = blockIdx.x, r = blockIdx.y, lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const double* X = x64 + (size_t)r * 3 * Np;
     int li = lb_start[lb] + lane;
     bool v = lane < lb_count[lb];
@@ -2226,42 +2228,67 @@ __global__ __launch_bounds__(64 * RW) void k_deltaA_red(
     __shared__ AtomTile64 T;
     __shared__ double4 part[RW][64];
     int cnt = 0;
-    for (int base = 0; base < L; base += 64) {
-        int n = min(64, L - base);
-        __syncthreads();  // the previous chunk has been read
-        if ((int)threadIdx.x < n)
-            stage_atom(T, threadIdx.x, load_atom64(X, Np, lig[base + threadIdx.x], cls, cdispl, q64,
-                                                   sig64, eps64));
-        __syncthreads();
-        for (int k = wv; k < n; k += RW) {
-            Atom64 J = tile_atom(T, k);
-            if (!v || J.cls == I.cls || excluded(ex_start, ex_list, I.idx, J.idx)) continue;
-            int iny;
-            du += 0.5 * delta_pair(I, J, g, fx, fy, fz, &iny);
-            cnt += (iny && I.idx < J.idx) ? 1 : 0;
+    if (ncls > 1) {  // uniform
+        const bool exI = v && ex_cross[I.idx] != 0;
+        for (int base = 0; base < L; base += 64) {
+            int n = min(64, L - base);
+            // (the list is in order of classes, and a ligand block is of one class)
+            const int own = cls[lig[lb_start[lb]]];
+            if (cls[lig[base]] == own && cls[lig[base + n - 1]] == own) continue;  // uniform
+            __syncthreads();  // the previous chunk has been read
+            if ((int)threadIdx.x < n)
+                stage_atom(T, threadIdx.x, load_atom64(X, Np, lig[base + threadIdx.x], cls, cdispl, q64,
+                                                       sig64, eps64));
+            __syncthreads();
+            for (int k = wv; k < n; k += RW) {
+                Atom64 J = tile_atom(T, k);
+                if (!v || J.cls == I.cls) continue;
+                if (exI && excluded(ex_start, ex_list, I.idx, J.idx)) continue;
+                int iny;
+                du += 0.5 * delta_pair(I, J, g, fx, fy, fz, &iny);
+                cnt += (iny && I.idx < J.idx) ? 1 : 0;
+            }
         }
     }
     if (pair_count) {
         double s = wave_sum((double)cnt);
         if (lane == 0) atomicAdd(&pair_count[r], (unsigned long long)(s + 0.5));
-        return;
+        return 0.0;
     }
     part[wv][lane] = make_double4(fx, fy, fz, du);
     __syncthreads();
-    if (wv == 0) {
-        double4 t = part[0][lane];
-        for (int w = 1; w < RW; w++) {
-            t.x += part[w][lane].x;
-            t.y += part[w][lane].y;
-            t.z += part[w][lane].z;
-            t.w += part[w][lane].w;
-        }
-        if (v) dlig[(size_t)r * L + li] = t;
-        double us = wave_sum(v ? t.w : 0.0);
-        if (lane == 0) u_part[(size_t)r * LB + lb] = us;
+    if (wv != 0) return 0.0;
+    double4 t = part[0][lane];
+    for (int w = 1; w < RW; w++) {
+        t.x += part[w][lane].x;
+        t.y += part[w][lane].y;
+        t.z += part[w][lane].z;
+        t.w += part[w][lane].w;
     }
+    if (v) dlig[(size_t)r * L + li] = t;
+    return wave_sum(v ? t.w : 0.0);
 }
-constexpr int DRED_WAVES = 4;
+
+// the sums of one ligand block (and, with pair_count, only the count of its pairs)
+template <int RW>
+__global__ __launch_bounds__(64 * RW) void k_deltaA_red(
+    int Np, int L, int LB, int ncls, const int* __restrict__ lig, const int* __restrict__ lb_start,
+    const int* __restrict__ lb_count, const int* __restrict__ cls,
+    const double* __restrict__ cdispl, const double* __restrict__ q64,
+    const double* __restrict__ sig64, const double* __restrict__ eps64,
+    const int* __restrict__ ex_start, const int* __restrict__ ex_list, const int* __restrict__ ex_cross,
+    const double* __restrict__ x64, const int* __restrict__ ncand, int maxc,
+    const double4* __restrict__ dA, double4* __restrict__ dlig, double* __restrict__ u_part,
+    Geom g, unsigned long long* __restrict__ pair_count) {
+    const double u = delta_sums<RW>(blockIdx.x, blockIdx.y, Np, L, LB, ncls, lig, lb_start, lb_count, cls,
+                                    cdispl, q64, sig64, eps64, ex_start, ex_list, ex_cross, x64, ncand,
+                                    maxc, dA, dlig, g, pair_count);
+    if (threadIdx.x == 0 && !pair_count) u_part[(size_t)blockIdx.y * LB + blockIdx.x] = u;
+}
+constexpr int DRED_WAVES = 16;
+// ligand blocks whose sums k_scalar takes itself; more of them get workgroups of their own (the
+// figures are at k_scalar)
+constexpr int DRED_FUSED = 1;
 
 // ---------------------------------------------------------------------------
 // scalar stage (one workgroup per replica): energies, SoftCoreF, bias, sp, schedule.
@@ -2287,51 +2314,83 @@ __device__ double softcore_dev(int method, double u, double umax, double a, doub
 }
 
 // ne: pair-energy slots per replica (i-blocks times the pair kernel's waves per block)
-__global__ __launch_bounds__(256) void k_scalar(
+// SUMS: first the sums on the displaced atoms (delta_sums), with one ligand block: a launch of
+// its own for them took 7.2 us of 22,750 atoms and 10 us of 22 replicas before this one's 9.9
+// and 7.5 us; together, and with the state and the Langevin parameters off the last thread's
+// chain of loads and divisions, 9.3 and 12.7 us.  Two ligand blocks one after the other took
+// 36 us of 8 x 99,920 atoms, in workgroups of their own 13.5 us and 8 us here.
+template <bool SUMS>
+__global__ __launch_bounds__(64 * DRED_WAVES) void k_scalar(
     int ne, int nbw, int LB, const double* __restrict__ e_pair,
     const double* __restrict__ e_bond, const double* __restrict__ u_part,
     DevState* __restrict__ state, DevRecord* __restrict__ rec, int* __restrict__ flags,
     int advance, int energy, int hist_every, int hist_cap, double* __restrict__ uhist,
     const double* __restrict__ e_rest, int nrest, const double* __restrict__ e_t1,
-    const double* __restrict__ e_t2, int ntb, float* __restrict__ dmax) {
-    __shared__ double red[256];
+    const double* __restrict__ e_t2, int ntb, float* __restrict__ dmax, int Np, int L, int ncls,
+    const int* __restrict__ lig, const int* __restrict__ lb_start,
+    const int* __restrict__ lb_count, const int* __restrict__ cls,
+    const double* __restrict__ cdispl, const double* __restrict__ q64,
+    const double* __restrict__ sig64, const double* __restrict__ eps64,
+    const int* __restrict__ ex_start, const int* __restrict__ ex_list, const int* __restrict__ ex_cross,
+    const double* __restrict__ x64, const int* __restrict__ ncand, int maxc,
+    const double4* __restrict__ dA, double4* __restrict__ dlig, Geom g) {
+    constexpr int T = 64 * DRED_WAVES;
+    __shared__ double red[2][DRED_WAVES];
+    __shared__ DevState S;  // in flight with the sums
     int r = blockIdx.x, t = threadIdx.x;
+    constexpr int words = sizeof(DevState) / 4;
+    static_assert(sizeof(DevState) % 4 == 0 && words <= 192, "DevState");
+    if (t >= 64 && t < 64 + words) ((int*)&S)[t - 64] = ((const int*)&state[r])[t - 64];
+    const double old_U0 = t == 0 ? rec[r].U0 : 0.0;
     // the displacement record of kept tile lists restarts with the next slot refresh:
     // this evaluation's k_tiles has read it and kept or rebuilt the lists (after a sort,
     // rebuilt), and the next refresh measures the displacement since that build again
     if (t == 0) dmax[(size_t)r * DISP_STRIDE] = 0.f;
     double s0 = 0.0, s1 = 0.0;
-    // energy == 0: the pair kernel left the pair energies out; U0, U1 and pot_energy
-    // keep the values of the last evaluation that had them (nothing else depends on U0)
-    double U0 = rec[r].U0;
-    if (energy) {
-        for (int k = t; k < ne; k += 256) s0 += e_pair[(size_t)r * ne + k];
-        red[t] = s0;
-        __syncthreads();
-        for (int o = 128; o > 0; o >>= 1) {
-            if (t < o) red[t] += red[t + o];
-            __syncthreads();
+    if (energy)
+        for (int k = t; k < ne; k += T) s0 += e_pair[(size_t)r * ne + k];
+    for (int k = t; k < nbw; k += T) s1 += e_bond[(size_t)r * nbw + k];
+    s0 = wave_sum(s0);
+    s1 = wave_sum(s1);
+    if ((t & 63) == 0) {
+        red[0][t >> 6] = s0;
+        red[1][t >> 6] = s1;
+    }
+    double u = 0.0;
+    if constexpr (SUMS) {
+        for (int lb = 0; lb < LB; lb++) {
+            u += delta_sums<DRED_WAVES>(lb, r, Np, L, LB, ncls, lig, lb_start, lb_count, cls, cdispl, q64,
+                                        sig64, eps64, ex_start, ex_list, ex_cross, x64, ncand, maxc, dA,
+                                        dlig, g, nullptr);
+            __syncthreads();  // its LDS is used again
         }
-        U0 = red[0];
-        __syncthreads();
     }
-    for (int k = t; k < nbw; k += 256) s1 += e_bond[(size_t)r * nbw + k];
-    red[t] = s1;
     __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if (t < o) red[t] += red[t + o];
-        __syncthreads();
+    if (t == 64) {
+        // Langevin parameters (OpenCLSDMKernels.cpp:331-355; equal to
+        // ReferenceStochasticDynamicsSDM.cpp:144-148 for friction > 0)
+        const double vscale = exp(-S.step_size * S.friction);
+        rec[r].vscale = vscale;
+        rec[r].fscale = (S.friction == 0.0) ? S.step_size : (1.0 - vscale) / S.friction;
+        rec[r].noisescale = sqrt(SDM_BOLTZ * S.temperature * (1.0 - vscale * vscale));
+        rec[r].dt = S.step_size;
     }
-    double Ub = red[0];
     if (t != 0) return;
+    double U0 = 0.0, Ub = 0.0;
+    for (int w = 0; w < DRED_WAVES; w++) {
+        U0 += red[0][w];
+        Ub += red[1][w];
+    }
+    // energy == 0: the pair energies were left out; U0, U1 and pot_energy keep the values of
+    // the last evaluation that had them (nothing else depends on U0)
+    if (!energy) U0 = old_U0;
     for (int k = 0; k < nrest; k++) Ub += e_rest[(size_t)r * nrest + k];  // restraints
     for (int k = 0; k < ntb; k++) {  // further force-field terms: groups 1 and 2
         Ub += e_t1[(size_t)r * ntb + k];
         if (energy) U0 += e_t2[(size_t)r * ntb + k];
     }
-    double u = 0.0;
-    for (int k = 0; k < LB; k++) u += u_part[(size_t)r * LB + k];
-    DevState& S = state[r];
+    if constexpr (!SUMS)
+        for (int k = 0; k < LB; k++) u += u_part[(size_t)r * LB + k];
     DevRecord& Rr = rec[r];
     // nonequilibrium schedule (ReferenceSDMKernels.cpp:221-245)
     double stepSize = S.step_size;
@@ -2413,14 +2472,6 @@ __global__ __launch_bounds__(256) void k_scalar(
     Rr.u0 = (method == 2) ? u0 : S.u0;
     Rr.w0 = S.w0coeff;
     Rr.work = S.work;
-    // Langevin parameters (OpenCLSDMKernels.cpp:331-355; equal to
-    // ReferenceStochasticDynamicsSDM.cpp:144-148 for friction > 0)
-    double kT = SDM_BOLTZ * S.temperature;
-    double vscale = exp(-stepSize * S.friction);
-    Rr.vscale = vscale;
-    Rr.fscale = (S.friction == 0.0) ? stepSize : (1.0 - vscale) / S.friction;
-    Rr.noisescale = sqrt(kT * (1.0 - vscale * vscale));
-    Rr.dt = stepSize;
     Rr.noise_step = S.step;
     if (hist_every > 0 && advance && (S.step % hist_every) == 0) {
         uhist[(size_t)r * hist_cap + (size_t)(S.hist_n % hist_cap)] = be;
@@ -2433,6 +2484,7 @@ __global__ __launch_bounds__(256) void k_scalar(
     Rr.time = S.time;
     Rr.step = S.step;
     Rr.flags = flags[r];
+    state[r] = S;
 }
 
 // F += sp (F1 - F0): candidate-block atoms from dB, displaced atoms from dlig (the

@@ -78,3 +78,10 @@ def test_parts_take_every_pair_once(hip_device, waters, box, skin):
         assert got[0] == ref[0] and abs(got[1] - ref[1]) <= 1e-12 * max(abs(ref[1]), 1e3 * s.n)
         rms = np.sqrt(np.mean(ref[2] ** 2))
         assert np.sqrt(np.mean((got[2] - ref[2]) ** 2)) <= 1e-6 * rms
+
+
+@pytest.mark.parametrize("cells", [10, 20, 21, 33])
+def test_sort_grid_sizes(hip_device, cells):
+    """Sort grids of fewer and more cells than one round of the scan (8 x 1,024) takes."""
+    print(f"case cells={cells}", flush=True)
+    _check(systems.make_small(40, 7, frame=5), dict(cell_cells_per_dim=cells))
