@@ -2556,45 +2556,58 @@ __global__ __launch_bounds__(256) void k_langevin(int N, int Np, const double* _
     int r = blockIdx.y;
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= N) return;
+    // everything that is read is asked for first, and the noise computed meanwhile: a thread's
+    // time is its chain of loads and FP64 logarithms, square roots and sines (22,750 atoms 9.0 ->
+    // 6.9 us)
     const DevRecord& Rr = rec[r];
-    if (mg.lig_of) {
-        const int li = mg.lig_of[i];
-        const int sl = slot_of[(size_t)r * Np + i];
-        const int cb = li >= 0 ? 0 : mg.cmap[(size_t)r * mg.NB + (sl >> 6)];
-        if (cb >= 0) {
-            const double4 d = li >= 0 ? mg.dlig[(size_t)r * mg.L + li]
-                                      : env_force(mg.dB, mg.parts, (size_t)r * mg.maxc + cb, sl & 63);
-            const double sp = Rr.sp;
-            long long* Fm = F + (size_t)r * 3 * Np;
-            int bad = 0;
-            Fm[sl] += to_fixed(sp * d.x, &bad);
-            Fm[Np + sl] += to_fixed(sp * d.y, &bad);
-            Fm[2 * Np + sl] += to_fixed(sp * d.z, &bad);
-            if (bad) atomicOr(&flags[r], 2);
-        }
+    const int slot = slot_of[(size_t)r * Np + i];
+    const double im = invm[i];
+    const bool con = cflag && cflag[i];
+    long long* Fr = F + (size_t)r * 3 * Np;
+    double* X = x64 + (size_t)r * 3 * Np;
+    double* V = v64 + (size_t)r * 3 * Np;
+    long long fi[3];
+    double fb[3], x[3], v[3];
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        x[d] = X[d * Np + i];
+        v[d] = V[d * Np + i];
+        fb[d] = Fb ? Fb[((size_t)r * 3 + d) * Np + i] : 0.0;
+        fi[d] = Fr[d * Np + slot];
     }
-    double im = invm[i];
+    int li = -1, cb = -1;
+    if (mg.lig_of) {
+        li = mg.lig_of[i];
+        cb = li >= 0 ? 0 : mg.cmap[(size_t)r * mg.NB + (slot >> 6)];
+    }
+    double gz[3];
+    gauss3(state[r].seed, (uint32_t)r, (uint64_t)Rr.noise_step, (uint32_t)i, gz);
+    if (cb >= 0) {  // the displaced-state forces, into the accumulator too
+        const double4 d = li >= 0 ? mg.dlig[(size_t)r * mg.L + li]
+                                  : env_force(mg.dB, mg.parts, (size_t)r * mg.maxc + cb, slot & 63);
+        const double sp = Rr.sp;
+        int bad = 0;
+        fi[0] += to_fixed(sp * d.x, &bad);
+        fi[1] += to_fixed(sp * d.y, &bad);
+        fi[2] += to_fixed(sp * d.z, &bad);
+#pragma unroll
+        for (int k = 0; k < 3; k++) Fr[k * Np + slot] = fi[k];
+        if (bad) atomicOr(&flags[r], 2);
+    }
     if (im == 0.0) return;
     double vscale = Rr.vscale, fscale = Rr.fscale, noise = Rr.noisescale, dt = Rr.dt;
     double sim = sqrt(im);
-    double gz[3];
-    gauss3(state[r].seed, (uint32_t)r, (uint64_t)Rr.noise_step, (uint32_t)i, gz);
-    const long long* Fr = F + (size_t)r * 3 * Np;
-    double* X = x64 + (size_t)r * 3 * Np;
-    double* V = v64 + (size_t)r * 3 * Np;
     double inv = 1.0 / dt;
-    int slot = slot_of[(size_t)r * Np + i];
-    bool con = cflag && cflag[i];
 #pragma unroll
     for (int d = 0; d < 3; d++) {
-        double f = from_fixed(Fr[d * Np + slot]);
-        if (Fb) f += Fb[((size_t)r * 3 + d) * Np + i];
-        double vel = vscale * V[d * Np + i] + fscale * im * f + noise * sim * gz[d];
+        double f = from_fixed(fi[d]);
+        if (Fb) f += fb[d];
+        double vel = vscale * v[d] + fscale * im * f + noise * sim * gz[d];
         double delta = dt * vel;
         if (con) {
             dxs[(size_t)r * 3 * Np + d * Np + i] = delta;
         } else {
-            X[d * Np + i] += delta;
+            X[d * Np + i] = x[d] + delta;
             V[d * Np + i] = inv * delta;
         }
     }
