@@ -584,7 +584,8 @@ bool mix_in_langevin(const sdm_context* c, bool advance) {
 // for long (many_waves).  Measured, energies in k_forces against on the side stream: 5 steps
 // of 22 x 22,750 atoms with energies 5.32 against 5.01 ms, but one evaluation of 22,750 atoms
 // 0.40 against 0.44 ms.
-void enqueue_eval(sdm_context* c, bool advance, bool components, bool full, bool energy) {
+void enqueue_eval(sdm_context* c, bool advance, bool components, bool full, bool energy,
+                  bool ordered = false) {
     // tuning.side_fork: restraints and force-field terms need the slot order and cleared
     // accumulator, not the tile lists.  0: they start after the tile lists, 1, 3 and 4:
     // before them, 2: there is no side stream, everything runs on the main one.
@@ -598,7 +599,7 @@ void enqueue_eval(sdm_context* c, bool advance, bool components, bool full, bool
         (void)hipEventRecord(c->ev_fork, s);
         (void)hipStreamWaitEvent(s1, c->ev_fork, 0);
     };
-    enqueue_order(c, full, energy);
+    if (!ordered) enqueue_order(c, full, energy);  // (k_move has done it)
     fork(terms && mode != 0);
     enqueue_tiles(c);
     fork((terms && mode == 0) || apart);
@@ -642,8 +643,16 @@ void enqueue_eval(sdm_context* c, bool advance, bool components, bool full, bool
                                                        displaced_parts(c), c->dB, c->dlig, c->rec, c->slot_of, c->F, c->flags);
 }
 
-void enqueue_step(sdm_context* c, bool full, bool energy) {
-    enqueue_eval(c, true, false, full, energy);
+// Whether a step ends with the next one's slot records (k_move): nothing else moves atoms, and
+// the GPU is short of work, so that a launch less counts for more than gathered positions (22
+// replicas of 22,750 atoms: k_move 45 us, the Langevin kernel and the records 23 + 14 us).
+bool can_move(const sdm_context* c) { return c->ncl == 0 && c->nvs == 0 && few_blocks(c); }
+
+// ordered: the step before has made the slot records (k_move); move: this one makes the next
+// one's, which keeps the order and has energies or not like this one
+void enqueue_step(sdm_context* c, bool full, bool energy, bool ordered = false,
+                  bool move = false) {
+    enqueue_eval(c, true, false, full, energy, ordered);
     if (c->cm_every > 0)
         k_cm_remove<<<c->R, 1024, 0, c->stream>>>(c->N, c->Np, c->cm_every, c->mass, c->v64,
                                                    c->state);
@@ -654,6 +663,13 @@ void enqueue_step(sdm_context* c, bool full, bool energy) {
     MixGather mg{};
     if (mix_in_langevin(c, true))
         mg = MixGather{c->lig_of, c->cmap, c->dB, c->dlig, c->NB, c->maxc, c->L, displaced_parts(c)};
+    if (move) {
+        k_move<<<dim3(c->NB, c->R), 64, 0, c->stream>>>(
+            c->N, c->Np, c->NB, c->invm, c->F, c->Fb, c->x64, c->v64, c->rec, c->state, c->orig_s,
+            mg, c->flags, c->qs, c->g, c->arec, c->bb_lo, c->bb_hi, c->cbox, c->par64,
+            energy ? c->rec64 : nullptr, lists_kept(c) ? c->xb : nullptr, c->dmax, c->bfirst);
+        return;
+    }
     k_langevin<<<g2(c->N, 256, c->R), 256, 0, c->stream>>>(c->N, c->Np, c->invm, c->F, c->Fb,
                                                            c->x64, c->v64, c->rec, c->state,
                                                            c->slot_of, c->cflag, c->dxs, mg,
@@ -683,8 +699,10 @@ int build_graph(sdm_context* c, int kind, bool energy) {
     hipGraph_t& graph = c->graph[kind][energy];
     hipGraphExec_t& gexec = c->gexec[kind][energy];
     HIPCHK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-    for (int k = 0; k < (kind == GRAPH_RUN ? GRAPH_STEPS : 1); k++)
-        enqueue_step(c, kind == GRAPH_SORT, energy);
+    const int n = kind == GRAPH_RUN ? GRAPH_STEPS : 1;
+    const bool move = can_move(c);
+    for (int k = 0; k < n; k++)
+        enqueue_step(c, kind == GRAPH_SORT, energy, move && k > 0, move && k < n - 1);
     hipError_t e = hipStreamEndCapture(c->stream, &graph);
     if (e != hipSuccess) return fail(SDM_ERR_HIP, std::string("hipStreamEndCapture: ") + hipGetErrorString(e));
     HIPCHK(hipGraphInstantiate(&gexec, graph, nullptr, nullptr, 0));
