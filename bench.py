@@ -88,7 +88,7 @@ def read_profile_value(name, key):
 
 def read_traffic():
     """HBM bytes per pair-kernel launch from the committed rocprofv3 --pmc summary."""
-    return read_profile_value("k_pair_n3_config3_pmc.md", "traffic_bytes_per_launch")
+    return read_profile_value("k_forces_pairs_config3_pmc.md", "traffic_bytes_per_launch")
 
 
 def note(msg):
@@ -295,7 +295,7 @@ def main():
     traffic = read_traffic()
     # VALU evidence from the committed counter summary (SQ_INSTS_VALU per launch, and the
     # busy fraction derived from SQ_ACTIVE_INST_VALU and GRBM_GUI_ACTIVE)
-    vname = "k_pair_n3_config3_valu.md"
+    vname = "k_forces_pairs_config3_valu.md"
     valu_busy = read_profile_value(vname, "valu_busy")
     vinst = read_profile_value(vname, "valu_insts_per_launch")
     valu_per_pair = 64.0 * vinst / pairs if vinst else None
@@ -400,7 +400,7 @@ def main():
         "batched_over_plain": agg / single,
         "all_finite_no_flags": ok,
         "roofline": {
-            "bound": "valu", "kernel": "k_pair_n3 (forces only)", "achieved": achieved,
+            "bound": "valu", "kernel": "k_forces pairs (forces only)", "achieved": achieved,
             "peak": FP32_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": achieved / FP32_PEAK_TFLOPS,
             "traffic": traffic, "pair_kernel_ms": pair_ms,
             "pairs_per_launch": pairs, "flop_per_pair": FLOP_PER_PAIR_FORCES,

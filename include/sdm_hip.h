@@ -143,12 +143,11 @@ typedef struct {
     int32_t pair_waves_per_group; /* 1, 2 or 4 wave64s per workgroup in the pair kernel */
     int32_t cell_cells_per_dim;   /* sort-grid resolution; 0 = automatic */
     int32_t use_graph;            /* 1: replay steps from captured hipGraphs; 0: launch each
-                                     kernel directly.  Either way the bonded terms and the
-                                     displaced-state chain run beside the pair kernel on
-                                     two side streams. */
+                                     kernel directly.  Runs of steps in the
+                                     kept slot order are captured eight at a time. */
     int32_t pair_newton3;         /* 0 or 1: accepted for callers that choose between pair
                                      kernels.  One kernel (each pair once) serves both;
-                                     with 0 an i-block has one wave */
+                                     with 0 an i-block has one part */
     int32_t pair_group;           /* 0, 8 or 16: as pair_newton3; with 8 or 16 an i-block has
                                      one wave and list_skin is ignored */
     int32_t sort_interval;        /* steps between full spatial sorts (1: every step); the

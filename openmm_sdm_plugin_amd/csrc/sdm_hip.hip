@@ -1,8 +1,8 @@
 // sdm_hip.hip -- host runtime and C ABI (include/sdm_hip.h) of the SDM HIP path.
 //
 // A context owns every device buffer of R replicas and one HIP stream (default
-// priority).  sdm_step replays a captured hipGraph of one step (all replicas in every
-// launch); no memset nodes are captured (counters are cleared by kernels).
+// priority).  sdm_step replays captured hipGraphs of one sorted step or of eight steps in the kept
+// order (all replicas in every launch); no memset nodes are captured (counters are cleared by kernels).
 #include "sdm_hip.h"
 
 #include <algorithm>
@@ -113,7 +113,7 @@ struct sdm_context {
     int* bfirst = nullptr;   // [R][NB] atom that a kept block's images are taken about
     int *ccount = nullptr, *cstart = nullptr, *cfill = nullptr;
     float4 *bb_lo = nullptr, *bb_hi = nullptr;
-    int* exs = nullptr;      // [R][NB][max_ex][64] exclusion partners in slot order (k_bbox)
+    int* exs = nullptr;      // [R][NB][max_ex][64] exclusion partners in slot order (k_refresh)
     unsigned long long* exblocks = nullptr;  // [R][NB] set of the j-blocks that hold any
     float4* cbox = nullptr;  // [R][NB][16] centres and half extents of the 8-slot clusters
     int* tiles = nullptr;
@@ -124,7 +124,7 @@ struct sdm_context {
     float4* xb = nullptr;   // [R][Np] slot coordinates when the tile lists were built
     float* dmax = nullptr;  // [R][DISP_STRIDE] (first float used) largest squared
                             // displacement of the replica's atoms since then (k_refresh),
-                            // or stale after a sort (k_bbox)
+                            // or stale after a sort (k_refresh)
     long long* F = nullptr;
     double *e_bond = nullptr, *u_part = nullptr;
     double* e64 = nullptr;  // FP64 pair-energy slots, one per wave of energy64_wave
@@ -479,7 +479,7 @@ int pair_parts(const sdm_context* c) {
 }
 
 // whether the tile lists hold the tiles' shifts (pack_tile)
-int packed_tiles(const sdm_context* c) { return !lists_kept(c) && c->NB <= TILE_BLOCK; }
+int packed_tiles(const sdm_context* c) { return !lists_kept(c); }
 
 // tile lists of the pairs and pair energies, candidate blocks of the displaced atoms.  With a skin, k_tiles keeps a replica's lists
 // while its atoms have moved less than half the skin since they were built.
@@ -489,8 +489,8 @@ void enqueue_tiles(sdm_context* c) {
                      c->cdispl, c->x64, c->cand, c->ncand, c->cmap};
     // One workgroup per (replica, i-block).  Its time is the serial path through it, so
     // when the workgroups do not fill the GPU (fewer than 8 per CU) each gets 8 waves for
-    // the candidate masks, otherwise 4 (measured: one replica of 22,750 atoms +6%, 22
-    // replicas -1% with 8).
+    // the candidate masks, otherwise 2 (4 waves at 73 registers against 2 at 64, measured
+    // together: 22 replicas of 22,750 atoms 55 and 44 us, 8 of 99,920 atoms 142 and 109 us).
 #define SDM_TILES(NW)                                                                         \
     k_tiles<NW><<<dim3(c->NB + lc.groups, c->R), 64 * NW, 0, c->stream>>>(                    \
         c->N, c->Np, c->NB, c->maxj, c->arec, c->bb_lo, c->bb_hi, c->cbox, c->tiles,          \

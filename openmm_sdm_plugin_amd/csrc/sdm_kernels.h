@@ -759,14 +759,15 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_num_vgpr(64))) void 
 // the j atoms' offset, took 5% less time but rounded otherwise than the box's coordinates.
 // Fixed-point atomics commute, so results are bit-reproducible.
 //
-// What bounds it: VALU issue (89% of the cycles of 22 x 22,750 atoms, 4 waves per SIMD at
+// What bounds it: VALU issue (93% of the cycles of 22 x 22,750 atoms, 4 waves per SIMD at
 // 123 registers).  A step takes 7 instructions to the distance test and 21 after it.  One
 // lane per i atom against one j atom at a time, the form before, took 37 instructions per 64
 // pairs with 22% of them within the cutoff; pairs of clusters have 30% (40% after the
 // distance test's early end) and no sum over the wave for each j atom.  Measured alone, 22
 // x 22,750 atoms: 532 -> 405 us (297M -> 201M VALU instructions); 8 x 99,920 atoms:
 // 1,054 -> 850 us; one replica of 22,750 atoms: 55 -> 44 us (before the tiles were shared out
-// in parts, share_tiles).  Where the i atoms' charges and
+// in parts, share_tiles; 22 x 22,750 atoms now 347 us, 191M
+// instructions).  Where the i atoms' charges and
 // LJ parameters came from LDS instead (122 registers), or the j forces of four clusters were
 // summed together (as many instructions in all, 30% more code), it was 4% and 14% slower.
 // ---------------------------------------------------------------------------
