@@ -179,7 +179,6 @@ struct sdm_context {
     sdm_tuning tune{1, 0, 1, 1, 0, 20, 0, 4, 1, 0.f};
     // steps evaluated in the current slot order (0: stale, the next evaluation sorts)
     int since_sort = 0;
-    // captured steps: [with a full sort][with the pair energies]
     // captured steps [kind][with energies]: with a sort, in the kept order, and GRAPH_STEPS
     // steps in the kept order
     hipGraph_t graph[3][2] = {};
@@ -187,7 +186,7 @@ struct sdm_context {
     bool components_valid = false;
     std::vector<void*> allocs;
     // pinned host memory (IO_SLOTS slots for data on its way to the device, in turn, and one
-    // for data on its way back), of io_cap bytes each; 0: none (very large systems)
+    // for data on its way back), of io_cap bytes each; 0: none (very large systems, or none to be had)
     char* io = nullptr;
     size_t io_cap = 0;
     int io_next = 0;
@@ -926,10 +925,13 @@ int sdm_create(const sdm_system_desc* sys, int32_t n_replicas, sdm_context** out
     const size_t io_cap = std::max((size_t)3 * ((N + 63) / 64 * 64) * sizeof(double),
                                    (size_t)n_replicas * (sizeof(DevRecord) + sizeof(int)));
     if (io_cap <= IO_MAX) {
-        if (hipHostMalloc((void**)&c->io, (IO_SLOTS + 1) * io_cap, hipHostMallocDefault) != hipSuccess)
-            return bail(fail(SDM_ERR_HIP, "hipHostMalloc failed"));
-        c->io_cap = io_cap;
-        std::memset(c->io, 0, (IO_SLOTS + 1) * io_cap);  // maps its pages (1 us each)
+        if (hipHostMalloc((void**)&c->io, (IO_SLOTS + 1) * io_cap, hipHostMallocDefault) == hipSuccess) {
+            c->io_cap = io_cap;
+            std::memset(c->io, 0, (IO_SLOTS + 1) * io_cap);  // maps its pages (1 us each)
+        } else {  // no pinned memory to be had: copies of pageable memory, as above IO_MAX
+            c->io = nullptr;
+            (void)hipGetLastError();
+        }
     }
     c->N = N;
     c->max_ex = max_ex;
