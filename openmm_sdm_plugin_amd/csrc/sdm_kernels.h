@@ -215,6 +215,10 @@ __global__ __launch_bounds__(64) void k_blockorder(int N, int Np, const double* 
         const double w = X[(size_t)d * Np + (v ? idx : O[b * 64])];
         const double dw = w - __shfl(w, 0, 64);
         p[d] = (float)(dw - L[d] * rint(dw * iL[d]));
+        // The lanes of a comparison decide apart, so keys have to be in a total order, and
+        // below the key of the empty slots: NaN, infinities and what is beyond FP32 (a replica
+        // that has blown up) count as one far coordinate, ordered by the atoms' indices.
+        if (!(fabsf(p[d]) <= 1.0e30f)) p[d] = 1.0e30f;
     }
 #pragma unroll
     for (int n = 64; n >= 16; n >>= 1) {
