@@ -415,11 +415,13 @@ int sdm_count_pairs(sdm_context* ctx, int64_t* p0, int64_t* pdelta /* [n_replica
 int sdm_time_pair_kernel(sdm_context* ctx, int32_t nsteps, double* avg_ms);
 
 /* Launch-configuration search (project-written autotuner): times each candidate (waves
-   per workgroup and per i-block of the pair kernel, sort grid) on the context's own replicas
-   for `steps` steps, then times the three fastest, each with and without graph replay
-   and with the placements of the side work that differ (side_fork), for 3 x `steps`
+   per workgroup and parts per i-block of the pair kernel, sort grid) on the context's own
+   replicas for `steps` steps, then times the three fastest, each with and without graph
+   replay and with the placements of the side work that differ (side_fork), for 3 x `steps`
    steps in two rounds, and keeps the one with the smallest total; it then times that one
-   with list_skin 0, 0.01, 0.02, 0.03 and 0.04 nm the same way.  The state the context had before the call is restored. */
+   with list_skin 0, 0.01, 0.02, 0.03 and 0.04 nm the same way.  Settings that are the same
+   step (pair_split, side_fork) are timed once, under the smallest value.  The state the
+   context had before the call is restored. */
 int sdm_autotune(sdm_context* ctx, int32_t steps, sdm_tuning* chosen);
 int sdm_get_tuning(sdm_context* ctx, sdm_tuning* t);
 int sdm_set_tuning(sdm_context* ctx, const sdm_tuning* t);

@@ -472,10 +472,11 @@ int block_parts(const sdm_context* c) {
 // Parts of the pair kernel: tuning.pair_split, or more where block_parts has more (one where
 // tuning asks for one, or for the full tile lists or the grouped form, for which pair_split
 // has no meaning).
-int pair_parts(const sdm_context* c) {
-    const int split = c->tune.pair_group == 0 && c->tune.pair_newton3 ? c->tune.pair_split : 1;
+int pair_parts(const sdm_context* c, const sdm_tuning& t) {
+    const int split = t.pair_group == 0 && t.pair_newton3 ? t.pair_split : 1;
     return split == 1 ? 1 : std::max(split, block_parts(c));
 }
+int pair_parts(const sdm_context* c) { return pair_parts(c, c->tune); }
 
 // whether the tile lists hold the tiles' shifts (pack_tile)
 int packed_tiles(const sdm_context* c) { return !lists_kept(c); }
@@ -508,9 +509,10 @@ void enqueue_sort(sdm_context* c, bool full) {
 
 // Whether the pairs alone run for several generations of waves (4,096 are resident): 20 x
 // 2,976 atoms have 15,000 parts, 22 x 22,750 and 8 x 99,920 atoms 78,000 and 50,000.
-bool many_waves(const sdm_context* c) {
-    return (long long)c->R * c->NB * pair_parts(c) >= 6 * 4096;
+bool many_waves(const sdm_context* c, const sdm_tuning& t) {
+    return (long long)c->R * c->NB * pair_parts(c, t) >= 6 * 4096;
 }
+bool many_waves(const sdm_context* c) { return many_waves(c, c->tune); }
 
 // parts of the displaced-state forces on a candidate block (env_force)
 int displaced_parts(const sdm_context* c) { return many_waves(c) ? 1 : DISP_WAVES; }
@@ -2019,11 +2021,26 @@ int sdm_autotune(sdm_context* c, int32_t steps, sdm_tuning* chosen) {
         CHK(upload(c, c->flags, fl.data(), c->R));
         return SDM_OK;
     };
-    // waves per i-block of the pair kernel
-    const int splits[] = {1, 2, 4, 8, 16, 32};
+    // parts of an i-block's tiles, one value of pair_split for each number that comes of them,
+    // and grids: settings that are the same step are tried once, or the three fastest would be
+    // one setting three times
+    std::vector<int> splits, parts, grids;
+    for (int split : {1, 2, 4, 8, 16, 32}) {
+        sdm_tuning t = c->tune;
+        t.pair_group = 0;
+        t.pair_newton3 = 1;
+        t.pair_split = split;
+        if (std::find(parts.begin(), parts.end(), pair_parts(c, t)) != parts.end()) continue;
+        parts.push_back(pair_parts(c, t));
+        splits.push_back(split);
+    }
+    for (double side : cell_sides) {
+        const int n = std::max(1, (int)std::floor(L / side));
+        if (std::find(grids.begin(), grids.end(), n) == grids.end()) grids.push_back(n);
+    }
     std::vector<std::pair<double, sdm_tuning>> timed;
     int rc = SDM_OK;
-    for (double side : cell_sides)
+    for (int cells : grids)
         for (int w : waves)
             for (int split : splits) {
                 if (rc != SDM_OK) break;
@@ -2032,7 +2049,7 @@ int sdm_autotune(sdm_context* c, int32_t steps, sdm_tuning* chosen) {
                 t.pair_group = 0;
                 t.pair_newton3 = 1;
                 t.pair_split = split;
-                t.cell_cells_per_dim = std::max(1, (int)std::floor(L / side));
+                t.cell_cells_per_dim = cells;
                 double ms = 0.0;
                 rc = trial(t, steps, ms);
                 if (rc == SDM_OK) timed.push_back({ms, t});
@@ -2049,12 +2066,14 @@ int sdm_autotune(sdm_context* c, int32_t steps, sdm_tuning* chosen) {
     std::vector<sdm_tuning> finalists;
     const bool terms = c->ncen + c->nali + c->nterm > 0;
     for (size_t k = 0; k < timed.size() && k < 3; k++)
-        for (int variant = 0; variant < 10; variant++) {
+        for (int variant = 0; variant < 6; variant++) {
             sdm_tuning t = timed[k].second;
             t.use_graph = variant & 1;
             t.side_fork = variant >> 1;
-            // without restraints and force-field terms 0, 1, 3 and 4 are the same step
-            if (!terms && t.side_fork != 1 && t.side_fork != 2) continue;
+            // 1, 3 and 4 are the same step; without restraints and force-field terms 0 is, too,
+            // and 2 unless pair energies have a stream of their own
+            if (!terms && t.side_fork == 0) continue;
+            if (!terms && t.side_fork == 2 && !many_waves(c, t)) continue;
             finalists.push_back(t);
         }
     std::vector<double> total(finalists.size(), 0.0);
