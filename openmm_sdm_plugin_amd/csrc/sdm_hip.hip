@@ -2003,10 +2003,17 @@ int sdm_autotune(sdm_context* c, int32_t steps, sdm_tuning* chosen) {
     const int hist_every = c->hist_every;
     c->hist_every = 0;
     // one trial: n steps from the saved state after two unmeasured ones (the first
-    // sorts and, with use_graph, captures), then the saved state back
+    // sorts) and, with use_graph, the capture of every graph that they replay, which a
+    // program pays once and a trial of some dozen steps is shorter than; then the saved
+    // state back
     auto trial = [&](const sdm_tuning& t, int n, double& ms_out) -> int {
         CHK(sdm_set_tuning(c, &t));
         CHK(sdm_step(c, 2));
+        for (int kind = 0; kind < 3 && t.use_graph; kind++)
+            for (int energy = t.energy_every_step; energy < 2; energy++) {
+                if (kind == GRAPH_RUN && energy != t.energy_every_step) continue;  // not replayed
+                if (!c->gexec[kind][energy]) CHK(build_graph(c, kind, energy));
+            }
         HIPCHK(hipEventRecord(e0, c->stream));
         CHK(sdm_step(c, n));
         HIPCHK(hipEventRecord(e1, c->stream));

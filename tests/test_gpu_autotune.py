@@ -1,6 +1,9 @@
 """What the autotuner times: every configuration once, by what it runs as and not by its
-setting.  The times are not compared; the test looks at which of the settings that are one
-configuration is reported."""
+setting, and steps only, without the capture of the graphs that replay them.
+
+The times themselves are not compared with bounds: the first test looks at which of the
+settings that are one configuration is reported, the second at whether replay from graphs,
+a few percent faster than launches for this system, is ever found to be."""
 import pytest
 
 from openmm_sdm_plugin_amd import _native, systems
@@ -30,3 +33,12 @@ def test_one_setting_for_each_configuration(hip_device, waters, box, replicas):
         t = ctx.autotune(8)
         assert t["pair_split"] in (1, 2) and t["side_fork"] == 1
         assert ctx.get_tuning() == t
+
+
+def test_graphs_are_not_timed_with_their_capture(hip_device):
+    s = systems.make_config1(frame=0)
+    picks = []
+    for k in range(6):
+        picks.append(_context(s, 1).autotune(20)["use_graph"])
+        print(f"case autotune {k}: use_graph={picks[-1]}", flush=True)
+    assert any(picks)
