@@ -44,7 +44,7 @@ struct Geom {
     float oix, oiy, oiz;
     // LJ sigma combining: 0 Lorentz-Berthelot, 1 geometric (OPLS).  The per-atom FP32 and
     // FP64-record sigma entries hold s/2 for the first, s for the second (the FP64 sigma
-    // array always s); the FP32 block kernel takes it as a template parameter
+    // array always s); the pair kernel takes it as a template parameter
     int geo;
     // sort grid: cell c_d = floor((w_d - go_d) * gs_d), clamped to the grid, w the
     // (wrapped, if periodic) coordinate.  Periodic: go = 0, gs = cells / L; otherwise
@@ -114,7 +114,7 @@ __device__ __forceinline__ int wave_scan(int v) {
 
 // exclusive scan of the cell counts, one 1024-thread workgroup per replica; clears the
 // counters for the next step.  8 x 1024 cells at a time, coalesced and in flight together,
-// with two barriers: the launch is one workgroup's latency, 19.6 us for 8,000 cells with a
+// with one barrier a round: the launch is one workgroup's latency, 19.6 us for 8,000 cells with a
 // run of cells per thread and a barrier per doubling, 3.8 us so.
 __global__ __launch_bounds__(1024) void k_scan(int NC, int* __restrict__ ccount,
                                                int* __restrict__ cstart, int* __restrict__ cfill) {
@@ -750,8 +750,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_num_vgpr(64))) void 
 // clusters, 64 pairs on 64 lanes, taken for the bits of the tile's mask (uniform branches).
 // A step none of whose pairs is within the cutoff ends after the distance test.
 //   i forces: FP32 in the lane (24 registers), added up over the eight lanes that share an
-//     i atom and over to the int64 accumulator at the end of each part and after every
-//     PAIRS_PER_FLUSH pairs or more (pairs within the cutoff), rounded to nearest.
+//     i atom and over to the int64 accumulator, rounded to nearest, at the end of each part
+//     and by PAIRS_PER_FLUSH and TILES_PER_FLUSH.
 //   j forces: FP32 over the cluster's steps, added up over the eight lanes that share a j
 //     atom, kept in registers over the tile and added to the slot-ordered int64 accumulator
 //     once per tile with coalesced atomics.
@@ -770,7 +770,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_num_vgpr(64))) void 
 // distance test's early end) and no sum over the wave for each j atom.  Measured alone, 22
 // x 22,750 atoms: 532 -> 405 us (297M -> 201M VALU instructions); 8 x 99,920 atoms:
 // 1,054 -> 850 us; one replica of 22,750 atoms: 55 -> 44 us (before the tiles were shared out
-// in parts, share_tiles; 22 x 22,750 atoms now 347 us, 191M
+// in parts, share_tiles; 22 x 22,750 atoms now 351 us, 195M
 // instructions).  Where the i atoms' charges and
 // LJ parameters came from LDS instead (122 registers), or the j forces of four clusters were
 // summed together (as many instructions in all, 30% more code), it was 4% and 14% slower.
@@ -855,16 +855,17 @@ __device__ __forceinline__ void scatter_clusters24(const float (&v)[24], int lan
     }
 }
 
-// Pairs of a block (within the cutoff) after which the FP32 sums of its i forces go to the
-// 64-bit accumulator, at the next tile: an atom that has all of them (alone in its block) then
-// has 384 and one more tile's 63, in eight lanes at most 56 additions in a row, as few as a
-// tile's 64 terms in one lane; on average it is 9 terms an atom.  The error of the forces
-// against 64 bits, 32 frames of 22,750, 21,005 and 9,005 atoms, as a ratio to FP32 sums of one
-// tile added up in FP64: 0.989, 0.996, 0.993 (0.989, 0.996, 0.994 with one part per block);
-// with 4,096 pairs (20 frames) 0.991, 1.001, 0.996 (0.995, 1.008, 1.002), and 5.5e-8 where one
-// atom has all pairs, so 1.8e-8.  Pair kernel of 22 x 22,750 and 8 x 99,920 atoms: 401 and 817
-// us, with 512 pairs 397 and 809, with 4,096 386 and 778.
-constexpr int PAIRS_PER_FLUSH = 384;
+// Pairs of a block (within the cutoff), and tiles with any, after which the FP32 sums of its i
+// forces go to the 64-bit accumulator, at the next tile.  A lane adds at most 8 terms to an i
+// atom's sum in a tile, so 7 tiles leave 56 additions in a row and three over the lanes,
+// whatever the geometry: no more than a tile's 64 terms in one lane.  The pairs bound the mean (16 to 20
+// terms an atom).  The error of the forces against 64 bits, 32 frames of 22,750, 21,005 and 9,005
+// atoms, as a ratio to FP32 sums of one tile added up in FP64: 0.989, 0.997, 0.994 (0.990, 0.997,
+// 0.994 with one part per block); with 4,096 pairs and any number of tiles (20 frames) 0.991, 1.001,
+// 0.996 (0.995, 1.008, 1.002), and 5.5e-8 where one atom has all pairs, so 1.4e-8.  Pair kernel of
+// 22 x 22,750 and 8 x 99,920 atoms: 391 and 797 us, with 4,096 pairs 386 and 778, with 512 397 and 807,
+// with tiles alone 387 and 781 (but 1.000, 1.004, 1.009 with one part per block).
+constexpr int PAIRS_PER_FLUSH = 1024, TILES_PER_FLUSH = 7;
 
 // m without its r lowest bits
 __device__ __forceinline__ unsigned long long drop_bits(unsigned long long m, int r) {
@@ -1050,7 +1051,7 @@ __device__ __forceinline__ void pair_wave(
 #pragma unroll
         for (int k = 0; k < 24; k++) fi[k] = 0.f;
     };
-    int npair = 0, buf = 0;
+    int npair = 0, used = 0, buf = 0;  // pairs, and tiles with any, in the sums
     // lane that holds the sum of j atom `lane` of a tile (cluster lane >> 3 in lanes with
     // il = that cluster), as a byte address for ds_bpermute
     const int transpose = 4 * ((lane >> 3) + 8 * (lane & 7));
@@ -1100,10 +1101,11 @@ __device__ __forceinline__ void pair_wave(
             }
             stage(__builtin_amdgcn_readlane(tj, next & 63) & TILE_BLOCK, buf ^ 1);
         }
-        if (!COUNT && npair >= PAIRS_PER_FLUSH) {
+        if (!COUNT && (npair >= PAIRS_PER_FLUSH || used == TILES_PER_FLUSH)) {
             flush_i();
-            npair = 0;
+            npair = used = 0;
         }
+        const int in_tile = npair;
         // pairs of the tile that need more than the shift (uniform): their own minimum
         // image, or a look at the exclusions and empty slots
         const bool mi = (jt & TILE_MI) != 0;
@@ -1117,8 +1119,8 @@ __device__ __forceinline__ void pair_wave(
         float fjx = 0.f, fjy = 0.f, fjz = 0.f;  // sum of cluster il, atom jl
         unsigned long long rest = m, done = 0ull;
         do {
-            // the last cluster first: the order of the FP32 sums.  Errors as at PAIRS_PER_FLUSH,
-            // 32 frames: 0.989, 0.996, 0.993, with the first one first 0.991, 0.997, 0.995
+            // the last cluster first: the order of the FP32 sums.  Errors as at PAIRS_PER_FLUSH (with
+            // 384 pairs) 0.989, 0.996, 0.993, with the first one first 0.991, 0.997, 0.995
             const int jc8 = (63 - __builtin_clzll(rest)) & 56;  // 8 jc
             const unsigned ics = (unsigned)(m >> jc8) & 0xffu;
             rest &= ~(0xffull << jc8);
@@ -1219,7 +1221,9 @@ __device__ __forceinline__ void pair_wave(
         // on how many parts a wave takes
         if (!COUNT && part_ends) {
             flush_i();
-            npair = 0;
+            npair = used = 0;
+        } else {
+            used += npair > in_tile ? 1 : 0;
         }
         if (next < 0) break;
         buf ^= next > t ? 1 : 0;
@@ -2341,7 +2345,7 @@ __device__ double softcore_dev(int method, double u, double umax, double a, doub
     return (umax - ub) * (zetap - 1.0) / (zetap + 1.0) + ub;
 }
 
-// ne: pair-energy slots per replica (i-blocks times the pair kernel's waves per block)
+// ne: pair-energy slots per replica (one per part of an i-block's tiles)
 // SUMS: first the sums on the displaced atoms (delta_sums), with one ligand block: a launch of
 // its own for them took 7.2 us of 22,750 atoms and 10 us of 22 replicas before this one's 9.9
 // and 7.5 us; together, and with the state and the Langevin parameters off the last thread's

@@ -10,8 +10,8 @@ place.  A chain of n additions of like terms is off by rms 0.29 2^-23.5 sqrt(n /
 errors of half a last place of sums that grow evenly): 1.2e-7 for chains of 72, of
 which the eight lanes of an atom make eight in each of at least 4,096 / 576 sums: 1.6e-8 of the
 half of the force that comes from the atom's own tiles, 8e-9 of the force (and less for
-shorter chains).  Added up: below
-3e-8 rms.  Chains of 512 (sums over 4,096 pairs) are off by 6e-8."""
+shorter chains).  Added up: below 3e-8 rms.  Chains of 512 (sums over 4,096 pairs) are off by
+6e-8."""
 import numpy as np
 import pytest
 
