@@ -80,9 +80,9 @@ typedef struct {
                                    sigma_ij = sqrt(s_i s_j): the CustomNonbondedForce the
                                    reference's DMS reader builds for OPLS,
                                    desmonddmsfile75.py:780-793); epsilon_ij =
-                                   sqrt(e_i e_j) either way.  Geometric runs on the block
-                                   Newton-3 pair kernel (sdm_tuning.pair_group 0,
-                                   pair_newton3 1). */
+                                   sqrt(e_i e_j) either way.  With geometric,
+                                   sdm_set_tuning takes pair_group 0 and pair_newton3 1
+                                   only. */
 } sdm_system_desc;
 #define SDM_LJ_ARITHMETIC 0
 #define SDM_LJ_GEOMETRIC 1

@@ -409,9 +409,9 @@ int setup_cells(sdm_context* c, int per_dim) {
 
 dim3 g2(int n, int per, int R) { return dim3((unsigned)((n + per - 1) / per), (unsigned)R); }
 
-// Tile lists are kept over steps (tuning.list_skin > 0) except where tuning asks for the
-// grouped form.  Every slot refresh is followed by a k_tiles launch, which rebuilds after a
-// sort, so the build coordinates (xb) always belong to the lists in use.
+// Tile lists are kept over steps (tuning.list_skin > 0) except with a pair_group, which always
+// had lists of its own evaluation.  Every slot refresh is followed by a k_tiles launch, which
+// rebuilds after a sort, so the build coordinates (xb) always belong to the lists in use.
 bool lists_kept(const sdm_context* c) { return c->tune.list_skin > 0.f && c->tune.pair_group == 0; }
 
 // slot order (a full spatial sort, or the last sort's order refreshed) and block boxes
@@ -441,8 +441,11 @@ void enqueue_order(sdm_context* c, bool full, bool energy = false) {
 #undef SDM_REFRESH
 }
 
-// whether a launch of one workgroup per (replica, 64-atom block) leaves the GPU short of
-// work (fewer than 8 workgroups per CU)
+// Whether a launch of one workgroup per (replica, 64-atom block) leaves the GPU short of
+// work (fewer than 8 workgroups per CU): k_tiles then has 8 waves per block, and k_move is used.
+// Steps (us) with and without, either side of the line: 47 blocks x 20, 43, 64 replicas 105 / 101,
+// 155 / 141, 212 / 189; 128 x 8, 16: 100 / 98, 149 / 137; 356 x 1, 4, 6, 8: 61 / 68, 123 / 124, 158 / 155,
+// 196 / 187; 1,562 x 1, 2: 226 / 229, 275 / 268.
 bool few_blocks(const sdm_context* c) { return (long)c->NB * c->R < 2048; }
 
 // build radius and reuse threshold of the tile lists for a skin of tuning.list_skin nm
@@ -462,16 +465,20 @@ TileRadius tile_radius(const sdm_context* c) {
 // of few blocks have short tile lists but leave most of the GPU idle with few waves; each
 // part costs about 3 us of a wave (loads, and the sums of the i forces) in large launches.
 // The number of replicas does not enter, so that a replica in a batch gives the bits of the
-// same replica alone.  Measured (us), 8 / 10 / 12 / 16 parts of 356 blocks: 20 steps of one
-// replica 1,953 / 1,874 / 1,900 / -, pair kernel of 22 replicas 379 / 392 / 402 / 426.  16 / 32
-// parts: 47 blocks 17.9 / 15.1 but 20 replicas of them 61 / 88, 174 blocks 22 / 31.
+// same replica alone; the lines are between what one replica and what a batch would want.
+// Steps (us, cutoff 0.9 nm) with this rule and with the best of 4 to 64 parts, one replica and
+// a batch: 16 blocks 32 / 32 and (16 replicas) 65 / 51 (16 parts); 33 39 / 35 (32) and (20) 84 / 82;
+// 64 44 / 40 (32) and (20) 133 / 127 (8); 128 43 / 42 and (20) 162 / 155 (10); 256 66 / 56 (32) and (20)
+// 309 / 308; 356 61 / 60 (16) and (22) 400 / 394 (6); 511 71 / 67 (16) and (12) 336 / 329 (6); 512 105 / 66
+// (12) and (12) 324 / 324; 800 107 / 84 (8) and (8) 322 / 321; 1,562 226 / 154 (16) and (6) 512 / 512.  A
+// single large replica gets more by tuning.pair_split, which the autotuner tries.
 int block_parts(const sdm_context* c) {
     return c->NB <= 16 ? 64 : c->NB <= 32 ? 32 : c->NB < 256 ? 16 : c->NB < TILE_SLOPE_BLOCKS ? 10 : 4;
 }
 
 // Parts of the pair kernel: tuning.pair_split, or more where block_parts has more (one where
-// tuning asks for one, or for the full tile lists or the grouped form, for which pair_split
-// has no meaning).
+// tuning asks for one, or with pair_newton3 0 or a pair_group, for which pair_split has no
+// meaning).
 int pair_parts(const sdm_context* c, const sdm_tuning& t) {
     const int split = t.pair_group == 0 && t.pair_newton3 ? t.pair_split : 1;
     return split == 1 ? 1 : std::max(split, block_parts(c));
@@ -508,7 +515,11 @@ void enqueue_sort(sdm_context* c, bool full) {
 }
 
 // Whether the pairs alone run for several generations of waves (4,096 are resident): 20 x
-// 2,976 atoms have 15,000 parts, 22 x 22,750 and 8 x 99,920 atoms 78,000 and 50,000.
+// 2,976 atoms have 15,000 parts, 22 x 22,750 and 8 x 99,920 atoms 78,000 and 50,000.  Steps (us)
+// with and without the line drawn so, by parts: 16 blocks 16,384 60 / 65, 24,576 72 / 82; 47 blocks
+// 12,032 85 / 90, 18,048 114 / 117, 24,064 131 / 144, 36,096 154 / 184; 128 blocks 16,384 96 / 101, 24,576
+// 125 / 131; 356 blocks 21,360 170 / 155, 24,920 180 / 169, 32,040 203 / 205, 42,720 248 / 258; 511 blocks
+// 20,440 158 / 156, 30,660 200 / 204.  With energies on every step it pays from about 16,000 on.
 bool many_waves(const sdm_context* c, const sdm_tuning& t) {
     return (long long)c->R * c->NB * pair_parts(c, t) >= 6 * 4096;
 }
@@ -525,6 +536,11 @@ void launch_forces(sdm_context* c, int parts) {
     // workgroups of W waves for n waves, a multiple of 8 (k_forces)
     auto groups = [](int part, int n) { return part ? ((n + W - 1) / W + 7) / 8 * 8 : 0; };
     const int pparts = pair_parts(c), ewaves = block_parts(c);  // energies: one wave per part
+    // Where the waves are many a wave takes several parts (part_of), 7 / 3 of them on average (from
+    // TILE_SLOPE_BLOCKS on the parts themselves fall in size).  Steps (us) with 25, 33, 43, 60 and
+    // 100 waves for 100 parts: 64 replicas of 16 blocks 143, 144, 141, 145, 145; 64 of 47 195, 188, 189,
+    // 192, 198; 24 of 128 190, 184, 187, 189, 194; 20 of 256 324, 325, 309, 312, 319; 22 of 356 412, 411,
+    // 402, 408, 418; 10 of 511 300, 299, 290, 296, 302
     const int waves = many_waves(c) && c->NB < TILE_SLOPE_BLOCKS ? std::max(1, (3 * pparts + 3) / 7) : pparts;
     // A wave per group of displaced atoms where the launch is short, one for all groups of a
     // candidate block where it is long: fewer waves then wait for their atoms while others
@@ -1967,9 +1983,9 @@ int sdm_set_tuning(sdm_context* c, const sdm_tuning* t) {
         return fail(SDM_ERR_INVALID, "side_fork must be 0, 1, 2, 3 or 4");
     if (!(t->list_skin >= 0.f && t->list_skin <= (float)SDM_MAX_LIST_SKIN))
         return fail(SDM_ERR_INVALID, "list_skin must be in [0, 0.1] nm");
+    // (one kernel serves all of these now; callers that rely on the refusal keep it)
     if (c->g.geo && (t->pair_group != 0 || t->pair_newton3 != 1))
-        return fail(SDM_ERR_INVALID, "the geometric LJ rule runs on the block Newton-3 pair "
-                                     "kernel (pair_group 0, pair_newton3 1)");
+        return fail(SDM_ERR_INVALID, "the geometric LJ rule needs pair_group 0 and pair_newton3 1");
     HIPCHK(hipStreamSynchronize(c->stream));
     if (t->cell_cells_per_dim != c->tune.cell_cells_per_dim) CHK(setup_cells(c, t->cell_cells_per_dim));
     c->tune = *t;
@@ -2095,8 +2111,8 @@ int sdm_autotune(sdm_context* c, int32_t steps, sdm_tuning* chosen) {
             best_ms = total[k];
             best = finalists[k];
         }
-    // then the Verlet skin of the tile lists for the chosen configuration (block kernels
-    // only): a wider skin keeps the lists longer but the pair kernel evaluates more pairs
+    // then the Verlet skin of the tile lists for the chosen configuration: a wider skin
+    // keeps the lists longer but the pair kernel evaluates more pairs
     // outside the cutoff.  Two rounds again, ranked by the sum.
     if (rc == SDM_OK) {
         const float skins[] = {0.f, 0.01f, 0.02f, 0.03f, 0.04f};
