@@ -164,7 +164,7 @@ def cpu_baseline(n_steps, warmup=10, runs=3, omp_steps=2):
 
 # the launch configurations sdm_autotune picks on MI355X for the 22-replica 22,750-atom
 # ladder and the 8-replica 99,920-atom ladder (used by the profiling modes, which do not
-# autotune)
+# autotune; pair_split 2, 4 and 8 are one configuration at the first size, 2 and 4 at the second)
 LADDER_TUNING = dict(pair_group=0, pair_newton3=1, pair_split=4, pair_waves_per_group=1,
                      cell_cells_per_dim=20, sort_interval=20, use_graph=0, energy_every_step=0,
                      side_fork=1)
